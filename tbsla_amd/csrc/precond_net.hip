@@ -229,6 +229,37 @@ __global__ __launch_bounds__(kBlock) void k_layer0(long long n, const int *__res
 
 typedef float floatq __attribute__((ext_vector_type(4)));
 
+// acc + sum over a node's deg edges (from beg) of ev * row eci of `rows`
+// (`stride` floats a row, channels 4q .. 4q + 3), in edge order.  The node's
+// 16 lanes read 16 edges at once and pass them round by shuffles, so that the
+// gathers of four edges are in flight.
+__device__ inline floatq neighbour_sum(floatq acc, int beg, int deg, const int *__restrict__ eci,
+                                       const float *__restrict__ ev,
+                                       const float *__restrict__ rows, int stride, int q) {
+  for (int b0 = 0; b0 < deg; b0 += 16) {
+    const bool in = b0 + q < deg;
+    const int c = in ? eci[beg + b0 + q] : 0;
+    const float e = in ? ev[beg + b0 + q] : 0.f;
+    const int m = min(16, deg - b0);
+    for (int k0 = 0; k0 < m; k0 += 4) {
+      floatq u[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const long long cj = __shfl(c, k0 + k, 16);
+        u[k] = *reinterpret_cast<const floatq *>(rows + cj * stride + 4 * q);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float ek = __shfl(e, k0 + k, 16);
+        if (k0 + k >= m) continue;
+#pragma unroll
+        for (int x = 0; x < 4; x++) acc[x] = fmaf(ek, u[k][x], acc[x]);
+      }
+    }
+  }
+  return acc;
+}
+
 // h' = relu(U[:, :64] + E U[:, 64:] + b); the last layer also gives the
 // diagonal head g^_ii = exp(wd . h + bd).  Four nodes per wavefront, 16
 // lanes per node, four channels per lane (16-byte loads).
@@ -246,15 +277,10 @@ __global__ __launch_bounds__(kBlock) void k_aggregate(long long n, const int *__
   const floatq wd = {th[owd + 4 * q], th[owd + 4 * q + 1], th[owd + 4 * q + 2], th[owd + 4 * q + 3]};
   const float bd = th[obd];
   for (long long i = (long long)blockIdx.x * (kBlock / 16) + threadIdx.x / 16; i < n; i += groups) {
-    floatq pre = *reinterpret_cast<const floatq *>(U + i * H2 + 4 * q) + bias;
-    for (int j = erp[i]; j < erp[i + 1]; j++) {
-      const float e = ev[j];
-      const floatq u = *reinterpret_cast<const floatq *>(U + (long long)eci[j] * H2 + H + 4 * q);
-      pre.x = fmaf(e, u.x, pre.x);
-      pre.y = fmaf(e, u.y, pre.y);
-      pre.z = fmaf(e, u.z, pre.z);
-      pre.w = fmaf(e, u.w, pre.w);
-    }
+    const int beg = erp[i], deg = erp[i + 1] - beg;
+    const floatq pre =
+        neighbour_sum(*reinterpret_cast<const floatq *>(U + i * H2 + 4 * q) + bias, beg, deg, eci,
+                      ev, U + H, H2, q);
     floatq hv;
     hv.x = fmaxf(pre.x, 0.f);
     hv.y = fmaxf(pre.y, 0.f);
@@ -518,123 +544,149 @@ __global__ __launch_bounds__(kBlock) void k_dghat(long long n, const int *__rest
 // backward
 // ---------------------------------------------------------------------------
 
-// Head, row pass (wave per row i): diagonal head, and the lower edges (i, j)
-// for dP_i[:64]; parameter partials for wd, bd, wo, bo, ve, c per workgroup.
+// Head, one pass over the nodes: the diagonal head, the lower edges (i, j)
+// for dP_i[:64] and the upper ones (i' > i) for dP_i[64:]; parameter partials
+// for wd, bd, wo, bo, ve, c per workgroup (each edge counted at its lower end).
 // Partial layout per workgroup: [wd 64 | bd | wo 64 | bo | ve 64 | c 64].
+// 16 lanes per node, four channels per lane: a node's edges are read by its
+// lanes at once and handed round by shuffles, so the gathers of four edges are
+// in flight instead of one chain of three dependent loads per edge.  64^3
+// grid: a wave-per-row pass per triangle took 248 + 203 us, this 107.
 constexpr int kHeadPart = 4 * H + 2;
+constexpr int kNodes = kBlock / 16;  // nodes per workgroup of the 16-lane kernels
 
-__global__ __launch_bounds__(kBlock) void k_head_bwd_rows(
-    long long n, const int *__restrict__ erp, const int *__restrict__ eci,
-    const float *__restrict__ ev, const int *__restrict__ nlow, const int *__restrict__ grp,
-    const float *__restrict__ P, const float *__restrict__ h3, const float *__restrict__ th,
-    const float *__restrict__ ghat, const float *__restrict__ dg, float *__restrict__ dh3,
-    float *__restrict__ dP, bf16_t *__restrict__ dPb, float *__restrict__ part) {
-  __shared__ float lds[kBlock / kWave][kHeadPart];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const long long waves = (long long)gridDim.x * (kBlock / kWave);
-  const float ve = th[ove + lane], cc = th[oc + lane], wo = th[owo + lane], wd = th[owd + lane];
-  float a_wd = 0.f, a_bd = 0.f, a_wo = 0.f, a_bo = 0.f, a_ve = 0.f, a_c = 0.f;
-  for (long long i = (long long)blockIdx.x * (kBlock / kWave) + wave; i < n; i += waves) {
-    const int lo = nlow[i], g0 = grp[i];
-    const float dq = dg[g0 + lo] * ghat[g0 + lo];
-    a_wd = fmaf(dq, h3[i * H + lane], a_wd);
-    a_bd += dq;
-    dh3[i * H + lane] = dq * wd;
-    const float pi = P[i * H2 + lane];
-    float dpi = 0.f;
-    for (int k = 0; k < lo; k++) {
-      const int j = eci[erp[i] + k];
-      const float e = ev[erp[i] + k];
-      const float sv = pi + P[(long long)j * H2 + H + lane] + e * ve + cc;
-      const float d = dg[g0 + k];
-      a_wo = fmaf(d, fmaxf(sv, 0.f), a_wo);
-      a_bo += d;
-      const float ds = sv > 0.f ? d * wo : 0.f;
-      a_ve = fmaf(ds, e, a_ve);
-      a_c += ds;
-      dpi += ds;
-    }
-    dP[i * H2 + lane] = dpi;
-    dPb[i * H2 + lane] = to_bf16(dpi);
-  }
-  // workgroup partials (waves in order)
-  lds[wave][lane] = a_wd;
-  lds[wave][H + 1 + lane] = a_wo;
-  lds[wave][2 * H + 2 + lane] = a_ve;
-  lds[wave][3 * H + 2 + lane] = a_c;
-  // a_bd and a_bo hold the same per-node / per-edge sums in every lane
-  const float bd = __shfl(a_bd, 0, kWave), bo = __shfl(a_bo, 0, kWave);
-  if (lane == 0) {
-    lds[wave][H] = bd;
-    lds[wave][2 * H + 1] = bo;
+__device__ inline void store_bf16x4(bf16_t *p, floatq v) {
+  const uint32_t lo = (uint32_t)to_bf16(v.x) | ((uint32_t)to_bf16(v.y) << 16);
+  const uint32_t hi = (uint32_t)to_bf16(v.z) | ((uint32_t)to_bf16(v.w) << 16);
+  *reinterpret_cast<uint2 *>(p) = make_uint2(lo, hi);
+}
+
+// sums over the 16-lane groups of the workgroup, per channel quad: the four
+// groups of each wavefront, then the wavefronts in order; lds holds H floats
+// per wavefront, thread c < H receives channel c's total
+__device__ inline float quad_total(floatq v, float *lds) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    v[k] += __shfl_xor(v[k], 16, kWave);
+    v[k] += __shfl_xor(v[k], 32, kWave);
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < kHeadPart; e += kBlock) {
-    float t = 0.f;
-    for (int w = 0; w < kBlock / kWave; w++) t += lds[w][e];
-    part[(long long)blockIdx.x * kHeadPart + e] = t;
-  }
+  if (lane < 16) *reinterpret_cast<floatq *>(lds + wave * H + 4 * lane) = v;
+  __syncthreads();
+  float t = 0.f;
+  if (threadIdx.x < H)
+    for (int w = 0; w < kBlock / kWave; w++) t += lds[w * H + threadIdx.x];
+  return t;
 }
 
-// Head, column pass (wave per row j): edges (i, j), i > j, are the upper
-// entries of row j; they give dP_j[64:].
-__global__ __launch_bounds__(kBlock) void k_head_bwd_cols(
-    long long n, const int *__restrict__ trp, const int *__restrict__ tci,
-    const int *__restrict__ tmap, const int *__restrict__ erp, const int *__restrict__ eci,
-    const float *__restrict__ ev, const int *__restrict__ nlow, const float *__restrict__ P,
-    const float *__restrict__ th, const float *__restrict__ dg, float *__restrict__ dP,
-    bf16_t *__restrict__ dPb) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const long long waves = (long long)gridDim.x * (kBlock / kWave);
-  const float ve = th[ove + lane], cc = th[oc + lane], wo = th[owo + lane];
-  for (long long j = (long long)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; j < n;
-       j += waves) {
-    const float pj = P[j * H2 + H + lane];
-    float dpj = 0.f;
-    // G^T row j: the diagonal, then upper columns i (the same order as the
-    // upper part of E's row j, whose values are e_ji = e_ij)
-    const int t0 = trp[j];
-    const int eu = erp[j] + nlow[j];
-    for (int t = t0 + 1; t < trp[j + 1]; t++) {
-      const long long i = tci[t];
-      const float e = ev[eu + (t - t0 - 1)];
-      const float sv = P[i * H2 + lane] + pj + e * ve + cc;
-      const float d = dg[tmap[t]];
-      dpj += sv > 0.f ? d * wo : 0.f;
+__global__ __launch_bounds__(kBlock) void k_head_bwd(
+    long long n, const int *__restrict__ erp, const int *__restrict__ eci,
+    const float *__restrict__ ev, const int *__restrict__ nlow, const int *__restrict__ grp,
+    const int *__restrict__ trp, const int *__restrict__ tmap, const float *__restrict__ P,
+    const float *__restrict__ h3, const float *__restrict__ th, const float *__restrict__ ghat,
+    const float *__restrict__ dg, float *__restrict__ dh3, bf16_t *__restrict__ dPb,
+    float *__restrict__ part) {
+  __shared__ __align__(16) float lds[kBlock / kWave * H];
+  const int q = threadIdx.x & 15;
+  const long long groups = (long long)gridDim.x * kNodes;
+  const floatq ve = *reinterpret_cast<const floatq *>(th + ove + 4 * q);
+  const floatq cc = *reinterpret_cast<const floatq *>(th + oc + 4 * q);
+  const floatq wo = *reinterpret_cast<const floatq *>(th + owo + 4 * q);
+  const floatq wd = {th[owd + 4 * q], th[owd + 4 * q + 1], th[owd + 4 * q + 2], th[owd + 4 * q + 3]};
+  floatq a_wd = {0.f, 0.f, 0.f, 0.f}, a_wo = a_wd, a_ve = a_wd, a_c = a_wd;
+  float a_bd = 0.f, a_bo = 0.f;
+  for (long long i = (long long)blockIdx.x * kNodes + threadIdx.x / 16; i < n; i += groups) {
+    const int lo = nlow[i], g0 = grp[i], beg = erp[i], deg = erp[i + 1] - beg, t0 = trp[i];
+    const floatq pi = *reinterpret_cast<const floatq *>(P + i * H2 + 4 * q);
+    const floatq pj = *reinterpret_cast<const floatq *>(P + i * H2 + H + 4 * q);
+    const floatq hv = *reinterpret_cast<const floatq *>(h3 + i * H + 4 * q);
+    const float dq = dg[g0 + lo] * ghat[g0 + lo];
+    a_bd += dq;
+    *reinterpret_cast<floatq *>(dh3 + i * H + 4 * q) = dq * wd;
+    floatq dpi = {0.f, 0.f, 0.f, 0.f}, dpj = dpi;
+#pragma unroll
+    for (int k = 0; k < 4; k++) a_wd[k] = fmaf(dq, hv[k], a_wd[k]);
+    for (int b0 = 0; b0 < deg; b0 += 16) {
+      // edge b0 + q: neighbour, value, dL/dg^ of its entry of G
+      const int kq = b0 + q;
+      const bool in = kq < deg;
+      const int c = in ? eci[beg + kq] : 0;
+      const float e = in ? ev[beg + kq] : 0.f;
+      const float d = in ? dg[kq < lo ? g0 + kq : tmap[t0 + 1 + kq - lo]] : 0.f;
+      const int m = min(16, deg - b0);
+      for (int k0 = 0; k0 < m; k0 += 4) {
+        floatq u[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const long long cj = __shfl(c, k0 + k, 16);
+          u[k] = *reinterpret_cast<const floatq *>(P + cj * H2 + (b0 + k0 + k < lo ? H : 0) + 4 * q);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const float ek = __shfl(e, k0 + k, 16), dk = __shfl(d, k0 + k, 16);
+          if (k0 + k >= m) continue;
+          const bool lower = b0 + k0 + k < lo;
+          const floatq sv = (lower ? pi : pj) + u[k] + ek * ve + cc;
+          if (lower) a_bo += dk;
+#pragma unroll
+          for (int x = 0; x < 4; x++) {
+            const float ds = sv[x] > 0.f ? dk * wo[x] : 0.f;
+            if (lower) {
+              a_wo[x] = fmaf(dk, fmaxf(sv[x], 0.f), a_wo[x]);
+              a_ve[x] = fmaf(ds, ek, a_ve[x]);
+              a_c[x] += ds;
+              dpi[x] += ds;
+            } else {
+              dpj[x] += ds;
+            }
+          }
+        }
+      }
     }
-    dP[j * H2 + H + lane] = dpj;
-    dPb[j * H2 + H + lane] = to_bf16(dpj);
+    store_bf16x4(dPb + i * H2 + 4 * q, dpi);
+    store_bf16x4(dPb + i * H2 + H + 4 * q, dpj);
+  }
+  float *out = part + (long long)blockIdx.x * kHeadPart;
+  const float t_wd = quad_total(a_wd, lds), t_wo = quad_total(a_wo, lds);
+  const float t_ve = quad_total(a_ve, lds), t_c = quad_total(a_c, lds);
+  // every lane of a node's group holds the same a_bd and a_bo
+  const floatq two = {a_bd, a_bo, 0.f, 0.f};
+  const float t_b = quad_total(two, lds);
+  if (threadIdx.x < H) {
+    out[threadIdx.x] = t_wd;
+    out[H + 1 + threadIdx.x] = t_wo;
+    out[2 * H + 2 + threadIdx.x] = t_ve;
+    out[3 * H + 2 + threadIdx.x] = t_c;
+    if (threadIdx.x == 0) out[H] = t_b;
+    if (threadIdx.x == 1) out[2 * H + 1] = t_b;
   }
 }
 
-// dU = [dpre, E dpre] (BF16) and per-workgroup partials of db = sum dpre
+// dU = [dpre, E dpre] (BF16) and per-workgroup partials of db = sum dpre:
+// 16 lanes per node, edges as in k_head_bwd (64^3 grid: 195 us with a
+// wavefront per node and one edge at a time, this 44; the bytes, dpre
+// once and dU once, take 30 us)
 __global__ __launch_bounds__(kBlock) void k_aggregate_bwd(long long n, const int *__restrict__ erp,
                                                           const int *__restrict__ eci,
                                                           const float *__restrict__ ev,
                                                           const float *__restrict__ dpre,
                                                           bf16_t *__restrict__ dUb,
                                                           float *__restrict__ part) {
-  __shared__ float lds[kBlock / kWave][H];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const long long waves = (long long)gridDim.x * (kBlock / kWave);
-  float ab = 0.f;
-  for (long long i = (long long)blockIdx.x * (kBlock / kWave) + wave; i < n; i += waves) {
-    const float d = dpre[i * H + lane];
+  __shared__ __align__(16) float lds[kBlock / kWave * H];
+  const int q = threadIdx.x & 15;
+  const long long groups = (long long)gridDim.x * kNodes;
+  floatq ab = {0.f, 0.f, 0.f, 0.f};
+  for (long long i = (long long)blockIdx.x * kNodes + threadIdx.x / 16; i < n; i += groups) {
+    const int beg = erp[i], deg = erp[i + 1] - beg;
+    const floatq d = *reinterpret_cast<const floatq *>(dpre + i * H + 4 * q);
     ab += d;
-    float nb = 0.f;
-    for (int j = erp[i]; j < erp[i + 1]; j++) nb = fmaf(ev[j], dpre[(long long)eci[j] * H + lane], nb);
-    dUb[i * H2 + lane] = to_bf16(d);
-    dUb[i * H2 + H + lane] = to_bf16(nb);
+    const floatq nb = neighbour_sum(floatq{0.f, 0.f, 0.f, 0.f}, beg, deg, eci, ev, dpre, H, q);
+    store_bf16x4(dUb + i * H2 + 4 * q, d);
+    store_bf16x4(dUb + i * H2 + H + 4 * q, nb);
   }
-  lds[wave][lane] = ab;
-  __syncthreads();
-  if (threadIdx.x < H) {
-    float t = 0.f;
-    for (int w = 0; w < kBlock / kWave; w++) t += lds[w][threadIdx.x];
-    part[(long long)blockIdx.x * H + threadIdx.x] = t;
-  }
+  const float t = quad_total(ab, lds);
+  if (threadIdx.x < H) part[(long long)blockIdx.x * H + threadIdx.x] = t;
 }
 
 // layer 0: partials of dW0 = z0^T dpre1 (8 x 64) and db0 = sum dpre1
@@ -784,7 +836,7 @@ unsigned sgrid(long long n, int per = kBlock) {
   return (unsigned)std::max<long long>(1, std::min<long long>(g, 65536));
 }
 
-constexpr unsigned kRowGrid = 1024;  // workgroups of the wave-per-row kernels (partials)
+constexpr unsigned kRowGrid = 2048;  // workgroups of the kernels that leave partials
 
 template <typename T>
 struct DBuf {
@@ -824,7 +876,7 @@ struct tbsla_hip_precond_net_s {
   DBuf<float> ev, x, z0;
   DBuf<char> scan_ws;
   // activations and gradients
-  DBuf<float> h1, h2, h3, U, P, gdiag, ghat, dg, dh, dP;
+  DBuf<float> h1, h2, h3, U, P, gdiag, ghat, dg, dh;
   DBuf<bf16_t> hb1, hb2, hb3, Ub, dPb;
   DBuf<float> Z, T1, Vv, W, R, T2, Y;
   DBuf<double> lpart, lsum;
@@ -888,7 +940,7 @@ int prepare(tbsla_hip_precond_net_s *net, tbsla_hip_matrix_s *A, hipStream_t s) 
 }
 
 unsigned row_grid(long long n) {
-  return (unsigned)std::min<long long>(kRowGrid, std::max<long long>(1, (n + 3) / 4));
+  return (unsigned)std::min<long long>(kRowGrid, std::max<long long>(1, (n + kNodes - 1) / kNodes));
 }
 
 int forward(tbsla_hip_precond_net_s *net, double *gval, hipStream_t s) {
@@ -966,7 +1018,6 @@ int backward(tbsla_hip_precond_net_s *net, hipStream_t s) {
   const unsigned gg = (unsigned)((n + 63) / 64);
   const unsigned wg = (unsigned)((n + kWgRows - 1) / kWgRows);
   TBSLA_TRY(net->dh.ensure(n * H));
-  TBSLA_TRY(net->dP.ensure(n * H2));
   TBSLA_TRY(net->dPb.ensure(n * H2));
   TBSLA_TRY(net->Ub.ensure(n * H2));
   TBSLA_TRY(net->grad.ensure(kParams));
@@ -977,14 +1028,11 @@ int backward(tbsla_hip_precond_net_s *net, hipStream_t s) {
   const float *th = net->th.p;
   float *grad = net->grad.p;
   // head
-  k_head_bwd_rows<<<rg, kBlock, 0, s>>>(n, net->erp.p, net->eci.p, net->ev.p, net->nlow.p,
-                                        net->grp.p, net->P.p, net->h3.p, th, net->ghat.p, net->dg.p,
-                                        net->dh.p, net->dP.p, net->dPb.p, net->part.p);
+  k_head_bwd<<<rg, kBlock, 0, s>>>(n, net->erp.p, net->eci.p, net->ev.p, net->nlow.p, net->grp.p,
+                                   net->trp.p, net->tmap.p, net->P.p, net->h3.p, th, net->ghat.p,
+                                   net->dg.p, net->dh.p, net->dPb.p, net->part.p);
   reduce_parts(net->part.p, (int)rg, kHeadPart, net->red.p, s);
   k_head_scatter<<<1, kBlock, 0, s>>>(net->red.p, grad);
-  k_head_bwd_cols<<<rg, kBlock, 0, s>>>(n, net->trp.p, net->tci.p, net->tmap.p, net->erp.p,
-                                        net->eci.p, net->ev.p, net->nlow.p, net->P.p, th, net->dg.p,
-                                        net->dP.p, net->dPb.p);
   // V: dV = h3^T dP; dh3 += dP V^T, masked -> dpre3
   k_gemm_wgrad<<<wg, kBlock, 0, s>>>(n, net->hb3.p, net->dPb.p, net->part.p);
   reduce_parts(net->part.p, (int)wg, H * H2, grad + oV, s);
