@@ -349,45 +349,74 @@ __global__ __launch_bounds__(kBlock) void k_gemm_rows(long long n, const bf16_t 
 }
 
 // Split-K weight gradient: part[blk] = A[rows]^T B[rows] (M = 64, N = 128)
-// over the workgroup's chunk of rows, staged through LDS (transposed) in
-// steps of 32 rows.  Each wave owns 16 rows of the 64 x 128 result.
+// over the workgroup's chunk of rows.  The product contracts over rows, while
+// both operands are stored by rows, so a stage of 64 rows goes through LDS
+// transposed: a thread loads 8 channels (16 bytes) of rows 2p and 2p + 1 and
+// writes the 8 channels' row pairs as dwords (lanes p consecutive: no bank
+// conflicts), and a fragment is one 16-byte LDS read (a channel's stride of 36
+// dwords spreads 16 channels over all banks).  Two stages of LDS and the next
+// stage's loads in registers: one barrier a stage.  Each wave owns 16 rows of
+// the 64 x 128 result.  Bound by the 384 bytes a row; n = 262,144: 143 us with
+// 2-byte loads and stores, 20 so.
 constexpr int kWgRows = 512;
+constexpr int kWgStage = 64;                // rows per stage
+constexpr int kWgStride = kWgStage / 2 + 4;  // dwords per channel
 
 __global__ __launch_bounds__(kBlock) void k_gemm_wgrad(long long n, const bf16_t *__restrict__ A,
                                                        const bf16_t *__restrict__ B,
                                                        float *__restrict__ part) {
-  __shared__ bf16_t At[H][32 + 8];   // At[m][k]
-  __shared__ bf16_t Bs[H2][32 + 8];  // Bs[nn][k]
+  typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
+  __shared__ __align__(16) unsigned int At[2][H][kWgStride];   // [m][row pair]
+  __shared__ __align__(16) unsigned int Bs[2][H2][kWgStride];  // [nn][row pair]
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const long long row0 = (long long)blockIdx.x * kWgRows;
+  // this thread's row pair and channel octets: A's oct, B's oct and oct + 8
+  const int p = threadIdx.x & 31, oct = threadIdx.x / 32;
+  uintx4 ra[2], rb[2][2];
+  auto load = [&](int ks) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const long long r = row0 + ks + 2 * p + h;
+      const bool in = r < n;
+      ra[h] = in ? *reinterpret_cast<const uintx4 *>(A + r * H + 8 * oct) : uintx4{};
+#pragma unroll
+      for (int o = 0; o < 2; o++)
+        rb[o][h] = in ? *reinterpret_cast<const uintx4 *>(B + r * H2 + 8 * (oct + 8 * o)) : uintx4{};
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int w = k >> 1, sh = (k & 1) * 16;
+      At[buf][8 * oct + k][p] = ((ra[0][w] >> sh) & 0xFFFFu) | ((ra[1][w] >> sh) << 16);
+#pragma unroll
+      for (int o = 0; o < 2; o++)
+        Bs[buf][8 * (oct + 8 * o) + k][p] =
+            ((rb[o][0][w] >> sh) & 0xFFFFu) | ((rb[o][1][w] >> sh) << 16);
+    }
+  };
   floatx4 acc[8];
 #pragma unroll
   for (int t = 0; t < 8; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int ks = 0; ks < kWgRows; ks += 32) {
-    // stage 32 rows: A (32 x 64) and B (32 x 128), transposed
-    for (int e = threadIdx.x; e < 32 * H; e += kBlock) {
-      const int k = e / H, m = e % H;
-      const long long r = row0 + ks + k;
-      At[m][k] = r < n ? A[r * H + m] : (bf16_t)0;
-    }
-    for (int e = threadIdx.x; e < 32 * H2; e += kBlock) {
-      const int k = e / H2, c = e % H2;
-      const long long r = row0 + ks + k;
-      Bs[c][k] = r < n ? B[r * H2 + c] : (bf16_t)0;
-    }
-    __syncthreads();
-    const int kq = (lane >> 4) * 8;
-    bf16x8 a;
+  load(0);
+  stage(0);
+  __syncthreads();
+  for (int ks = 0, buf = 0; ks < kWgRows; ks += kWgStage, buf ^= 1) {
+    const bool more = ks + kWgStage < kWgRows;
+    if (more) load(ks + kWgStage);
 #pragma unroll
-    for (int q = 0; q < 8; q++) a[q] = __builtin_bit_cast(__bf16, At[wave * 16 + (lane & 15)][kq + q]);
+    for (int kk = 0; kk < kWgStage / 2; kk += 16) {
+      const int kq = kk + (lane >> 4) * 4;  // in row pairs
+      const bf16x8 a =
+          *reinterpret_cast<const bf16x8 *>(&At[buf][wave * 16 + (lane & 15)][kq]);
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-      bf16x8 b;
-#pragma unroll
-      for (int q = 0; q < 8; q++) b[q] = __builtin_bit_cast(__bf16, Bs[t * 16 + (lane & 15)][kq + q]);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+      for (int t = 0; t < 8; t++) {
+        const bf16x8 b = *reinterpret_cast<const bf16x8 *>(&Bs[buf][t * 16 + (lane & 15)][kq]);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+      }
     }
+    if (more) stage(buf ^ 1);
     __syncthreads();
   }
   float *out = part + (long long)blockIdx.x * H * H2;
