@@ -1379,7 +1379,7 @@ struct Buf {
     if (count <= n && p) return TBSLA_HIP_SUCCESS;
     if (p) {
       (void)hipDeviceSynchronize();
-      (void)hipFree(p);
+      device_free(p);
     }
     p = nullptr;
     n = 0;
@@ -1388,7 +1388,7 @@ struct Buf {
     return TBSLA_HIP_SUCCESS;
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) device_free(p);
     p = nullptr;
     n = 0;
   }
@@ -1471,11 +1471,11 @@ struct CgCache {
   std::vector<int> host_blocks;
 
   void drop_factor() {
-    (void)hipFree(t_rp);
-    (void)hipFree(t_ci);
-    (void)hipFree(t_v64);
-    (void)hipFree(g_v32);
-    (void)hipFree(t_v32);
+    device_free(t_rp);
+    device_free(t_ci);
+    device_free(t_v64);
+    device_free(g_v32);
+    device_free(t_v32);
     t_rp = t_ci = nullptr;
     t_v64 = nullptr;
     g_v32 = t_v32 = nullptr;
@@ -1504,8 +1504,8 @@ struct CgCache {
       if (e) (void)hipEventDestroy(e);
     if (own) (void)hipStreamDestroy(own);
     drop_factor();
-    (void)hipFree(a_v32);
-    (void)hipFree(dv32);
+    device_free(a_v32);
+    device_free(dv32);
   }
 };
 
@@ -1895,7 +1895,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
     const size_t need = (size_t)std::max(m->stored, 1LL);
     if (c.a_v32_len < need) {
       TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-      (void)hipFree(c.a_v32);
+      device_free(c.a_v32);
       c.a_v32 = nullptr;
       c.a_v32_len = 0;
       TBSLA_TRY(device_alloc((void **)&c.a_v32, need * 4));
@@ -1932,9 +1932,9 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
       tbsla_hip_matrix_s *GT = o.factor_t;
       if (!GT) {
         TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-        (void)hipFree(c.t_rp);
-        (void)hipFree(c.t_ci);
-        (void)hipFree(c.t_v64);
+        device_free(c.t_rp);
+        device_free(c.t_ci);
+        device_free(c.t_v64);
         c.t_rp = c.t_ci = nullptr;
         c.t_v64 = nullptr;
         TBSLA_TRY(csr_transpose_arrays(G, &c.t_rp, &c.t_ci, &c.t_v64, s));
@@ -1942,8 +1942,8 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
       if (mixed) {
         if (c.f32_len < (size_t)std::max(G->stored, 1LL)) {
           TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-          (void)hipFree(c.g_v32);
-          (void)hipFree(c.t_v32);
+          device_free(c.g_v32);
+          device_free(c.t_v32);
           c.g_v32 = c.t_v32 = nullptr;
           c.f32_len = 0;
           TBSLA_TRY(device_alloc((void **)&c.g_v32, (size_t)std::max(G->stored, 1LL) * 4));
@@ -2025,7 +2025,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
     if (mixed) {
       if (c.dv32_len < (size_t)dv_len) {
         TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-        (void)hipFree(c.dv32);
+        device_free(c.dv32);
         c.dv32 = nullptr;
         c.dv32_len = 0;
         TBSLA_TRY(device_alloc((void **)&c.dv32, (size_t)dv_len * 4));

@@ -235,5 +235,9 @@ int ensure_scratch(tbsla_hip_matrix_s *m, size_t bytes);
 void release_arrays(tbsla_hip_matrix_s *m);
 void cg_cache_release(tbsla_hip_matrix_s *m);
 void split_release(tbsla_hip_matrix_s *m);
+// Device memory of the library's own objects (capi.hip): device_free waits for
+// the device's queued work, as hipFree does, and keeps the block for a later
+// device_alloc of about its size.
 int device_alloc(void **p, size_t bytes);
+void device_free(void *p);
 }  // namespace tbsla_hip

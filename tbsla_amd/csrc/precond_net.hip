@@ -875,7 +875,7 @@ struct DBuf {
     if (p && count <= n) return TBSLA_HIP_SUCCESS;
     if (p) {
       (void)hipDeviceSynchronize();
-      (void)hipFree(p);
+      device_free(p);
     }
     p = nullptr;
     n = 0;
@@ -884,7 +884,7 @@ struct DBuf {
     return TBSLA_HIP_SUCCESS;
   }
   ~DBuf() {
-    if (p) (void)hipFree(p);
+    if (p) device_free(p);
   }
 };
 

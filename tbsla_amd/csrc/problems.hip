@@ -339,7 +339,7 @@ int counts_to_rowptr(const int *cnt, int *rowptr, long long n, long long *total,
     if (e != hipSuccess) st = fail(TBSLA_HIP_ERR_HIP, hipGetErrorString(e));
   }
   (void)hipStreamSynchronize(s);
-  (void)hipFree(ws);
+  device_free(ws);
   if (st) return st;
   if (t > INT32_MAX) return fail(TBSLA_HIP_ERR_RANGE, "more than 2^31-1 entries");
   int ti = (int)t;
@@ -360,9 +360,9 @@ int csr_transpose_arrays(const tbsla_hip_matrix_s *src, int **rowptr_t, int **co
   unsigned long long *keys = nullptr;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    (void)hipFree(cnt);
-    (void)hipFree(pay);
-    (void)hipFree(keys);
+    device_free(cnt);
+    device_free(pay);
+    device_free(keys);
   };
   int st;
   if ((st = device_alloc((void **)&cnt, (size_t)(nc + 1) * 4)) ||
@@ -372,9 +372,9 @@ int csr_transpose_arrays(const tbsla_hip_matrix_s *src, int **rowptr_t, int **co
       (st = device_alloc((void **)&pay, (size_t)std::max(m, 1LL) * 4)) ||
       (st = device_alloc((void **)&keys, (size_t)std::max(m, 1LL) * 8))) {
     cleanup();
-    (void)hipFree(rp);
-    (void)hipFree(ci);
-    (void)hipFree(v);
+    device_free(rp);
+    device_free(ci);
+    device_free(v);
     return st;
   }
   (void)hipMemsetAsync(cnt, 0, (size_t)(nc + 1) * 4, s);
@@ -394,9 +394,9 @@ int csr_transpose_arrays(const tbsla_hip_matrix_s *src, int **rowptr_t, int **co
   }
   cleanup();
   if (st) {
-    (void)hipFree(rp);
-    (void)hipFree(ci);
-    (void)hipFree(v);
+    device_free(rp);
+    device_free(ci);
+    device_free(v);
     return st;
   }
   *rowptr_t = rp;
@@ -426,7 +426,7 @@ extern "C" int tbsla_hip_fill_poisson3d(tbsla_hip_matrix_t m, int nx, int ny, in
   k_poisson_count<<<sgrid(n), kBlock, 0, s>>>(g, n, cnt);
   long long total = 0;
   int st = counts_to_rowptr(cnt, m->rowptr, n, &total, s);
-  (void)hipFree(cnt);
+  device_free(cnt);
   if (st) return st;
   TBSLA_TRY(device_alloc((void **)&m->colidx, (size_t)total * 4));
   TBSLA_TRY(device_alloc((void **)&m->values, (size_t)total * 8));
@@ -478,7 +478,7 @@ extern "C" int tbsla_hip_fill_lognormal_field(double *d_kappa, int nx, int ny, i
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(d_kappa, tmp, (size_t)n * 8, hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(tmp);
+  device_free(tmp);
   if (e != hipSuccess) return fail(TBSLA_HIP_ERR_HIP, hipGetErrorString(e));
   return TBSLA_HIP_SUCCESS;
 }
@@ -517,10 +517,10 @@ extern "C" int tbsla_hip_fill_sym_cqmat(tbsla_hip_matrix_t m, int n, int c, doub
   int *pay = nullptr, *cnt = nullptr, *start = nullptr;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    (void)hipFree(keys);
-    (void)hipFree(pay);
-    (void)hipFree(cnt);
-    (void)hipFree(start);
+    device_free(keys);
+    device_free(pay);
+    device_free(cnt);
+    device_free(start);
     tbsla_hip_destroy(B);
   };
   const long long m2 = std::max(2 * mb, 1LL);

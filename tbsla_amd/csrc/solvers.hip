@@ -455,7 +455,7 @@ unsigned stride_grid(long long n) {
 template <typename T>
 struct DevBuf {
   T *p = nullptr;
-  ~DevBuf() { if (p) (void)hipFree(p); }
+  ~DevBuf() { if (p) device_free(p); }
   int alloc(long long n) { return device_alloc((void **)&p, (size_t)std::max(n, 1LL) * sizeof(T)); }
 };
 
@@ -484,7 +484,7 @@ extern "C" int tbsla_hip_values_changed(tbsla_hip_matrix_t m, void *stream) {
   // the COO/SCOO row pointer is derived from the row array: rebuilt (and the
   // triplets' order checked again) at the next SpMV
   if (m->coo_rowptr) {
-    (void)hipFree(m->coo_rowptr);
+    device_free(m->coo_rowptr);
     m->coo_rowptr = nullptr;
   }
   if (m->format == TBSLA_HIP_COO || m->format == TBSLA_HIP_SCOO) {

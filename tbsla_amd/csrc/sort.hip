@@ -199,10 +199,10 @@ int radix_sort_pairs(unsigned long long *keys, int *payload, long long n, int ke
   int st = TBSLA_HIP_SUCCESS;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    (void)hipFree(keys_alt);
-    (void)hipFree(pay_alt);
-    (void)hipFree(hist);
-    (void)hipFree(ws);
+    device_free(keys_alt);
+    device_free(pay_alt);
+    device_free(hist);
+    device_free(ws);
   };
   if ((st = device_alloc((void **)&keys_alt, (size_t)n * 8)) ||
       (st = device_alloc((void **)&pay_alt, (size_t)n * 4)) ||
@@ -248,7 +248,7 @@ static int coo_order(const tbsla_hip_matrix_s *coo, int *perm, hipStream_t s) {
   k_iota<<<grid_for(n), kBlock, 0, s>>>(perm, n);
   int st = radix_sort_pairs(keys, perm, n, col_bits + row_bits, s);
   (void)hipStreamSynchronize(s);
-  (void)hipFree(keys);
+  device_free(keys);
   return st;
 }
 
@@ -328,7 +328,7 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
       // key = row only (col_bits 0 and row OR row == row)
       int st = radix_sort_pairs(keys, perm, n, bits_for(std::max(coo->n_row, 1)), s);
       (void)hipStreamSynchronize(s);
-      (void)hipFree(keys);
+      device_free(keys);
       if (st) return st;
     }
     const size_t cells = (size_t)rows * (size_t)dst->ln_col;
@@ -341,8 +341,8 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
     dst->stored = (long long)cells;
     dst->has_arrays = 1;
     TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-    (void)hipFree(perm);
-    (void)hipFree(rowptr);
+    device_free(perm);
+    device_free(rowptr);
     return TBSLA_HIP_SUCCESS;
   }
 
@@ -356,7 +356,7 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
     TBSLA_HIP_LAUNCH_CHECK();
   }
   (void)hipStreamSynchronize(s);
-  (void)hipFree(perm);
+  device_free(perm);
   if (format == TBSLA_HIP_CSR) {
     dst->rowptr = rowptr;
     dst->colidx = scol;
@@ -377,7 +377,7 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
   int width = 0;
   TBSLA_HIP_CHECK(hipMemcpyAsync(&width, d_w, 4, hipMemcpyDeviceToHost, s));
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-  (void)hipFree(lens);
+  device_free(lens);
   dst->max_col = width;
   const size_t slots = (size_t)rows * (size_t)width;
   TBSLA_TRY(device_alloc((void **)&dst->colidx, std::max<size_t>(slots, 1) * 4));
@@ -389,8 +389,8 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
   dst->stored = (long long)slots;
   dst->has_arrays = 1;
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-  (void)hipFree(rowptr);
-  (void)hipFree(scol);
-  (void)hipFree(sval);
+  device_free(rowptr);
+  device_free(scol);
+  device_free(sval);
   return TBSLA_HIP_SUCCESS;
 }

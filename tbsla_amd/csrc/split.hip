@@ -85,24 +85,24 @@ struct SplitCsr {
   int *sst = nullptr, *pst = nullptr, *pb = nullptr;
   ~SplitCsr() {
     (void)hipDeviceSynchronize();
-    (void)hipFree(c16);
-    (void)hipFree(q16);
-    (void)hipFree(d16);
-    (void)hipFree(rs16);
-    (void)hipFree(sst);
-    (void)hipFree(pst);
-    (void)hipFree(pb);
-    (void)hipFree(lrp);
-    (void)hipFree(lci);
-    (void)hipFree(lv);
-    (void)hipFree(sr);
-    (void)hipFree(sc);
-    (void)hipFree(sv);
-    (void)hipFree(boff);
-    (void)hipFree(P);
-    (void)hipFree(R);
-    (void)hipFree(doff);
-    (void)hipFree(dv);
+    device_free(c16);
+    device_free(q16);
+    device_free(d16);
+    device_free(rs16);
+    device_free(sst);
+    device_free(pst);
+    device_free(pb);
+    device_free(lrp);
+    device_free(lci);
+    device_free(lv);
+    device_free(sr);
+    device_free(sc);
+    device_free(sv);
+    device_free(boff);
+    device_free(P);
+    device_free(R);
+    device_free(doff);
+    device_free(dv);
   }
 };
 
@@ -851,7 +851,7 @@ static int pick_block_rows(const int *rp, long long n, hipStream_t s, int *h_out
                   hipMemcpyAsync(hb.data(), d, (size_t)(nb + 1) * 4, hipMemcpyDeviceToHost, s) ==
                       hipSuccess &&
                   hipStreamSynchronize(s) == hipSuccess;
-  (void)hipFree(d);
+  device_free(d);
   if (!ok) return fail(TBSLA_HIP_ERR_HIP, "diagonal layout: block sizes");
   for (int h = 4096; h >= kWave && *h_out == 0; h /= 2) {
     const long long step = h / kWave;
@@ -888,17 +888,17 @@ int split_build(tbsla_hip_matrix_s *m, int window, int slices, hipStream_t s, in
   int tot32[2] = {0, 0};  // rptr[n] and lrp[n], copied from here before the stream syncs
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    (void)hipFree(lcnt);
-    (void)hipFree(rcnt);
-    (void)hipFree(rptr);
-    (void)hipFree(rc);
-    (void)hipFree(pay);
-    (void)hipFree(scount);
-    (void)hipFree(rv);
-    (void)hipFree(keys);
-    (void)hipFree(ws);
-    (void)hipFree(hist);
-    (void)hipFree(dmap);
+    device_free(lcnt);
+    device_free(rcnt);
+    device_free(rptr);
+    device_free(rc);
+    device_free(pay);
+    device_free(scount);
+    device_free(rv);
+    device_free(keys);
+    device_free(ws);
+    device_free(hist);
+    device_free(dmap);
   };
   auto failed = [&](int st) {
     cleanup();

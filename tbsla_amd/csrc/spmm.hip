@@ -802,12 +802,12 @@ extern "C" int tbsla_hip_personalized_page_rank(tbsla_hip_matrix_t m, double bet
   PprState *st = nullptr;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    (void)hipFree(buf);
-    (void)hipFree(part);
-    (void)hipFree(S);
-    (void)hipFree(src);
-    (void)hipFree(st);
-    (void)hipFree(bins);
+    device_free(buf);
+    device_free(part);
+    device_free(S);
+    device_free(src);
+    device_free(st);
+    device_free(bins);
   };
   // the first failing HIP call of the set-up and iteration loop
   hipError_t herr = hipSuccess;
