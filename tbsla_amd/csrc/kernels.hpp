@@ -27,11 +27,16 @@ int pick_csr_nt(const tbsla_hip_matrix_s *m);
 int launch_fill(double *d, long long n, double v, hipStream_t s);
 int launch_axpy_inplace(double *y, const double *x, long long n, hipStream_t s);  // y += x
 
-// sort.hip: stable LSD radix sort of 64-bit keys carrying a 32-bit payload
-// (the original position); key_bits significant bits.  Buffers of n
-// elements; the result lands in keys/payload.
-int radix_sort_pairs(unsigned long long *keys, int *payload, long long n, int key_bits,
-                     hipStream_t s);
+// sort.hip: stable LSD radix sort of 32- or 64-bit keys (key_bits significant
+// bits), *payload receiving each key's original position.  Buffers of n
+// elements from device_alloc; the sort works between them and two of its own
+// and leaves in *keys / *payload the pair that holds the result (it frees the
+// other).  Synchronises the stream.
+template <typename K>
+int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s);
+// ptr[b] = the first k with (keys[k] >> shift) >= b, b in [0, nb], of n sorted keys
+template <typename K>
+int bucket_starts(const K *keys, long long n, int shift, long long nb, int *ptr, hipStream_t s);
 
 // problems.hip: row pointers from per-row counts (exclusive scan; *total,
 // host, receives the sum; synchronises the stream)

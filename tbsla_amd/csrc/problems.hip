@@ -171,23 +171,17 @@ __global__ __launch_bounds__(kBlock) void k_sym_keys(long long n, long long m,
                                                      const int *__restrict__ rowptr,
                                                      const int *__restrict__ colidx, int cb,
                                                      unsigned long long sentinel,
-                                                     unsigned long long *__restrict__ keys,
-                                                     int *__restrict__ payload,
-                                                     int *__restrict__ cnt) {
+                                                     unsigned long long *__restrict__ keys) {
   for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r < n;
        r += (long long)gridDim.x * kBlock) {
     for (int j = rowptr[r]; j < rowptr[r + 1]; j++) {
       const long long c = colidx[j];
-      payload[j] = j;
-      payload[m + j] = (int)(m + j);
       if (c == r) {
         keys[j] = sentinel;
         keys[m + j] = sentinel;
       } else {
         keys[j] = ((unsigned long long)r << cb) | (unsigned long long)c;
         keys[m + j] = ((unsigned long long)c << cb) | (unsigned long long)r;
-        atomicAdd(cnt + r, 1);
-        atomicAdd(cnt + c, 1);
       }
     }
   }
@@ -256,16 +250,12 @@ __global__ __launch_bounds__(kBlock) void k_transpose_keys(long long n_rows,
                                                            const int *__restrict__ rowptr,
                                                            const int *__restrict__ colidx,
                                                            int f_col, int rb,
-                                                           unsigned long long *__restrict__ keys,
-                                                           int *__restrict__ payload,
-                                                           int *__restrict__ cnt) {
+                                                           unsigned long long *__restrict__ keys) {
   for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r < n_rows;
        r += (long long)gridDim.x * kBlock) {
     for (int j = rowptr[r]; j < rowptr[r + 1]; j++) {
       const long long c = colidx[j] - f_col;
       keys[j] = ((unsigned long long)c << rb) | (unsigned long long)r;
-      payload[j] = j;
-      atomicAdd(cnt + c, 1);
     }
   }
 }
@@ -355,18 +345,16 @@ int counts_to_rowptr(const int *cnt, int *rowptr, long long n, long long *total,
 int csr_transpose_arrays(const tbsla_hip_matrix_s *src, int **rowptr_t, int **colidx_t,
                          double **values_t, hipStream_t s) {
   const long long nr = src->ln_row, nc = src->ln_col, m = src->stored;
-  int *cnt = nullptr, *rp = nullptr, *ci = nullptr, *pay = nullptr;
+  int *rp = nullptr, *ci = nullptr, *pay = nullptr;
   double *v = nullptr;
   unsigned long long *keys = nullptr;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
-    device_free(cnt);
     device_free(pay);
     device_free(keys);
   };
   int st;
-  if ((st = device_alloc((void **)&cnt, (size_t)(nc + 1) * 4)) ||
-      (st = device_alloc((void **)&rp, (size_t)(nc + 1) * 4)) ||
+  if ((st = device_alloc((void **)&rp, (size_t)(nc + 1) * 4)) ||
       (st = device_alloc((void **)&ci, (size_t)std::max(m, 1LL) * 4)) ||
       (st = device_alloc((void **)&v, (size_t)std::max(m, 1LL) * 8)) ||
       (st = device_alloc((void **)&pay, (size_t)std::max(m, 1LL) * 4)) ||
@@ -377,16 +365,14 @@ int csr_transpose_arrays(const tbsla_hip_matrix_s *src, int **rowptr_t, int **co
     device_free(v);
     return st;
   }
-  (void)hipMemsetAsync(cnt, 0, (size_t)(nc + 1) * 4, s);
   const int rb = bits_of(std::max(nr, 1LL));
   const int cbits = bits_of(std::max(nc, 1LL));
   if (m > 0) {
     k_transpose_keys<<<sgrid(nr), kBlock, 0, s>>>(nr, src->rowptr, src->colidx, src->f_col, rb,
-                                                  keys, pay, cnt);
-    st = radix_sort_pairs(keys, pay, m, rb + cbits, s);
+                                                  keys);
+    st = radix_sort_pairs<unsigned long long>(&keys, &pay, m, rb + cbits, s);
   }
-  long long total = 0;
-  if (!st) st = counts_to_rowptr(cnt, rp, nc, &total, s);
+  if (!st) st = bucket_starts<unsigned long long>(keys, m, rb, nc, rp, s);
   if (!st && m > 0) {
     k_transpose_fill<<<sgrid(m), kBlock, 0, s>>>(m, keys, pay, src->values, rb, src->f_row, ci, v);
     hipError_t e = hipGetLastError();
@@ -531,11 +517,10 @@ extern "C" int tbsla_hip_fill_sym_cqmat(tbsla_hip_matrix_t m, int n, int c, doub
     cleanup();
     return st;
   }
-  (void)hipMemsetAsync(cnt, 0, (size_t)(n + 1) * 4, s);
-  k_sym_keys<<<sgrid(n), kBlock, 0, s>>>(n, mb, B->rowptr, B->colidx, cb, sentinel, keys, pay, cnt);
-  if (2 * mb > 1) st = radix_sort_pairs(keys, pay, 2 * mb, 2 * cb, s);
-  long long total = 0;
-  if (!st) st = counts_to_rowptr(cnt, start, n, &total, s);
+  k_sym_keys<<<sgrid(n), kBlock, 0, s>>>(n, mb, B->rowptr, B->colidx, cb, sentinel, keys);
+  st = radix_sort_pairs<unsigned long long>(&keys, &pay, 2 * mb, 2 * cb, s);
+  // the sentinel's row, (1 << cb) - 1 >= n, lies after the last
+  if (!st) st = bucket_starts<unsigned long long>(keys, 2 * mb, cb, n, start, s);
   release_arrays(m);
   set_square(m, n);
   if (!st) {

@@ -137,26 +137,14 @@ __global__ __launch_bounds__(kBlock) void k_scoo_normalize_rows(long long n, lon
 }
 
 // SCOO row sums: key = row[k] - f_row (entries of other rows get the key
-// ln_row, a bucket no sum reads), payload = k.
+// ln_row, a bucket no sum reads); the sort's payload is k.
 __global__ __launch_bounds__(kBlock) void k_scoo_rowkeys(long long n, const int *__restrict__ row,
                                                          int f_row, long long ln_row,
-                                                         unsigned long long *__restrict__ keys,
-                                                         int *__restrict__ pos) {
+                                                         unsigned *__restrict__ keys) {
   long long k = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (k >= n) return;
   const long long r = (long long)row[k] - f_row;
-  keys[k] = (r >= 0 && r < ln_row) ? (unsigned long long)r : (unsigned long long)ln_row;
-  pos[k] = (int)k;
-}
-
-__global__ __launch_bounds__(kBlock) void k_count_keys(const unsigned long long *__restrict__ keys,
-                                                       long long n, long long nb,
-                                                       int *__restrict__ counts) {
-  for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (long long)gridDim.x * kBlock) {
-    const unsigned long long k = keys[i];
-    if (k <= (unsigned long long)nb) atomicAdd(counts + k, 1);
-  }
+  keys[k] = (r >= 0 && r < ln_row) ? (unsigned)r : (unsigned)ln_row;
 }
 
 // s[b] += the bucket's values in entry order (MatrixSCOO.cpp:701-705)
@@ -463,24 +451,17 @@ struct Buf {
 
 int scoo_row_sums(tbsla_hip_matrix_s *m, double *d_s, hipStream_t s) {
   const long long n = m->stored, nb = m->ln_row;
-  Buf<unsigned long long> keys;
+  Buf<unsigned> keys;
   Buf<int> pos, ptr;
-  Buf<char> ws;
   TBSLA_TRY(keys.alloc(n));
   TBSLA_TRY(pos.alloc(n));
-  TBSLA_TRY(ptr.alloc(nb + 2));  // ln_row buckets + the bucket of other rows
-  k_scoo_rowkeys<<<grid_for(n), kBlock, 0, s>>>(n, m->rowidx, m->f_row, nb, keys.p, pos.p);
+  TBSLA_TRY(ptr.alloc(nb + 1));
+  k_scoo_rowkeys<<<grid_for(n), kBlock, 0, s>>>(n, m->rowidx, m->f_row, nb, keys.p);
   TBSLA_HIP_LAUNCH_CHECK();
   int bits = 1;
-  while (bits < 62 && (1LL << bits) <= nb) bits++;  // keys <= ln_row < 2^bits
-  TBSLA_TRY(radix_sort_pairs(keys.p, pos.p, n, bits, s));
-  TBSLA_HIP_CHECK(hipMemsetAsync(ptr.p, 0, (size_t)(nb + 2) * 4, s));
-  k_count_keys<<<rgrid(n), kBlock, 0, s>>>(keys.p, n, nb, ptr.p + 1);
-  TBSLA_HIP_LAUNCH_CHECK();
-  const size_t wsb = scan_workspace_bytes(nb + 1);
-  TBSLA_TRY(ws.alloc((long long)wsb + 64));
-  TBSLA_TRY(scan<int>(ptr.p + 1, ptr.p + 1, nb + 1, true,
-                      reinterpret_cast<long long *>(ws.p + wsb), ws.p, s));
+  while (bits < 32 && (1LL << bits) <= nb) bits++;  // keys <= ln_row < 2^bits
+  TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s));
+  TBSLA_TRY(bucket_starts<unsigned>(keys.p, n, 0, nb, ptr.p, s));
   if (nb > 0) {
     k_bucket_sums<<<grid_for(nb), kBlock, 0, s>>>(nb, ptr.p, pos.p, m->values, d_s + m->f_row);
     TBSLA_HIP_LAUNCH_CHECK();

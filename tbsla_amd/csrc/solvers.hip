@@ -53,8 +53,8 @@ unsigned red_grid(long long n) {
 
 // ---- column sums --------------------------------------------------------
 
-// key = local column, payload = the entry's position in the reference's loop
-// order (CSR/SCOO: storage order; ELL: row-major slot i*max_col+j).  Entries
+// key = local column; the sort's payload is the entry's position in the
+// reference's loop order (CSR/SCOO: storage order; ELL: row-major slot i*max_col+j).  Entries
 // the reference skips -- ELL slots whose value is not positive
 // (MatrixELL.cpp:812), which include the padding (column 0, possibly left of
 // the block) -- and any column outside [0, ln_col) get the key ln_col, a
@@ -63,51 +63,68 @@ __global__ __launch_bounds__(kBlock) void k_colkeys(long long n, int fmt, long l
                                                     long long ln_col, int max_col,
                                                     const int *__restrict__ cols,
                                                     const double *__restrict__ vals, int f_col,
-                                                    unsigned long long *__restrict__ keys,
-                                                    int *__restrict__ pos) {
+                                                    unsigned *__restrict__ keys) {
   long long p = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (p >= n) return;
   long long src = p;
   if (fmt == TBSLA_HIP_ELL) src = (p % max_col) * ln_row + p / max_col;
   long long c = (long long)cols[src] - f_col;
   bool keep = c >= 0 && c < ln_col && (fmt != TBSLA_HIP_ELL || vals[src] > 0);
-  keys[p] = keep ? (unsigned long long)c : (unsigned long long)ln_col;
-  pos[p] = (int)p;
-}
-
-// counts[key]++ for keys <= ln_col (the last bucket collects skipped entries)
-__global__ __launch_bounds__(kBlock) void k_count_cols(const unsigned long long *__restrict__ keys,
-                                                       long long n, long long ln_col,
-                                                       int *__restrict__ counts) {
-  for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (long long)gridDim.x * kBlock) {
-    unsigned long long k = keys[i];
-    if (k <= (unsigned long long)ln_col) atomicAdd(counts + k, 1);
-  }
+  keys[p] = keep ? (unsigned)c : (unsigned)ln_col;
 }
 
 // s[c] += the column's values in reference order (one thread per column):
 // the serial loop of MatrixCSR::get_col_sums (MatrixCSR.cpp:1200-1206) and
 // MatrixSCOO::get_col_sums (MatrixSCOO.cpp:719-723); ELL adds positive
 // values only (MatrixELL.cpp:809-815).
+//
+// A workgroup takes 256 columns, whose sorted positions are one contiguous
+// run: it goes through LDS in chunks, loaded by consecutive lanes with the
+// gathers of eight values in flight each, and every thread then adds its own
+// column's values from LDS, in order (one spare double per 16 keeps the
+// columns of a regular matrix on different banks).  24 M entries: 107 us,
+// against 554 with each thread walking its positions in memory.
+constexpr int kSumChunk = 4096;
+
 __global__ __launch_bounds__(kBlock) void k_col_sums(long long ln_col, int fmt, long long ln_row,
                                                      int max_col, const int *__restrict__ colptr,
                                                      const int *__restrict__ pos,
                                                      const double *__restrict__ vals,
                                                      double *__restrict__ s) {
-  long long c = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (c >= ln_col) return;
-  double acc = s[c];
-  for (int j = colptr[c]; j < colptr[c + 1]; j++) {
-    long long p = pos[j];
-    if (fmt == TBSLA_HIP_ELL) {
-      double v = vals[(p % max_col) * ln_row + p / max_col];
-      if (v > 0) acc += v;
-    } else {
-      acc += vals[p];
+  __shared__ double buf[kSumChunk + kSumChunk / 16];
+  const long long c0 = (long long)blockIdx.x * kBlock;
+  const long long c = c0 + threadIdx.x;
+  const bool live = c < ln_col;
+  const int first = colptr[c0], last = colptr[min(c0 + kBlock, ln_col)];
+  const int beg = live ? colptr[c] : last, end = live ? colptr[c + 1] : last;
+  double acc = live ? s[c] : 0.0;
+  int j = beg;
+  for (int b = first; b < last; b += kSumChunk) {
+    const int m = min(kSumChunk, last - b);
+    for (int i0 = threadIdx.x; i0 < m; i0 += 8 * kBlock) {
+      long long p[8];
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) p[k] = pos[b + min(i0 + k * kBlock, m - 1)];
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        v[k] = vals[fmt == TBSLA_HIP_ELL ? (p[k] % max_col) * ln_row + p[k] / max_col : p[k]];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int i = i0 + k * kBlock;
+        if (i < m) buf[i + (i >> 4)] = v[k];
+      }
     }
+    __syncthreads();
+    const int stop = min(end, b + m);
+    for (; j < stop; j++) {
+      const int i = j - b;
+      const double v = buf[i + (i >> 4)];
+      if (fmt != TBSLA_HIP_ELL || v > 0) acc += v;
+    }
+    __syncthreads();
   }
-  s[c] = acc;
+  if (live) s[c] = acc;
 }
 
 // normalize_cols: CSR (MatrixCSR.cpp:1221-1231) and SCOO
@@ -510,25 +527,18 @@ extern "C" int tbsla_hip_get_col_sums(tbsla_hip_matrix_t m, double *d_s, void *s
   const long long n = fmt == TBSLA_HIP_ELL ? (long long)m->ln_row * m->max_col : m->stored;
   const long long ln_col = m->ln_col;
   if (n == 0) return TBSLA_HIP_SUCCESS;
-  DevBuf<unsigned long long> keys;
+  DevBuf<unsigned> keys;
   DevBuf<int> pos, colptr;
   TBSLA_TRY(keys.alloc(n));
   TBSLA_TRY(pos.alloc(n));
-  TBSLA_TRY(colptr.alloc(ln_col + 2));  // ln_col columns + the skipped-entry bucket
+  TBSLA_TRY(colptr.alloc(ln_col + 1));
   k_colkeys<<<grid_for(n), kBlock, 0, s>>>(n, fmt, m->ln_row, ln_col, m->max_col, m->colidx,
-                                           m->values, m->f_col, keys.p, pos.p);
+                                           m->values, m->f_col, keys.p);
   TBSLA_HIP_LAUNCH_CHECK();
   int bits = 1;
-  while (bits < 62 && (1LL << bits) <= ln_col) bits++;  // keys <= ln_col < 2^bits
-  TBSLA_TRY(radix_sort_pairs(keys.p, pos.p, n, bits, s));
-  TBSLA_HIP_CHECK(hipMemsetAsync(colptr.p, 0, (size_t)(ln_col + 2) * 4, s));
-  k_count_cols<<<stride_grid(n), kBlock, 0, s>>>(keys.p, n, ln_col, colptr.p + 1);
-  TBSLA_HIP_LAUNCH_CHECK();
-  DevBuf<char> ws;
-  TBSLA_TRY(ws.alloc((long long)scan_workspace_bytes(ln_col + 1) + 64));
-  TBSLA_TRY(scan<int>(colptr.p + 1, colptr.p + 1, ln_col + 1, true,
-                      reinterpret_cast<long long *>(ws.p + scan_workspace_bytes(ln_col + 1)), ws.p,
-                      s));
+  while (bits < 32 && (1LL << bits) <= ln_col) bits++;  // keys <= ln_col < 2^bits
+  TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s));
+  TBSLA_TRY(bucket_starts<unsigned>(keys.p, n, 0, ln_col, colptr.p, s));
   if (ln_col > 0) {
     k_col_sums<<<grid_for(ln_col), kBlock, 0, s>>>(ln_col, fmt, m->ln_row, m->max_col, colptr.p,
                                                    pos.p, m->values, d_s);

@@ -1,12 +1,15 @@
 // sort.hip -- stable LSD radix sort and the COO conversion constructors.
 //
-// Radix sort of 64-bit keys with a 32-bit payload, 8-bit digits.  Per pass:
-// a per-tile digit histogram, one exclusive scan over the digit-major
-// histogram, and a stable scatter.  Stability inside a tile comes from
-// processing elements in index order: each wavefront owns a contiguous
-// 1024-element sub-tile, walks it in 64-element rounds, finds the lanes that
-// share its digit with eight ballots and ranks itself among them; per-wave
-// running bases live in LDS.  Integer work only: the permutation is unique.
+// Radix sort of 32- or 64-bit keys carrying each key's original position, in
+// digits of at most 8 bits.  Per pass: a per-tile digit histogram, one
+// exclusive scan over the digit-major histogram, and a stable scatter.
+// Stability inside a tile comes from processing elements in index order: each
+// wavefront owns a contiguous sub-tile, walks it in 64-element rounds, finds
+// the lanes that share its digit with one ballot per digit bit and ranks itself
+// among them; per-wave counts live in LDS.  The tile's elements are then put
+// into LDS in digit order and written from there, so that an output run of one
+// digit is written by consecutive lanes.  Integer work only: the permutation is
+// unique.
 #include <algorithm>
 #include <vector>
 
@@ -18,116 +21,211 @@ namespace tbsla_hip {
 namespace {
 
 constexpr int kRadix = 256;
-constexpr int kRounds = 16;                       // rounds of 64 per wave
-constexpr int kSubTile = kWave * kRounds;         // 1024 elements per wave
-constexpr int kTileElems = kSubTile * (kBlock / kWave);  // 4096 per workgroup
+constexpr int kItems = 16;  // keys per thread of a tile
 
-__global__ __launch_bounds__(kBlock) void k_digit_hist(const unsigned long long *__restrict__ keys,
-                                                       long long n, int shift, long long ntiles,
-                                                       int *__restrict__ hist) {
-  __shared__ int h[kRadix];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  const long long base = (long long)blockIdx.x * kTileElems;
-  for (int i = threadIdx.x; i < kTileElems; i += kBlock) {
-    long long e = base + i;
-    if (e < n) atomicAdd(&h[(keys[e] >> shift) & 0xFF], 1);
-  }
-  __syncthreads();
-  hist[(long long)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
-}
+// Tiles: 512 threads for 32-bit keys, 256 for 64-bit ones; both put 32 KB of
+// keys through LDS (four, or for 64-bit keys three to four, workgroups per CU).
+template <typename K>
+struct SortTile {
+  static constexpr int threads = sizeof(K) == 4 ? 512 : 256;
+  static constexpr int elems = threads * kItems;
+  static constexpr int waves = threads / kWave;
+};
 
-__global__ __launch_bounds__(kBlock) void k_digit_scatter(
-    const unsigned long long *__restrict__ keys_in, const int *__restrict__ pay_in,
-    unsigned long long *__restrict__ keys_out, int *__restrict__ pay_out, long long n, int shift,
-    long long ntiles, const int *__restrict__ offsets) {
-  __shared__ int wbase[kBlock / kWave][kRadix];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  for (int i = threadIdx.x; i < (kBlock / kWave) * kRadix; i += kBlock) (&wbase[0][0])[i] = 0;
+// Digit counts of each tile.  Per-wave counters in LDS; a round whose lanes all
+// hold one digit (the high digits of a banded or sorted input) is counted by
+// one lane instead of 64 additions to one address.
+template <typename K>
+__global__ __launch_bounds__(SortTile<K>::threads) void k_digit_hist(
+    const K *__restrict__ keys, long long n, int shift, int mask, long long ntiles,
+    int *__restrict__ hist) {
+  typedef SortTile<K> T;
+  __shared__ int h[T::waves][kRadix];
+  for (int i = threadIdx.x; i < T::waves * kRadix; i += T::threads) (&h[0][0])[i] = 0;
   __syncthreads();
-  const long long sub = (long long)blockIdx.x * kTileElems + (long long)wave * kSubTile;
-  // phase A: digit counts of each wave's sub-tile
-  for (int r = 0; r < kRounds; r++) {
-    long long e = sub + r * kWave + lane;
-    if (e < n) atomicAdd(&wbase[wave][(keys_in[e] >> shift) & 0xFF], 1);
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const long long base = (long long)blockIdx.x * T::elems + threadIdx.x;
+  K key[kItems];
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const long long e = base + i * T::threads;
+    key[i] = e < n ? keys[e] : (K)0;
   }
-  __syncthreads();
-  // per-wave starting position of each digit
-  {
-    const int d = threadIdx.x;
-    int run = offsets[(long long)d * ntiles + blockIdx.x];
-    for (int w = 0; w < kBlock / kWave; w++) {
-      int c = wbase[w][d];
-      wbase[w][d] = run;
-      run += c;
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const bool valid = base + i * T::threads < n;
+    const int d = (int)(key[i] >> shift) & mask;
+    const unsigned long long in = __ballot(valid);
+    const int first = __builtin_amdgcn_readfirstlane(d);
+    if (in == ~0ull && __ballot(d == first) == ~0ull) {
+      if (lane == 0) atomicAdd(&h[wave][first], kWave);
+    } else if (valid) {
+      atomicAdd(&h[wave][d], 1);
     }
   }
   __syncthreads();
-  // phase B: stable scatter, rounds in index order
-  const unsigned long long lanes_below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
-  for (int r = 0; r < kRounds; r++) {
-    long long e = sub + r * kWave + lane;
-    const bool valid = e < n;
-    unsigned long long key = valid ? keys_in[e] : 0ull;
-    int d = (int)((key >> shift) & 0xFF);
-    unsigned long long peers = __ballot(valid);
+  for (int d = threadIdx.x; d <= mask; d += T::threads) {
+    int c = 0;
+    for (int w = 0; w < T::waves; w++) c += h[w][d];
+    hist[(long long)d * ntiles + blockIdx.x] = c;
+  }
+}
+
+// The stable scatter of one pass; pay_in null: the payload of element e is e
+// (the first pass).  Bound by its bytes once the output runs are whole: 24 M
+// 32-bit keys take 101 us a pass (16 bytes an element, 3.8 TB/s) where
+// the scatter from registers, with 64-bit keys read twice, took 290 (2.0 TB/s).
+template <typename K>
+__global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
+    const K *__restrict__ keys_in, const int *__restrict__ pay_in, K *__restrict__ keys_out,
+    int *__restrict__ pay_out, long long n, int shift, int bits, long long ntiles,
+    const int *__restrict__ offsets) {
+  typedef SortTile<K> T;
+  __shared__ int wcnt[T::waves][kRadix];  // counts, then each wave's first position
+  __shared__ int gofs[kRadix];            // output position minus tile position
+  __shared__ int wsum[T::waves];
+  __shared__ K stage[T::elems];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int mask = (1 << bits) - 1;
+  const long long tile0 = (long long)blockIdx.x * T::elems;
+  const int count = (int)min((long long)T::elems, n - tile0);
+  const int sub = wave * kWave * kItems + lane;  // this lane's first element of the tile
+  for (int i = threadIdx.x; i < T::waves * kRadix; i += T::threads) (&wcnt[0][0])[i] = 0;
+  K key[kItems];
+  int pay[kItems], pos[kItems];
 #pragma unroll
-    for (int b = 0; b < 8; b++) {
+  for (int i = 0; i < kItems; i++) {
+    const int e = sub + i * kWave;
+    key[i] = e < count ? keys_in[tile0 + e] : (K)0;
+  }
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const int e = sub + i * kWave;
+    pay[i] = pay_in ? (e < count ? pay_in[tile0 + e] : 0) : (int)(tile0 + e);
+  }
+  __syncthreads();
+  // rank of every element among its wave's elements of the same digit
+  const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const bool valid = sub + i * kWave < count;
+    const int d = (int)(key[i] >> shift) & mask;
+    unsigned long long peers = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
       const bool bit = (d >> b) & 1;
       const unsigned long long m = __ballot(bit);
       peers &= bit ? m : ~m;
     }
-    const int rank = __popcll(peers & lanes_below);
-    const int base = valid ? wbase[wave][d] : 0;
-    if (valid) {
-      keys_out[base + rank] = key;
-      pay_out[base + rank] = pay_in[e];
+    const int rank = __popcll(peers & below);
+    const int before = valid ? wcnt[wave][d] : 0;
+    pos[i] = before + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && rank == 0) wcnt[wave][d] = before + __popcll(peers);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  // digit starts within the tile (exclusive scan over digits), wave starts
+  // within each digit; thread d < kRadix owns digit d
+  int total = 0, incl = 0;
+  if (threadIdx.x < kRadix) {
+    for (int w = 0; w < T::waves; w++) {
+      const int c = wcnt[w][threadIdx.x];
+      wcnt[w][threadIdx.x] = total;
+      total += c;
     }
-    __builtin_amdgcn_wave_barrier();
-    if (valid && rank == 0) wbase[wave][d] = base + __popcll(peers);
-    __builtin_amdgcn_wave_barrier();
+    incl = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int o = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += o;
+    }
+    if (lane == kWave - 1) wsum[wave] = incl;
+  }
+  __syncthreads();
+  if (threadIdx.x < kRadix) {
+    int start = incl - total;
+    for (int w = 0; w < wave; w++) start += wsum[w];
+    for (int w = 0; w < T::waves; w++) wcnt[w][threadIdx.x] += start;
+    if ((int)threadIdx.x <= mask)
+      gofs[threadIdx.x] = offsets[(long long)threadIdx.x * ntiles + blockIdx.x] - start;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const int d = (int)(key[i] >> shift) & mask;
+    pos[i] += wcnt[wave][d];
+    if (sub + i * kWave < count) stage[pos[i]] = key[i];
+  }
+  __syncthreads();
+  int dst[kItems];
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const int t = threadIdx.x + i * T::threads;
+    if (t < count) {
+      const K k = stage[t];
+      dst[i] = gofs[(int)(k >> shift) & mask] + t;
+      keys_out[dst[i]] = k;
+    }
+  }
+  __syncthreads();
+  int *pstage = reinterpret_cast<int *>(stage);
+#pragma unroll
+  for (int i = 0; i < kItems; i++)
+    if (sub + i * kWave < count) pstage[pos[i]] = pay[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const int t = threadIdx.x + i * T::threads;
+    if (t < count) pay_out[dst[i]] = pstage[t];
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_iota(int *__restrict__ p, long long n) {
-  long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) p[i] = (int)i;
+// ptr[b] = the first k with (keys[k] >> shift) >= b, for b in [0, nb]: the
+// bucket starts of sorted keys, by binary search (no atomics: counting 24 M
+// banded keys by atomic additions took 1053 us, and 4.8 M with hub rows 317).
+template <typename K>
+__global__ __launch_bounds__(kBlock) void k_bucket_starts(const K *__restrict__ keys, long long n,
+                                                          int shift, long long nb,
+                                                          int *__restrict__ ptr) {
+  const long long b = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (b > nb) return;
+  long long lo = 0, hi = n;
+  while (lo < hi) {
+    const long long mid = (lo + hi) >> 1;
+    if ((long long)(keys[mid] >> shift) < b) lo = mid + 1;
+    else hi = mid;
+  }
+  ptr[b] = (int)lo;
 }
 
+template <typename K>
 __global__ __launch_bounds__(kBlock) void k_coo_keys(const int *__restrict__ rows,
                                                      const int *__restrict__ cols, long long n,
-                                                     int col_bits,
-                                                     unsigned long long *__restrict__ keys) {
+                                                     int col_bits, K *__restrict__ keys) {
   long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) keys[i] = ((unsigned long long)(unsigned)rows[i] << col_bits) | (unsigned)cols[i];
+  if (i < n) keys[i] = ((K)(unsigned)rows[i] << col_bits) | (K)(cols ? (unsigned)cols[i] : 0u);
 }
 
-__global__ __launch_bounds__(kBlock) void k_gather_sorted(const int *__restrict__ perm,
-                                                          const int *__restrict__ cols,
+// columns from the keys' low bits, values by the sorted positions
+template <typename K>
+__global__ __launch_bounds__(kBlock) void k_gather_sorted(const K *__restrict__ keys, int col_bits,
+                                                          const int *__restrict__ perm,
                                                           const double *__restrict__ vals,
                                                           long long n, int *__restrict__ cols_out,
                                                           double *__restrict__ vals_out) {
   long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  int p = perm[i];
-  cols_out[i] = cols[p];
-  vals_out[i] = vals[p];
+  cols_out[i] = (int)(keys[i] & (((K)1 << col_bits) - 1));
+  vals_out[i] = vals[perm[i]];
 }
 
-__global__ __launch_bounds__(kBlock) void k_count_keys(const int *__restrict__ idx, long long n,
-                                                       int *__restrict__ counts) {
-  for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (long long)gridDim.x * kBlock)
-    atomicAdd(counts + idx[i], 1);
-}
-
-__global__ __launch_bounds__(kBlock) void k_max_int(const int *__restrict__ a, long long n,
+// the longest row
+__global__ __launch_bounds__(kBlock) void k_max_row(const int *__restrict__ rowptr, long long n,
                                                     int *__restrict__ out) {
   int m = 0;
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n;
        i += (long long)gridDim.x * kBlock)
-    m = max(m, a[i]);
+    m = max(m, rowptr[i + 1] - rowptr[i]);
   if (m > 0) atomicMax(out, m);
 }
 
@@ -187,16 +285,17 @@ int bits_for(long long v) {
 
 }  // namespace
 
-int radix_sort_pairs(unsigned long long *keys, int *payload, long long n, int key_bits,
-                     hipStream_t s) {
-  if (n <= 1) return TBSLA_HIP_SUCCESS;
-  const long long ntiles = (n + kTileElems - 1) / kTileElems;
-  const long long hist_n = (long long)kRadix * ntiles;
-  unsigned long long *keys_alt = nullptr;
+template <typename K>
+int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s) {
+  typedef SortTile<K> T;
+  if (n <= 0) return TBSLA_HIP_SUCCESS;
+  const long long ntiles = (n + T::elems - 1) / T::elems;
+  const int passes = std::max(1, (key_bits + 7) / 8);
+  const int bits = std::max(1, (key_bits + passes - 1) / passes);
+  const long long hist_n = (1LL << bits) * ntiles;
+  K *keys_alt = nullptr;
   int *pay_alt = nullptr, *hist = nullptr;
   void *ws = nullptr;
-  long long *d_total = nullptr;
-  int st = TBSLA_HIP_SUCCESS;
   auto cleanup = [&]() {
     (void)hipStreamSynchronize(s);
     device_free(keys_alt);
@@ -204,30 +303,24 @@ int radix_sort_pairs(unsigned long long *keys, int *payload, long long n, int ke
     device_free(hist);
     device_free(ws);
   };
-  if ((st = device_alloc((void **)&keys_alt, (size_t)n * 8)) ||
+  int st = TBSLA_HIP_SUCCESS;
+  if ((st = device_alloc((void **)&keys_alt, (size_t)n * sizeof(K))) ||
       (st = device_alloc((void **)&pay_alt, (size_t)n * 4)) ||
       (st = device_alloc((void **)&hist, (size_t)hist_n * 4)) ||
-      (st = device_alloc(&ws, scan_workspace_bytes(hist_n) + 64))) {
+      (st = device_alloc(&ws, scan_workspace_bytes(hist_n)))) {
     cleanup();
     return st;
   }
-  d_total = reinterpret_cast<long long *>(static_cast<char *>(ws) + scan_workspace_bytes(hist_n));
-  unsigned long long *kin = keys, *kout = keys_alt;
-  int *pin = payload, *pout = pay_alt;
-  const int passes = (key_bits + 7) / 8;
-  for (int p = 0; p < passes && st == TBSLA_HIP_SUCCESS; p++) {
-    const int shift = 8 * p;
-    k_digit_hist<<<(unsigned)ntiles, kBlock, 0, s>>>(kin, n, shift, ntiles, hist);
-    st = scan<int>(hist, hist, hist_n, false, d_total, ws, s);
+  for (int p = 0; p < passes; p++) {
+    const int shift = bits * p, b = std::min(bits, std::max(1, key_bits - shift));
+    k_digit_hist<K><<<(unsigned)ntiles, T::threads, 0, s>>>(*keys, n, shift, (1 << b) - 1, ntiles,
+                                                            hist);
+    st = scan<int>(hist, hist, (1LL << b) * ntiles, false, nullptr, ws, s);
     if (st) break;
-    k_digit_scatter<<<(unsigned)ntiles, kBlock, 0, s>>>(kin, pin, kout, pout, n, shift, ntiles,
-                                                        hist);
-    std::swap(kin, kout);
-    std::swap(pin, pout);
-  }
-  if (st == TBSLA_HIP_SUCCESS && kin != keys) {
-    (void)hipMemcpyAsync(keys, kin, (size_t)n * 8, hipMemcpyDeviceToDevice, s);
-    (void)hipMemcpyAsync(payload, pin, (size_t)n * 4, hipMemcpyDeviceToDevice, s);
+    k_digit_scatter<K><<<(unsigned)ntiles, T::threads, 0, s>>>(
+        *keys, p > 0 ? *payload : nullptr, keys_alt, pay_alt, n, shift, b, ntiles, hist);
+    std::swap(*keys, keys_alt);
+    std::swap(*payload, pay_alt);
   }
   hipError_t e = hipGetLastError();
   cleanup();
@@ -236,19 +329,46 @@ int radix_sort_pairs(unsigned long long *keys, int *payload, long long n, int ke
   return TBSLA_HIP_SUCCESS;
 }
 
-// Stable permutation of COO triplets by (row, col) (csr::compare_row,
-// src/cpp/utils/csr.cpp:3-8).  perm receives n ints.
-static int coo_order(const tbsla_hip_matrix_s *coo, int *perm, hipStream_t s) {
-  const long long n = std::min(coo->nnz, coo->stored);
-  unsigned long long *keys = nullptr;
-  TBSLA_TRY(device_alloc((void **)&keys, (size_t)std::max(n, 1LL) * 8));
-  const int col_bits = bits_for(std::max(coo->n_col, 1));
-  const int row_bits = bits_for(std::max(coo->n_row, 1));
-  k_coo_keys<<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, coo->colidx, n, col_bits, keys);
-  k_iota<<<grid_for(n), kBlock, 0, s>>>(perm, n);
-  int st = radix_sort_pairs(keys, perm, n, col_bits + row_bits, s);
+template int radix_sort_pairs<unsigned>(unsigned **, int **, long long, int, hipStream_t);
+template int radix_sort_pairs<unsigned long long>(unsigned long long **, int **, long long, int,
+                                                  hipStream_t);
+
+template <typename K>
+int bucket_starts(const K *keys, long long n, int shift, long long nb, int *ptr, hipStream_t s) {
+  k_bucket_starts<K><<<grid_for(nb + 1), kBlock, 0, s>>>(keys, n, shift, nb, ptr);
+  TBSLA_HIP_LAUNCH_CHECK();
+  return TBSLA_HIP_SUCCESS;
+}
+
+template int bucket_starts<unsigned>(const unsigned *, long long, int, long long, int *,
+                                     hipStream_t);
+template int bucket_starts<unsigned long long>(const unsigned long long *, long long, int,
+                                               long long, int *, hipStream_t);
+
+// The CSR arrays of n COO triplets: stable order by (row, col)
+// (csr::compare_row, src/cpp/utils/csr.cpp:3-8), 32-bit keys where both
+// indices fit.
+template <typename K>
+static int coo_rows(const tbsla_hip_matrix_s *coo, long long n, int row_bits, int col_bits,
+                    int *rowptr, int *cols, double *vals, hipStream_t s) {
+  K *keys = nullptr;
+  int *perm = nullptr;
+  int st;
+  if (!(st = device_alloc((void **)&keys, (size_t)std::max(n, 1LL) * sizeof(K))) &&
+      !(st = device_alloc((void **)&perm, (size_t)std::max(n, 1LL) * 4))) {
+    if (n > 0)
+      k_coo_keys<K><<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, coo->colidx, n, col_bits, keys);
+    st = radix_sort_pairs<K>(&keys, &perm, n, col_bits + row_bits, s);
+    if (!st) st = bucket_starts<K>(keys, n, col_bits, coo->n_row, rowptr, s);
+    if (!st && n > 0)
+      k_gather_sorted<K><<<grid_for(n), kBlock, 0, s>>>(keys, col_bits, perm, coo->values, n, cols,
+                                                        vals);
+    const hipError_t e = hipGetLastError();
+    if (!st && e != hipSuccess) st = fail(TBSLA_HIP_ERR_HIP, hipGetErrorString(e));
+  }
   (void)hipStreamSynchronize(s);
   device_free(keys);
+  device_free(perm);
   return st;
 }
 
@@ -305,44 +425,42 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
     return TBSLA_HIP_SUCCESS;
   }
 
-  // row pointers from the row counts; stable (row, col) order
-  int *rowptr = nullptr, *perm = nullptr;
+  int *rowptr = nullptr;
   TBSLA_TRY(device_alloc((void **)&rowptr, (size_t)(rows + 1) * 4));
-  TBSLA_TRY(device_alloc((void **)&perm, (size_t)std::max(n, 1LL) * 4));
-  TBSLA_HIP_CHECK(hipMemsetAsync(rowptr, 0, (size_t)(rows + 1) * 4, s));
-  if (n > 0) {
-    k_count_keys<<<stride_grid(n), kBlock, 0, s>>>(coo->rowidx, n, rowptr + 1);
-    TBSLA_HIP_LAUNCH_CHECK();
-  }
-  TBSLA_TRY(ensure_scratch(dst, scan_workspace_bytes(rows) + 256));
-  TBSLA_TRY(scan<int>(rowptr + 1, rowptr + 1, rows, true,
-                      reinterpret_cast<long long *>(dst->scratch),
-                      static_cast<char *>(dst->scratch) + 256, s));
   if (format == TBSLA_HIP_DENSE) {
     // DENSE needs only a stable row order (cells add in COO order)
-    if (n > 0) {
-      unsigned long long *keys = nullptr;
-      TBSLA_TRY(device_alloc((void **)&keys, (size_t)n * 8));
-      k_coo_keys<<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, coo->rowidx, n, 0, keys);
-      k_iota<<<grid_for(n), kBlock, 0, s>>>(perm, n);
-      // key = row only (col_bits 0 and row OR row == row)
-      int st = radix_sort_pairs(keys, perm, n, bits_for(std::max(coo->n_row, 1)), s);
+    unsigned *keys = nullptr;
+    int *perm = nullptr;
+    auto drop = [&]() {
       (void)hipStreamSynchronize(s);
       device_free(keys);
-      if (st) return st;
-    }
+      device_free(perm);
+      device_free(rowptr);
+    };
     const size_t cells = (size_t)rows * (size_t)dst->ln_col;
-    TBSLA_TRY(device_alloc((void **)&dst->values, std::max<size_t>(cells, 1) * 8));
+    int st;
+    if ((st = device_alloc((void **)&keys, (size_t)std::max(n, 1LL) * 4)) ||
+        (st = device_alloc((void **)&perm, (size_t)std::max(n, 1LL) * 4)) ||
+        (st = device_alloc((void **)&dst->values, std::max<size_t>(cells, 1) * 8))) {
+      drop();
+      return st;
+    }
+    if (n > 0)
+      k_coo_keys<unsigned><<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, nullptr, n, 0, keys);
+    if ((st = radix_sort_pairs<unsigned>(&keys, &perm, n, bits_for(std::max(coo->n_row, 1)), s)) ||
+        (st = bucket_starts<unsigned>(keys, n, 0, rows, rowptr, s))) {
+      drop();
+      return st;
+    }
     k_zero_d<<<stride_grid((long long)cells), kBlock, 0, s>>>(dst->values, (long long)cells);
     if (rows > 0)
       k_rows_to_dense<<<grid_for(rows), kBlock, 0, s>>>(rows, dst->ln_col, rowptr, perm,
                                                         coo->colidx, coo->values, dst->values);
-    TBSLA_HIP_LAUNCH_CHECK();
+    const hipError_t e = hipGetLastError();
+    drop();
+    if (e != hipSuccess) return fail(TBSLA_HIP_ERR_HIP, hipGetErrorString(e));
     dst->stored = (long long)cells;
     dst->has_arrays = 1;
-    TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-    device_free(perm);
-    device_free(rowptr);
     return TBSLA_HIP_SUCCESS;
   }
 
@@ -350,13 +468,20 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
   double *sval = nullptr;
   TBSLA_TRY(device_alloc((void **)&scol, (size_t)std::max(n, 1LL) * 4));
   TBSLA_TRY(device_alloc((void **)&sval, (size_t)std::max(n, 1LL) * 8));
-  if (n > 0) {
-    TBSLA_TRY(coo_order(coo, perm, s));
-    k_gather_sorted<<<grid_for(n), kBlock, 0, s>>>(perm, coo->colidx, coo->values, n, scol, sval);
-    TBSLA_HIP_LAUNCH_CHECK();
+  {
+    const int col_bits = bits_for(std::max(coo->n_col, 1));
+    const int row_bits = bits_for(std::max(coo->n_row, 1));
+    const int st = col_bits + row_bits <= 32
+                       ? coo_rows<unsigned>(coo, n, row_bits, col_bits, rowptr, scol, sval, s)
+                       : coo_rows<unsigned long long>(coo, n, row_bits, col_bits, rowptr, scol,
+                                                      sval, s);
+    if (st) {
+      device_free(rowptr);
+      device_free(scol);
+      device_free(sval);
+      return st;
+    }
   }
-  (void)hipStreamSynchronize(s);
-  device_free(perm);
   if (format == TBSLA_HIP_CSR) {
     dst->rowptr = rowptr;
     dst->colidx = scol;
@@ -366,18 +491,13 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
     return TBSLA_HIP_SUCCESS;
   }
   // ELL: width = longest row
+  TBSLA_TRY(ensure_scratch(dst, 256));
   int *d_w = reinterpret_cast<int *>(dst->scratch);
   TBSLA_HIP_CHECK(hipMemsetAsync(d_w, 0, 4, s));
-  // row lengths = rowptr differences: recount into a temporary
-  int *lens = nullptr;
-  TBSLA_TRY(device_alloc((void **)&lens, (size_t)std::max(rows, 1LL) * 4));
-  TBSLA_HIP_CHECK(hipMemsetAsync(lens, 0, (size_t)std::max(rows, 1LL) * 4, s));
-  k_count_keys<<<stride_grid(n), kBlock, 0, s>>>(coo->rowidx, n, lens);
-  k_max_int<<<stride_grid(rows), kBlock, 0, s>>>(lens, rows, d_w);
+  k_max_row<<<stride_grid(rows), kBlock, 0, s>>>(rowptr, rows, d_w);
   int width = 0;
   TBSLA_HIP_CHECK(hipMemcpyAsync(&width, d_w, 4, hipMemcpyDeviceToHost, s));
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-  device_free(lens);
   dst->max_col = width;
   const size_t slots = (size_t)rows * (size_t)width;
   TBSLA_TRY(device_alloc((void **)&dst->colidx, std::max<size_t>(slots, 1) * 4));

@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_split_fill(
     const int *__restrict__ ci, const double *__restrict__ v, const int *__restrict__ dmap,
     int ndiag, const int *__restrict__ lrp, const int *__restrict__ rptr, int *__restrict__ lci,
     double *__restrict__ lv, double *__restrict__ dv, int *__restrict__ rc,
-    double *__restrict__ rv, unsigned long long *__restrict__ keys, int *__restrict__ payload,
+    double *__restrict__ rv, unsigned long long *__restrict__ keys,
     int *__restrict__ scount) {
   for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r < n;
        r += (long long)gridDim.x * kBlock) {
@@ -315,7 +315,6 @@ __global__ __launch_bounds__(kBlock) void k_split_fill(
         rc[pr] = (int)c;
         rv[pr] = val;
         keys[pr] = (s << rb) | (unsigned long long)r;
-        payload[pr] = pr;
         atomicAdd(scount + s, 1);
         pr++;
       }
@@ -991,7 +990,7 @@ int split_build(tbsla_hip_matrix_s *m, int window, int slices, hipStream_t s, in
   const int rb = bits_of(std::max(n, 1LL));
   k_split_fill<<<sgrid(n), kBlock, 0, s>>>(n, nc, f_col, lr.r0, window, slices,
                                            H > 0 ? kSliceCols : 0, rb, src, m->colidx, m->values, dmap, sp->ndiag, sp->lrp,
-                                           rptr, sp->lci, sp->lv, sp->dv, rc, rv, keys, pay, scount);
+                                           rptr, sp->lci, sp->lv, sp->dv, rc, rv, keys, scount);
   if (H > 0) {
     const int S = s_lds, R = (int)((n + H - 1) / H);
     sp->lds_h = H;
@@ -1009,7 +1008,8 @@ int split_build(tbsla_hip_matrix_s *m, int window, int slices, hipStream_t s, in
         (st = device_alloc((void **)&sp->pb, (size_t)(R + 1) * 4)) ||
         (st = device_alloc((void **)&sp->rs16, (size_t)R * (size_t)(H + 1) * 2)))
       return failed(st);
-    if (sp->nr > 1 && (st = radix_sort_pairs(keys, pay, sp->nr, rb + bits_of(S), s))) return failed(st);
+    if ((st = radix_sort_pairs<unsigned long long>(&keys, &pay, sp->nr, rb + bits_of(S), s)))
+      return failed(st);
     k_slice_place<<<sgrid(sp->nr), kBlock, 0, s>>>(sp->nr, keys, rb, H, pay, rc, rv, sp->c16,
                                                    sp->q16, sp->sv);
     k_block_starts<<<sgrid(R + 1), kBlock, 0, s>>>(n, H, R, rptr, sp->pb);
@@ -1030,7 +1030,8 @@ int split_build(tbsla_hip_matrix_s *m, int window, int slices, hipStream_t s, in
       // P, followed by the device copy of the slice offsets
       (st = device_alloc((void **)&sp->P, (size_t)nr1 * 8 + (size_t)(slices + 1) * 8)))
     return failed(st);
-  if (sp->nr > 1 && (st = radix_sort_pairs(keys, pay, sp->nr, rb + bits_of(slices), s))) return failed(st);
+  if ((st = radix_sort_pairs<unsigned long long>(&keys, &pay, sp->nr, rb + bits_of(slices), s)))
+    return failed(st);
   if (sp->nr > 0)
     k_split_place<<<sgrid(sp->nr), kBlock, 0, s>>>(sp->nr, keys, rb, pay, rc, rv, sp->sr, sp->sc,
                                                    sp->sv);
