@@ -77,20 +77,55 @@ struct CqmatParams {
   uint64_t nr, nc, c, nfull;  // nfull = min(nc - c + 1, nr)
   double q;
   uint32_t seed_mult;
+  // the tests on q as tests on the draw (set_q): a full row's entry is rewired
+  // when draw < below; a tail row's when tail0 (draw < RAND_MAX) or tail1
+  int64_t below;
+  int tail0, tail1;
+  // draw / RAND_MAX < q is monotone in the draw: `below` is the first draw that
+  // fails it, found with the reference's own expression (:36)
+  void set_q(double q_) {
+    q = q_;
+    int64_t lo = 0, hi = (int64_t)2147483647 + 1;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) / 2;
+      if ((double)mid / 2147483647.0 < q) lo = mid + 1;
+      else hi = mid;
+    }
+    below = lo;
+    tail0 = 0.0 < q;
+    tail1 = 1.0 < q;
+  }
 };
+
+// column of a tail row's entry (row cur, position it): integer division, as
+// the reference (:45), so the draw matters only at RAND_MAX
+__host__ __device__ inline int64_t cqmat_tail_col(const CqmatParams &p, uint32_t seed, uint64_t cur,
+                                                  uint64_t it) {
+  const int draw = rand_r32(seed);
+  if (draw == 2147483647 ? p.tail1 : p.tail0)
+    return (int64_t)((uint32_t)rand_r32(seed) % (uint32_t)p.nc);
+  return (int64_t)(cur + it);
+}
+
+// column of a full row's entry j of row r
+__host__ __device__ inline int64_t cqmat_full_col(const CqmatParams &p, uint32_t seed, uint64_t r,
+                                                  uint64_t j) {
+  const int draw = rand_r32(seed);
+  if (draw < p.below) return (int64_t)((uint32_t)rand_r32(seed) % (uint32_t)p.nc);
+  return (int64_t)(r + j);
+}
+
+__host__ __device__ inline uint32_t cqmat_seed(const CqmatParams &p, uint64_t k) {
+  return p.seed_mult > 0 ? (uint32_t)((uint64_t)p.seed_mult * k) : (uint32_t)k;
+}
 
 __host__ __device__ inline void cqmat_decode(const CqmatParams &p, uint64_t k, int64_t &row,
                                              int64_t &col) {
-  uint32_t seed = (uint32_t)k;
-  if (p.seed_mult > 0) seed = (uint32_t)((uint64_t)p.seed_mult * k);
+  const uint32_t seed = cqmat_seed(p, k);
   if (k < p.c * p.nfull) {
-    uint64_t r = k / p.c;
-    int draw = rand_r32(seed);
+    const uint64_t r = k / p.c;
     row = (int64_t)r;
-    if ((double)draw / 2147483647.0 < p.q)
-      col = (int64_t)((uint64_t)rand_r32(seed) % p.nc);
-    else
-      col = (int64_t)(r + k % p.c);
+    col = cqmat_full_col(p, seed, r, k - r * p.c);
   } else {
     uint64_t it = k - p.c * p.nfull;
     uint64_t cur = 1;
@@ -99,13 +134,8 @@ __host__ __device__ inline void cqmat_decode(const CqmatParams &p, uint64_t k, i
       cur++;
     }
     cur += p.nfull - 1;
-    int draw = rand_r32(seed);
     row = (int64_t)cur;
-    // integer division, as the reference (:45): true for every draw < RAND_MAX
-    if ((double)(draw / 2147483647) < p.q)
-      col = (int64_t)((uint64_t)rand_r32(seed) % p.nc);
-    else
-      col = (int64_t)(cur + it);
+    col = cqmat_tail_col(p, seed, cur, it);
   }
 }
 

@@ -132,6 +132,101 @@ __global__ __launch_bounds__(kBlock) void k_cqmat_fill_rows(CqmatBlock b, const 
   }
 }
 
+// ---- blocks as wide as the matrix -----------------------------------------
+//
+// A block with every column (f_col = 0, ln_col = n_col) holds every entry its
+// rows generate: the row pointer is arithmetic on the generator indices and
+// entry e of the block is generator index incr + e, so nothing is counted and
+// consecutive lanes write consecutive entries.  Bound by the integer work (some
+// 150 instructions an entry: the rand_r steps and the value's two 64-bit
+// multiplications) beside 12 bytes written; n = 1.5 M, c = 16: 62 us with its
+// row pointer, against 75 (counts) + 300 with a thread walking each row.
+
+// x / d for 32-bit x by a precomputed multiplication (Granlund and Montgomery,
+// "Division by invariant integers using multiplication", PLDI 1994, figure 4.1)
+struct Div32 {
+  uint32_t mul, sh1, sh2;
+};
+
+Div32 make_div32(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32 && (1ull << l) < d) l++;
+  Div32 r;
+  r.mul = (uint32_t)((((1ull << l) - d) << 32) / d + 1);
+  r.sh1 = l < 1 ? l : 1;
+  r.sh2 = l < 1 ? 0 : l - 1;
+  return r;
+}
+
+__device__ inline uint32_t div32(uint32_t x, const Div32 &d) {
+  const uint32_t t = __umulhi(d.mul, x);
+  return (t + ((x - t) >> d.sh1)) >> d.sh2;
+}
+
+__global__ __launch_bounds__(kBlock) void k_cqmat_rowptr(CqmatBlock b, int *__restrict__ offs) {
+  const long long r = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (r > b.ln_row) return;
+  const long long i = b.f_row + r;
+  long long k0, cnt;
+  row_range(b, i, k0, cnt);
+  offs[r] = r < b.ln_row && i < b.row_end ? (int)(k0 - b.incr) : (int)b.nv;
+}
+
+constexpr int kFillItems = 4;  // consecutive entries per thread: 16-byte stores
+
+__global__ __launch_bounds__(kBlock) void k_cqmat_fill_wide(CqmatBlock b, Div32 by_cc, long long n,
+                                                            long long nfull, int *__restrict__ rows,
+                                                            int *__restrict__ cols,
+                                                            double *__restrict__ vals, int unit,
+                                                            uint64_t seed_hash) {
+  typedef int intx4 __attribute__((ext_vector_type(4)));
+  typedef double doublex2 __attribute__((ext_vector_type(2)));
+  const long long e0 = ((long long)blockIdx.x * kBlock + threadIdx.x) * kFillItems;
+  if (e0 >= n) return;
+  int row[kFillItems], col[kFillItems];
+  double val[kFillItems];
+  const uint64_t k0 = (uint64_t)(b.incr + e0);
+  if (e0 + kFillItems <= nfull) {
+    uint32_t r = div32((uint32_t)e0, by_cc);
+    uint32_t j = (uint32_t)e0 - r * (uint32_t)b.cc;
+#pragma unroll
+    for (int k = 0; k < kFillItems; k++) {
+      const uint64_t gr = (uint64_t)b.f_row + r;
+      row[k] = (int)gr;
+      col[k] = (int)cqmat_full_col(b.p, cqmat_seed(b.p, k0 + k), gr, j);
+      if (++j == (uint32_t)b.cc) {
+        j = 0;
+        r++;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < kFillItems; k++) {
+      row[k] = col[k] = 0;
+      if (e0 + k < n) {
+        int64_t ii, jj;
+        cqmat_decode(b.p, k0 + k, ii, jj);
+        row[k] = (int)ii;
+        col[k] = (int)jj;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kFillItems; k++) val[k] = entry_value(unit, seed_hash, (long long)k0 + k);
+  if (e0 + kFillItems <= n) {
+    *reinterpret_cast<intx4 *>(cols + e0) = intx4{col[0], col[1], col[2], col[3]};
+    if (rows) *reinterpret_cast<intx4 *>(rows + e0) = intx4{row[0], row[1], row[2], row[3]};
+    *reinterpret_cast<doublex2 *>(vals + e0) = doublex2{val[0], val[1]};
+    *reinterpret_cast<doublex2 *>(vals + e0 + 2) = doublex2{val[2], val[3]};
+  } else {
+    for (int k = 0; k < (int)(n - e0); k++) {
+      cols[e0 + k] = col[k];
+      if (rows) rows[e0 + k] = row[k];
+      vals[e0 + k] = val[k];
+    }
+  }
+}
+
 // ELL (MatrixELL.cpp:426-465), column-major slots; padding (col 0, value 0).
 __global__ __launch_bounds__(kBlock) void k_cqmat_fill_ell(CqmatBlock b, int max_col,
                                                            int *__restrict__ cols,
@@ -304,22 +399,18 @@ void set_geometry(tbsla_hip_matrix_s *m, int n_row, int n_col, int pr, int pc, i
   m->f_col = (int)pflv(n_col, pc, NC);
 }
 
-// MatrixCSR.cpp:393-417 (identical loops in every format).
+// MatrixCSR.cpp:393-417 (identical loops in every format), summed in closed
+// form: cc entries for each of the first min_ rows, cc - 1 - u for tail row u.
 void prescan(long long n_row, long long n_col, long long cc, long long f_row, long long ln_row,
              long long &incr, long long &nv) {
-  long long min_ = std::min(n_col - cc + 1, n_row);
-  incr = 0;
-  nv = 0;
-  for (long long i = 0; i < min_; i++) {
-    if (i < f_row) incr += cc;
-    if (i >= f_row && i < f_row + ln_row) nv += cc;
-    if (i >= f_row + ln_row) break;
-  }
-  for (long long i = 0; i < std::min(n_row, n_col) - min_; i++) {
-    if (i + min_ < f_row) incr += cc - i - 1;
-    if (i + min_ >= f_row && i + min_ < f_row + ln_row) nv += cc - i - 1;
-    if (i + min_ >= f_row + ln_row) break;
-  }
+  const long long min_ = std::min(n_col - cc + 1, n_row);
+  const long long tails = std::max<long long>(0, std::min(n_row, n_col) - min_);
+  auto before = [&](long long row) {  // entries of the rows before `row`
+    return cc * std::min(row, min_) +
+           tail_prefix(cc, std::min(std::max<long long>(0, row - min_), tails));
+  };
+  incr = before(f_row);
+  nv = before(f_row + ln_row) - incr;
 }
 
 CqmatBlock make_block(const tbsla_hip_matrix_s *m, int c, double q, unsigned seed_mult) {
@@ -329,7 +420,7 @@ CqmatBlock make_block(const tbsla_hip_matrix_s *m, int c, double q, unsigned see
   b.p.nc = (uint64_t)m->n_col;
   b.p.c = (uint64_t)cc;
   b.p.nfull = (uint64_t)std::min<long long>((long long)m->n_col - cc + 1, m->n_row);
-  b.p.q = q;
+  b.p.set_q(q);
   b.p.seed_mult = seed_mult;
   b.f_row = m->f_row;
   b.ln_row = m->ln_row;
@@ -446,7 +537,7 @@ extern "C" int tbsla_hip_fill_cqmat(tbsla_hip_matrix_t m, int n_row, int n_col, 
     p.nc = (uint64_t)n_col;
     p.c = (uint64_t)cc;
     p.nfull = (uint64_t)full;
-    p.q = q;
+    p.set_q(q);
     p.seed_mult = seed_mult;
     k_cqmat_fill_coo<<<grid_for(n), kBlock, 0, s>>>(p, st, n, m->rowidx, m->colidx, m->values,
                                                      unit, seed_hash);
@@ -465,7 +556,35 @@ extern "C" int tbsla_hip_fill_cqmat(tbsla_hip_matrix_t m, int n_row, int n_col, 
   const long long walk_end = b.incr + std::max<long long>(0, b.row_end - b.f_row) * b.cc;
   unsigned long long *d_counter = nullptr;
 
-  // per-row in-block counts (every format needs them)
+  // a CSR or SCOO block with every column: no counts (see k_cqmat_fill_wide)
+  if ((fmt == TBSLA_HIP_CSR || fmt == TBSLA_HIP_SCOO) && b.nv > 0 && ln_row > 0 && m->f_col == 0 &&
+      m->ln_col == m->n_col && b.nv <= INT32_MAX) {
+    long long extra = 0;
+    if (fmt == TBSLA_HIP_CSR) {
+      TBSLA_TRY(fill_scratch(m, 0));
+      // nnz field: as below
+      TBSLA_TRY(count_range(b, b.incr + b.nv, walk_end, extra, scratch_counter(m), s));
+      TBSLA_TRY(device_alloc((void **)&m->rowptr, (size_t)(ln_row + 1) * sizeof(int)));
+      k_cqmat_rowptr<<<grid_for(ln_row + 1), kBlock, 0, s>>>(b, m->rowptr);
+      TBSLA_HIP_LAUNCH_CHECK();
+    } else {
+      TBSLA_TRY(device_alloc((void **)&m->rowidx, (size_t)b.nv * sizeof(int)));
+    }
+    TBSLA_TRY(device_alloc((void **)&m->colidx, (size_t)b.nv * sizeof(int)));
+    TBSLA_TRY(device_alloc((void **)&m->values, (size_t)b.nv * sizeof(double)));
+    const long long nfull = std::max<long long>(0, b.full_end - b.f_row) * b.cc;
+    k_cqmat_fill_wide<<<grid_for((b.nv + kFillItems - 1) / kFillItems), kBlock, 0, s>>>(
+        b, make_div32((uint32_t)b.cc), b.nv, nfull, m->rowidx, m->colidx, m->values, unit,
+        seed_hash);
+    TBSLA_HIP_LAUNCH_CHECK();
+    TBSLA_HIP_CHECK(hipStreamSynchronize(s));
+    m->nnz = b.nv + extra;
+    m->stored = b.nv;
+    m->has_arrays = 1;
+    return TBSLA_HIP_SUCCESS;
+  }
+
+  // per-row in-block counts (every other block needs them)
   int *offs = nullptr;
   TBSLA_TRY(device_alloc((void **)&offs, (size_t)(ln_row + 1) * sizeof(int)));
   int *d_width = nullptr;
