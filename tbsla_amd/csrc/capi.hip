@@ -649,9 +649,9 @@ int tbsla_hip_set_csr_schedule(tbsla_hip_matrix_t m, int lanes, int rows) {
 
 int tbsla_hip_get_csr_schedule(tbsla_hip_matrix_t m, int *lanes, int *rows) {
   if (!m) return fail(TBSLA_HIP_ERR_INVALID, "null matrix handle");
-  int L = pick_csr_lanes(m);
-  if (lanes) *lanes = L;
-  if (rows) *rows = pick_csr_rows(m, L);
+  const CsrKernel k = pick_csr(m);
+  if (lanes) *lanes = k.L;
+  if (rows) *rows = k.R;
   return TBSLA_HIP_SUCCESS;
 }
 
@@ -672,11 +672,11 @@ int tbsla_hip_set_csr_kernel(tbsla_hip_matrix_t m, int lanes, int rows, int vec,
 int tbsla_hip_get_csr_kernel(tbsla_hip_matrix_t m, int *lanes, int *rows, int *vec,
                              int *nontemporal) {
   if (!m) return fail(TBSLA_HIP_ERR_INVALID, "null matrix handle");
-  const int L = pick_csr_lanes(m);
-  if (lanes) *lanes = L;
-  if (rows) *rows = pick_csr_rows(m, L);
-  if (vec) *vec = pick_csr_vec(m);
-  if (nontemporal) *nontemporal = pick_csr_nt(m);
+  const CsrKernel k = pick_csr(m);
+  if (lanes) *lanes = k.L;
+  if (rows) *rows = k.R;
+  if (vec) *vec = k.V;
+  if (nontemporal) *nontemporal = k.NT;
   return TBSLA_HIP_SUCCESS;
 }
 

@@ -18,10 +18,13 @@ size_t scan_workspace_bytes(long long n);
 int spmv_launch(tbsla_hip_matrix_s *m, double *d_r, const double *d_v, int vect_incr,
                 bool zero_first, hipStream_t s, const int *d_done = nullptr,
                 const int *seg_offs = nullptr, int nseg = 0, const int *seg_done = nullptr);
-int pick_csr_lanes(const tbsla_hip_matrix_s *m);
-int pick_csr_rows(const tbsla_hip_matrix_s *m, int lanes);
-int pick_csr_vec(const tbsla_hip_matrix_s *m);
-int pick_csr_nt(const tbsla_hip_matrix_s *m);
+// the CSR row kernel (csr_rows.hpp) of a block: what was set on the handle,
+// else csr_default of its mean row length
+struct CsrKernel {
+  int V, L, R, NT;
+};
+CsrKernel csr_default(double mean, double entries);
+CsrKernel pick_csr(const tbsla_hip_matrix_s *m);
 
 // vec.hip
 int launch_fill(double *d, long long n, double v, hipStream_t s);

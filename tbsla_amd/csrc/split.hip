@@ -829,8 +829,8 @@ int split_launch(tbsla_hip_matrix_s *m, double *y, const double *x, const int *d
                                                          sp->sr, sp->P, sp->R, done);
   // the near-diagonal entries with the block's CSR schedule, plus R[row]
   CsrRowsArgs a{n, sp->lrp, sp->lci, sp->lv, x, 0, y, done, sp->R};
-  const int L = pick_csr_lanes(m);
-  csr_rows_launch<true>(a, pick_csr_vec(m), L, pick_csr_rows(m, L), pick_csr_nt(m), s);
+  const CsrKernel k = pick_csr(m);
+  csr_rows_launch<true>(a, k.V, k.L, k.R, k.NT, s);
   TBSLA_HIP_LAUNCH_CHECK();
   return TBSLA_HIP_SUCCESS;
 }

@@ -278,8 +278,6 @@ int launch_axpy_inplace(double *y, const double *x, long long n, hipStream_t s) 
   return TBSLA_HIP_SUCCESS;
 }
 
-// Lanes per row from the mean row length (two entries per lane per row,
-// clamped to 1..64) unless set; rows per group from the lanes.
 // The row pointer of a row-sorted COO/SCOO block (built once; false when
 // the triplets turn out not to be sorted, which also clears row_sorted).
 int coo_rowptr(tbsla_hip_matrix_s *m, long long n, bool *ok, hipStream_t s) {
@@ -330,23 +328,41 @@ int coo_rowptr(tbsla_hip_matrix_s *m, long long n, bool *ok, hipStream_t s) {
   return TBSLA_HIP_SUCCESS;
 }
 
-int pick_csr_lanes(const tbsla_hip_matrix_s *m) {
-  if (m->lanes_per_row > 0) return m->lanes_per_row;
-  double mean = m->ln_row > 0 ? (double)m->stored / m->ln_row : 1.0;
-  int L = 1;
-  while (L < 64 && L < mean / 2) L <<= 1;
-  return L;
+// The row kernel for a mean row length.  Every compiled kernel was timed on
+// cqmats (q = 0.1) of 20,000 to 2.5 M rows with 3 to 34 entries, three matrices
+// in turn; the line lies where the neighbours meet, and each choice is within
+// 6 % of the best at 10^6 rows.  A quad of entries per lane (V = 4) makes a
+// row's lines whole per instruction, and pays from ten entries on; below, the
+// quads of short rows are mostly slack.  One million rows, against V = 1 with
+// two entries per lane, four rows in flight and the non-temporal hint (the rule
+// before): 5 entries 32 -> 22 us, 8: 44 -> 29, 12: 63 -> 40, 17: 99 -> 72, 24:
+// 109 -> 73, 34: 183 -> 120.  The hint pays (3 to 5 %) only where the entries
+// are more than the 256 MB MALL keeps from one product to the next, and not for
+// short rows, whose lines are shared between instructions.
+CsrKernel csr_default(double mean, double entries) {
+  const int nt = 12.0 * entries > 256e6 && mean >= 8 ? 1 : 0;
+  if (mean < 2.5) return {1, mean <= 2 ? 1 : 2, 4, 1};  // hypersparse: not timed, as before
+  if (mean < 4) return {1, 4, 2, nt};
+  if (mean < 10) return {2, 4, 2, nt};
+  if (mean < 15) return {4, 4, 2, nt};
+  if (mean < 20) return {4, 4, 1, nt};
+  if (mean < 28) return {4, 8, 2, nt};
+  if (mean < 48) return {4, 8, 1, nt};
+  if (mean < 128) return {4, 16, 1, nt};
+  return {1, 64, 1, 1};  // long rows: a wavefront per row, as before
 }
 
-int pick_csr_rows(const tbsla_hip_matrix_s *m, int L) {
-  if (m->rows_per_group > 0) return m->rows_per_group;
-  return L >= 64 ? 1 : (L >= 32 ? 2 : 4);
+CsrKernel pick_csr(const tbsla_hip_matrix_s *m) {
+  const double mean = m->ln_row > 0 ? (double)m->stored / m->ln_row : 1.0;
+  if (m->lanes_per_row <= 0 && m->rows_per_group <= 0) return csr_default(mean, (double)m->stored);
+  int L = m->lanes_per_row;
+  if (L <= 0) {
+    L = 1;
+    while (L < 64 && L < mean / 2) L <<= 1;
+  }
+  const int R = m->rows_per_group > 0 ? m->rows_per_group : (L >= 64 ? 1 : (L >= 32 ? 2 : 4));
+  return {m->csr_vec > 0 ? m->csr_vec : 1, L, R, m->csr_nt >= 0 ? m->csr_nt : 1};
 }
-
-// entries per lane load (1 unless set) and the non-temporal load hint (on
-// unless set)
-int pick_csr_vec(const tbsla_hip_matrix_s *m) { return m->csr_vec > 0 ? m->csr_vec : 1; }
-int pick_csr_nt(const tbsla_hip_matrix_s *m) { return m->csr_nt >= 0 ? m->csr_nt : 1; }
 
 // Scratch of the segmented COO/SCOO accumulation of n row-sorted triplets:
 // each chunk's head and tail keys (int) and values (double).
@@ -388,8 +404,8 @@ int spmv_launch(tbsla_hip_matrix_s *m, double *d_r, const double *d_v, int vect_
       if (m->split) return split_launch(m, d_r, d_v, d_done, s);
       CsrRowsArgs a{m->ln_row, m->rowptr, m->colidx, m->values, d_v, m->f_col, d_r, d_done,
                     nullptr, seg_offs, nseg, seg_done};
-      const int L = pick_csr_lanes(m);
-      csr_rows_launch<false>(a, pick_csr_vec(m), L, pick_csr_rows(m, L), pick_csr_nt(m), s);
+      const CsrKernel k = pick_csr(m);
+      csr_rows_launch<false>(a, k.V, k.L, k.R, k.NT, s);
       TBSLA_HIP_LAUNCH_CHECK();
       return TBSLA_HIP_SUCCESS;
     }
@@ -422,18 +438,11 @@ int spmv_launch(tbsla_hip_matrix_s *m, double *d_r, const double *d_v, int vect_
         return split_launch(m, d_r + ((long long)m->coo_row0 + row_off), d_v, nullptr, s);
       if (rows_ok) {
         // y is zero: the row kernel's stores over the triplets' row range
-        // equal the accumulation.  V from the mean row length, L the
-        // fewest lanes whose V L entries cover a mean row in one trip.
-        const double mean = (double)n / m->coo_nrows;
-        int V = mean >= 16 ? 4 : (mean >= 6 ? 2 : 1);
-        int L = 1;
-        while (L < 64 && L * V < mean) L <<= 1;
-        if (V == 2) L = std::min(std::max(L, 4), 32);
-        if (V == 4) L = std::min(std::max(L, 4), 16);
-        const int R = V > 1 ? 1 : (L >= 64 ? 1 : (L >= 32 ? 2 : 4));
+        // equal the accumulation.
+        const CsrKernel k = csr_default((double)n / m->coo_nrows, (double)n);
         CsrRowsArgs a{m->coo_nrows, m->coo_rowptr, m->colidx, m->values, d_v, -col_off,
                       d_r + ((long long)m->coo_row0 + row_off), nullptr, nullptr};
-        csr_rows_launch<false>(a, V, L, R, 1, s);
+        csr_rows_launch<false>(a, k.V, k.L, k.R, k.NT, s);
         TBSLA_HIP_LAUNCH_CHECK();
         return TBSLA_HIP_SUCCESS;
       }
