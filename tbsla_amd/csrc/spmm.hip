@@ -1,13 +1,13 @@
 // spmm.hip -- C = A B (MatrixCSR::dense_multiply) and personalised PageRank
 // over k teleport vectors as one SpMM per iteration.
 //
-// One wavefront per row, lane t owning columns t, t+64, ... of the dense
-// operands (row-major n x k).  A row's (column, value) pairs are
-// wave-uniform and come through the scalar cache; each nonzero reads one
-// contiguous k-double row of B.  Products are added in the row's storage
-// order with separate multiply and add (no FMA), so C is bit-identical to
-// the reference's loop (src/mpi/matrix/MatrixCSR.cpp:11-30).
+// The product takes the columns of the dense operands (row-major n x k) in
+// chunks (k_csr_spmm).  Products are added in the row's storage order with
+// separate multiply and add (no FMA), so C is bit-identical to the reference's
+// loop (src/mpi/matrix/MatrixCSR.cpp:11-30).
 #include <algorithm>
+#include <climits>
+#include <cstdint>
 #include <type_traits>
 #include <vector>
 
@@ -18,72 +18,138 @@ namespace tbsla_hip {
 
 namespace {
 
-constexpr int kMaxTiles = 4;  // columns per launch row: 256; wider B in chunks (grid y)
+// C = A B.  A group of LPR lanes takes one row and one chunk of LPR V columns (V
+// doubles per lane load), up to eight entries' pieces of B in flight.  Every
+// entry gathers its row's chunk of B, so the kernel is bound by where those come
+// from, and the chunk is narrow: 32 columns (256 bytes, two lines) keep the
+// chunk's slice of B small enough to be met again in a cache.  Chunks are the
+// outer order of the grid: the whole chip works on one slice (MALL: 51 MB at
+// 200,003 columns, where whole rows of 512 doubles are 819 MB).  Up to
+// kSpmmXcdCols columns, whose slices are a few times an XCD's 4 MB L2 at most,
+// each XCD (workgroup b runs on XCD b mod 8) takes its own chunks instead,
+// when the chunks divide evenly.  Ten random columns per row, k = 512, whole
+// rows against this: n = 5,003: 28 -> 14 us, 20,011: 114 -> 65, 50,021: 308 ->
+// 245, 100,003: 648 -> 579, 200,003: 1229 -> 1091 (7.5 TB/s gathered); a chunk
+// of 16 columns took 81, 297, 670 and 1380 (one line per gather).  C is written
+// past the caches (1 to 5 %): nothing here reads it again.
+struct SpmmArgs {
+  long long n_rows;
+  int k, f_col, ln_col;
+  const int *rowptr;
+  const int *colidx;
+  const double *vals;
+  const double *B;
+  double *C;
+  unsigned nchunks;  // column chunks
+  unsigned rblocks;  // row blocks
+  int xcd;           // chunks dealt to the XCDs (one-dimensional grid)
+  unsigned chunk0;   // else: grid y is the chunk, from here on
+};
 
-template <int KT>
-__global__ __launch_bounds__(kBlock) void k_csr_spmm(long long n_rows, int k, int f_col, int ln_col,
-                                                     const int *__restrict__ rowptr,
-                                                     const int *__restrict__ colidx,
-                                                     const double *__restrict__ vals,
-                                                     const double *__restrict__ B,
-                                                     double *__restrict__ C) {
+constexpr int kSpmmXcdCols = 65536;
+
+// E entries from j on: their pieces of B are in flight together, the products
+// are added in entry order
+template <int E, int V>
+__device__ inline void spmm_step(const SpmmArgs &a, int j, int col, bool on, double (&acc)[V]) {
   TBSLA_NO_FMA
-  const long long row = __builtin_amdgcn_readfirstlane(
-      (int)(((long long)blockIdx.x * kBlock + threadIdx.x) / kWave));
-  const int lane = threadIdx.x & (kWave - 1);
-  if (row >= n_rows) return;
-  const int k0 = blockIdx.y * (kMaxTiles * kWave);  // this launch row's column chunk
-  double acc[KT];
+  typedef double vd __attribute__((ext_vector_type(V)));
+  bool in[E];
+  double v[E], x[E][V];
+  const double *bp[E];
 #pragma unroll
-  for (int t = 0; t < KT; t++) acc[t] = 0.0;
-  const int beg = rowptr[row], end = rowptr[row + 1];
-  int j = beg;
-  // E entries per step: their B rows' loads are in flight together; the
-  // products are still added in entry order
-  constexpr int E = 4;
-  for (; j + E <= end; j += E) {
-    bool in[E];
-    double v[E];
-    const double *bp[E];
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-      const int c = colidx[j + e] - f_col;
-      in[e] = c >= 0 && c < ln_col;  // block filter (:19)
-      v[e] = vals[j + e];
-      bp[e] = B + (size_t)(in[e] ? c : 0) * k;
-    }
-    double xv[E][KT];
-#pragma unroll
-    for (int e = 0; e < E; e++)
-#pragma unroll
-      for (int t = 0; t < KT; t++) {
-        const int col = k0 + lane + t * kWave;
-        xv[e][t] = col < k ? bp[e][col] : 0.0;
-      }
-#pragma unroll
-    for (int e = 0; e < E; e++)
-#pragma unroll
-      for (int t = 0; t < KT; t++)
-        if (in[e]) acc[t] = acc[t] + v[e] * xv[e][t];
+  for (int e = 0; e < E; e++) {
+    const int c = a.colidx[j + e] - a.f_col;
+    in[e] = c >= 0 && c < a.ln_col;  // block filter (:19)
+    v[e] = a.vals[j + e];
+    bp[e] = a.B + (size_t)(in[e] ? c : 0) * a.k + col;
   }
-  for (; j < end; j++) {
-    const int c = colidx[j] - f_col;
-    if (c >= 0 && c < ln_col) {
-      const double v = vals[j];
-      const double *b = B + (size_t)c * k;
 #pragma unroll
-      for (int t = 0; t < KT; t++) {
-        const int col = k0 + lane + t * kWave;
-        if (col < k) acc[t] = acc[t] + v * b[col];
-      }
+  for (int e = 0; e < E; e++) {
+    if constexpr (V == 1) {
+      x[e][0] = on ? *bp[e] : 0.0;
+    } else {
+      const vd b = on ? *reinterpret_cast<const vd *>(bp[e]) : vd{};
+#pragma unroll
+      for (int q = 0; q < V; q++) x[e][q] = b[q];
     }
   }
-  double *out = C + (size_t)row * k;
 #pragma unroll
-  for (int t = 0; t < KT; t++) {
-    const int col = k0 + lane + t * kWave;
-    if (col < k) out[col] = acc[t];
+  for (int e = 0; e < E; e++)
+#pragma unroll
+    for (int q = 0; q < V; q++)
+      if (in[e]) acc[q] = acc[q] + v[e] * x[e][q];
+}
+
+template <int LPR, int V>
+__global__ __launch_bounds__(kBlock) void k_csr_spmm(SpmmArgs a) {
+  typedef double vd __attribute__((ext_vector_type(V)));
+  unsigned chunk, rb;
+  if (a.xcd && a.nchunks >= 8) {  // nchunks a multiple of 8
+    const unsigned i = blockIdx.x / 8;
+    chunk = blockIdx.x % 8 + 8 * (i / a.rblocks);
+    rb = i % a.rblocks;
+  } else if (a.xcd) {  // 8 / nchunks XCDs share a chunk and split its row blocks
+    const unsigned x = blockIdx.x % 8;
+    chunk = x % a.nchunks;
+    rb = blockIdx.x / 8 * (8 / a.nchunks) + x / a.nchunks;
+  } else {
+    chunk = a.chunk0 + blockIdx.y;
+    rb = blockIdx.x;
   }
+  const long long row = (long long)rb * (kBlock / LPR) + threadIdx.x / LPR;
+  if (rb >= a.rblocks || row >= a.n_rows) return;
+  const int col = (int)chunk * LPR * V + (threadIdx.x & (LPR - 1)) * V;
+  const bool on = col < a.k;  // V = 2: k is even
+  double acc[V];
+#pragma unroll
+  for (int q = 0; q < V; q++) acc[q] = 0.0;
+  int j = a.rowptr[row];
+  const int end = a.rowptr[row + 1];
+  for (; j + 8 <= end; j += 8) spmm_step<8, V>(a, j, col, on, acc);
+  if (j + 4 <= end) {
+    spmm_step<4, V>(a, j, col, on, acc);
+    j += 4;
+  }
+  if (j + 2 <= end) {
+    spmm_step<2, V>(a, j, col, on, acc);
+    j += 2;
+  }
+  if (j < end) spmm_step<1, V>(a, j, col, on, acc);
+  if (!on) return;
+  double *out = a.C + (size_t)row * a.k + col;
+  if constexpr (V == 1) {
+    __builtin_nontemporal_store(acc[0], out);
+  } else {
+    vd o;
+#pragma unroll
+    for (int q = 0; q < V; q++) o[q] = acc[q];
+    __builtin_nontemporal_store(o, reinterpret_cast<vd *>(out));
+  }
+}
+
+// the launch of one (LPR, V)
+template <int LPR, int V>
+int spmm_go(SpmmArgs a, hipStream_t s) {
+  const long long rb = (a.n_rows + kBlock / LPR - 1) / (kBlock / LPR);
+  a.nchunks = (unsigned)(((long long)a.k + LPR * V - 1) / (LPR * V));
+  a.rblocks = (unsigned)rb;
+  a.xcd = a.ln_col <= kSpmmXcdCols && rb * a.nchunks < (1 << 20) && a.nchunks > 1 &&
+          (a.nchunks % 8 == 0 || 8 % a.nchunks == 0);
+  if (a.xcd) {
+    const unsigned share = a.nchunks < 8 ? 8 / a.nchunks : 1;  // XCDs to a chunk
+    const unsigned grid =
+        a.nchunks < 8 ? 8 * ((a.rblocks + share - 1) / share) : a.rblocks * a.nchunks;
+    k_csr_spmm<LPR, V><<<grid, kBlock, 0, s>>>(a);
+    TBSLA_HIP_LAUNCH_CHECK();
+    return TBSLA_HIP_SUCCESS;
+  }
+  constexpr unsigned kMostY = 65535;
+  for (a.chunk0 = 0; a.chunk0 < a.nchunks; a.chunk0 += kMostY) {
+    k_csr_spmm<LPR, V><<<dim3(a.rblocks, std::min(kMostY, a.nchunks - a.chunk0)), kBlock, 0, s>>>(a);
+    TBSLA_HIP_LAUNCH_CHECK();
+  }
+  return TBSLA_HIP_SUCCESS;
 }
 
 struct PprState {
@@ -759,17 +825,12 @@ extern "C" int tbsla_hip_spmm(tbsla_hip_matrix_t m, const double *d_B, double *d
   if (rows == 0) return TBSLA_HIP_SUCCESS;
   if (m->ln_col == 0 || !m->has_arrays || m->stored == 0)  // no products: C = 0
     return launch_fill(d_C, rows * (long long)k, 0.0, s);
-  const int chunk = kMaxTiles * kWave;
-  const dim3 grid(grid_for(rows * kWave), (unsigned)((k + chunk - 1) / chunk));
-  const int tiles = k > chunk ? kMaxTiles : (k + kWave - 1) / kWave;
-  switch (tiles) {
-    case 1: k_csr_spmm<1><<<grid, kBlock, 0, s>>>(rows, k, m->f_col, m->ln_col, m->rowptr, m->colidx, m->values, d_B, d_C); break;
-    case 2: k_csr_spmm<2><<<grid, kBlock, 0, s>>>(rows, k, m->f_col, m->ln_col, m->rowptr, m->colidx, m->values, d_B, d_C); break;
-    case 3: k_csr_spmm<3><<<grid, kBlock, 0, s>>>(rows, k, m->f_col, m->ln_col, m->rowptr, m->colidx, m->values, d_B, d_C); break;
-    default: k_csr_spmm<4><<<grid, kBlock, 0, s>>>(rows, k, m->f_col, m->ln_col, m->rowptr, m->colidx, m->values, d_B, d_C); break;
-  }
-  TBSLA_HIP_LAUNCH_CHECK();
-  return TBSLA_HIP_SUCCESS;
+  const SpmmArgs a{rows, k,   m->f_col, m->ln_col, m->rowptr, m->colidx, m->values,
+                   d_B,  d_C, 0,        0,         0,         0};
+  // 16-byte pieces where every row of B and C starts on one
+  const bool pairs = k % 2 == 0 && ((uintptr_t)d_B | (uintptr_t)d_C) % 16 == 0;
+  if (pairs) return k <= 16 ? spmm_go<8, 2>(a, s) : spmm_go<16, 2>(a, s);
+  return k <= 16 ? spmm_go<16, 1>(a, s) : spmm_go<32, 1>(a, s);
 }
 
 extern "C" int tbsla_hip_personalized_page_rank(tbsla_hip_matrix_t m, double beta, double epsilon,
