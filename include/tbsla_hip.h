@@ -382,7 +382,8 @@ typedef struct {
                             system and 256 when tbsla_hip_cg_batched solves more
                             than one.  Every workgroup reads all of its system's
                             dot-product partials, so a batch, whose systems fill the GPU
-                            together, takes fewer; a system solved alone and in a batch
+                            together, takes fewer (and, as with any value up to 256,
+                            no workgroup under 256 rows); a system solved alone and in a batch
                             gives bitwise the same iterates when both use the same value
                             (and the same lanes_per_row) */
   int spmv_passes;       /* K1 (p = z + beta p, then A p) on A's CSR rows: 1 forms p at every

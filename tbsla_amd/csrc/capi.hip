@@ -71,10 +71,12 @@ Pool &pool() {
   return *p;
 }
 
-// whole pages of the allocator: 4 KiB, or 2 MiB for large blocks
+// whole pages of the allocator: 4 KiB, or 2 MiB for large blocks; 32 bytes of
+// slack after the bytes asked for
 size_t pool_size(size_t bytes) {
+  bytes += 32;
   const size_t unit = bytes >= (size_t(1) << 23) ? (size_t(1) << 21) : 4096;
-  return (std::max<size_t>(bytes, 1) + unit - 1) / unit * unit;
+  return (bytes + unit - 1) / unit * unit;
 }
 
 // hipMalloc, once more after the idle blocks are given back

@@ -63,6 +63,7 @@ struct CgSeg {
   int row0, row1;    // rows of the system
   int blk0, blk1;    // workgroups of the system (same in every kernel)
   int rpb;           // rows per workgroup
+  int ent0;          // the first entry of row0
 };
 
 struct CgCom {
@@ -128,7 +129,67 @@ struct CgArgs {
 // buffer, so one instantiated graph serves every later solve of the same
 // shape and no graph can refer to memory that has been freed since.
 #define CG_ARGS const CgArgs *__restrict__ pa_
-#define CG_BIND const CgArgs &a = *pa_
+#define CG_BIND const CgArgs a = cg_bind(pa_)
+
+// The argument block read as constant memory, by scalar loads, and its pointers
+// as pointers to global memory.  A pointer that is itself loaded would otherwise
+// be a generic one, and what is read through it would go by flat instructions,
+// which count as LDS accesses too, take no uniform base and hold a 64-bit
+// address each.
+#define TBSLA_CONST __attribute__((address_space(4))) const
+template <typename T>
+__device__ inline T *arg(T *TBSLA_CONST *slot) {
+  typedef __attribute__((address_space(1))) T G;
+  return (T *)*(G *TBSLA_CONST *)slot;
+}
+
+// element `i` of one of the block's pointer pairs
+#define CG_AT(field, i) arg(&((TBSLA_CONST CgArgs *)pa_)->field[i])
+
+// the block's other fields
+__device__ inline CgArgs cg_bind(const CgArgs *pa) {
+  TBSLA_CONST CgArgs *c = (TBSLA_CONST CgArgs *)pa;
+  CgArgs a;
+  a.rowptr = arg(&c->rowptr);
+  a.colidx = arg(&c->colidx);
+  a.val64 = arg(&c->val64);
+  a.val32 = arg(&c->val32);
+  a.f_col = c->f_col;
+  a.g_rp = arg(&c->g_rp);
+  a.g_ci = arg(&c->g_ci);
+  a.g_v64 = arg(&c->g_v64);
+  a.g_v32 = arg(&c->g_v32);
+  a.t_rp = arg(&c->t_rp);
+  a.t_ci = arg(&c->t_ci);
+  a.t_v64 = arg(&c->t_v64);
+  a.t_v32 = arg(&c->t_v32);
+  a.dinv = arg(&c->dinv);
+  a.gdoff = arg(&c->gdoff);
+  a.gd64 = arg(&c->gd64);
+  a.gd32 = arg(&c->gd32);
+  a.gndiag = c->gndiag;
+  a.b = arg(&c->b);
+  a.x = arg(&c->x);
+  a.z = arg(&c->z);
+  a.ap = arg(&c->ap);
+  a.ax = arg(&c->ax);
+  a.t64 = arg(&c->t64);
+  a.t32 = arg(&c->t32);
+  a.ppap = arg(&c->ppap);
+  a.seg = arg(&c->seg);
+  a.com = arg(&c->com);
+  a.block_seg = arg(&c->block_seg);
+  a.verify = c->verify;
+  a.stall_window = c->stall_window;
+  a.a_nnz = c->a_nnz;
+  a.g_nnz = c->g_nnz;
+  a.doff = arg(&c->doff);
+  a.dv64 = arg(&c->dv64);
+  a.dv32 = arg(&c->dv32);
+  a.ndiag = c->ndiag;
+  a.ncol = c->ncol;
+  return a;
+}
 
 // Sums of a system's workgroup partials are taken in one fixed order:
 // thread k adds partials k, k+256, ... in order; waves reduce by xor
@@ -205,6 +266,75 @@ struct RowPrefetch {
   int col[P];
   V v[P];
   double s[P], t[P];
+};
+
+// One row of A as a group of L lanes reads it in K1: 8 entries per lane.  L = 1:
+// the row's first 8, one by one (short rows).  L >= 2: two 16-byte loads of
+// column indices (and 16 or 32 bytes of values), 4 entries each, from the row's
+// first entry rounded down to a multiple of 4 of its system's entries (so that a
+// system is summed alike alone and in a batch, where its quads may lie on any
+// 4-byte boundary); lane l's quads are l and l + L, so a row's lines are read
+// whole by one instruction instead of 4 L bytes at a time.  Slots outside the row
+// have column 0 of the block and are not summed.  Longer rows continue with the
+// entries from `rest` on.
+template <int L, typename V>
+struct CgRow {
+  static constexpr int P = 8;
+  int beg, end, first;
+  int col[P];
+  V v[P];
+
+  __device__ inline void extent(const int *__restrict__ rowptr, int row, int ent0) {
+    beg = rowptr[row];
+    end = rowptr[row + 1];
+    first = L == 1 ? beg : beg - ((beg - ent0) & 3);
+  }
+  __device__ inline int at(int lane, int k) const {
+    return L == 1 ? beg + k : first + 4 * (lane + (k >> 2) * L) + (k & 3);
+  }
+  __device__ inline bool in(int lane, int k) const {
+    const int e = at(lane, k);
+    return e >= beg && e < end;
+  }
+  __device__ inline int rest(int lane) const {
+    return L == 1 ? beg + P : first + 4 * (lane + 2 * L);
+  }
+  // the entries, clamped into the arrays (the last quad may end up to three
+  // entries after the last one: device_alloc's blocks have room for them)
+  template <bool NT>
+  __device__ inline void load(const int *__restrict__ ci, const V *__restrict__ va, int nnz,
+                              int f_col, int lane) {
+    if constexpr (L == 1) {
+#pragma unroll
+      for (int k = 0; k < P; k++) {
+        const int j = min(at(lane, k), nnz - 1);
+        col[k] = ci[j];
+        v[k] = va[j];
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; h++) quad<NT>(ci, va, min(at(lane, 4 * h), nnz - 1), 4 * h);
+    }
+#pragma unroll
+    for (int k = 0; k < P; k++) col[k] = in(lane, k) ? col[k] - f_col : 0;
+  }
+  template <bool NT>
+  __device__ inline void quad(const int *__restrict__ ci, const V *__restrict__ va, int j, int k) {
+    typedef int vi __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int W = 16 / sizeof(V);  // values per 16 bytes
+    typedef V vv __attribute__((ext_vector_type(W), aligned(sizeof(V))));
+    const vi *pc = reinterpret_cast<const vi *>(ci + j);
+    const vi c = NT ? __builtin_nontemporal_load(pc) : *pc;
+#pragma unroll
+    for (int q = 0; q < 4; q++) col[k + q] = c[q];
+#pragma unroll
+    for (int q = 0; q < 4; q += W) {
+      const vv *pv = reinterpret_cast<const vv *>(va + j + q);
+      const vv x = NT ? __builtin_nontemporal_load(pv) : *pv;
+#pragma unroll
+      for (int w = 0; w < W; w++) v[k + q + w] = x[w];
+    }
+  }
 };
 
 // A system's workgroup partials as loaded by seg_issue (raw, unmasked) and
@@ -308,7 +438,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
   TBSLA_NO_FMA
   CG_BIND;
   typedef typename std::conditional<MIX, float, double>::type V;
-  constexpr int P = L == 1 ? 8 : 4;
+  typedef CgRow<L, V> Row;
+  constexpr int P = Row::P;
   constexpr int NP = ZBUF ? 3 : 2;
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
@@ -319,34 +450,27 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
   const int r0 = S->row0 + (b - b0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
   const int lane = threadIdx.x & (L - 1);
-  const double *zv = ZBUF ? a.z : a.r[par];
-  const double *po = a.p[par];
+  const double *zv = ZBUF ? a.z : CG_AT(r, par);
+  const double *po = CG_AT(p, par);
   const V *val = MIX ? (const V *)a.val32 : (const V *)a.val64;
   const int row_first = r0 + (int)threadIdx.x / L;
   const int rowc = min(row_first, r1 - 1);
-  // row extent and own entries, then the row's first entries (indices
-  // clamped into the arrays, which hold at least one entry; entries past the
-  // row end are never used), then the partials, then the gathers.  No
-  // branches between them: a join would make the partials' wait cover the
-  // gathers.
-  RowPrefetch<P, V> f;
-  f.beg = a.rowptr[rowc];
-  f.end = a.rowptr[rowc + 1];
+  // row extent and own entries, then the row's first entries, then the
+  // partials, then the gathers.  No branches between them: a join would make
+  // the partials' wait cover the gathers.
+  Row f;
+  double fs[P], ft[P];
+  f.extent(a.rowptr, rowc, S->ent0);
   const double own_z = zv[rowc], own_p = po[rowc];
-#pragma unroll
-  for (int k = 0; k < P; k++) {
-    const int j = min(f.beg + lane + k * L, a.a_nnz - 1);
-    f.col[k] = a.colidx[j];
-    f.v[k] = val[j];
-  }
+  f.template load<false>(a.colidx, val, a.a_nnz, a.f_col, lane);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
   SegLoad sl;
-  seg_issue(a.prz[par ^ 1], a.prz[par], a.prr[par ^ 1], NP, b0, b1, sl);
+  seg_issue(CG_AT(prz, par ^ 1), CG_AT(prz, par), CG_AT(prr, par ^ 1), NP, b0, b1, sl);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int k = 0; k < P; k++) {
-    f.s[k] = zv[f.col[k] - a.f_col];
-    f.t[k] = po[f.col[k] - a.f_col];
+    fs[k] = zv[f.col[k]];
+    ft[k] = po[f.col[k]];
   }
   __builtin_amdgcn_sched_barrier(0);  // keep the loads above issued in this order
   double t[3];
@@ -358,89 +482,64 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
     if (fin != kRunning || check_only) return;
   }
   const double beta = rz_new / fmax(rz_old, S->near_zero);
-  double *pn = a.p[par ^ 1];
+  double *pn = CG_AT(p, par ^ 1);
   double pap = 0.0;
   constexpr int PASS = kBlock / L;
-  if (row_first < r1) {
+  // the sum of a loaded row, the entries past its 8 per lane from memory
+  auto finish = [&](const Row &w, const double (&sv)[P], const double (&tv)[P], int row, double oz,
+                    double op) {
     V acc = 0;
+    auto term = [&](V av, double s, double t) {
+      const double v = s + beta * t;
+      if (MIX) acc = fmaf((float)av, (float)v, (float)acc);
+      else acc = fma((double)av, v, (double)acc);
+    };
 #pragma unroll
-    for (int k = 0; k < P; k++) {
-      if (f.beg + lane + k * L < f.end) {
-        const double v = f.s[k] + beta * f.t[k];
-        if (MIX) acc = fmaf((float)f.v[k], (float)v, (float)acc);
-        else acc = fma((double)f.v[k], v, (double)acc);
-      }
-    }
-    for (int j = f.beg + lane + P * L; j < f.end; j += L) {
-      const int c = a.colidx[j] - a.f_col;
-      const double v = zv[c] + beta * po[c];
-      if (MIX) acc = fmaf((float)val[j], (float)v, (float)acc);
-      else acc = fma((double)val[j], v, (double)acc);
-    }
+    for (int k = 0; k < P; k++)
+      if (w.in(lane, k)) term(w.v[k], sv[k], tv[k]);
+    constexpr int Q = L == 1 ? 1 : 4;  // consecutive entries of a lane
+    for (int j = w.rest(lane); j < w.end; j += Q * L)
+#pragma unroll
+      for (int q = 0; q < Q; q++)
+        if (j + q < w.end) {
+          const int c = a.colidx[j + q] - a.f_col;
+          term(val[j + q], zv[c], po[c]);
+        }
     acc = lane_sum<L>(acc);
-    const double own = own_z + beta * own_p;
+    const double own = oz + beta * op;
     if (lane == 0) {
-      pn[row_first] = own;
-      a.ap[row_first] = (double)acc;
+      pn[row] = own;
+      a.ap[row] = (double)acc;
       pap += own * (double)acc;
     }
-  }
+  };
+  if (row_first < r1) finish(f, fs, ft, row_first, own_z, own_p);
   // the later rows two at a time: both rows' extents, then entries, then
   // gathers are issued before either is summed
   constexpr int R2 = 2;
   for (int row = row_first + PASS; row < r1; row += R2 * PASS) {
-    RowPrefetch<P, V> g[R2];
-    double oz[R2], op[R2];
+    Row g[R2];
+    double gs[R2][P], gt[R2][P], oz[R2], op[R2];
     int rw[R2];
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       rw[r] = min(row + r * PASS, r1 - 1);
-      g[r].beg = a.rowptr[rw[r]];
-      g[r].end = a.rowptr[rw[r] + 1];
+      g[r].extent(a.rowptr, rw[r], S->ent0);
       oz[r] = zv[rw[r]];
       op[r] = po[rw[r]];
     }
 #pragma unroll
-    for (int r = 0; r < R2; r++)
-#pragma unroll
-      for (int k = 0; k < P; k++) {
-        const int j = min(g[r].beg + lane + k * L, a.a_nnz - 1);
-        g[r].col[k] = a.colidx[j];
-        g[r].v[k] = val[j];
-      }
+    for (int r = 0; r < R2; r++) g[r].template load<false>(a.colidx, val, a.a_nnz, a.f_col, lane);
 #pragma unroll
     for (int r = 0; r < R2; r++)
 #pragma unroll
       for (int k = 0; k < P; k++) {
-        g[r].s[k] = zv[g[r].col[k] - a.f_col];
-        g[r].t[k] = po[g[r].col[k] - a.f_col];
+        gs[r][k] = zv[g[r].col[k]];
+        gt[r][k] = po[g[r].col[k]];
       }
 #pragma unroll
-    for (int r = 0; r < R2; r++) {
-      if (row + r * PASS >= r1) break;
-      V acc = 0;
-#pragma unroll
-      for (int k = 0; k < P; k++) {
-        if (g[r].beg + lane + k * L < g[r].end) {
-          const double v = g[r].s[k] + beta * g[r].t[k];
-          if (MIX) acc = fmaf((float)g[r].v[k], (float)v, (float)acc);
-          else acc = fma((double)g[r].v[k], v, (double)acc);
-        }
-      }
-      for (int j = g[r].beg + lane + P * L; j < g[r].end; j += L) {
-        const int c = a.colidx[j] - a.f_col;
-        const double v = zv[c] + beta * po[c];
-        if (MIX) acc = fmaf((float)val[j], (float)v, (float)acc);
-        else acc = fma((double)val[j], v, (double)acc);
-      }
-      acc = lane_sum<L>(acc);
-      const double own = oz[r] + beta * op[r];
-      if (lane == 0) {
-        pn[rw[r]] = own;
-        a.ap[rw[r]] = (double)acc;
-        pap += own * (double)acc;
-      }
-    }
+    for (int r = 0; r < R2; r++)
+      if (row + r * PASS < r1) finish(g[r], gs[r], gt[r], rw[r], oz[r], op[r]);
   }
   pap = wg_sum(pap, lds);
   if (threadIdx.x == 0) a.ppap[b] = pap;
@@ -463,11 +562,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_pnew(CG_ARGS, int par_g, int chec
   const int b0 = S->blk0, b1 = S->blk1;
   const int r0 = S->row0 + (b - b0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
-  const double *zv = ZBUF ? a.z : a.r[par];
-  const double *po = a.p[par];
+  const double *zv = ZBUF ? a.z : CG_AT(r, par);
+  const double *po = CG_AT(p, par);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
   SegLoad sl;
-  seg_issue(a.prz[par ^ 1], a.prz[par], a.prr[par ^ 1], NP, b0, b1, sl);
+  seg_issue(CG_AT(prz, par ^ 1), CG_AT(prz, par), CG_AT(prr, par ^ 1), NP, b0, b1, sl);
   double t[3];
   if (seg_finish(flag, sl, NP, b0, b1, sh, t) != kRunning) return;
   const double rz_new = t[0], rz_old = t[1];
@@ -477,7 +576,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_pnew(CG_ARGS, int par_g, int chec
     if (fin != kRunning || check_only) return;
   }
   const double beta = rz_new / fmax(rz_old, S->near_zero);
-  double *pn = a.p[par ^ 1];
+  double *pn = CG_AT(p, par ^ 1);
   for (int row = r0 + (int)threadIdx.x; row < r1; row += 2 * kBlock) {
     const int row2 = row + kBlock;
     const double z0 = zv[row], p0 = po[row];
@@ -496,7 +595,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
   TBSLA_NO_FMA  // p'.Ap' partials added as k_cg_spmv_p adds them
   CG_BIND;
   typedef typename std::conditional<MIX, float, double>::type V;
-  constexpr int P = L == 1 ? 8 : 4;
+  typedef CgRow<L, V> Row;
+  constexpr int P = Row::P;
   __shared__ double lds[kBlock / kWave];
   const int b = blockIdx.x;
   CgSeg *S = a.seg + a.block_seg[b];
@@ -506,7 +606,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
   const int r0 = S->row0 + (b - b0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
   const int lane = threadIdx.x & (L - 1);
-  const double *pn = a.p[par ^ 1];
+  const double *pn = CG_AT(p, par ^ 1);
   const V *val = MIX ? (const V *)a.val32 : (const V *)a.val64;
   constexpr int PASS = kBlock / L;
   constexpr int R2 = 2;
@@ -514,44 +614,37 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
   // rows two at a time: both rows' extents, then entries, then gathers are
   // issued before either is summed
   for (int row = r0 + (int)threadIdx.x / L; row < r1; row += R2 * PASS) {
-    int beg[R2], end[R2], rw[R2], col[R2][P];
-    V v[R2][P];
+    Row w[R2];
+    int rw[R2];
     double g[R2][P], own[R2];
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       rw[r] = min(row + r * PASS, r1 - 1);
-      beg[r] = a.rowptr[rw[r]];
-      end[r] = a.rowptr[rw[r] + 1];
+      w[r].extent(a.rowptr, rw[r], S->ent0);
       own[r] = pn[rw[r]];
     }
 #pragma unroll
-    for (int r = 0; r < R2; r++)
-#pragma unroll
-      for (int k = 0; k < P; k++) {
-        const int j = min(beg[r] + lane + k * L, a.a_nnz - 1);
-        col[r][k] = a.colidx[j];
-        v[r][k] = val[j];
-      }
+    for (int r = 0; r < R2; r++) w[r].template load<L != 1>(a.colidx, val, a.a_nnz, a.f_col, lane);
 #pragma unroll
     for (int r = 0; r < R2; r++)
 #pragma unroll
-      for (int k = 0; k < P; k++) g[r][k] = pn[col[r][k] - a.f_col];
+      for (int k = 0; k < P; k++) g[r][k] = pn[w[r].col[k]];
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       if (row + r * PASS >= r1) break;
       V acc = 0;
+      auto term = [&](V av, double x) {
+        if (MIX) acc = fmaf((float)av, (float)x, (float)acc);
+        else acc = fma((double)av, x, (double)acc);
+      };
 #pragma unroll
-      for (int k = 0; k < P; k++) {
-        if (beg[r] + lane + k * L < end[r]) {
-          if (MIX) acc = fmaf((float)v[r][k], (float)g[r][k], (float)acc);
-          else acc = fma((double)v[r][k], g[r][k], (double)acc);
-        }
-      }
-      for (int j = beg[r] + lane + P * L; j < end[r]; j += L) {
-        const double x = pn[a.colidx[j] - a.f_col];
-        if (MIX) acc = fmaf((float)val[j], (float)x, (float)acc);
-        else acc = fma((double)val[j], x, (double)acc);
-      }
+      for (int k = 0; k < P; k++)
+        if (w[r].in(lane, k)) term(w[r].v[k], g[r][k]);
+      constexpr int Q = L == 1 ? 1 : 4;
+      for (int j = w[r].rest(lane); j < w[r].end; j += Q * L)
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+          if (j + q < w[r].end) term(val[j + q], pn[a.colidx[j + q] - a.f_col]);
       acc = lane_sum<L>(acc);
       if (lane == 0) {
         a.ap[rw[r]] = (double)acc;
@@ -563,19 +656,40 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
   if (threadIdx.x == 0) a.ppap[b] = pap;
 }
 
+// base[i] by a 32-bit byte offset (one register of address beside the uniform
+// base): arrays below 4 GiB
+template <typename T>
+__device__ inline T ld32(const T *__restrict__ base, unsigned i) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) +
+                                      (size_t)(i * (unsigned)sizeof(T)));
+}
+// the same, or by a 64-bit one where an array may be larger
+template <bool WIDE, typename T>
+__device__ inline T ldi(const T *__restrict__ base, long long i) {
+  if constexpr (WIDE) return base[i];
+  else return ld32(base, (unsigned)i);
+}
+
 // K1 on A in the diagonal layout: the same steps as k_cg_spmv_p (the
 // partials of the previous iteration, the convergence test, beta), then per
 // row p' = z + beta p and (A p')_row = sum over the stored diagonals
 // (ascending offset, zero slots skipped) of A's slot times p' at the slot's
-// column, one row per thread, eight diagonals' loads in flight.
-template <bool MIX, bool ZBUF>
+// column.  KD 3, 5, 7: exactly that many diagonals (the stencils of one to three
+// dimensions) in arrays below 4 GiB, a row's loads all in flight; the first row's
+// loads (which need no sum) go out before the partials', so the reductions and
+// the test run under them.  KD 0: any number of diagonals and any size, eight
+// diagonals at a time.  Bound by latency (flag and partials, then a trip per row)
+// at 64^3, FP64: 9.7 -> 8.0 us an iteration (KD and the early loads, 0.9; global
+// loads for flat ones, 0.8); 10^6 rows, mixed: 19.4 -> 17.1.  Two rows in flight per
+// thread were slower (8.3 and 18.6: 204 registers, half the wavefronts).
+template <bool MIX, bool ZBUF, int KD>
 __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int check,
                                                         int check_only) {
   TBSLA_NO_FMA
   CG_BIND;
   typedef typename std::conditional<MIX, float, double>::type V;
   constexpr int NP = ZBUF ? 3 : 2;
-  constexpr int U = 8;
+  constexpr int U = KD > 0 ? KD : 8;
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
   const int b = blockIdx.x;
@@ -584,12 +698,47 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
   const int b0 = S->blk0, b1 = S->blk1;
   const int r0 = S->row0 + (b - b0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
-  const double *zv = ZBUF ? a.z : a.r[par];
-  const double *po = a.p[par];
+  const double *zv = ZBUF ? a.z : CG_AT(r, par);
+  const double *po = CG_AT(p, par);
   const V *dv = MIX ? (const V *)a.dv32 : (const V *)a.dv64;
+  const int row_first = r0 + (int)threadIdx.x;
+  struct Row {
+    V v[U];
+    double z[U], p[U], oz, op;
+  } f;
+  // slots k0 .. k0 + U - 1 of one row (past the last diagonal: the last one
+  // again, not used)
+  auto load = [&](int row, int k0, Row &w) {
+    if constexpr (KD > 0) {
+      const unsigned at = (unsigned)dia_at(row, 0, KD);
+#pragma unroll
+      for (int i = 0; i < U; i++) {
+        const unsigned c = (unsigned)min(max(row + a.doff[i], 0), a.ncol - 1);
+        w.v[i] = ld32(dv, at + i * kWave);
+        w.z[i] = ld32(zv, c);
+        w.p[i] = ld32(po, c);
+      }
+      w.oz = ld32(zv, (unsigned)row);
+      w.op = ld32(po, (unsigned)row);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const int kk = min(k0 + i, a.ndiag - 1);
+      const int c = min(max(row + a.doff[kk], 0), a.ncol - 1);
+      w.v[i] = dv[dia_at(row, kk, a.ndiag)];
+      w.z[i] = zv[c];
+      w.p[i] = po[c];
+    }
+  };
+  if (KD > 0) {
+    load(min(row_first, r1 - 1), 0, f);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
   SegLoad sl;
-  seg_issue(a.prz[par ^ 1], a.prz[par], a.prr[par ^ 1], NP, b0, b1, sl);
+  seg_issue(CG_AT(prz, par ^ 1), CG_AT(prz, par), CG_AT(prr, par ^ 1), NP, b0, b1, sl);
+  __builtin_amdgcn_sched_barrier(0);  // keep the loads above issued in this order
   double t[3];
   if (seg_finish(flag, sl, NP, b0, b1, sh, t) != kRunning) return;
   const double rz_new = t[0], rz_old = t[1];
@@ -599,34 +748,38 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
     if (fin != kRunning || check_only) return;
   }
   const double beta = rz_new / fmax(rz_old, S->near_zero);
-  double *pn = a.p[par ^ 1];
+  double *pn = CG_AT(p, par ^ 1);
   double pap = 0.0;
-  for (int row = r0 + (int)threadIdx.x; row < r1; row += kBlock) {
-    V acc = 0;
-    for (int k = 0; k < a.ndiag; k += U) {
-      V v[U];
-      double zs[U], ps[U];
+  auto add = [&](const Row &w, int k0, V acc) {
 #pragma unroll
-      for (int i = 0; i < U; i++) {
-        const int kk = min(k + i, a.ndiag - 1);
-        const int c = min(max(row + a.doff[kk], 0), a.ncol - 1);
-        v[i] = dv[dia_at(row, kk, a.ndiag)];
-        zs[i] = zv[c];
-        ps[i] = po[c];
-      }
-#pragma unroll
-      for (int i = 0; i < U; i++) {
-        if (k + i < a.ndiag && v[i] != (V)0) {
-          const double pc = zs[i] + beta * ps[i];
-          if (MIX) acc = fmaf((float)v[i], (float)pc, (float)acc);
-          else acc = fma((double)v[i], pc, (double)acc);
-        }
+    for (int i = 0; i < U; i++) {
+      if ((KD > 0 || k0 + i < a.ndiag) && w.v[i] != (V)0) {
+        const double pc = w.z[i] + beta * w.p[i];
+        if (MIX) acc = fmaf((float)w.v[i], (float)pc, (float)acc);
+        else acc = fma((double)w.v[i], pc, (double)acc);
       }
     }
-    const double own = zv[row] + beta * po[row];
+    return acc;
+  };
+  auto store = [&](int row, double own, V acc) {
     pn[row] = own;
     a.ap[row] = (double)acc;
     pap += own * (double)acc;
+  };
+  if (KD > 0) {
+    for (int row = row_first; row < r1; row += kBlock) {
+      if (row != row_first) load(row, 0, f);
+      store(row, f.oz + beta * f.op, add(f, 0, (V)0));
+    }
+  } else {
+    for (int row = row_first; row < r1; row += kBlock) {
+      V acc = 0;
+      for (int k = 0; k < a.ndiag; k += U) {
+        load(row, k, f);
+        acc = add(f, k, acc);
+      }
+      store(row, zv[row] + beta * po[row], acc);
+    }
   }
   pap = wg_sum(pap, lds);
   if (threadIdx.x == 0) a.ppap[b] = pap;
@@ -646,9 +799,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   CgSeg *S = a.seg + a.block_seg[b];
   const int par = (par_g ^ S->shift) & 1;
   const int b0 = S->blk0, b1 = S->blk1;
-  const double *rc = a.r[par];
-  double *rn = a.r[par ^ 1];
-  const double *pn = a.p[par ^ 1];
+  const double *rc = CG_AT(r, par);
+  double *rn = CG_AT(r, par ^ 1);
+  const double *pn = CG_AT(p, par ^ 1);
   const V *tv = MIX ? (const V *)a.t_v32 : (const V *)a.t_v64;
   const int r0 = S->row0 + (b - b0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
@@ -658,6 +811,16 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   // gathers of t = G^T r'
   const double fx = a.x[rowc], fp = pn[rowc], fr = rc[rowc], fap = a.ap[rowc];
   const double fd = PRE == 1 ? a.dinv[rowc] : 0.0;
+  // and, without a factor, the second row's
+  const int row2 = min(row_first + kBlock, r1 - 1);
+  double fx2 = 0.0, fp2 = 0.0, fr2 = 0.0, fap2 = 0.0, fd2 = 0.0;
+  if (PRE != 2) {
+    fx2 = a.x[row2];
+    fp2 = pn[row2];
+    fr2 = rc[row2];
+    fap2 = a.ap[row2];
+    if (PRE == 1) fd2 = a.dinv[row2];
+  }
   RowPrefetch<P, V> f;
   f.beg = f.end = 0;
   if (PRE == 2) {
@@ -672,7 +835,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   }
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
   SegLoad sl;
-  seg_issue(a.prz[par ^ 1], a.ppap, nullptr, 2, b0, b1, sl);
+  seg_issue(CG_AT(prz, par ^ 1), a.ppap, nullptr, 2, b0, b1, sl);
   __builtin_amdgcn_sched_barrier(0);
   if (PRE == 2) {
 #pragma unroll
@@ -691,17 +854,17 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   // loads issued before either is updated; sums in row order)
   const int row_end = PRE == 2 ? min(r1, row_first + 1) : r1;
   for (int row = row_first; row < row_end; row += kBlock) {
-    const bool first = row == row_first;
-    const double xv = first ? fx : a.x[row];
-    const double pv = first ? fp : pn[row];
-    const double rv = first ? fr : rc[row];
-    const double apv = first ? fap : a.ap[row];
+    const bool first = row == row_first, second = PRE != 2 && row == row_first + kBlock;
+    const double xv = first ? fx : second ? fx2 : a.x[row];
+    const double pv = first ? fp : second ? fp2 : pn[row];
+    const double rv = first ? fr : second ? fr2 : rc[row];
+    const double apv = first ? fap : second ? fap2 : a.ap[row];
     a.x[row] = xv + alpha * pv;
     const double ri = rv + (-alpha) * apv;
     rn[row] = ri;
     rr += ri * ri;
     if (PRE == 1) {
-      const double zi = ri * (first ? fd : a.dinv[row]);
+      const double zi = ri * (first ? fd : second ? fd2 : a.dinv[row]);
       a.z[row] = zi;
       rzp += ri * zi;
     }
@@ -787,9 +950,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   rr = wg_sum(rr, lds);
   if (PRE == 1) rzp = wg_sum(rzp, lds);
   if (threadIdx.x == 0) {
-    a.prr[par][b] = rr;
-    if (PRE == 0) a.prz[par][b] = rr;
-    if (PRE == 1) a.prz[par][b] = rzp;
+    CG_AT(prr, par)[b] = rr;
+    if (PRE == 0) CG_AT(prz, par)[b] = rr;
+    if (PRE == 1) CG_AT(prz, par)[b] = rzp;
     if (b == b0) {
       S->true_res = 0;
       if (count) S->iters += 1;  // the test K1 made on this iteration passed
@@ -807,24 +970,25 @@ __device__ inline V gd_slot(const V *__restrict__ gd, long long src, int k, int 
 // K2 with M = G G^T and G on diagonals: t_i = sum over G^T's row i in
 // ascending column (descending offset o_k <= 0) of G_{i-o_k, i} r'_{i-o_k},
 // zero slots skipped -- the order and the products of K2's CSR form, so the
-// two forms give bitwise the same iterates.  Rows go two per thread and
-// trip, all their loads issued before either row is updated.
-template <bool MIX, int KD>
+// two forms give bitwise the same iterates.  All of a row's loads are issued
+// before it is updated, the first row's (which need no sum) before the partials'.
+// Two rows in flight per thread are slower: 10^6 rows, mixed, 17.3 -> 23.4 us (170
+// registers for 100).
+template <bool MIX, int KD, bool WIDE>
 __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, int count) {
   TBSLA_NO_FMA
   CG_BIND;
   typedef typename std::conditional<MIX, float, double>::type V;
   // KD: at most that many diagonals of G (4 or 8, chosen on the host)
-  constexpr int R2 = 2;
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
   const int b = blockIdx.x;
   CgSeg *S = a.seg + a.block_seg[b];
   const int par = (par_g ^ S->shift) & 1;
   const int b0 = S->blk0, b1 = S->blk1;
-  const double *rc = a.r[par];
-  double *rn = a.r[par ^ 1];
-  const double *pn = a.p[par ^ 1];
+  const double *rc = CG_AT(r, par);
+  double *rn = CG_AT(r, par ^ 1);
+  const double *pn = CG_AT(p, par ^ 1);
   const V *gd = MIX ? (const V *)a.gd32 : (const V *)a.gd64;
   const int ndg = a.gndiag;
   const long long n = a.ncol;
@@ -833,59 +997,58 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, i
   int off[KD];
 #pragma unroll
   for (int k = 0; k < KD; k++) off[k] = k < ndg ? a.gdoff[k] : 0;
+  const int row_first = r0 + (int)threadIdx.x;
+  double xv, pv, rv, apv, rs[KD], as[KD];
+  V gv[KD];
+  auto load = [&](int row) {
+    xv = ldi<WIDE>(a.x, row);
+    pv = ldi<WIDE>(pn, row);
+    rv = ldi<WIDE>(rc, row);
+    apv = ldi<WIDE>(a.ap, row);
+#pragma unroll
+    for (int k = 0; k < KD; k++) {
+      if (k < ndg) {
+        const long long src = (long long)row - off[k];
+        const long long sc = src < n ? src : row;
+        const V g = ldi<WIDE>(gd, dia_at(sc, k, ndg));
+        gv[k] = src < n ? g : (V)0;
+        rs[k] = ldi<WIDE>(rc, sc);
+        as[k] = ldi<WIDE>(a.ap, sc);
+      }
+    }
+  };
+  load(min(row_first, r1 - 1));
+  __builtin_amdgcn_sched_barrier(0);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
   SegLoad sl;
-  seg_issue(a.prz[par ^ 1], a.ppap, nullptr, 2, b0, b1, sl);
+  seg_issue(CG_AT(prz, par ^ 1), a.ppap, nullptr, 2, b0, b1, sl);
+  __builtin_amdgcn_sched_barrier(0);
   double t[3];
   if (seg_finish(flag, sl, 2, b0, b1, sh, t) != kRunning) return;
   const double rz = t[0], pap = t[1];
   const double alpha = rz / fmax(pap, S->near_zero);
   double rr = 0.0;
-  for (int row = r0 + (int)threadIdx.x; row < r1; row += R2 * kBlock) {
-    double xv[R2], pv[R2], rv[R2], apv[R2], rs[R2][KD], as[R2][KD];
-    V gv[R2][KD];
-    int rw[R2];
+  for (int row = row_first; row < r1; row += kBlock) {
+    if (row != row_first) load(row);
+    a.x[row] = xv + alpha * pv;
+    const double ri = rv + (-alpha) * apv;
+    rn[row] = ri;
+    rr += ri * ri;
+    V acc = 0;
 #pragma unroll
-    for (int r = 0; r < R2; r++) {
-      rw[r] = min(row + r * kBlock, r1 - 1);
-      xv[r] = a.x[rw[r]];
-      pv[r] = pn[rw[r]];
-      rv[r] = rc[rw[r]];
-      apv[r] = a.ap[rw[r]];
-#pragma unroll
-      for (int k = 0; k < KD; k++) {
-        if (k < ndg) {
-          const long long src = (long long)rw[r] - off[k];
-          const long long sc = src < n ? src : rw[r];
-          gv[r][k] = gd_slot(gd, src, k, ndg, n);
-          rs[r][k] = rc[sc];
-          as[r][k] = a.ap[sc];
-        }
+    for (int k = KD - 1; k >= 0; k--) {
+      if (k < ndg && gv[k] != (V)0) {
+        const double rcv = rs[k] + (-alpha) * as[k];
+        if (MIX) acc = fmaf((float)gv[k], (float)rcv, (float)acc);
+        else acc = fma((double)gv[k], rcv, (double)acc);
       }
     }
-#pragma unroll
-    for (int r = 0; r < R2; r++) {
-      if (row + r * kBlock >= r1) break;
-      a.x[rw[r]] = xv[r] + alpha * pv[r];
-      const double ri = rv[r] + (-alpha) * apv[r];
-      rn[rw[r]] = ri;
-      rr += ri * ri;
-      V acc = 0;
-#pragma unroll
-      for (int k = KD - 1; k >= 0; k--) {
-        if (k < ndg && gv[r][k] != (V)0) {
-          const double rcv = rs[r][k] + (-alpha) * as[r][k];
-          if (MIX) acc = fmaf((float)gv[r][k], (float)rcv, (float)acc);
-          else acc = fma((double)gv[r][k], rcv, (double)acc);
-        }
-      }
-      if (MIX) a.t32[rw[r]] = (float)acc;
-      else a.t64[rw[r]] = (double)acc;
-    }
+    if (MIX) a.t32[row] = (float)acc;
+    else a.t64[row] = (double)acc;
   }
   rr = wg_sum(rr, lds);
   if (threadIdx.x == 0) {
-    a.prr[par][b] = rr;
+    CG_AT(prr, par)[b] = rr;
     if (b == b0) {
       S->true_res = 0;
       if (count) S->iters += 1;  // the test K1 made on this iteration passed
@@ -932,7 +1095,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz(CG_ARGS, int par_g, int mode) 
   const int rsel = mode == kAfterIter ? ((par_g ^ S->shift) & 1) ^ 1
                    : mode == kVerify  ? S->stop_par
                                       : 0;
-  const double *rc = a.r[rsel];
+  const double *rc = CG_AT(r, rsel);
   const V *gv = MIX ? (const V *)a.g_v32 : (const V *)a.g_v64;
   const V *tv = MIX ? (const V *)a.t32 : (const V *)a.t64;
   const int b0 = S->blk0;
@@ -1025,7 +1188,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz(CG_ARGS, int par_g, int mode) 
     }
   }
   rz = wg_sum(rz, lds);
-  if (threadIdx.x == 0) a.prz[rsel ^ 1][b] = rz;
+  if (threadIdx.x == 0) CG_AT(prz, rsel ^ 1)[b] = rz;
 }
 
 // t = G^T r for the current residual (replacement, verification, start).
@@ -1038,7 +1201,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_gtr(CG_ARGS, int par_g, int mode)
   CgSeg *S = a.seg + a.block_seg[b];
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
-  const double *rc = a.r[rsel];
+  const double *rc = CG_AT(r, rsel);
   const int r0 = S->row0 + (b - S->blk0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
   for (int row = r0 + (int)threadIdx.x; row < r1; row += kBlock) {
@@ -1068,7 +1231,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_gtr_gdia(CG_ARGS, int par_g, int 
   CgSeg *S = a.seg + a.block_seg[b];
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
-  const double *rc = a.r[rsel];
+  const double *rc = CG_AT(r, rsel);
   const V *gd = MIX ? (const V *)a.gd32 : (const V *)a.gd64;
   const int ndg = a.gndiag;
   const long long n = a.ncol;
@@ -1092,7 +1255,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_gtr_gdia(CG_ARGS, int par_g, int 
 // K3 with G on diagonals: z_i = sum over G's row i in ascending column
 // (ascending offset) of G_{i,i+o_k} t_{i+o_k}, zero slots skipped; r.z
 // partials.  Rows two per thread and trip, loads of both issued first.
-template <bool MIX, int KD>
+template <bool MIX, int KD, bool WIDE>
 __global__ __launch_bounds__(kBlock) void k_cg_gz_gdia(CG_ARGS, int par_g, int mode) {
   TBSLA_NO_FMA
   CG_BIND;
@@ -1102,9 +1265,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz_gdia(CG_ARGS, int par_g, int m
   __shared__ int s_flag;
   const int b = blockIdx.x;
   CgSeg *S = a.seg + a.block_seg[b];
-  int rsel;
-  if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
-  const double *rc = a.r[rsel];
+  const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
+  const int rsel = mode == kAfterIter ? ((par_g ^ S->shift) & 1) ^ 1
+                   : mode == kVerify  ? S->stop_par
+                                      : 0;
+  const double *rc = CG_AT(r, rsel);
   const V *gd = MIX ? (const V *)a.gd32 : (const V *)a.gd64;
   const V *tv = MIX ? (const V *)a.t32 : (const V *)a.t64;
   const int ndg = a.gndiag;
@@ -1113,24 +1278,37 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz_gdia(CG_ARGS, int par_g, int m
   int off[KD];
 #pragma unroll
   for (int k = 0; k < KD; k++) off[k] = k < ndg ? a.gdoff[k] : 0;
-  double rz = 0.0;
-  for (int row = r0 + (int)threadIdx.x; row < r1; row += R2 * kBlock) {
-    V gv[R2][KD], tq[R2][KD];
-    double rv[R2];
-    int rw[R2];
+  const int row_first = r0 + (int)threadIdx.x;
+  V gv[R2][KD], tq[R2][KD];
+  double rv[R2];
+  int rw[R2];
+  auto load = [&](int row) {
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       rw[r] = min(row + r * kBlock, r1 - 1);
-      rv[r] = rc[rw[r]];
+      rv[r] = ldi<WIDE>(rc, rw[r]);
 #pragma unroll
       for (int k = 0; k < KD; k++) {
         if (k < ndg) {
           const int c = rw[r] + off[k];
-          gv[r][k] = gd[dia_at(rw[r], k, ndg)];
-          tq[r][k] = tv[c >= 0 ? c : rw[r]];
+          gv[r][k] = ldi<WIDE>(gd, dia_at(rw[r], k, ndg));
+          tq[r][k] = ldi<WIDE>(tv, c >= 0 ? c : rw[r]);
         }
       }
     }
+  };
+  load(row_first);  // before the done flag is shared, as k_cg_gz
+  __builtin_amdgcn_sched_barrier(0);
+  if (threadIdx.x == 0) s_flag = flag;
+  __syncthreads();
+  const int fl = s_flag;
+  const bool part = mode == kAfterIter ? fl == kRunning
+                    : mode == kVerify  ? fl == kPending
+                                       : fl != kInactive;
+  if (!part) return;
+  double rz = 0.0;
+  for (int row = row_first; row < r1; row += R2 * kBlock) {
+    if (row != row_first) load(row);
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       if (row + r * kBlock >= r1) break;
@@ -1147,7 +1325,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz_gdia(CG_ARGS, int par_g, int m
     }
   }
   rz = wg_sum(rz, lds);
-  if (threadIdx.x == 0) a.prz[rsel ^ 1][b] = rz;
+  if (threadIdx.x == 0) CG_AT(prz, rsel ^ 1)[b] = rz;
 }
 
 // The entries' offsets col - row of kProbeRows rows spread over the block
@@ -1211,7 +1389,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_residual(CG_ARGS, int use_ax, int
   CgSeg *S = a.seg + sid;
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
-  double *rc = a.r[rsel];
+  double *rc = CG_AT(r, rsel);
   const int b0 = S->blk0;
   const int r0 = S->row0 + (b - b0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
@@ -1228,7 +1406,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_residual(CG_ARGS, int use_ax, int
     }
     if (mode == kStart) {
       if (zero_x) a.x[row] = 0.0;
-      a.p[0][row] = 0.0;
+      CG_AT(p, 0)[row] = 0.0;
       bb += bi * bi;
     }
   }
@@ -1236,11 +1414,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_residual(CG_ARGS, int use_ax, int
   if (PRE == 1) rz = wg_sum(rz, lds);
   if (mode == kStart) bb = wg_sum(bb, lds);
   if (threadIdx.x == 0) {
-    a.prr[rsel ^ 1][b] = rr;
-    if (PRE == 0) a.prz[rsel ^ 1][b] = rr;
-    if (PRE == 1) a.prz[rsel ^ 1][b] = rz;
+    CG_AT(prr, rsel ^ 1)[b] = rr;
+    if (PRE == 0) CG_AT(prz, rsel ^ 1)[b] = rr;
+    if (PRE == 1) CG_AT(prz, rsel ^ 1)[b] = rz;
     if (mode == kStart) {
-      a.prz[0][b] = b == b0 ? INFINITY : 0.0;  // the first beta is 0
+      CG_AT(prz, 0)[b] = b == b0 ? INFINITY : 0.0;  // the first beta is 0
       a.ppap[b] = bb;
     }
     if (b == b0) S->true_res = 1;
@@ -1262,7 +1440,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_start(CG_ARGS, double tol, int re
   (void)lds;
   (void)sid;
   double t[3];
-  seg_sums(a.ppap, a.prr[1], nullptr, 2, S->blk0, S->blk1, t);
+  seg_sums(a.ppap, CG_AT(prr, 1), nullptr, 2, S->blk0, S->blk1, t);
   const double bb = t[0], rr = t[1];
   if (threadIdx.x == 0) {
     S->stop = relative ? tol * sqrt(bb) : tol;
@@ -1270,6 +1448,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_start(CG_ARGS, double tol, int re
     S->rnorm0 = sqrt(rr);
     S->rnorm = S->rnorm0;
     S->iters = 0;
+    S->ent0 = a.rowptr[S->row0];
     S->shift = 0;
     S->true_res = 1;
     S->t_done = 0;
@@ -1291,7 +1470,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_vcheck(CG_ARGS, int j) {
   (void)lds;
   (void)sid;
   double t[3];
-  seg_sums(a.prr[S->stop_par ^ 1], nullptr, nullptr, 1, S->blk0, S->blk1, t);
+  seg_sums(CG_AT(prr, S->stop_par ^ 1), nullptr, nullptr, 1, S->blk0, S->blk1, t);
   const double rr = t[0];
   if (threadIdx.x == 0) {
     const double rn = sqrt(rr);
@@ -1311,7 +1490,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_vcheck(CG_ARGS, int j) {
   }
   __syncthreads();
   if (!(sqrt(rr) < S->stop)) {
-    double *old_rz = a.prz[S->stop_par];
+    double *old_rz = CG_AT(prz, S->stop_par);
     for (int k = S->blk0 + (int)threadIdx.x; k < S->blk1; k += kBlock)
       old_rz[k] = k == S->blk0 ? INFINITY : 0.0;
   }
@@ -1332,10 +1511,24 @@ __global__ __launch_bounds__(kBlock) void k_cg_ax(CG_ARGS, int par_g, int mode) 
   const int r0 = S->row0 + (b - S->blk0) * S->rpb;
   const int r1 = min(S->row1, r0 + S->rpb);
   const int lane = threadIdx.x & (L - 1);
-  for (int row = r0 + (int)threadIdx.x / L; row < r1; row += kBlock / L) {
+  typedef CgRow<L, double> Row;
+  constexpr int PASS = kBlock / L;
+  for (int row = r0 + (int)threadIdx.x / L; row < r1; row += PASS) {
+    Row w;
+    w.extent(a.rowptr, row, S->ent0);
+    w.template load<false>(a.colidx, a.val64, a.a_nnz, a.f_col, lane);
+    double g[Row::P];
+#pragma unroll
+    for (int k = 0; k < Row::P; k++) g[k] = a.x[w.col[k]];
     double acc = 0.0;
-    for (int j = a.rowptr[row] + lane; j < a.rowptr[row + 1]; j += L)
-      acc = fma(a.val64[j], a.x[a.colidx[j] - a.f_col], acc);
+#pragma unroll
+    for (int k = 0; k < Row::P; k++)
+      if (w.in(lane, k)) acc = fma(w.v[k], g[k], acc);
+    constexpr int Q = L == 1 ? 1 : 4;
+    for (int j = w.rest(lane); j < w.end; j += Q * L)
+#pragma unroll
+      for (int q = 0; q < Q; q++)
+        if (j + q < w.end) acc = fma(a.val64[j + q], a.x[a.colidx[j + q] - a.f_col], acc);
     acc = lane_sum<L>(acc);
     if (lane == 0) ax[row] = acc;
   }
@@ -1567,9 +1760,11 @@ namespace {
 struct Plan {
   int L, pre, mixed, replace, verify, stall;
   bool dia;   // K1 reads A's diagonal layout
+  int dkd;    // its kernel's diagonals: 3, 5 or 7, or 0 for any number
   bool two;   // K1 in two passes (k_cg_pnew, then k_cg_ap) on A's CSR rows
   bool gdia;  // M = G G^T applied from G's diagonals
   int gkd;    // their kernels' capacity: 4 or 8 diagonals
+  bool wide;  // vectors or G's diagonals of 4 GiB or more (64-bit offsets)
   long long n;
   int nblocks;
   const CgArgs *args;  // device argument block
@@ -1586,16 +1781,27 @@ void launch_k1(const Plan &p, int par, int check, int check_only) {
   if (!check_only) k_cg_ap<L, MIX><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par);
 }
 
+template <int KD>
+void launch_k1_dia(const Plan &p, bool zbuf, int par, int check, int check_only) {
+  const int g = p.nblocks;
+  if (p.mixed) {
+    if (zbuf) k_cg_spmv_dia<true, true, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+    else k_cg_spmv_dia<true, false, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+  } else {
+    if (zbuf) k_cg_spmv_dia<false, true, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+    else k_cg_spmv_dia<false, false, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+  }
+}
+
 template <int L>
 void launch_k1_l(const Plan &p, int par, int check, int check_only) {
   const bool zbuf = p.pre != 0;
   if (p.dia) {
-    if (p.mixed) {
-      if (zbuf) k_cg_spmv_dia<true, true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, check, check_only);
-      else k_cg_spmv_dia<true, false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, check, check_only);
-    } else {
-      if (zbuf) k_cg_spmv_dia<false, true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, check, check_only);
-      else k_cg_spmv_dia<false, false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+    switch (p.dkd) {
+      case 3: launch_k1_dia<3>(p, zbuf, par, check, check_only); break;
+      case 5: launch_k1_dia<5>(p, zbuf, par, check, check_only); break;
+      case 7: launch_k1_dia<7>(p, zbuf, par, check, check_only); break;
+      default: launch_k1_dia<0>(p, zbuf, par, check, check_only); break;
     }
     return;
   }
@@ -1620,6 +1826,18 @@ void launch_k1_any(const Plan &p, int par, int check, int check_only) {
   }
 }
 
+template <bool WIDE>
+void launch_k2_gdia(const Plan &p, int par, int count) {
+  const int g = p.nblocks;
+  if (p.gkd == 4) {
+    if (p.mixed) k_cg_update_gdia<true, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    else k_cg_update_gdia<false, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+  } else {
+    if (p.mixed) k_cg_update_gdia<true, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    else k_cg_update_gdia<false, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+  }
+}
+
 void launch_k2(const Plan &p, int par, int count) {
   const int g = p.nblocks;
   if (p.pre == 0) {
@@ -1629,28 +1847,30 @@ void launch_k2(const Plan &p, int par, int count) {
     if (p.mixed) k_cg_update<1, true><<<g, kBlock, 0, p.s>>>(p.args, par, count);
     else k_cg_update<1, false><<<g, kBlock, 0, p.s>>>(p.args, par, count);
   } else if (p.gdia) {
-    if (p.gkd == 4) {
-      if (p.mixed) k_cg_update_gdia<true, 4><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-      else k_cg_update_gdia<false, 4><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    } else {
-      if (p.mixed) k_cg_update_gdia<true, 8><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-      else k_cg_update_gdia<false, 8><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    }
+    if (p.wide) launch_k2_gdia<true>(p, par, count);
+    else launch_k2_gdia<false>(p, par, count);
   } else {
     if (p.mixed) k_cg_update<2, true><<<g, kBlock, 0, p.s>>>(p.args, par, count);
     else k_cg_update<2, false><<<g, kBlock, 0, p.s>>>(p.args, par, count);
   }
 }
 
+template <bool WIDE>
+void launch_gz_gdia(const Plan &p, int par, int mode) {
+  const int g = p.nblocks;
+  if (p.gkd == 4) {
+    if (p.mixed) k_cg_gz_gdia<true, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
+    else k_cg_gz_gdia<false, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
+  } else {
+    if (p.mixed) k_cg_gz_gdia<true, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
+    else k_cg_gz_gdia<false, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
+  }
+}
+
 void launch_gz(const Plan &p, int par, int mode) {
   if (p.gdia) {
-    if (p.gkd == 4) {
-      if (p.mixed) k_cg_gz_gdia<true, 4><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-      else k_cg_gz_gdia<false, 4><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-    } else {
-      if (p.mixed) k_cg_gz_gdia<true, 8><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-      else k_cg_gz_gdia<false, 8><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-    }
+    if (p.wide) launch_gz_gdia<true>(p, par, mode);
+    else launch_gz_gdia<false>(p, par, mode);
   } else {
     if (p.mixed) k_cg_gz<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
     else k_cg_gz<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
@@ -1859,9 +2079,18 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   hs.assign(nsys, CgSeg{});
   hb.clear();
   const long long pass_rows = kBlock / L;
+  // A batch (or the same cap asked for, so that a system alone and in a batch
+  // is laid out alike): at least kBlock rows per workgroup, a row per thread in
+  // K2 and in the first pass of K1.  96 systems of 4,096 to 65,536 rows, L = 8:
+  // 96 rows a workgroup left five threads in eight idle there (over a solve K1a
+  // took 40 and K2 54 us on average, 21 and 28 so).
+  const bool batch_layout = o.max_blocks_per_system > 0
+                                ? o.max_blocks_per_system <= kBatchBlocksPerSystem
+                                : nsys > 1;
+  const long long min_rpb = batch_layout ? kBlock : pass_rows;
   for (int k = 0; k < nsys; k++) {
     const long long rows = h_rows[k + 1] - h_rows[k];
-    long long rpb = std::max<long long>(pass_rows, (rows + cap - 1) / cap);
+    long long rpb = std::max<long long>(min_rpb, (rows + cap - 1) / cap);
     rpb = (rpb + pass_rows - 1) / pass_rows * pass_rows;
     const int nb = (int)((rows + rpb - 1) / rpb);
     CgSeg &S = hs[k];
@@ -2074,6 +2303,10 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   p.verify = a.verify;
   p.stall = o.stall_window;
   p.dia = dia;
+  const long long most = 1LL << 32;
+  const bool narrow_a = (n + kWave) * std::max(ndiag, 1) * 8 < most;
+  p.dkd = dia && narrow_a && (ndiag == 3 || ndiag == 5 || ndiag == 7) ? ndiag : 0;
+  p.wide = (n + kWave) * std::max(gndiag, 1) * 8 >= most;
   p.two = two;
   p.gdia = gdia;
   p.gkd = gndiag <= 4 ? 4 : 8;
@@ -2145,8 +2378,8 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   key.batch = B;
   key.nblocks = nblocks;
   key.verify = p.verify;
-  key.dia = p.dia ? 1 : 0;
-  key.gdia = p.gdia ? p.gkd : 0;
+  key.dia = p.dia ? 1 + p.dkd : 0;
+  key.gdia = p.gdia ? p.gkd + (p.wide ? 16 : 0) : 0;
   key.two = p.two ? 1 : 0;
   // the graph set of this plan, captured and instantiated once; the least
   // recently used set is destroyed when kGraphSets are held (the stream is

@@ -267,7 +267,9 @@ void cg_cache_release(tbsla_hip_matrix_s *m);
 void split_release(tbsla_hip_matrix_s *m);
 // Device memory of the library's own objects (capi.hip): device_free waits for
 // the device's queued work, as hipFree does, and keeps the block for a later
-// device_alloc of about its size.
+// device_alloc of about its size.  At least 32 readable bytes follow the bytes
+// asked for, so a load of four entries that starts inside an array stays in the
+// block.
 int device_alloc(void **p, size_t bytes);
 void device_free(void *p);
 }  // namespace tbsla_hip
