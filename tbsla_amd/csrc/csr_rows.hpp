@@ -72,20 +72,12 @@ __device__ inline void csr_load(const int *ci, const double *va, int j, int (&c)
   }
 }
 
-template <int V, int L, int R, int NT, bool SPLIT>
-__global__ __launch_bounds__(kBlock) void k_csr_rows(CsrRowsArgs a) {
-  if (a.done && *a.done) return;
+// The sums of the wavefront's rows base + r G + g, r < R (G = 64 / L), in every
+// lane of group g
+template <int V, int L, int R, int NT>
+__device__ inline void csr_row_sums(const CsrRowsArgs &a, long long base, int lane, int g,
+                                    double (&sum)[R]) {
   constexpr int G = kWave / L;
-  const int lane = threadIdx.x & (L - 1);
-  const int g = (threadIdx.x & (kWave - 1)) / L;
-  const long long wave = ((long long)blockIdx.x * kBlock + threadIdx.x) / kWave;
-  const long long base = wave * (G * R);
-  if (base >= a.n_rows) return;
-  if (a.seg_offs) {  // wave-uniform
-    const long long last = min(base + G * R, a.n_rows) - 1;
-    const int k0 = seg_of_row(a.seg_offs, a.nseg, base);
-    if (a.seg_done[k0] && (last < a.seg_offs[k0 + 1])) return;
-  }
   int beg[R], end[R];
   int len = 0;
 #pragma unroll
@@ -102,7 +94,6 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows(CsrRowsArgs a) {
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) len = max(len, __shfl_xor(len, off, kWave));
   const int trips = (len + V * L - 1) / (V * L);
-  double sum[R];
 #pragma unroll
   for (int r = 0; r < R; r++) sum[r] = 0.0;
   for (int t = 0; t < trips; t++) {
@@ -133,10 +124,29 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows(CsrRowsArgs a) {
       for (int k = 0; k < V; k++) sum[r] = fma(v[r][k], a.x[c[r][k]], sum[r]);
   }
 #pragma unroll
+  for (int r = 0; r < R; r++) sum[r] = group_sum<L>(sum[r]);
+}
+
+template <int V, int L, int R, int NT, bool SPLIT>
+__global__ __launch_bounds__(kBlock) void k_csr_rows(CsrRowsArgs a) {
+  if (a.done && *a.done) return;
+  constexpr int G = kWave / L;
+  const int lane = threadIdx.x & (L - 1);
+  const int g = (threadIdx.x & (kWave - 1)) / L;
+  const long long wave = ((long long)blockIdx.x * kBlock + threadIdx.x) / kWave;
+  const long long base = wave * (G * R);
+  if (base >= a.n_rows) return;
+  if (a.seg_offs) {  // wave-uniform
+    const long long last = min(base + G * R, a.n_rows) - 1;
+    const int k0 = seg_of_row(a.seg_offs, a.nseg, base);
+    if (a.seg_done[k0] && (last < a.seg_offs[k0 + 1])) return;
+  }
+  double sum[R];
+  csr_row_sums<V, L, R, NT>(a, base, lane, g, sum);
+#pragma unroll
   for (int r = 0; r < R; r++) {
-    const double s = group_sum<L>(sum[r]);
     const long long row = base + r * G + g;
-    if (lane == 0 && row < a.n_rows) a.y[row] = SPLIT ? s + a.add[row] : s;
+    if (lane == 0 && row < a.n_rows) a.y[row] = SPLIT ? sum[r] + a.add[row] : sum[r];
   }
 }
 

@@ -69,6 +69,12 @@ struct PrFuse {
   double *p_err, *p_sum;
 };
 int split_pr_blocks(const tbsla_hip_matrix_s *m);
+// The same on the CSR row kernel (spmv.hip): for a square block on the diagonal
+// whose row kernel has a fused form; nb workgroups and partials, those of
+// k_pr_update on its grid of nb
+bool csr_pr_fits(const tbsla_hip_matrix_s *m);
+int csr_pr_launch(const tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf, const int *done,
+                  unsigned nb, hipStream_t s);
 int split_launch_pr(tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf, const int *done,
                     hipStream_t s);
 // The row pointer of a COO / SCOO block's n row-sorted triplets over their

@@ -18,7 +18,8 @@ namespace tbsla_hip {
 
 namespace {
 
-constexpr int kRedBlocks = 512;  // reduction grid (fixed: the partial layout is part of the order)
+// reduction grid (fixed: the partial layout is part of the order)
+constexpr int kRedBlocks = 2048;
 
 struct SolverState {
   double S;      // sum of the current iterate
@@ -280,11 +281,26 @@ __global__ __launch_bounds__(kBlock) void k_prm_max(PrmState *__restrict__ st,
                                                     const double *__restrict__ p_min, int nb,
                                                     double beta) {
   TBSLA_NO_FMA
-  if (st->done || threadIdx.x != 0) return;
+  __shared__ double lmax[kBlock / kWave], lmin[kBlock / kWave];
+  if (st->done) return;
   double hi = -INFINITY, lo = INFINITY;
-  for (int i = 0; i < nb; i++) {
+  for (int i = threadIdx.x; i < nb; i += kBlock) {
     hi = fmax(hi, p_max[i]);
     lo = fmin(lo, p_min[i]);
+  }
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    hi = fmax(hi, __shfl_xor(hi, o, kWave));
+    lo = fmin(lo, __shfl_xor(lo, o, kWave));
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    lmax[threadIdx.x / kWave] = hi;
+    lmin[threadIdx.x / kWave] = lo;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < kBlock / kWave; w++) {
+    hi = fmax(hi, lmax[w]);
+    lo = fmin(lo, lmin[w]);
   }
   const double e = beta >= 0 ? hi : lo;
   st->maxv = beta * e + st->T;
@@ -593,15 +609,17 @@ extern "C" int tbsla_hip_page_rank(tbsla_hip_matrix_t m, double beta, double eps
   }
   // a square block on the diagonal in the diagonal layout's LDS-slice form:
   // SpMV and update in one pass (split_launch_pr), one partial per row block
-  const int fused = (r_start == 0 && s_start == 0 && length == ln_col && ln_row == ln_col)
-                        ? split_pr_blocks(m)
-                        : 0;
+  const bool diagonal = r_start == 0 && s_start == 0 && length == ln_col && ln_row == ln_col;
+  const int fused = diagonal ? split_pr_blocks(m) : 0;
+  // such a block on its rows: SpMV and update in one pass too, with the
+  // partials of the separate update
+  const bool rows_fused = diagonal && !fused && csr_pr_fits(m);
   const long long np = std::max<long long>(kRedBlocks, fused);  // partials of each kind
   DevBuf<double> bufA, bufB, y, part;
   DevBuf<SolverState> st;
   TBSLA_TRY(bufA.alloc(ln_col));
   TBSLA_TRY(bufB.alloc(ln_col));
-  if (!fused) TBSLA_TRY(y.alloc(ylen));
+  if (!fused && !rows_fused) TBSLA_TRY(y.alloc(ylen));
   TBSLA_TRY(part.alloc(2 * np + 8));
   TBSLA_TRY(st.alloc(1));
   TBSLA_TRY(launch_fill(bufA.p, ln_col, 1.0, s));  // b = 1 (Matrix.cpp:549-552)
@@ -618,6 +636,9 @@ extern "C" int tbsla_hip_page_rank(tbsla_hip_matrix_t m, double beta, double eps
       if (fused) {
         const PrFuse pf{bn, &st.p->S, beta, (double)m->n_col, part.p, part.p + np};
         TBSLA_TRY(split_launch_pr(m, bt, pf, &st.p->done, s));
+      } else if (rows_fused) {
+        const PrFuse pf{bn, &st.p->S, beta, (double)m->n_col, part.p, part.p + np};
+        TBSLA_TRY(csr_pr_launch(m, bt, pf, &st.p->done, nb, s));
       } else {
         TBSLA_TRY(spmv_launch(m, y.p, bt, 0, true, s, &st.p->done));
         k_pr_update<<<nb, kBlock, 0, s>>>(ln_col, y.p, bt, bn, r_start, s_start, length, beta,
