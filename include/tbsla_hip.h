@@ -199,7 +199,8 @@ int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_matrix_t coo
  * b = col; v = values.  For zero-copy interoperation: read them freely;
  * writes through them bypass the copies the library derives from the
  * arrays (the split and diagonal CSR layouts, the mixed CG's FP32 values,
- * the COO row pointer): call tbsla_hip_values_changed after them. */
+ * the COO row pointer, the triplets' order): call tbsla_hip_values_changed after
+ * them. */
 int tbsla_hip_device_arrays(tbsla_hip_matrix_t m, void **d_a, void **d_b, void **d_v);
 /* After writes through tbsla_hip_device_arrays (values or indices): rebuilds
  * the split/diagonal execution layout from the arrays, drops the COO row

@@ -203,6 +203,7 @@ void release_arrays(tbsla_hip_matrix_s *m) {
   m->rowptr = m->colidx = m->rowidx = nullptr;
   m->values = nullptr;
   m->values_version++;
+  m->col_sorted = 0;
   m->has_arrays = 0;
   m->stored = 0;
 }
@@ -534,6 +535,7 @@ int tbsla_hip_import(tbsla_hip_matrix_t m, int format, const tbsla_hip_geometry 
           m->row_sorted = 0;
           break;
         }
+      m->col_sorted = h_b != nullptr && std::is_sorted(h_b, h_b + st);
       TBSLA_TRY(h2d((void **)&m->rowidx, h_a, st * sizeof(int)));
       TBSLA_TRY(h2d((void **)&m->colidx, h_b, st * sizeof(int)));
       TBSLA_TRY(h2d((void **)&m->values, h_v, st * sizeof(double)));

@@ -232,6 +232,7 @@ struct tbsla_hip_matrix_s {
   int max_col = 0;       // ELL
   int has_arrays = 0;    // the reference allocated its arrays (fills can skip it)
   int row_sorted = 1;    // COO/SCOO triplets in nondecreasing row order
+  int col_sorted = 0;    // COO triplets known to be in nondecreasing column order
   // device arrays (owned)
   int *rowptr = nullptr;     // CSR: ln_row + 1
   int *colidx = nullptr;     // CSR: stored;  ELL: max_col * ln_row, column-major

@@ -37,6 +37,20 @@ int launch_axpy_inplace(double *y, const double *x, long long n, hipStream_t s);
 // other).  Synchronises the stream.
 template <typename K>
 int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s);
+// Keys taken from column indices: the local column, or ln_col outside the block.
+struct ColumnKeys {
+  const int *cols;
+  int f_col;
+  unsigned ln_col;
+  __device__ inline unsigned operator[](long long i) const {
+    const unsigned c = (unsigned)(cols[i] - f_col);
+    return c < ln_col ? c : ln_col;
+  }
+};
+// radix_sort_pairs<unsigned> of src's n keys, read by the first pass in place of
+// *keys (whose contents are ignored)
+int radix_sort_columns(const ColumnKeys &src, unsigned **keys, int **payload, long long n,
+                       int key_bits, hipStream_t s);
 // ptr[b] = the first k with (keys[k] >> shift) >= b, b in [0, nb], of n sorted keys
 template <typename K>
 int bucket_starts(const K *keys, long long n, int shift, long long nb, int *ptr, hipStream_t s);

@@ -54,23 +54,23 @@ unsigned red_grid(long long n) {
 
 // ---- column sums --------------------------------------------------------
 
-// key = local column; the sort's payload is the entry's position in the
-// reference's loop order (CSR/SCOO: storage order; ELL: row-major slot i*max_col+j).  Entries
+// The sort's keys are the local columns, its payload the entry's position in the
+// reference's loop order (CSR/SCOO: storage order, keys read from the column
+// array by the first pass; ELL: row-major slot i*max_col+j, here).  Entries
 // the reference skips -- ELL slots whose value is not positive
 // (MatrixELL.cpp:812), which include the padding (column 0, possibly left of
 // the block) -- and any column outside [0, ln_col) get the key ln_col, a
 // bucket after the last column that no sum reads.
-__global__ __launch_bounds__(kBlock) void k_colkeys(long long n, int fmt, long long ln_row,
-                                                    long long ln_col, int max_col,
-                                                    const int *__restrict__ cols,
-                                                    const double *__restrict__ vals, int f_col,
-                                                    unsigned *__restrict__ keys) {
+__global__ __launch_bounds__(kBlock) void k_ell_colkeys(long long n, long long ln_row,
+                                                        long long ln_col, int max_col,
+                                                        const int *__restrict__ cols,
+                                                        const double *__restrict__ vals, int f_col,
+                                                        unsigned *__restrict__ keys) {
   long long p = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (p >= n) return;
-  long long src = p;
-  if (fmt == TBSLA_HIP_ELL) src = (p % max_col) * ln_row + p / max_col;
-  long long c = (long long)cols[src] - f_col;
-  bool keep = c >= 0 && c < ln_col && (fmt != TBSLA_HIP_ELL || vals[src] > 0);
+  const long long src = (p % max_col) * ln_row + p / max_col;
+  const long long c = (long long)cols[src] - f_col;
+  const bool keep = c >= 0 && c < ln_col && vals[src] > 0;
   keys[p] = keep ? (unsigned)c : (unsigned)ln_col;
 }
 
@@ -522,6 +522,7 @@ extern "C" int tbsla_hip_values_changed(tbsla_hip_matrix_t m, void *stream) {
   }
   if (m->format == TBSLA_HIP_COO || m->format == TBSLA_HIP_SCOO) {
     m->row_sorted = 1;
+    m->col_sorted = 0;
     // a derived layout over the triplets' rows is rebuilt from the new row
     // pointer, or dropped when the triplets are no longer sorted by row
     if (m->split) {
@@ -548,12 +549,17 @@ extern "C" int tbsla_hip_get_col_sums(tbsla_hip_matrix_t m, double *d_s, void *s
   TBSLA_TRY(keys.alloc(n));
   TBSLA_TRY(pos.alloc(n));
   TBSLA_TRY(colptr.alloc(ln_col + 1));
-  k_colkeys<<<grid_for(n), kBlock, 0, s>>>(n, fmt, m->ln_row, ln_col, m->max_col, m->colidx,
-                                           m->values, m->f_col, keys.p);
-  TBSLA_HIP_LAUNCH_CHECK();
   int bits = 1;
   while (bits < 32 && (1LL << bits) <= ln_col) bits++;  // keys <= ln_col < 2^bits
-  TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s));
+  if (fmt == TBSLA_HIP_ELL) {
+    k_ell_colkeys<<<grid_for(n), kBlock, 0, s>>>(n, m->ln_row, ln_col, m->max_col, m->colidx,
+                                                 m->values, m->f_col, keys.p);
+    TBSLA_HIP_LAUNCH_CHECK();
+    TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s));
+  } else {
+    const ColumnKeys src{m->colidx, m->f_col, (unsigned)ln_col};
+    TBSLA_TRY(radix_sort_columns(src, &keys.p, &pos.p, n, bits, s));
+  }
   TBSLA_TRY(bucket_starts<unsigned>(keys.p, n, 0, ln_col, colptr.p, s));
   if (ln_col > 0) {
     k_col_sums<<<grid_for(ln_col), kBlock, 0, s>>>(ln_col, fmt, m->ln_row, m->max_col, colptr.p,

@@ -32,13 +32,13 @@ struct SortTile {
   static constexpr int waves = threads / kWave;
 };
 
-// Digit counts of each tile.  Per-wave counters in LDS; a round whose lanes all
-// hold one digit (the high digits of a banded or sorted input) is counted by
-// one lane instead of 64 additions to one address.
-template <typename K>
+// Digit counts of each tile.  Per-wave counters in LDS; the lanes of a round that
+// hold its first lane's digit (most of them in the high digits of a banded or
+// sorted input) are counted by that lane instead of added one by one to one
+// address.  keys: an array, or a source with its operator[] (ColumnKeys).
+template <typename K, typename Src>
 __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_hist(
-    const K *__restrict__ keys, long long n, int shift, int mask, long long ntiles,
-    int *__restrict__ hist) {
+    const Src keys, long long n, int shift, int mask, long long ntiles, int *__restrict__ hist) {
   typedef SortTile<K> T;
   __shared__ int h[T::waves][kRadix];
   for (int i = threadIdx.x; i < T::waves * kRadix; i += T::threads) (&h[0][0])[i] = 0;
@@ -55,13 +55,10 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_hist(
   for (int i = 0; i < kItems; i++) {
     const bool valid = base + i * T::threads < n;
     const int d = (int)(key[i] >> shift) & mask;
-    const unsigned long long in = __ballot(valid);
     const int first = __builtin_amdgcn_readfirstlane(d);
-    if (in == ~0ull && __ballot(d == first) == ~0ull) {
-      if (lane == 0) atomicAdd(&h[wave][first], kWave);
-    } else if (valid) {
-      atomicAdd(&h[wave][d], 1);
-    }
+    const unsigned long long same = __ballot(valid && d == first);
+    if (lane == 0 && same) atomicAdd(&h[wave][first], __popcll(same));
+    if (valid && d != first) atomicAdd(&h[wave][d], 1);
   }
   __syncthreads();
   for (int d = threadIdx.x; d <= mask; d += T::threads) {
@@ -75,9 +72,9 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_hist(
 // (the first pass).  Bound by its bytes once the output runs are whole: 24 M
 // 32-bit keys take 101 us a pass (16 bytes an element, 3.8 TB/s) where
 // the scatter from registers, with 64-bit keys read twice, took 290 (2.0 TB/s).
-template <typename K>
+template <typename K, typename Src>
 __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
-    const K *__restrict__ keys_in, const int *__restrict__ pay_in, K *__restrict__ keys_out,
+    const Src keys_in, const int *__restrict__ pay_in, K *__restrict__ keys_out,
     int *__restrict__ pay_out, long long n, int shift, int bits, long long ntiles,
     const int *__restrict__ offsets) {
   typedef SortTile<K> T;
@@ -183,19 +180,30 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
 // ptr[b] = the first k with (keys[k] >> shift) >= b, for b in [0, nb]: the
 // bucket starts of sorted keys, by binary search (no atomics: counting 24 M
 // banded keys by atomic additions took 1053 us, and 4.8 M with hub rows 317).
+// Two threads find the ends of their workgroup's 256 buckets among all keys,
+// the others search between them.
 template <typename K>
-__global__ __launch_bounds__(kBlock) void k_bucket_starts(const K *__restrict__ keys, long long n,
-                                                          int shift, long long nb,
-                                                          int *__restrict__ ptr) {
-  const long long b = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (b > nb) return;
-  long long lo = 0, hi = n;
+__device__ inline long long first_at_least(const K *__restrict__ keys, int shift, long long lo,
+                                           long long hi, long long b) {
   while (lo < hi) {
     const long long mid = (lo + hi) >> 1;
     if ((long long)(keys[mid] >> shift) < b) lo = mid + 1;
     else hi = mid;
   }
-  ptr[b] = (int)lo;
+  return lo;
+}
+
+template <typename K>
+__global__ __launch_bounds__(kBlock) void k_bucket_starts(const K *__restrict__ keys, long long n,
+                                                          int shift, long long nb,
+                                                          int *__restrict__ ptr) {
+  __shared__ long long ends[2];
+  const long long b0 = (long long)blockIdx.x * kBlock, b = b0 + threadIdx.x;
+  if (threadIdx.x % kWave == 0 && threadIdx.x < 2 * kWave)
+    ends[threadIdx.x / kWave] =
+        first_at_least(keys, shift, 0, n, threadIdx.x ? b0 + kBlock : b0);
+  __syncthreads();
+  if (b <= nb) ptr[b] = (int)first_at_least(keys, shift, ends[0], ends[1], b);
 }
 
 template <typename K>
@@ -206,17 +214,20 @@ __global__ __launch_bounds__(kBlock) void k_coo_keys(const int *__restrict__ row
   if (i < n) keys[i] = ((K)(unsigned)rows[i] << col_bits) | (K)(cols ? (unsigned)cols[i] : 0u);
 }
 
-// columns from the keys' low bits, values by the sorted positions
+// columns from the keys' low bits (col_bits 0: by the sorted positions), values
+// by the sorted positions
 template <typename K>
 __global__ __launch_bounds__(kBlock) void k_gather_sorted(const K *__restrict__ keys, int col_bits,
                                                           const int *__restrict__ perm,
+                                                          const int *__restrict__ cols,
                                                           const double *__restrict__ vals,
                                                           long long n, int *__restrict__ cols_out,
                                                           double *__restrict__ vals_out) {
   long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  cols_out[i] = (int)(keys[i] & (((K)1 << col_bits) - 1));
-  vals_out[i] = vals[perm[i]];
+  const int p = perm[i];
+  cols_out[i] = col_bits ? (int)(keys[i] & (((K)1 << col_bits) - 1)) : cols[p];
+  vals_out[i] = vals[p];
 }
 
 // the longest row
@@ -285,8 +296,9 @@ int bits_for(long long v) {
 
 }  // namespace
 
-template <typename K>
-int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s) {
+template <typename K, typename Src>
+static int radix_sort_from(const Src *first, K **keys, int **payload, long long n, int key_bits,
+                           hipStream_t s) {
   typedef SortTile<K> T;
   if (n <= 0) return TBSLA_HIP_SUCCESS;
   const long long ntiles = (n + T::elems - 1) / T::elems;
@@ -313,12 +325,21 @@ int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStre
   }
   for (int p = 0; p < passes; p++) {
     const int shift = bits * p, b = std::min(bits, std::max(1, key_bits - shift));
-    k_digit_hist<K><<<(unsigned)ntiles, T::threads, 0, s>>>(*keys, n, shift, (1 << b) - 1, ntiles,
-                                                            hist);
+    const K *kin = *keys;
+    if (p == 0 && first)
+      k_digit_hist<K><<<(unsigned)ntiles, T::threads, 0, s>>>(*first, n, shift, (1 << b) - 1,
+                                                              ntiles, hist);
+    else
+      k_digit_hist<K><<<(unsigned)ntiles, T::threads, 0, s>>>(kin, n, shift, (1 << b) - 1, ntiles,
+                                                              hist);
     st = scan<int>(hist, hist, (1LL << b) * ntiles, false, nullptr, ws, s);
     if (st) break;
-    k_digit_scatter<K><<<(unsigned)ntiles, T::threads, 0, s>>>(
-        *keys, p > 0 ? *payload : nullptr, keys_alt, pay_alt, n, shift, b, ntiles, hist);
+    if (p == 0 && first)
+      k_digit_scatter<K><<<(unsigned)ntiles, T::threads, 0, s>>>(*first, nullptr, keys_alt, pay_alt,
+                                                                 n, shift, b, ntiles, hist);
+    else
+      k_digit_scatter<K><<<(unsigned)ntiles, T::threads, 0, s>>>(
+          kin, p > 0 ? *payload : nullptr, keys_alt, pay_alt, n, shift, b, ntiles, hist);
     std::swap(*keys, keys_alt);
     std::swap(*payload, pay_alt);
   }
@@ -327,6 +348,16 @@ int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStre
   if (st) return st;
   if (e != hipSuccess) return fail(TBSLA_HIP_ERR_HIP, std::string("radix sort: ") + hipGetErrorString(e));
   return TBSLA_HIP_SUCCESS;
+}
+
+template <typename K>
+int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s) {
+  return radix_sort_from<K, const K *>(nullptr, keys, payload, n, key_bits, s);
+}
+
+int radix_sort_columns(const ColumnKeys &src, unsigned **keys, int **payload, long long n,
+                       int key_bits, hipStream_t s) {
+  return radix_sort_from<unsigned, ColumnKeys>(&src, keys, payload, n, key_bits, s);
 }
 
 template int radix_sort_pairs<unsigned>(unsigned **, int **, long long, int, hipStream_t);
@@ -347,7 +378,10 @@ template int bucket_starts<unsigned long long>(const unsigned long long *, long 
 
 // The CSR arrays of n COO triplets: stable order by (row, col)
 // (csr::compare_row, src/cpp/utils/csr.cpp:3-8), 32-bit keys where both
-// indices fit.
+// indices fit.  col_bits 0: the triplets are in column order already (known from
+// the import, as a column-ordered file gives them), and the stable sort by row
+// keeps it -- three 32-bit passes instead of five 64-bit ones at 300,007 rows
+// (4.8 M triplets in column order: 450 -> 368 us with the two-launch prefix sums).
 template <typename K>
 static int coo_rows(const tbsla_hip_matrix_s *coo, long long n, int row_bits, int col_bits,
                     int *rowptr, int *cols, double *vals, hipStream_t s) {
@@ -357,12 +391,13 @@ static int coo_rows(const tbsla_hip_matrix_s *coo, long long n, int row_bits, in
   if (!(st = device_alloc((void **)&keys, (size_t)std::max(n, 1LL) * sizeof(K))) &&
       !(st = device_alloc((void **)&perm, (size_t)std::max(n, 1LL) * 4))) {
     if (n > 0)
-      k_coo_keys<K><<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, coo->colidx, n, col_bits, keys);
+      k_coo_keys<K><<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, col_bits ? coo->colidx : nullptr, n,
+                                                   col_bits, keys);
     st = radix_sort_pairs<K>(&keys, &perm, n, col_bits + row_bits, s);
     if (!st) st = bucket_starts<K>(keys, n, col_bits, coo->n_row, rowptr, s);
     if (!st && n > 0)
-      k_gather_sorted<K><<<grid_for(n), kBlock, 0, s>>>(keys, col_bits, perm, coo->values, n, cols,
-                                                        vals);
+      k_gather_sorted<K><<<grid_for(n), kBlock, 0, s>>>(keys, col_bits, perm, coo->colidx,
+                                                        coo->values, n, cols, vals);
     const hipError_t e = hipGetLastError();
     if (!st && e != hipSuccess) st = fail(TBSLA_HIP_ERR_HIP, hipGetErrorString(e));
   }
@@ -469,7 +504,7 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
   TBSLA_TRY(device_alloc((void **)&scol, (size_t)std::max(n, 1LL) * 4));
   TBSLA_TRY(device_alloc((void **)&sval, (size_t)std::max(n, 1LL) * 8));
   {
-    const int col_bits = bits_for(std::max(coo->n_col, 1));
+    const int col_bits = coo->col_sorted ? 0 : bits_for(std::max(coo->n_col, 1));
     const int row_bits = bits_for(std::max(coo->n_row, 1));
     const int st = col_bits + row_bits <= 32
                        ? coo_rows<unsigned>(coo, n, row_bits, col_bits, rowptr, scol, sval, s)
