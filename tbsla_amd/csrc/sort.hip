@@ -1,7 +1,7 @@
 // sort.hip -- stable LSD radix sort and the COO conversion constructors.
 //
-// Radix sort of 32- or 64-bit keys carrying each key's original position, in
-// digits of at most 8 bits.  Per pass: a per-tile digit histogram, one
+// Radix sort of 32- or 64-bit keys carrying each key's original position, and of
+// matrix entries by an index of theirs, in digits of at most 8 bits.  Per pass: a per-tile digit histogram, one
 // exclusive scan over the digit-major histogram, and a stable scatter.
 // Stability inside a tile comes from processing elements in index order: each
 // wavefront owns a contiguous sub-tile, walks it in 64-element rounds, finds
@@ -27,8 +27,18 @@ constexpr int kItems = 16;  // keys per thread of a tile
 // keys through LDS (four, or for 64-bit keys three to four, workgroups per CU).
 template <typename K>
 struct SortTile {
+  typedef K key;
+  static constexpr int items = kItems;
   static constexpr int threads = sizeof(K) == 4 ? 512 : 256;
   static constexpr int elems = threads * kItems;
+  static constexpr int waves = threads / kWave;
+};
+// of matrix entries (k_entry_scatter)
+struct EntryTile {
+  typedef unsigned key;
+  static constexpr int items = 8;
+  static constexpr int threads = 512;
+  static constexpr int elems = threads * items;
   static constexpr int waves = threads / kWave;
 };
 
@@ -36,10 +46,11 @@ struct SortTile {
 // hold its first lane's digit (most of them in the high digits of a banded or
 // sorted input) are counted by that lane instead of added one by one to one
 // address.  keys: an array, or a source with its operator[] (ColumnKeys).
-template <typename K, typename Src>
-__global__ __launch_bounds__(SortTile<K>::threads) void k_digit_hist(
+template <typename T, typename Src>
+__global__ __launch_bounds__(T::threads) void k_digit_hist(
     const Src keys, long long n, int shift, int mask, long long ntiles, int *__restrict__ hist) {
-  typedef SortTile<K> T;
+  typedef typename T::key K;
+  constexpr int kItems = T::items;
   __shared__ int h[T::waves][kRadix];
   for (int i = threadIdx.x; i < T::waves * kRadix; i += T::threads) (&h[0][0])[i] = 0;
   __syncthreads();
@@ -68,6 +79,81 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_hist(
   }
 }
 
+// Places of a tile's elements in digit order.  Thread t holds elements
+// sub + i * kWave (sub below); pos[i] is element i's place in the tile, and
+// sh.gofs[d] turns a place into the output position of digit d's elements.
+template <int THREADS>
+struct TileRank {
+  int wcnt[THREADS / kWave][kRadix];  // counts, then each wave's first position
+  int gofs[kRadix];                   // output position minus tile position
+  int wsum[THREADS / kWave];
+};
+
+// this lane's first element of the tile
+template <int ITEMS>
+__device__ inline int tile_sub() {
+  return threadIdx.x / kWave * kWave * ITEMS + (threadIdx.x & (kWave - 1));
+}
+
+template <int THREADS, int ITEMS, typename K>
+__device__ inline void rank_tile(TileRank<THREADS> &sh, const K (&key)[ITEMS], int (&pos)[ITEMS],
+                                 int count, int shift, int bits, long long ntiles,
+                                 const int *__restrict__ offsets) {
+  constexpr int waves = THREADS / kWave;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int mask = (1 << bits) - 1, sub = tile_sub<ITEMS>();
+  for (int i = threadIdx.x; i < waves * kRadix; i += THREADS) (&sh.wcnt[0][0])[i] = 0;
+  __syncthreads();
+  // rank of every element among its wave's elements of the same digit
+  const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+#pragma unroll
+  for (int i = 0; i < ITEMS; i++) {
+    const bool valid = sub + i * kWave < count;
+    const int d = (int)(key[i] >> shift) & mask;
+    unsigned long long peers = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
+      const bool bit = (d >> b) & 1;
+      const unsigned long long m = __ballot(bit);
+      peers &= bit ? m : ~m;
+    }
+    const int rank = __popcll(peers & below);
+    const int before = valid ? sh.wcnt[wave][d] : 0;
+    pos[i] = before + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && rank == 0) sh.wcnt[wave][d] = before + __popcll(peers);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  // digit starts within the tile (exclusive scan over digits), wave starts
+  // within each digit; thread d < kRadix owns digit d
+  int total = 0, incl = 0;
+  if (threadIdx.x < kRadix) {
+    for (int w = 0; w < waves; w++) {
+      const int c = sh.wcnt[w][threadIdx.x];
+      sh.wcnt[w][threadIdx.x] = total;
+      total += c;
+    }
+    incl = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int o = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += o;
+    }
+    if (lane == kWave - 1) sh.wsum[wave] = incl;
+  }
+  __syncthreads();
+  if (threadIdx.x < kRadix) {
+    int start = incl - total;
+    for (int w = 0; w < wave; w++) start += sh.wsum[w];
+    for (int w = 0; w < waves; w++) sh.wcnt[w][threadIdx.x] += start;
+    if ((int)threadIdx.x <= mask)
+      sh.gofs[threadIdx.x] = offsets[(long long)threadIdx.x * ntiles + blockIdx.x] - start;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITEMS; i++) pos[i] += sh.wcnt[wave][(int)(key[i] >> shift) & mask];
+}
+
 // The stable scatter of one pass; pay_in null: the payload of element e is e
 // (the first pass).  Bound by its bytes once the output runs are whole: 24 M
 // 32-bit keys take 101 us a pass (16 bytes an element, 3.8 TB/s) where
@@ -78,16 +164,12 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
     int *__restrict__ pay_out, long long n, int shift, int bits, long long ntiles,
     const int *__restrict__ offsets) {
   typedef SortTile<K> T;
-  __shared__ int wcnt[T::waves][kRadix];  // counts, then each wave's first position
-  __shared__ int gofs[kRadix];            // output position minus tile position
-  __shared__ int wsum[T::waves];
+  __shared__ TileRank<T::threads> sh;
   __shared__ K stage[T::elems];
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int mask = (1 << bits) - 1;
   const long long tile0 = (long long)blockIdx.x * T::elems;
   const int count = (int)min((long long)T::elems, n - tile0);
-  const int sub = wave * kWave * kItems + lane;  // this lane's first element of the tile
-  for (int i = threadIdx.x; i < T::waves * kRadix; i += T::threads) (&wcnt[0][0])[i] = 0;
+  const int sub = tile_sub<kItems>();
   K key[kItems];
   int pay[kItems], pos[kItems];
 #pragma unroll
@@ -100,59 +182,10 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
     const int e = sub + i * kWave;
     pay[i] = pay_in ? (e < count ? pay_in[tile0 + e] : 0) : (int)(tile0 + e);
   }
-  __syncthreads();
-  // rank of every element among its wave's elements of the same digit
-  const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+  rank_tile<T::threads, kItems, K>(sh, key, pos, count, shift, bits, ntiles, offsets);
 #pragma unroll
-  for (int i = 0; i < kItems; i++) {
-    const bool valid = sub + i * kWave < count;
-    const int d = (int)(key[i] >> shift) & mask;
-    unsigned long long peers = __ballot(valid);
-    for (int b = 0; b < bits; b++) {
-      const bool bit = (d >> b) & 1;
-      const unsigned long long m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
-    const int rank = __popcll(peers & below);
-    const int before = valid ? wcnt[wave][d] : 0;
-    pos[i] = before + rank;
-    __builtin_amdgcn_wave_barrier();
-    if (valid && rank == 0) wcnt[wave][d] = before + __popcll(peers);
-    __builtin_amdgcn_wave_barrier();
-  }
-  __syncthreads();
-  // digit starts within the tile (exclusive scan over digits), wave starts
-  // within each digit; thread d < kRadix owns digit d
-  int total = 0, incl = 0;
-  if (threadIdx.x < kRadix) {
-    for (int w = 0; w < T::waves; w++) {
-      const int c = wcnt[w][threadIdx.x];
-      wcnt[w][threadIdx.x] = total;
-      total += c;
-    }
-    incl = total;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int o = __shfl_up(incl, off, kWave);
-      if (lane >= off) incl += o;
-    }
-    if (lane == kWave - 1) wsum[wave] = incl;
-  }
-  __syncthreads();
-  if (threadIdx.x < kRadix) {
-    int start = incl - total;
-    for (int w = 0; w < wave; w++) start += wsum[w];
-    for (int w = 0; w < T::waves; w++) wcnt[w][threadIdx.x] += start;
-    if ((int)threadIdx.x <= mask)
-      gofs[threadIdx.x] = offsets[(long long)threadIdx.x * ntiles + blockIdx.x] - start;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kItems; i++) {
-    const int d = (int)(key[i] >> shift) & mask;
-    pos[i] += wcnt[wave][d];
+  for (int i = 0; i < kItems; i++)
     if (sub + i * kWave < count) stage[pos[i]] = key[i];
-  }
   __syncthreads();
   int dst[kItems];
 #pragma unroll
@@ -160,7 +193,7 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
     const int t = threadIdx.x + i * T::threads;
     if (t < count) {
       const K k = stage[t];
-      dst[i] = gofs[(int)(k >> shift) & mask] + t;
+      dst[i] = sh.gofs[(int)(k >> shift) & mask] + t;
       keys_out[dst[i]] = k;
     }
   }
@@ -174,6 +207,72 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
   for (int i = 0; i < kItems; i++) {
     const int t = threadIdx.x + i * T::threads;
     if (t < count) pay_out[dst[i]] = pstage[t];
+  }
+}
+
+// A pass over matrix entries: key (the index sorted by), other (the other index)
+// and value move together, so no gather by sorted position follows (4.8 M
+// entries: 171 us, a cache line for each value and column).  Tiles of 4096, a
+// value of each through LDS at a time: 32 KB.  4.8 M entries take 32 us a pass (32
+// bytes an entry, 4.8 TB/s).
+constexpr int kEntThreads = EntryTile::threads, kEntItems = EntryTile::items;
+constexpr int kEntTile = EntryTile::elems;
+
+__global__ __launch_bounds__(kEntThreads) void k_entry_scatter(
+    const int *__restrict__ key_in, const int *__restrict__ other_in,
+    const double *__restrict__ val_in, int *__restrict__ key_out, int *__restrict__ other_out,
+    double *__restrict__ val_out, long long n, int shift, int bits, long long ntiles,
+    const int *__restrict__ offsets) {
+  __shared__ TileRank<kEntThreads> sh;
+  __shared__ double stage[kEntTile];
+  const int mask = (1 << bits) - 1;
+  const long long tile0 = (long long)blockIdx.x * kEntTile;
+  const int count = (int)min((long long)kEntTile, n - tile0);
+  const int sub = tile_sub<kEntItems>();
+  unsigned key[kEntItems];
+  int other[kEntItems], pos[kEntItems], dst[kEntItems];
+  double val[kEntItems];
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++) {
+    const int e = min(sub + i * kWave, count - 1);
+    key[i] = key_in[tile0 + e];
+    other[i] = other_in[tile0 + e];
+    val[i] = val_in[tile0 + e];
+  }
+  rank_tile<kEntThreads, kEntItems, unsigned>(sh, key, pos, count, shift, bits, ntiles, offsets);
+  int *istage = reinterpret_cast<int *>(stage);
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++)
+    if (sub + i * kWave < count) istage[pos[i]] = (int)key[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++) {
+    const int t = threadIdx.x + i * kEntThreads;
+    if (t < count) {
+      const unsigned k = istage[t];
+      dst[i] = sh.gofs[(int)(k >> shift) & mask] + t;
+      key_out[dst[i]] = (int)k;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++)
+    if (sub + i * kWave < count) istage[pos[i]] = other[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++) {
+    const int t = threadIdx.x + i * kEntThreads;
+    if (t < count) other_out[dst[i]] = istage[t];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++)
+    if (sub + i * kWave < count) stage[pos[i]] = val[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kEntItems; i++) {
+    const int t = threadIdx.x + i * kEntThreads;
+    if (t < count) val_out[dst[i]] = stage[t];
   }
 }
 
@@ -204,30 +303,6 @@ __global__ __launch_bounds__(kBlock) void k_bucket_starts(const K *__restrict__ 
         first_at_least(keys, shift, 0, n, threadIdx.x ? b0 + kBlock : b0);
   __syncthreads();
   if (b <= nb) ptr[b] = (int)first_at_least(keys, shift, ends[0], ends[1], b);
-}
-
-template <typename K>
-__global__ __launch_bounds__(kBlock) void k_coo_keys(const int *__restrict__ rows,
-                                                     const int *__restrict__ cols, long long n,
-                                                     int col_bits, K *__restrict__ keys) {
-  long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) keys[i] = ((K)(unsigned)rows[i] << col_bits) | (K)(cols ? (unsigned)cols[i] : 0u);
-}
-
-// columns from the keys' low bits (col_bits 0: by the sorted positions), values
-// by the sorted positions
-template <typename K>
-__global__ __launch_bounds__(kBlock) void k_gather_sorted(const K *__restrict__ keys, int col_bits,
-                                                          const int *__restrict__ perm,
-                                                          const int *__restrict__ cols,
-                                                          const double *__restrict__ vals,
-                                                          long long n, int *__restrict__ cols_out,
-                                                          double *__restrict__ vals_out) {
-  long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int p = perm[i];
-  cols_out[i] = col_bits ? (int)(keys[i] & (((K)1 << col_bits) - 1)) : cols[p];
-  vals_out[i] = vals[p];
 }
 
 // the longest row
@@ -327,10 +402,10 @@ static int radix_sort_from(const Src *first, K **keys, int **payload, long long 
     const int shift = bits * p, b = std::min(bits, std::max(1, key_bits - shift));
     const K *kin = *keys;
     if (p == 0 && first)
-      k_digit_hist<K><<<(unsigned)ntiles, T::threads, 0, s>>>(*first, n, shift, (1 << b) - 1,
+      k_digit_hist<T><<<(unsigned)ntiles, T::threads, 0, s>>>(*first, n, shift, (1 << b) - 1,
                                                               ntiles, hist);
     else
-      k_digit_hist<K><<<(unsigned)ntiles, T::threads, 0, s>>>(kin, n, shift, (1 << b) - 1, ntiles,
+      k_digit_hist<T><<<(unsigned)ntiles, T::threads, 0, s>>>(kin, n, shift, (1 << b) - 1, ntiles,
                                                               hist);
     st = scan<int>(hist, hist, (1LL << b) * ntiles, false, nullptr, ws, s);
     if (st) break;
@@ -377,33 +452,66 @@ template int bucket_starts<unsigned long long>(const unsigned long long *, long 
                                                long long, int *, hipStream_t);
 
 // The CSR arrays of n COO triplets: stable order by (row, col)
-// (csr::compare_row, src/cpp/utils/csr.cpp:3-8), 32-bit keys where both
-// indices fit.  col_bits 0: the triplets are in column order already (known from
-// the import, as a column-ordered file gives them), and the stable sort by row
-// keeps it -- three 32-bit passes instead of five 64-bit ones at 300,007 rows
-// (4.8 M triplets in column order: 450 -> 368 us with the two-launch prefix sums).
-template <typename K>
-static int coo_rows(const tbsla_hip_matrix_s *coo, long long n, int row_bits, int col_bits,
-                    int *rowptr, int *cols, double *vals, hipStream_t s) {
-  K *keys = nullptr;
-  int *perm = nullptr;
+// (csr::compare_row, src/cpp/utils/csr.cpp:3-8): passes over the columns' digits,
+// then over the rows'; those over the columns are left out where the triplets are
+// in column order already (known from the import, as a column-ordered file gives
+// them).  300,007 rows, 4.8 M triplets in column order: 368 -> 189 us (three passes
+// and a gather before).
+static int coo_rows(const tbsla_hip_matrix_s *coo, long long n, int *rowptr, int *cols,
+                    double *vals, hipStream_t s) {
+  const int row_bits = bits_for(std::max(coo->n_row, 1));
+  const int col_bits = coo->col_sorted ? 0 : bits_for(std::max(coo->n_col, 1));
+  const int row_passes = (row_bits + 7) / 8, col_passes = (col_bits + 7) / 8;
+  const int passes = row_passes + col_passes;
+  const int rb = (row_bits + row_passes - 1) / row_passes;
+  const int cb = col_passes ? (col_bits + col_passes - 1) / col_passes : 0;
+  const long long ntiles = (n + kEntTile - 1) / kEntTile;
+  const long long hist_n = (1LL << std::max(rb, cb)) * std::max(ntiles, 1LL);
+  const size_t len = (size_t)std::max(n, 1LL);
+  // where a pass's entries go: the result's arrays and others in turn, the last
+  // pass's to the result's (its rows, in order, to rows[0])
+  int *rows[2] = {nullptr, nullptr}, *oc[2] = {cols, nullptr}, *hist = nullptr;
+  double *ov[2] = {vals, nullptr};
+  void *ws = nullptr;
   int st;
-  if (!(st = device_alloc((void **)&keys, (size_t)std::max(n, 1LL) * sizeof(K))) &&
-      !(st = device_alloc((void **)&perm, (size_t)std::max(n, 1LL) * 4))) {
-    if (n > 0)
-      k_coo_keys<K><<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, col_bits ? coo->colidx : nullptr, n,
-                                                   col_bits, keys);
-    st = radix_sort_pairs<K>(&keys, &perm, n, col_bits + row_bits, s);
-    if (!st) st = bucket_starts<K>(keys, n, col_bits, coo->n_row, rowptr, s);
-    if (!st && n > 0)
-      k_gather_sorted<K><<<grid_for(n), kBlock, 0, s>>>(keys, col_bits, perm, coo->colidx,
-                                                        coo->values, n, cols, vals);
+  if (!(st = device_alloc((void **)&rows[0], len * 4)) &&
+      !(st = device_alloc((void **)&rows[1], passes > 1 ? len * 4 : 4)) &&
+      !(st = device_alloc((void **)&oc[1], passes > 1 ? len * 4 : 4)) &&
+      !(st = device_alloc((void **)&ov[1], passes > 1 ? len * 8 : 8)) &&
+      !(st = device_alloc((void **)&hist, (size_t)hist_n * 4)) &&
+      !(st = device_alloc(&ws, scan_workspace_bytes(hist_n)))) {
+    const int *r_in = coo->rowidx, *c_in = coo->colidx;
+    const double *v_in = coo->values;
+    for (int p = 0; n > 0 && !st && p < passes; p++) {
+      const bool by_row = p >= col_passes;
+      const int shift = by_row ? rb * (p - col_passes) : cb * p;
+      const int bits = by_row ? std::min(rb, row_bits - shift) : std::min(cb, col_bits - shift);
+      const int *key = by_row ? r_in : c_in, *other = by_row ? c_in : r_in;
+      const int to = (passes - 1 - p) % 2;
+      k_digit_hist<EntryTile><<<(unsigned)ntiles, kEntThreads, 0, s>>>(
+          key, n, shift, (1 << bits) - 1, ntiles, hist);
+      st = scan<int>(hist, hist, (1LL << bits) * ntiles, false, nullptr, ws, s);
+      if (st) break;
+      k_entry_scatter<<<(unsigned)ntiles, kEntThreads, 0, s>>>(
+          key, other, v_in, by_row ? rows[to] : oc[to], by_row ? oc[to] : rows[to], ov[to], n,
+          shift, bits, ntiles, hist);
+      r_in = rows[to];
+      c_in = oc[to];
+      v_in = ov[to];
+    }
+    if (!st)
+      st = bucket_starts<unsigned>(reinterpret_cast<unsigned *>(rows[0]), n, 0, coo->n_row, rowptr,
+                                   s);
     const hipError_t e = hipGetLastError();
     if (!st && e != hipSuccess) st = fail(TBSLA_HIP_ERR_HIP, hipGetErrorString(e));
   }
   (void)hipStreamSynchronize(s);
-  device_free(keys);
-  device_free(perm);
+  device_free(rows[0]);
+  device_free(rows[1]);
+  device_free(oc[1]);
+  device_free(ov[1]);
+  device_free(hist);
+  device_free(ws);
   return st;
 }
 
@@ -480,9 +588,9 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
       drop();
       return st;
     }
-    if (n > 0)
-      k_coo_keys<unsigned><<<grid_for(n), kBlock, 0, s>>>(coo->rowidx, nullptr, n, 0, keys);
-    if ((st = radix_sort_pairs<unsigned>(&keys, &perm, n, bits_for(std::max(coo->n_row, 1)), s)) ||
+    const unsigned *rows_in = reinterpret_cast<const unsigned *>(coo->rowidx);
+    if ((st = radix_sort_from<unsigned, const unsigned *>(&rows_in, &keys, &perm, n,
+                                                          bits_for(std::max(coo->n_row, 1)), s)) ||
         (st = bucket_starts<unsigned>(keys, n, 0, rows, rowptr, s))) {
       drop();
       return st;
@@ -504,12 +612,7 @@ extern "C" int tbsla_hip_convert(tbsla_hip_matrix_t dst, int format, tbsla_hip_m
   TBSLA_TRY(device_alloc((void **)&scol, (size_t)std::max(n, 1LL) * 4));
   TBSLA_TRY(device_alloc((void **)&sval, (size_t)std::max(n, 1LL) * 8));
   {
-    const int col_bits = coo->col_sorted ? 0 : bits_for(std::max(coo->n_col, 1));
-    const int row_bits = bits_for(std::max(coo->n_row, 1));
-    const int st = col_bits + row_bits <= 32
-                       ? coo_rows<unsigned>(coo, n, row_bits, col_bits, rowptr, scol, sval, s)
-                       : coo_rows<unsigned long long>(coo, n, row_bits, col_bits, rowptr, scol,
-                                                      sval, s);
+    const int st = coo_rows(coo, n, rowptr, scol, sval, s);
     if (st) {
       device_free(rowptr);
       device_free(scol);
