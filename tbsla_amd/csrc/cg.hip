@@ -121,15 +121,32 @@ struct CgArgs {
   const float *dv32;
   int ndiag;
   int ncol;
+  // the first 8 offsets of each again, at hand with the arguments (G's last one
+  // repeated)
+  int doff8[8];
+  int gdoff8[8];
 };
 
-// Every kernel reads its arguments from one CgArgs block in device memory
+// What the kernels find at one known address: the arguments, the status counts
+// and the state of a lone system (a batch's systems lie at args.seg).  A lone
+// system's kernels then load arguments and state in one trip to memory, before
+// the rows' data, where arguments, the workgroup's system, that system's state
+// and the diagonals' offsets took one each (10^6 rows, mixed: K1 17.1 -> 16.2 us,
+// K3 7.9 -> 7.4).
+struct CgBlock {
+  CgArgs args;
+  CgSeg seg;
+  CgCom com;
+};
+
+// Every kernel reads its arguments from one CgBlock in device memory
 // that the solve's cache owns for its whole lifetime: a captured graph then
 // names only that block (and its launch shape), never a matrix or work
 // buffer, so one instantiated graph serves every later solve of the same
 // shape and no graph can refer to memory that has been freed since.
-#define CG_ARGS const CgArgs *__restrict__ pa_
-#define CG_BIND const CgArgs a = cg_bind(pa_)
+// multi_: a batch of systems, whose workgroups look theirs up in block_seg.
+#define CG_ARGS const CgBlock *__restrict__ pa_, int multi_
+#define CG_BIND const CgArgs a = cg_bind(&pa_->args)
 
 // The argument block read as constant memory, by scalar loads, and its pointers
 // as pointers to global memory.  A pointer that is itself loaded would otherwise
@@ -143,8 +160,47 @@ __device__ inline T *arg(T *TBSLA_CONST *slot) {
   return (T *)*(G *TBSLA_CONST *)slot;
 }
 
-// element `i` of one of the block's pointer pairs
-#define CG_AT(field, i) arg(&((TBSLA_CONST CgArgs *)pa_)->field[i])
+// The workgroup's place in the layout.  A lone system's: the 8 XCDs, which take
+// workgroups in turn, each get a contiguous eighth of them, so that rows share an
+// L2 with most of the rows that their columns name (64^3, FP64: K1 8.3 -> 7.8 us,
+// K2 6.7 -> 5.6; 10^6 rows, mixed, factored: K1 16.2 -> 15.0, K2 15.2 -> 14.3, K3
+// 7.4 -> 6.5).  A batch's in turn: its systems differ in rows and iterations, and
+// eighths of it in work (96 systems, K1b: 115 us as it is, 135 in eighths; runs
+// of 16 or 64 workgroups an XCD, 115 and 119).
+__device__ inline int cg_block(int multi) {
+  const int i = blockIdx.x / 8, x = blockIdx.x % 8, n = gridDim.x;
+  return multi ? blockIdx.x : x * (n / 8) + min(x, n % 8) + i;
+}
+// pointer i (0 or 1) of a pair
+#define CG_AT(field, i) ((i) ? a.field[1] : a.field[0])
+// offset i < 8 of A's or of G's diagonals
+#define CG_OFF(field, i) ((TBSLA_CONST CgBlock *)pa_)->args.field[i]
+// The system of workgroup b: S, and in sg what a kernel of the iteration reads
+// of it and none of that launch writes (K1's test aside, which only writes iters
+// where it does not read it).  A lone system's is read at once, with the
+// arguments: CG_HAND names those a kernel needs first, so that the compiler asks
+// for all of them before it waits.
+#define CG_SYSTEM(b, ...)                                                              \
+  CgPart sg = cg_part(&((TBSLA_CONST CgBlock *)pa_)->seg);                             \
+  CG_HAND("s"(sg.shift), "s"(sg.row0), "s"(sg.row1), "s"(sg.blk0), "s"(sg.blk1),       \
+          "s"(sg.rpb), "s"(sg.near_zero), ##__VA_ARGS__);                              \
+  CgSeg *S = a.seg;                                                                    \
+  if (multi_) {                                                                        \
+    S += ((TBSLA_CONST int *)a.block_seg)[b];                                          \
+    sg = cg_part((TBSLA_CONST CgSeg *)S);                                              \
+  }
+#define CG_HAND(...) asm volatile("" : : __VA_ARGS__)
+
+struct CgPart {
+  double stop, near_zero, rnorm0;
+  int iters, shift, true_res, stop_par, done;
+  int row0, row1, blk0, blk1, rpb, ent0;
+};
+
+__device__ inline CgPart cg_part(TBSLA_CONST CgSeg *c) {
+  return CgPart{c->stop, c->near_zero, c->rnorm0, c->iters, c->shift, c->true_res, c->stop_par, c->done,
+                c->row0, c->row1, c->blk0, c->blk1, c->rpb, c->ent0};
+}
 
 // the block's other fields
 __device__ inline CgArgs cg_bind(const CgArgs *pa) {
@@ -170,6 +226,12 @@ __device__ inline CgArgs cg_bind(const CgArgs *pa) {
   a.gndiag = c->gndiag;
   a.b = arg(&c->b);
   a.x = arg(&c->x);
+  for (int i = 0; i < 2; i++) {
+    a.r[i] = arg(&c->r[i]);
+    a.p[i] = arg(&c->p[i]);
+    a.prr[i] = arg(&c->prr[i]);
+    a.prz[i] = arg(&c->prz[i]);
+  }
   a.z = arg(&c->z);
   a.ap = arg(&c->ap);
   a.ax = arg(&c->ax);
@@ -405,17 +467,17 @@ __device__ inline int seg_finish(int flag, const SegLoad &l, int np, int b0, int
 // The convergence test of the previous iteration (CG.cpp:66-72) on
 // |r| = sqrt(rr), made alike by every workgroup of the system from the same
 // sums; the system's first workgroup records the outcome.  Returns it.
-__device__ inline int k1_test(const CgArgs &a, CgSeg *S, int b, int b0, int par, double rz_new,
-                              double rr, int check_only) {
+__device__ inline int k1_test(const CgArgs &a, CgSeg *S, const CgPart &sg, int b, int par,
+                              double rz_new, double rr, int check_only) {
   const double rn = sqrt(rr);
   int fin = kRunning;
-  if (rn < S->stop || rn == 0.0)
-    fin = (a.verify && !S->true_res) ? kPending : kConverged;
+  if (rn < sg.stop || rn == 0.0)
+    fin = (a.verify && !sg.true_res) ? kPending : kConverged;
   else if (!(rz_new > 0.0) || !isfinite(rz_new) || !isfinite(rr))
     fin = kBreakdown;
-  else if (!check_only && a.stall_window > 0 && S->iters >= a.stall_window && rn >= S->rnorm0)
+  else if (!check_only && a.stall_window > 0 && sg.iters >= a.stall_window && rn >= sg.rnorm0)
     fin = kBreakdown;
-  if (b == b0 && threadIdx.x == 0) {
+  if (b == sg.blk0 && threadIdx.x == 0) {
     S->rnorm = rn;
     if (fin != kRunning) {
       S->stop_par = par;
@@ -443,12 +505,16 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
   constexpr int NP = ZBUF ? 3 : 2;
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
-  const int par = (par_g ^ S->shift) & 1;
-  const int b0 = S->blk0, b1 = S->blk1;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b, "s"(a.p[0]), "s"(a.p[1]), "s"(a.prz[0]), "s"(a.prz[1]), "s"(ZBUF ? a.prr[0] : a.r[0]),
+            "s"(ZBUF ? a.prr[1] : a.r[1]), "s"(a.z), "s"(a.ap), "s"(a.ppap),
+            "s"(a.rowptr), "s"(a.colidx),
+            "s"(MIX ? (const void *)a.val32 : (const void *)a.val64), "s"(a.a_nnz), "s"(a.f_col),
+            "s"(sg.stop), "s"(sg.iters), "s"(sg.true_res), "s"(sg.rnorm0), "s"(sg.ent0));
+  const int par = (par_g ^ sg.shift) & 1;
+  const int b0 = sg.blk0, b1 = sg.blk1;
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const int lane = threadIdx.x & (L - 1);
   const double *zv = ZBUF ? a.z : CG_AT(r, par);
   const double *po = CG_AT(p, par);
@@ -460,7 +526,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
   // the partials' wait cover the gathers.
   Row f;
   double fs[P], ft[P];
-  f.extent(a.rowptr, rowc, S->ent0);
+  f.extent(a.rowptr, rowc, sg.ent0);
   const double own_z = zv[rowc], own_p = po[rowc];
   f.template load<false>(a.colidx, val, a.a_nnz, a.f_col, lane);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
@@ -478,10 +544,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
   const double rz_new = t[0], rz_old = t[1];
   const double rr = ZBUF ? t[2] : rz_new;
   if (check) {
-    const int fin = k1_test(a, S, b, b0, par, rz_new, rr, check_only);
+    const int fin = k1_test(a, S, sg, b, par, rz_new, rr, check_only);
     if (fin != kRunning || check_only) return;
   }
-  const double beta = rz_new / fmax(rz_old, S->near_zero);
+  const double beta = rz_new / fmax(rz_old, sg.near_zero);
   double *pn = CG_AT(p, par ^ 1);
   double pap = 0.0;
   constexpr int PASS = kBlock / L;
@@ -524,7 +590,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       rw[r] = min(row + r * PASS, r1 - 1);
-      g[r].extent(a.rowptr, rw[r], S->ent0);
+      g[r].extent(a.rowptr, rw[r], sg.ent0);
       oz[r] = zv[rw[r]];
       op[r] = po[rw[r]];
     }
@@ -556,12 +622,13 @@ __global__ __launch_bounds__(kBlock) void k_cg_pnew(CG_ARGS, int par_g, int chec
   CG_BIND;
   constexpr int NP = ZBUF ? 3 : 2;
   __shared__ SegShared sh;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
-  const int par = (par_g ^ S->shift) & 1;
-  const int b0 = S->blk0, b1 = S->blk1;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
+  if (multi_ && sg.done != kRunning) return;  // finished before this launch
+  const int par = (par_g ^ sg.shift) & 1;
+  const int b0 = sg.blk0, b1 = sg.blk1;
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const double *zv = ZBUF ? a.z : CG_AT(r, par);
   const double *po = CG_AT(p, par);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
@@ -572,10 +639,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_pnew(CG_ARGS, int par_g, int chec
   const double rz_new = t[0], rz_old = t[1];
   const double rr = ZBUF ? t[2] : rz_new;
   if (check) {
-    const int fin = k1_test(a, S, b, b0, par, rz_new, rr, check_only);
+    const int fin = k1_test(a, S, sg, b, par, rz_new, rr, check_only);
     if (fin != kRunning || check_only) return;
   }
-  const double beta = rz_new / fmax(rz_old, S->near_zero);
+  const double beta = rz_new / fmax(rz_old, sg.near_zero);
   double *pn = CG_AT(p, par ^ 1);
   for (int row = r0 + (int)threadIdx.x; row < r1; row += 2 * kBlock) {
     const int row2 = row + kBlock;
@@ -598,13 +665,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
   typedef CgRow<L, V> Row;
   constexpr int P = Row::P;
   __shared__ double lds[kBlock / kWave];
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
+  if (multi_ && sg.done != kRunning) return;
   if (__atomic_load_n(&S->done, __ATOMIC_RELAXED) != kRunning) return;
-  const int par = (par_g ^ S->shift) & 1;
-  const int b0 = S->blk0;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int par = (par_g ^ sg.shift) & 1;
+  const int b0 = sg.blk0;
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const int lane = threadIdx.x & (L - 1);
   const double *pn = CG_AT(p, par ^ 1);
   const V *val = MIX ? (const V *)a.val32 : (const V *)a.val64;
@@ -620,7 +688,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
 #pragma unroll
     for (int r = 0; r < R2; r++) {
       rw[r] = min(row + r * PASS, r1 - 1);
-      w[r].extent(a.rowptr, rw[r], S->ent0);
+      w[r].extent(a.rowptr, rw[r], sg.ent0);
       own[r] = pn[rw[r]];
     }
 #pragma unroll
@@ -692,12 +760,17 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
   constexpr int U = KD > 0 ? KD : 8;
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
-  const int par = (par_g ^ S->shift) & 1;
-  const int b0 = S->blk0, b1 = S->blk1;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b, "s"(a.p[0]), "s"(a.p[1]), "s"(a.prz[0]), "s"(a.prz[1]), "s"(ZBUF ? a.prr[0] : a.r[0]),
+            "s"(ZBUF ? a.prr[1] : a.r[1]), "s"(a.z), "s"(a.ap),
+            "s"(MIX ? (const void *)a.dv32 : (const void *)a.dv64), "s"(a.ncol), "s"(a.ppap),
+            "s"(sg.stop), "s"(sg.iters), "s"(sg.true_res), "s"(sg.rnorm0), "s"(CG_OFF(doff8, 0)),
+            "s"(CG_OFF(doff8, 1)), "s"(CG_OFF(doff8, 2)), "s"(CG_OFF(doff8, 3)),
+            "s"(CG_OFF(doff8, 4)), "s"(CG_OFF(doff8, 5)), "s"(CG_OFF(doff8, 6)));
+  const int par = (par_g ^ sg.shift) & 1;
+  const int b0 = sg.blk0, b1 = sg.blk1;
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const double *zv = ZBUF ? a.z : CG_AT(r, par);
   const double *po = CG_AT(p, par);
   const V *dv = MIX ? (const V *)a.dv32 : (const V *)a.dv64;
@@ -713,7 +786,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
       const unsigned at = (unsigned)dia_at(row, 0, KD);
 #pragma unroll
       for (int i = 0; i < U; i++) {
-        const unsigned c = (unsigned)min(max(row + a.doff[i], 0), a.ncol - 1);
+        const unsigned c = (unsigned)min(max(row + CG_OFF(doff8, i), 0), a.ncol - 1);
         w.v[i] = ld32(dv, at + i * kWave);
         w.z[i] = ld32(zv, c);
         w.p[i] = ld32(po, c);
@@ -744,10 +817,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
   const double rz_new = t[0], rz_old = t[1];
   const double rr = ZBUF ? t[2] : rz_new;
   if (check) {
-    const int fin = k1_test(a, S, b, b0, par, rz_new, rr, check_only);
+    const int fin = k1_test(a, S, sg, b, par, rz_new, rr, check_only);
     if (fin != kRunning || check_only) return;
   }
-  const double beta = rz_new / fmax(rz_old, S->near_zero);
+  const double beta = rz_new / fmax(rz_old, sg.near_zero);
   double *pn = CG_AT(p, par ^ 1);
   double pap = 0.0;
   auto add = [&](const Row &w, int k0, V acc) {
@@ -795,16 +868,19 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   constexpr int P = 4;
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
-  const int par = (par_g ^ S->shift) & 1;
-  const int b0 = S->blk0, b1 = S->blk1;
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b, "s"(a.p[0]), "s"(a.p[1]), "s"(a.prz[0]), "s"(a.prz[1]), "s"(a.prr[0]),
+            "s"(a.prr[1]), "s"(a.r[0]), "s"(a.r[1]), "s"(a.x), "s"(a.ap), "s"(a.ppap),
+            "s"(a.dinv));
+  if (multi_ && sg.done != kRunning) return;  // finished before this launch
+  const int par = (par_g ^ sg.shift) & 1;
+  const int b0 = sg.blk0, b1 = sg.blk1;
   const double *rc = CG_AT(r, par);
   double *rn = CG_AT(r, par ^ 1);
   const double *pn = CG_AT(p, par ^ 1);
   const V *tv = MIX ? (const V *)a.t_v32 : (const V *)a.t_v64;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const int row_first = r0 + (int)threadIdx.x;
   const int rowc = min(row_first, r1 - 1);
   // the first row's operands (see RowPrefetch), then the partials, then the
@@ -848,7 +924,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   double t[3];
   if (seg_finish(flag, sl, 2, b0, b1, sh, t) != kRunning) return;
   const double rz = t[0], pap = t[1];
-  const double alpha = rz / fmax(pap, S->near_zero);
+  const double alpha = rz / fmax(pap, sg.near_zero);
   double rr = 0.0, rzp = 0.0;
   // PRE 2: the first row, then the later rows two at a time (each pair's
   // loads issued before either is updated; sums in row order)
@@ -971,9 +1047,9 @@ __device__ inline V gd_slot(const V *__restrict__ gd, long long src, int k, int 
 // ascending column (descending offset o_k <= 0) of G_{i-o_k, i} r'_{i-o_k},
 // zero slots skipped -- the order and the products of K2's CSR form, so the
 // two forms give bitwise the same iterates.  All of a row's loads are issued
-// before it is updated, the first row's (which need no sum) before the partials'.
-// Two rows in flight per thread are slower: 10^6 rows, mixed, 17.3 -> 23.4 us (170
-// registers for 100).
+// before it is updated, the first row's (which need no sum) before the partials';
+// past G's last diagonal that one's again, not used (with a branch around each
+// diagonal they took a trip to memory each: 10^6 rows, mixed, 17.3 -> 15.2 us).
 template <bool MIX, int KD, bool WIDE>
 __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, int count) {
   TBSLA_NO_FMA
@@ -982,21 +1058,26 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, i
   // KD: at most that many diagonals of G (4 or 8, chosen on the host)
   __shared__ double lds[kBlock / kWave];
   __shared__ SegShared sh;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
-  const int par = (par_g ^ S->shift) & 1;
-  const int b0 = S->blk0, b1 = S->blk1;
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b, "s"(a.p[0]), "s"(a.p[1]), "s"(a.prz[0]), "s"(a.prz[1]), "s"(a.prr[0]),
+            "s"(a.prr[1]), "s"(a.r[0]), "s"(a.r[1]), "s"(a.x), "s"(a.ap), "s"(a.ppap),
+            "s"(a.ncol), "s"(a.gndiag), "s"(MIX ? (const void *)a.gd32 : (const void *)a.gd64),
+            "s"(CG_OFF(gdoff8, 0)), "s"(CG_OFF(gdoff8, 1)), "s"(CG_OFF(gdoff8, 2)),
+            "s"(CG_OFF(gdoff8, 3)));
+  if (multi_ && sg.done != kRunning) return;  // finished before this launch
+  const int par = (par_g ^ sg.shift) & 1;
+  const int b0 = sg.blk0, b1 = sg.blk1;
   const double *rc = CG_AT(r, par);
   double *rn = CG_AT(r, par ^ 1);
   const double *pn = CG_AT(p, par ^ 1);
   const V *gd = MIX ? (const V *)a.gd32 : (const V *)a.gd64;
   const int ndg = a.gndiag;
   const long long n = a.ncol;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   int off[KD];
 #pragma unroll
-  for (int k = 0; k < KD; k++) off[k] = k < ndg ? a.gdoff[k] : 0;
+  for (int k = 0; k < KD; k++) off[k] = CG_OFF(gdoff8, k);
   const int row_first = r0 + (int)threadIdx.x;
   double xv, pv, rv, apv, rs[KD], as[KD];
   V gv[KD];
@@ -1007,14 +1088,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, i
     apv = ldi<WIDE>(a.ap, row);
 #pragma unroll
     for (int k = 0; k < KD; k++) {
-      if (k < ndg) {
-        const long long src = (long long)row - off[k];
-        const long long sc = src < n ? src : row;
-        const V g = ldi<WIDE>(gd, dia_at(sc, k, ndg));
-        gv[k] = src < n ? g : (V)0;
-        rs[k] = ldi<WIDE>(rc, sc);
-        as[k] = ldi<WIDE>(a.ap, sc);
-      }
+      const long long src = (long long)row - off[k];
+      const long long sc = src < n ? src : row;
+      gv[k] = ldi<WIDE>(gd, dia_at(sc, min(k, ndg - 1), ndg));
+      rs[k] = ldi<WIDE>(rc, sc);
+      as[k] = ldi<WIDE>(a.ap, sc);
     }
   };
   load(min(row_first, r1 - 1));
@@ -1026,7 +1104,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, i
   double t[3];
   if (seg_finish(flag, sl, 2, b0, b1, sh, t) != kRunning) return;
   const double rz = t[0], pap = t[1];
-  const double alpha = rz / fmax(pap, S->near_zero);
+  const double alpha = rz / fmax(pap, sg.near_zero);
   double rr = 0.0;
   for (int row = row_first; row < r1; row += kBlock) {
     if (row != row_first) load(row);
@@ -1037,7 +1115,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, i
     V acc = 0;
 #pragma unroll
     for (int k = KD - 1; k >= 0; k--) {
-      if (k < ndg && gv[k] != (V)0) {
+      if (k < ndg && (long long)row - off[k] < n && gv[k] != (V)0) {
         const double rcv = rs[k] + (-alpha) * as[k];
         if (MIX) acc = fmaf((float)gv[k], (float)rcv, (float)acc);
         else acc = fma((double)gv[k], rcv, (double)acc);
@@ -1090,17 +1168,17 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz(CG_ARGS, int par_g, int mode) 
   constexpr int P = 4;
   __shared__ double lds[kBlock / kWave];
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
-  const int rsel = mode == kAfterIter ? ((par_g ^ S->shift) & 1) ^ 1
-                   : mode == kVerify  ? S->stop_par
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
+  const int rsel = mode == kAfterIter ? ((par_g ^ sg.shift) & 1) ^ 1
+                   : mode == kVerify  ? sg.stop_par
                                       : 0;
   const double *rc = CG_AT(r, rsel);
   const V *gv = MIX ? (const V *)a.g_v32 : (const V *)a.g_v64;
   const V *tv = MIX ? (const V *)a.t32 : (const V *)a.t64;
-  const int b0 = S->blk0;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int b0 = sg.blk0;
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const int row_first = r0 + (int)threadIdx.x;
   const int rowc = min(row_first, r1 - 1);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
@@ -1197,13 +1275,13 @@ __global__ __launch_bounds__(kBlock) void k_cg_gtr(CG_ARGS, int par_g, int mode)
   TBSLA_NO_FMA
   CG_BIND;
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
   const double *rc = CG_AT(r, rsel);
-  const int r0 = S->row0 + (b - S->blk0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int r0 = sg.row0 + (b - sg.blk0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   for (int row = r0 + (int)threadIdx.x; row < r1; row += kBlock) {
     if (MIX) {
       float acc = 0.0f;
@@ -1227,16 +1305,16 @@ __global__ __launch_bounds__(kBlock) void k_cg_gtr_gdia(CG_ARGS, int par_g, int 
   CG_BIND;
   typedef typename std::conditional<MIX, float, double>::type V;
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
   const double *rc = CG_AT(r, rsel);
   const V *gd = MIX ? (const V *)a.gd32 : (const V *)a.gd64;
   const int ndg = a.gndiag;
   const long long n = a.ncol;
-  const int r0 = S->row0 + (b - S->blk0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int r0 = sg.row0 + (b - sg.blk0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   for (int row = r0 + (int)threadIdx.x; row < r1; row += kBlock) {
     V acc = 0;
     for (int k = ndg - 1; k >= 0; k--) {
@@ -1263,21 +1341,24 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz_gdia(CG_ARGS, int par_g, int m
   constexpr int R2 = 2;
   __shared__ double lds[kBlock / kWave];
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b, "s"(a.prz[0]), "s"(a.prz[1]), "s"(a.r[0]), "s"(a.r[1]), "s"(a.z), "s"(a.ncol),
+            "s"(a.gndiag), "s"(MIX ? (const void *)a.gd32 : (const void *)a.gd64),
+            "s"(MIX ? (const void *)a.t32 : (const void *)a.t64), "s"(CG_OFF(gdoff8, 0)),
+            "s"(CG_OFF(gdoff8, 1)), "s"(CG_OFF(gdoff8, 2)), "s"(CG_OFF(gdoff8, 3)));
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
-  const int rsel = mode == kAfterIter ? ((par_g ^ S->shift) & 1) ^ 1
-                   : mode == kVerify  ? S->stop_par
+  const int rsel = mode == kAfterIter ? ((par_g ^ sg.shift) & 1) ^ 1
+                   : mode == kVerify  ? sg.stop_par
                                       : 0;
   const double *rc = CG_AT(r, rsel);
   const V *gd = MIX ? (const V *)a.gd32 : (const V *)a.gd64;
   const V *tv = MIX ? (const V *)a.t32 : (const V *)a.t64;
   const int ndg = a.gndiag;
-  const int r0 = S->row0 + (b - S->blk0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int r0 = sg.row0 + (b - sg.blk0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   int off[KD];
 #pragma unroll
-  for (int k = 0; k < KD; k++) off[k] = k < ndg ? a.gdoff[k] : 0;
+  for (int k = 0; k < KD; k++) off[k] = CG_OFF(gdoff8, k);
   const int row_first = r0 + (int)threadIdx.x;
   V gv[R2][KD], tq[R2][KD];
   double rv[R2];
@@ -1289,11 +1370,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_gz_gdia(CG_ARGS, int par_g, int m
       rv[r] = ldi<WIDE>(rc, rw[r]);
 #pragma unroll
       for (int k = 0; k < KD; k++) {
-        if (k < ndg) {
-          const int c = rw[r] + off[k];
-          gv[r][k] = ldi<WIDE>(gd, dia_at(rw[r], k, ndg));
-          tq[r][k] = ldi<WIDE>(tv, c >= 0 ? c : rw[r]);
-        }
+        const int c = rw[r] + off[k];
+        gv[r][k] = ldi<WIDE>(gd, dia_at(rw[r], min(k, ndg - 1), ndg));
+        tq[r][k] = ldi<WIDE>(tv, c >= 0 ? c : rw[r]);
       }
     }
   };
@@ -1384,15 +1463,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_residual(CG_ARGS, int use_ax, int
   const double *ax = use_ax ? a.ax : nullptr;
   __shared__ double lds[kBlock / kWave];
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  const int sid = a.block_seg[b];
-  CgSeg *S = a.seg + sid;
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
   double *rc = CG_AT(r, rsel);
-  const int b0 = S->blk0;
-  const int r0 = S->row0 + (b - b0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int b0 = sg.blk0;
+  const int r0 = sg.row0 + (b - b0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   double rr = 0.0, rz = 0.0, bb = 0.0;
   for (int row = r0 + (int)threadIdx.x; row < r1; row += kBlock) {
     const double bi = a.b[row];
@@ -1406,7 +1484,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_residual(CG_ARGS, int use_ax, int
     }
     if (mode == kStart) {
       if (zero_x) a.x[row] = 0.0;
-      CG_AT(p, 0)[row] = 0.0;
+      a.p[0][row] = 0.0;
       bb += bi * bi;
     }
   }
@@ -1431,16 +1509,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_start(CG_ARGS, double tol, int re
   CG_BIND;
   __shared__ double lds[kBlock / kWave];
   __shared__ int s_flag;
-  const int b = blockIdx.x;
+  const int b = cg_block(multi_);
   if (b == 0 && threadIdx.x == 0) a.com->t0 = wall_clock64();
-  const int sid = a.block_seg[b];
-  CgSeg *S = a.seg + sid;
-  if (b != S->blk0) return;
+  CG_SYSTEM(b);
+  if (b != sg.blk0) return;
   if (seg_flag(S, &s_flag) == kInactive) return;
   (void)lds;
-  (void)sid;
   double t[3];
-  seg_sums(a.ppap, CG_AT(prr, 1), nullptr, 2, S->blk0, S->blk1, t);
+  seg_sums(a.ppap, CG_AT(prr, 1), nullptr, 2, sg.blk0, sg.blk1, t);
   const double bb = t[0], rr = t[1];
   if (threadIdx.x == 0) {
     S->stop = relative ? tol * sqrt(bb) : tol;
@@ -1448,7 +1524,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_start(CG_ARGS, double tol, int re
     S->rnorm0 = sqrt(rr);
     S->rnorm = S->rnorm0;
     S->iters = 0;
-    S->ent0 = a.rowptr[S->row0];
+    S->ent0 = a.rowptr[sg.row0];
     S->shift = 0;
     S->true_res = 1;
     S->t_done = 0;
@@ -1462,21 +1538,19 @@ __global__ __launch_bounds__(kBlock) void k_cg_vcheck(CG_ARGS, int j) {
   CG_BIND;
   __shared__ double lds[kBlock / kWave];
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  const int sid = a.block_seg[b];
-  CgSeg *S = a.seg + sid;
-  if (b != S->blk0) return;
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
+  if (b != sg.blk0) return;
   if (seg_flag(S, &s_flag) != kPending) return;
   (void)lds;
-  (void)sid;
   double t[3];
-  seg_sums(CG_AT(prr, S->stop_par ^ 1), nullptr, nullptr, 1, S->blk0, S->blk1, t);
+  seg_sums(CG_AT(prr, sg.stop_par ^ 1), nullptr, nullptr, 1, sg.blk0, sg.blk1, t);
   const double rr = t[0];
   if (threadIdx.x == 0) {
     const double rn = sqrt(rr);
     S->rnorm = rn;
     atomicAdd(&a.com->npending, -1);
-    if (rn < S->stop) {
+    if (rn < sg.stop) {
       // t_done keeps the time of the iteration whose test the recurrence
       // passed (k1_test), not the time of this verification
       S->done = kConverged;
@@ -1484,15 +1558,15 @@ __global__ __launch_bounds__(kBlock) void k_cg_vcheck(CG_ARGS, int j) {
     } else {
       // the recurrence had drifted from the true residual: restart from it
       // (beta = 0 at the next iteration: an infinite "old r.z")
-      S->shift = (j ^ S->stop_par) & 1;
+      S->shift = (j ^ sg.stop_par) & 1;
       S->done = kRunning;
     }
   }
   __syncthreads();
-  if (!(sqrt(rr) < S->stop)) {
-    double *old_rz = CG_AT(prz, S->stop_par);
-    for (int k = S->blk0 + (int)threadIdx.x; k < S->blk1; k += kBlock)
-      old_rz[k] = k == S->blk0 ? INFINITY : 0.0;
+  if (!(sqrt(rr) < sg.stop)) {
+    double *old_rz = CG_AT(prz, sg.stop_par);
+    for (int k = sg.blk0 + (int)threadIdx.x; k < sg.blk1; k += kBlock)
+      old_rz[k] = k == sg.blk0 ? INFINITY : 0.0;
   }
 }
 
@@ -1504,18 +1578,18 @@ __global__ __launch_bounds__(kBlock) void k_cg_ax(CG_ARGS, int par_g, int mode) 
   CG_BIND;
   double *ax = a.ax;
   __shared__ int s_flag;
-  const int b = blockIdx.x;
-  CgSeg *S = a.seg + a.block_seg[b];
+  const int b = cg_block(multi_);
+  CG_SYSTEM(b);
   int rsel;
   if (!mode_select(S, mode, par_g, &s_flag, &rsel)) return;
-  const int r0 = S->row0 + (b - S->blk0) * S->rpb;
-  const int r1 = min(S->row1, r0 + S->rpb);
+  const int r0 = sg.row0 + (b - sg.blk0) * sg.rpb;
+  const int r1 = min(sg.row1, r0 + sg.rpb);
   const int lane = threadIdx.x & (L - 1);
   typedef CgRow<L, double> Row;
   constexpr int PASS = kBlock / L;
   for (int row = r0 + (int)threadIdx.x / L; row < r1; row += PASS) {
     Row w;
-    w.extent(a.rowptr, row, S->ent0);
+    w.extent(a.rowptr, row, sg.ent0);
     w.template load<false>(a.colidx, a.val64, a.a_nnz, a.f_col, lane);
     double g[Row::P];
 #pragma unroll
@@ -1591,11 +1665,11 @@ struct Buf {
 // launch plan (kernel variants, grid, iteration indices).  Pointers are not
 // part of it -- every kernel reads them from the argument block at run time.
 struct GraphKey {
-  int L, pre, mixed, replace, batch, nblocks, verify, dia, gdia, two;
+  int L, pre, mixed, replace, batch, nblocks, verify, dia, gdia, two, multi;
   bool operator==(const GraphKey &o) const {
     return L == o.L && pre == o.pre && mixed == o.mixed && replace == o.replace &&
            batch == o.batch && nblocks == o.nblocks && verify == o.verify && dia == o.dia &&
-           gdia == o.gdia && two == o.two;
+           gdia == o.gdia && two == o.two && multi == o.multi;
   }
 };
 
@@ -1608,17 +1682,16 @@ struct CgCache {
   Buf<double> b, x, r0, r1, p0, p1, z, ap, t64, dinv, ax;
   Buf<float> t32;
   Buf<double> ppap, prr0, prr1, prz0, prz1;
-  Buf<CgSeg> seg;
-  Buf<CgCom> com;
+  Buf<CgSeg> seg;  // a batch's systems
   Buf<int> block_seg;
   // stand-ins for A's or G^T's entry arrays when they hold no entry: one
   // column index (the block's first column) and one zero value
   Buf<int> dummy_i;
   Buf<double> dummy_d;
-  // the kernels' argument block (one CgArgs, allocated once and never moved:
+  // the kernels' argument block (one CgBlock, allocated once and never moved:
   // captured graphs name it) and its pinned staging copy
-  Buf<CgArgs> args;
-  CgArgs *h_args = nullptr;
+  Buf<CgBlock> args;
+  CgBlock *h_args = nullptr;
   CgCom *h_com = nullptr;  // pinned status copies (2)
   int *h_probe = nullptr;  // pinned: G's probe rows (extents, columns) and the dia check
   hipEvent_t ev[2] = {nullptr, nullptr};
@@ -1642,6 +1715,7 @@ struct CgCache {
   size_t f32_len = 0;
   // factor G on diagonals: offsets, slots (FP64 or FP32), the check flag
   Buf<int> gdoff;
+  int host_gdoff[8] = {};
   Buf<double> gd64;
   Buf<float> gd32;
   Buf<int> gbad;
@@ -1683,7 +1757,6 @@ struct CgCache {
     t32.release();
     gd32.release();
     seg.release();
-    com.release();
     block_seg.release();
     dummy_i.release();
     dummy_d.release();
@@ -1767,29 +1840,30 @@ struct Plan {
   bool wide;  // vectors or G's diagonals of 4 GiB or more (64-bit offsets)
   long long n;
   int nblocks;
-  const CgArgs *args;  // device argument block
+  int multi;             // a batch of systems
+  const CgBlock *args;  // device argument block
   hipStream_t s;
 };
 
 template <int L, bool MIX, bool ZBUF>
 void launch_k1(const Plan &p, int par, int check, int check_only) {
   if (!p.two) {
-    k_cg_spmv_p<L, MIX, ZBUF><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+    k_cg_spmv_p<L, MIX, ZBUF><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
     return;
   }
-  k_cg_pnew<ZBUF><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, check, check_only);
-  if (!check_only) k_cg_ap<L, MIX><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par);
+  k_cg_pnew<ZBUF><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+  if (!check_only) k_cg_ap<L, MIX><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par);
 }
 
 template <int KD>
 void launch_k1_dia(const Plan &p, bool zbuf, int par, int check, int check_only) {
   const int g = p.nblocks;
   if (p.mixed) {
-    if (zbuf) k_cg_spmv_dia<true, true, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
-    else k_cg_spmv_dia<true, false, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+    if (zbuf) k_cg_spmv_dia<true, true, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+    else k_cg_spmv_dia<true, false, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
   } else {
-    if (zbuf) k_cg_spmv_dia<false, true, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
-    else k_cg_spmv_dia<false, false, KD><<<g, kBlock, 0, p.s>>>(p.args, par, check, check_only);
+    if (zbuf) k_cg_spmv_dia<false, true, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+    else k_cg_spmv_dia<false, false, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
   }
 }
 
@@ -1830,28 +1904,28 @@ template <bool WIDE>
 void launch_k2_gdia(const Plan &p, int par, int count) {
   const int g = p.nblocks;
   if (p.gkd == 4) {
-    if (p.mixed) k_cg_update_gdia<true, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    else k_cg_update_gdia<false, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    if (p.mixed) k_cg_update_gdia<true, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
+    else k_cg_update_gdia<false, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
   } else {
-    if (p.mixed) k_cg_update_gdia<true, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    else k_cg_update_gdia<false, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    if (p.mixed) k_cg_update_gdia<true, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
+    else k_cg_update_gdia<false, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
   }
 }
 
 void launch_k2(const Plan &p, int par, int count) {
   const int g = p.nblocks;
   if (p.pre == 0) {
-    if (p.mixed) k_cg_update<0, true><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    else k_cg_update<0, false><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    if (p.mixed) k_cg_update<0, true><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
+    else k_cg_update<0, false><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
   } else if (p.pre == 1) {
-    if (p.mixed) k_cg_update<1, true><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    else k_cg_update<1, false><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    if (p.mixed) k_cg_update<1, true><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
+    else k_cg_update<1, false><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
   } else if (p.gdia) {
     if (p.wide) launch_k2_gdia<true>(p, par, count);
     else launch_k2_gdia<false>(p, par, count);
   } else {
-    if (p.mixed) k_cg_update<2, true><<<g, kBlock, 0, p.s>>>(p.args, par, count);
-    else k_cg_update<2, false><<<g, kBlock, 0, p.s>>>(p.args, par, count);
+    if (p.mixed) k_cg_update<2, true><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
+    else k_cg_update<2, false><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, count);
   }
 }
 
@@ -1859,11 +1933,11 @@ template <bool WIDE>
 void launch_gz_gdia(const Plan &p, int par, int mode) {
   const int g = p.nblocks;
   if (p.gkd == 4) {
-    if (p.mixed) k_cg_gz_gdia<true, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
-    else k_cg_gz_gdia<false, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
+    if (p.mixed) k_cg_gz_gdia<true, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
+    else k_cg_gz_gdia<false, 4, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
   } else {
-    if (p.mixed) k_cg_gz_gdia<true, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
-    else k_cg_gz_gdia<false, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, par, mode);
+    if (p.mixed) k_cg_gz_gdia<true, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
+    else k_cg_gz_gdia<false, 8, WIDE><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
   }
 }
 
@@ -1872,37 +1946,37 @@ void launch_gz(const Plan &p, int par, int mode) {
     if (p.wide) launch_gz_gdia<true>(p, par, mode);
     else launch_gz_gdia<false>(p, par, mode);
   } else {
-    if (p.mixed) k_cg_gz<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-    else k_cg_gz<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
+    if (p.mixed) k_cg_gz<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
+    else k_cg_gz<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
   }
 }
 
 void launch_gtr(const Plan &p, int par, int mode) {
   if (p.gdia) {
-    if (p.mixed) k_cg_gtr_gdia<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-    else k_cg_gtr_gdia<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
+    if (p.mixed) k_cg_gtr_gdia<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
+    else k_cg_gtr_gdia<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
   } else {
-    if (p.mixed) k_cg_gtr<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
-    else k_cg_gtr<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode);
+    if (p.mixed) k_cg_gtr<true><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
+    else k_cg_gtr<false><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode);
   }
 }
 
 void launch_residual(const Plan &p, int use_ax, int par, int mode, int zero_x) {
-  if (p.pre == 1) k_cg_residual<1><<<p.nblocks, kBlock, 0, p.s>>>(p.args, use_ax, par, mode, zero_x);
-  else if (p.pre == 0) k_cg_residual<0><<<p.nblocks, kBlock, 0, p.s>>>(p.args, use_ax, par, mode, zero_x);
-  else k_cg_residual<2><<<p.nblocks, kBlock, 0, p.s>>>(p.args, use_ax, par, mode, zero_x);
+  if (p.pre == 1) k_cg_residual<1><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, use_ax, par, mode, zero_x);
+  else if (p.pre == 0) k_cg_residual<0><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, use_ax, par, mode, zero_x);
+  else k_cg_residual<2><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, use_ax, par, mode, zero_x);
 }
 
 // ax = A x with the FP64 matrix, for the systems the mode selects
 void launch_ax(const Plan &p, int par, int mode) {
   switch (p.L) {
-    case 1: k_cg_ax<1><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
-    case 2: k_cg_ax<2><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
-    case 4: k_cg_ax<4><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
-    case 8: k_cg_ax<8><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
-    case 16: k_cg_ax<16><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
-    case 32: k_cg_ax<32><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
-    default: k_cg_ax<64><<<p.nblocks, kBlock, 0, p.s>>>(p.args, par, mode); break;
+    case 1: k_cg_ax<1><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
+    case 2: k_cg_ax<2><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
+    case 4: k_cg_ax<4><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
+    case 8: k_cg_ax<8><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
+    case 16: k_cg_ax<16><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
+    case 32: k_cg_ax<32><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
+    default: k_cg_ax<64><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par, mode); break;
   }
 }
 
@@ -1932,7 +2006,7 @@ void enqueue_iteration(const Plan &p, int i, bool tail) {
   else if (p.pre == 2) launch_gz(p, par, kAfterIter);
   if (p.verify && (replace || tail)) {
     true_residual(p, par, kVerify);
-    k_cg_vcheck<<<p.nblocks, kBlock, 0, p.s>>>(p.args, (i + 1) & 1);
+    k_cg_vcheck<<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, (i + 1) & 1);
   }
 }
 
@@ -1970,7 +2044,8 @@ int build_gdia(CgCache &c, const tbsla_hip_matrix_s *G, bool mixed, hipStream_t 
   const int ndg = (int)off.size();
   const size_t slots = (size_t)((n + kWave - 1) / kWave) * kWave * ndg;
   TBSLA_TRY(c.gdoff.ensure(kMaxDiag));
-  for (int k = 0; k < ndg; k++) h[kProbeRows * 9 + k] = off[k];
+  static_assert(kMaxDiag <= sizeof c.host_gdoff / sizeof(int), "offsets at hand");
+  for (int k = 0; k < ndg; k++) h[kProbeRows * 9 + k] = c.host_gdoff[k] = off[k];
   TBSLA_HIP_CHECK(hipMemcpyAsync(c.gdoff.p, h + kProbeRows * 9, ndg * sizeof(int),
                                  hipMemcpyHostToDevice, s));
   TBSLA_HIP_CHECK(hipMemsetAsync(c.gbad.p, 0, sizeof(int), s));
@@ -2111,12 +2186,12 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   for (auto *v : vecs) TBSLA_TRY(v->ensure((size_t)n));
   Buf<double> *parts[] = {&c.ppap, &c.prr0, &c.prr1, &c.prz0, &c.prz1};
   for (auto *v : parts) TBSLA_TRY(v->ensure((size_t)nblocks));
-  TBSLA_TRY(c.seg.ensure(nsys));
-  TBSLA_TRY(c.com.ensure(1));
+  const bool multi = nsys > 1;
+  if (multi) TBSLA_TRY(c.seg.ensure(nsys));
   TBSLA_TRY(c.args.ensure(1));
-  TBSLA_TRY(c.block_seg.ensure(nblocks));
+  if (multi) TBSLA_TRY(c.block_seg.ensure(nblocks));
   if (!c.h_com) TBSLA_HIP_CHECK(hipHostMalloc((void **)&c.h_com, 2 * sizeof(CgCom), hipHostMallocDefault));
-  if (!c.h_args) TBSLA_HIP_CHECK(hipHostMalloc((void **)&c.h_args, sizeof(CgArgs), hipHostMallocDefault));
+  if (!c.h_args) TBSLA_HIP_CHECK(hipHostMalloc((void **)&c.h_args, sizeof(CgBlock), hipHostMallocDefault));
   for (auto &e : c.ev)
     if (!e) TBSLA_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   if (pre == TBSLA_HIP_PRECOND_JACOBI) TBSLA_TRY(c.dinv.ensure((size_t)n));
@@ -2201,6 +2276,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
       a.gd64 = c.gd64.p;
       a.gd32 = c.gd32.p;
       a.gndiag = gndiag;
+      for (int k = 0; k < 8; k++) a.gdoff8[k] = c.host_gdoff[std::min(k, gndiag - 1)];
     } else {
       a.g_rp = G->rowptr;
       a.g_ci = G->colidx;
@@ -2229,19 +2305,19 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   a.prr[1] = c.prr1.p;
   a.prz[0] = c.prz0.p;
   a.prz[1] = c.prz1.p;
-  a.seg = c.seg.p;
-  a.com = c.com.p;
+  a.seg = multi ? c.seg.p : &c.args.p->seg;
+  a.com = &c.args.p->com;
   a.block_seg = c.block_seg.p;
   a.verify = (mixed || o.replace_every > 0) ? 1 : 0;
   a.stall_window = o.stall_window;
   a.ncol = (int)m->ln_col;
   // A in the diagonal layout with no remote entries: K1 reads its diagonals
-  const int *d_off = nullptr;
+  const int *d_off = nullptr, *h_off = nullptr;
   const double *d_v = nullptr;
   int ndiag = 0;
   long long dv_len = 0;
   unsigned long long build = 0;
-  const bool dia = split_diag_only(m, &d_off, &d_v, &ndiag, &dv_len, &build) && m->ln_col > 0;
+  const bool dia = split_diag_only(m, &d_off, &h_off, &d_v, &ndiag, &dv_len, &build) && m->ln_col > 0;
   // K1 on CSR rows in two passes: asked for, or picked for large blocks,
   // whose gathers of z and p miss the caches (a random column then costs
   // one line fill instead of two)
@@ -2249,6 +2325,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
                             (o.spmv_passes == 0 && m->stored >= kTwoPassEntries));
   if (dia) {
     a.doff = d_off;
+    std::copy_n(h_off, std::min(ndiag, 8), a.doff8);
     a.dv64 = d_v;
     a.ndiag = ndiag;
     if (mixed) {
@@ -2312,6 +2389,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   p.gkd = gndiag <= 4 ? 4 : 8;
   p.n = n;
   p.nblocks = nblocks;
+  p.multi = multi ? 1 : 0;
   p.args = c.args.p;
   p.s = s;
 
@@ -2319,14 +2397,14 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   // work has finished with the previous contents, see the end of the solve),
   // layout, inputs, start
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-  *c.h_args = a;
+  *c.h_args = CgBlock{a, hs[0], CgCom{}};
   const int fcol = m->f_col;
-  CgCom com0{};
-  TBSLA_HIP_CHECK(hipMemcpyAsync(c.args.p, c.h_args, sizeof(CgArgs), hipMemcpyHostToDevice, s));
+  TBSLA_HIP_CHECK(hipMemcpyAsync(c.args.p, c.h_args, sizeof(CgBlock), hipMemcpyHostToDevice, s));
   TBSLA_HIP_CHECK(hipMemcpyAsync(c.dummy_i.p, &fcol, sizeof fcol, hipMemcpyHostToDevice, s));
-  TBSLA_HIP_CHECK(hipMemcpyAsync(c.seg.p, hs.data(), sizeof(CgSeg) * nsys, hipMemcpyHostToDevice, s));
-  TBSLA_HIP_CHECK(hipMemcpyAsync(c.block_seg.p, hb.data(), sizeof(int) * nblocks, hipMemcpyHostToDevice, s));
-  TBSLA_HIP_CHECK(hipMemcpyAsync(c.com.p, &com0, sizeof com0, hipMemcpyHostToDevice, s));
+  if (multi) {
+    TBSLA_HIP_CHECK(hipMemcpyAsync(c.seg.p, hs.data(), sizeof(CgSeg) * nsys, hipMemcpyHostToDevice, s));
+    TBSLA_HIP_CHECK(hipMemcpyAsync(c.block_seg.p, hb.data(), sizeof(int) * nblocks, hipMemcpyHostToDevice, s));
+  }
 
   TBSLA_HIP_CHECK(hipMemcpyAsync(c.b.p, d_rhs, (size_t)n * 8, hipMemcpyDeviceToDevice, s));
   // x of inactive systems stays as given; active ones start at 0 unless the
@@ -2348,7 +2426,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   const bool reference_setting = !o.relative && !mixed && pre == TBSLA_HIP_PRECOND_NONE;
   const double near_zero = o.near_zero > 0 ? o.near_zero
                            : (o.near_zero < 0 ? 1e-300 : (reference_setting ? kNearZero : 1e-300));
-  k_cg_start<<<nblocks, kBlock, 0, s>>>(p.args, o.tolerance, o.relative, near_zero);
+  k_cg_start<<<nblocks, kBlock, 0, s>>>(p.args, p.multi, o.tolerance, o.relative, near_zero);
   TBSLA_HIP_LAUNCH_CHECK();
 
   // Graph batches of B iterations starting at 1 + tB (B even, so every
@@ -2377,6 +2455,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   key.replace = p.replace;
   key.batch = B;
   key.nblocks = nblocks;
+  key.multi = p.multi;
   key.verify = p.verify;
   key.dia = p.dia ? 1 + p.dkd : 0;
   key.gdia = p.gdia ? p.gkd + (p.wide ? 16 : 0) : 0;
@@ -2446,7 +2525,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
     }
     TBSLA_HIP_LAUNCH_CHECK();
     const int slot = batches & 1;
-    TBSLA_HIP_CHECK(hipMemcpyAsync(c.h_com + slot, c.com.p, sizeof(CgCom), hipMemcpyDeviceToHost, s));
+    TBSLA_HIP_CHECK(hipMemcpyAsync(c.h_com + slot, a.com, sizeof(CgCom), hipMemcpyDeviceToHost, s));
     TBSLA_HIP_CHECK(hipEventRecord(c.ev[slot], s));
     if (batches > 0) {
       const int prev = slot ^ 1;
@@ -2454,7 +2533,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
       const CgCom h = c.h_com[prev];
       if (h.npending > 0 && p.verify) {
         true_residual(p, 0, kVerify);
-        k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, it);
+        k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, p.multi, it);
         TBSLA_HIP_LAUNCH_CHECK();
       }
       if (h.ndone >= nactive) finished = true;
@@ -2463,20 +2542,20 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   }
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   CgCom h{};
-  TBSLA_HIP_CHECK(hipMemcpy(&h, c.com.p, sizeof h, hipMemcpyDeviceToHost));
+  TBSLA_HIP_CHECK(hipMemcpy(&h, a.com, sizeof h, hipMemcpyDeviceToHost));
   if (h.ndone < nactive) {
     // the final test after the last iteration (CG.cpp:66-72), then the
     // true residual of systems whose recurrence converged
     if (max_it > 0) launch_k1_any(p, it & 1, 1, 1);
     if (p.verify) {
       true_residual(p, 0, kVerify);
-      k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, it);
+      k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, p.multi, it);
     }
     TBSLA_HIP_LAUNCH_CHECK();
   }
   TBSLA_HIP_CHECK(hipMemcpyAsync(d_x, c.x.p, (size_t)n * 8, hipMemcpyDeviceToDevice, s));
-  TBSLA_HIP_CHECK(hipMemcpyAsync(hs.data(), c.seg.p, sizeof(CgSeg) * nsys, hipMemcpyDeviceToHost, s));
-  TBSLA_HIP_CHECK(hipMemcpyAsync(&h, c.com.p, sizeof h, hipMemcpyDeviceToHost, s));
+  TBSLA_HIP_CHECK(hipMemcpyAsync(hs.data(), a.seg, sizeof(CgSeg) * nsys, hipMemcpyDeviceToHost, s));
+  TBSLA_HIP_CHECK(hipMemcpyAsync(&h, a.com, sizeof h, hipMemcpyDeviceToHost, s));
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   int dev = 0, khz = 0;
   (void)hipGetDevice(&dev);

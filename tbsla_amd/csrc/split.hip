@@ -75,6 +75,7 @@ struct SplitCsr {
   int ndiag = 0;  // diagonal layout: stored diagonals
   int *lrp = nullptr, *lci = nullptr, *sr = nullptr, *sc = nullptr, *boff = nullptr;
   int *doff = nullptr;  // their offsets c - r, ascending
+  std::vector<int> hoff;  // the same on the host
   double *lv = nullptr, *sv = nullptr, *P = nullptr, *R = nullptr;
   double *dv = nullptr;  // dv[k n + r]: row r's entry on diagonal k, or 0
   std::vector<long long> soff;  // slice boundaries (host)
@@ -768,12 +769,14 @@ int split_lds_block_rows(const tbsla_hip_matrix_s *m) {
   return sp ? sp->lds_h : 0;
 }
 
-int split_diag_only(const tbsla_hip_matrix_s *m, const int **doff, const double **dv, int *ndiag,
-                    long long *dv_len, unsigned long long *build_id) {
+int split_diag_only(const tbsla_hip_matrix_s *m, const int **doff, const int **hoff,
+                    const double **dv, int *ndiag, long long *dv_len,
+                    unsigned long long *build_id) {
   const SplitCsr *sp = static_cast<const SplitCsr *>(m->split);
   if (!sp || sp->layout != TBSLA_HIP_CSR_DIAG || sp->nr != 0 || sp->ndiag == 0) return 0;
   *build_id = sp->build_id;
   *doff = sp->doff;
+  *hoff = sp->hoff.data();
   *dv = sp->dv;
   *ndiag = sp->ndiag;
   *dv_len = (long long)sp->ndiag * ((layout_rows(m).n + kWave - 1) / kWave) * kWave;
@@ -946,6 +949,7 @@ int split_build(tbsla_hip_matrix_s *m, int window, int slices, hipStream_t s, in
       map[cand[k]] = (int)k;
       offs[k] = (int)(cand[k] - window + lr.r0);  // the kernels read x at r + offs[k]
     }
+    sp->hoff = offs;
     if ((st = device_alloc((void **)&sp->doff, offs.size() * 4)) ||
         (st = device_alloc((void **)&sp->dv, dia_bytes)))
       return failed(st);
