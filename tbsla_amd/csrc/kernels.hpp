@@ -31,12 +31,14 @@ int launch_fill(double *d, long long n, double v, hipStream_t s);
 int launch_axpy_inplace(double *y, const double *x, long long n, hipStream_t s);  // y += x
 
 // sort.hip: stable LSD radix sort of 32- or 64-bit keys (key_bits significant
-// bits), *payload receiving each key's original position.  Buffers of n
+// bits, the lowest `low` of which are left unsorted), *payload receiving each key's
+// original position.  Buffers of n
 // elements from device_alloc; the sort works between them and two of its own
 // and leaves in *keys / *payload the pair that holds the result (it frees the
 // other).  Synchronises the stream.
 template <typename K>
-int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s);
+int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s,
+                     int low = 0);
 // Keys taken from column indices: the local column, or ln_col outside the block.
 struct ColumnKeys {
   const int *cols;
@@ -50,7 +52,7 @@ struct ColumnKeys {
 // radix_sort_pairs<unsigned> of src's n keys, read by the first pass in place of
 // *keys (whose contents are ignored)
 int radix_sort_columns(const ColumnKeys &src, unsigned **keys, int **payload, long long n,
-                       int key_bits, hipStream_t s);
+                       int key_bits, hipStream_t s, int low = 0);
 // ptr[b] = the first k with (keys[k] >> shift) >= b, b in [0, nb], of n sorted keys
 template <typename K>
 int bucket_starts(const K *keys, long long n, int shift, long long nb, int *ptr, hipStream_t s);

@@ -13,6 +13,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "radix_tile.hpp"
 
 namespace tbsla_hip {
 
@@ -79,50 +80,51 @@ __global__ __launch_bounds__(kBlock) void k_ell_colkeys(long long n, long long l
 // MatrixSCOO::get_col_sums (MatrixSCOO.cpp:719-723); ELL adds positive
 // values only (MatrixELL.cpp:809-815).
 //
-// A workgroup takes 256 columns, whose sorted positions are one contiguous
-// run: it goes through LDS in chunks, loaded by consecutive lanes with the
-// gathers of eight values in flight each, and every thread then adds its own
-// column's values from LDS, in order (one spare double per 16 keeps the
-// columns of a regular matrix on different banks).  24 M entries: 107 us,
-// against 554 with each thread walking its positions in memory.
-constexpr int kSumChunk = 4096;
+// The entries come sorted by all but the keys' `low` bits: a workgroup takes 2^low
+// columns, whose entries are one contiguous run, in chunks of a tile.  It gathers
+// a chunk's values, puts them into LDS in the order of those last bits (a pass of
+// the sort that never leaves the CU), and thread d adds column d's values from
+// there, in order (one spare double per 16 spreads equal columns over the banks).
+// 24 M entries, 16 to a column: 148 us, where a third pass of the sort (155), the
+// starts of every column (57) and sums in sorted order (105) took 317.
+constexpr int kSumThreads = 512, kSumItems = 8, kSumChunk = kSumThreads * kSumItems;
 
-__global__ __launch_bounds__(kBlock) void k_col_sums(long long ln_col, int fmt, long long ln_row,
-                                                     int max_col, const int *__restrict__ colptr,
-                                                     const int *__restrict__ pos,
-                                                     const double *__restrict__ vals,
-                                                     double *__restrict__ s) {
+__global__ __launch_bounds__(kSumThreads) void k_col_sums(
+    long long ln_col, int fmt, long long ln_row, int max_col, int low,
+    const int *__restrict__ starts, const unsigned *__restrict__ keys,
+    const int *__restrict__ pos, const double *__restrict__ vals, double *__restrict__ s) {
+  __shared__ TileRank<kSumThreads> sh;
   __shared__ double buf[kSumChunk + kSumChunk / 16];
-  const long long c0 = (long long)blockIdx.x * kBlock;
-  const long long c = c0 + threadIdx.x;
-  const bool live = c < ln_col;
-  const int first = colptr[c0], last = colptr[min(c0 + kBlock, ln_col)];
-  const int beg = live ? colptr[c] : last, end = live ? colptr[c + 1] : last;
+  const long long c = ((long long)blockIdx.x << low) + threadIdx.x;
+  const bool live = (int)threadIdx.x < (1 << low) && c < ln_col;
+  const int first = starts[blockIdx.x], last = starts[blockIdx.x + 1];
+  const int sub = tile_sub<kSumItems>();
   double acc = live ? s[c] : 0.0;
-  int j = beg;
   for (int b = first; b < last; b += kSumChunk) {
-    const int m = min(kSumChunk, last - b);
-    for (int i0 = threadIdx.x; i0 < m; i0 += 8 * kBlock) {
-      long long p[8];
-      double v[8];
+    const int count = min(kSumChunk, last - b);
+    unsigned key[kSumItems];
+    long long p[kSumItems];
+    double v[kSumItems];
+    int at[kSumItems], start = 0, total = 0;
 #pragma unroll
-      for (int k = 0; k < 8; k++) p[k] = pos[b + min(i0 + k * kBlock, m - 1)];
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-        v[k] = vals[fmt == TBSLA_HIP_ELL ? (p[k] % max_col) * ln_row + p[k] / max_col : p[k]];
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const int i = i0 + k * kBlock;
-        if (i < m) buf[i + (i >> 4)] = v[k];
-      }
+    for (int k = 0; k < kSumItems; k++) {
+      const int e = b + min(sub + k * kWave, count - 1);
+      key[k] = keys[e];
+      p[k] = pos[e];
     }
+#pragma unroll
+    for (int k = 0; k < kSumItems; k++)
+      v[k] = vals[fmt == TBSLA_HIP_ELL ? (p[k] % max_col) * ln_row + p[k] / max_col : p[k]];
+    rank_tile<kSumThreads, kSumItems, unsigned>(sh, key, at, count, 0, low, start, total);
+#pragma unroll
+    for (int k = 0; k < kSumItems; k++)
+      if (sub + k * kWave < count) buf[at[k] + (at[k] >> 4)] = v[k];
     __syncthreads();
-    const int stop = min(end, b + m);
-    for (; j < stop; j++) {
-      const int i = j - b;
-      const double v = buf[i + (i >> 4)];
-      if (fmt != TBSLA_HIP_ELL || v > 0) acc += v;
-    }
+    if (live)
+      for (int i = start; i < start + total; i++) {
+        const double x = buf[i + (i >> 4)];
+        if (fmt != TBSLA_HIP_ELL || x > 0) acc += x;
+      }
     __syncthreads();
   }
   if (live) s[c] = acc;
@@ -548,22 +550,29 @@ extern "C" int tbsla_hip_get_col_sums(tbsla_hip_matrix_t m, double *d_s, void *s
   DevBuf<int> pos, colptr;
   TBSLA_TRY(keys.alloc(n));
   TBSLA_TRY(pos.alloc(n));
-  TBSLA_TRY(colptr.alloc(ln_col + 1));
   int bits = 1;
   while (bits < 32 && (1LL << bits) <= ln_col) bits++;  // keys <= ln_col < 2^bits
+  // the bits left to the sums: as many as spare the sort a pass, then as few as
+  // give a workgroup half a chunk or more
+  const int passes = std::max(1, (bits - 1) / 8);
+  int low = std::min(8, bits - 1);
+  while (low > std::max(0, bits - 8 * passes) && ((n << low) / std::max(ln_col, 1LL)) > 3 * kSumChunk / 4)
+    low--;
+  const long long nb = (ln_col >> low) + 1;
+  TBSLA_TRY(colptr.alloc(nb + 1));
   if (fmt == TBSLA_HIP_ELL) {
     k_ell_colkeys<<<grid_for(n), kBlock, 0, s>>>(n, m->ln_row, ln_col, m->max_col, m->colidx,
                                                  m->values, m->f_col, keys.p);
     TBSLA_HIP_LAUNCH_CHECK();
-    TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s));
+    TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s, low));
   } else {
     const ColumnKeys src{m->colidx, m->f_col, (unsigned)ln_col};
-    TBSLA_TRY(radix_sort_columns(src, &keys.p, &pos.p, n, bits, s));
+    TBSLA_TRY(radix_sort_columns(src, &keys.p, &pos.p, n, bits, s, low));
   }
-  TBSLA_TRY(bucket_starts<unsigned>(keys.p, n, 0, ln_col, colptr.p, s));
+  TBSLA_TRY(bucket_starts<unsigned>(keys.p, n, low, nb, colptr.p, s));
   if (ln_col > 0) {
-    k_col_sums<<<grid_for(ln_col), kBlock, 0, s>>>(ln_col, fmt, m->ln_row, m->max_col, colptr.p,
-                                                   pos.p, m->values, d_s);
+    k_col_sums<<<(unsigned)nb, kSumThreads, 0, s>>>(ln_col, fmt, m->ln_row, m->max_col, low,
+                                                    colptr.p, keys.p, pos.p, m->values, d_s);
     TBSLA_HIP_LAUNCH_CHECK();
   }
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));

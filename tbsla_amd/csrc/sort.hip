@@ -15,12 +15,12 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "radix_tile.hpp"
 
 namespace tbsla_hip {
 
 namespace {
 
-constexpr int kRadix = 256;
 constexpr int kItems = 16;  // keys per thread of a tile
 
 // Tiles: 512 threads for 32-bit keys, 256 for 64-bit ones; both put 32 KB of
@@ -79,81 +79,6 @@ __global__ __launch_bounds__(T::threads) void k_digit_hist(
   }
 }
 
-// Places of a tile's elements in digit order.  Thread t holds elements
-// sub + i * kWave (sub below); pos[i] is element i's place in the tile, and
-// sh.gofs[d] turns a place into the output position of digit d's elements.
-template <int THREADS>
-struct TileRank {
-  int wcnt[THREADS / kWave][kRadix];  // counts, then each wave's first position
-  int gofs[kRadix];                   // output position minus tile position
-  int wsum[THREADS / kWave];
-};
-
-// this lane's first element of the tile
-template <int ITEMS>
-__device__ inline int tile_sub() {
-  return threadIdx.x / kWave * kWave * ITEMS + (threadIdx.x & (kWave - 1));
-}
-
-template <int THREADS, int ITEMS, typename K>
-__device__ inline void rank_tile(TileRank<THREADS> &sh, const K (&key)[ITEMS], int (&pos)[ITEMS],
-                                 int count, int shift, int bits, long long ntiles,
-                                 const int *__restrict__ offsets) {
-  constexpr int waves = THREADS / kWave;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int mask = (1 << bits) - 1, sub = tile_sub<ITEMS>();
-  for (int i = threadIdx.x; i < waves * kRadix; i += THREADS) (&sh.wcnt[0][0])[i] = 0;
-  __syncthreads();
-  // rank of every element among its wave's elements of the same digit
-  const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
-#pragma unroll
-  for (int i = 0; i < ITEMS; i++) {
-    const bool valid = sub + i * kWave < count;
-    const int d = (int)(key[i] >> shift) & mask;
-    unsigned long long peers = __ballot(valid);
-    for (int b = 0; b < bits; b++) {
-      const bool bit = (d >> b) & 1;
-      const unsigned long long m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
-    const int rank = __popcll(peers & below);
-    const int before = valid ? sh.wcnt[wave][d] : 0;
-    pos[i] = before + rank;
-    __builtin_amdgcn_wave_barrier();
-    if (valid && rank == 0) sh.wcnt[wave][d] = before + __popcll(peers);
-    __builtin_amdgcn_wave_barrier();
-  }
-  __syncthreads();
-  // digit starts within the tile (exclusive scan over digits), wave starts
-  // within each digit; thread d < kRadix owns digit d
-  int total = 0, incl = 0;
-  if (threadIdx.x < kRadix) {
-    for (int w = 0; w < waves; w++) {
-      const int c = sh.wcnt[w][threadIdx.x];
-      sh.wcnt[w][threadIdx.x] = total;
-      total += c;
-    }
-    incl = total;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int o = __shfl_up(incl, off, kWave);
-      if (lane >= off) incl += o;
-    }
-    if (lane == kWave - 1) sh.wsum[wave] = incl;
-  }
-  __syncthreads();
-  if (threadIdx.x < kRadix) {
-    int start = incl - total;
-    for (int w = 0; w < wave; w++) start += sh.wsum[w];
-    for (int w = 0; w < waves; w++) sh.wcnt[w][threadIdx.x] += start;
-    if ((int)threadIdx.x <= mask)
-      sh.gofs[threadIdx.x] = offsets[(long long)threadIdx.x * ntiles + blockIdx.x] - start;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < ITEMS; i++) pos[i] += sh.wcnt[wave][(int)(key[i] >> shift) & mask];
-}
-
 // The stable scatter of one pass; pay_in null: the payload of element e is e
 // (the first pass).  Bound by its bytes once the output runs are whole: 24 M
 // 32-bit keys take 101 us a pass (16 bytes an element, 3.8 TB/s) where
@@ -182,7 +107,10 @@ __global__ __launch_bounds__(SortTile<K>::threads) void k_digit_scatter(
     const int e = sub + i * kWave;
     pay[i] = pay_in ? (e < count ? pay_in[tile0 + e] : 0) : (int)(tile0 + e);
   }
-  rank_tile<T::threads, kItems, K>(sh, key, pos, count, shift, bits, ntiles, offsets);
+  int start, total;
+  rank_tile<T::threads, kItems, K>(sh, key, pos, count, shift, bits, start, total);
+  if ((int)threadIdx.x <= mask)
+    sh.gofs[threadIdx.x] = offsets[(long long)threadIdx.x * ntiles + blockIdx.x] - start;
 #pragma unroll
   for (int i = 0; i < kItems; i++)
     if (sub + i * kWave < count) stage[pos[i]] = key[i];
@@ -239,7 +167,10 @@ __global__ __launch_bounds__(kEntThreads) void k_entry_scatter(
     other[i] = other_in[tile0 + e];
     val[i] = val_in[tile0 + e];
   }
-  rank_tile<kEntThreads, kEntItems, unsigned>(sh, key, pos, count, shift, bits, ntiles, offsets);
+  int start, total;
+  rank_tile<kEntThreads, kEntItems, unsigned>(sh, key, pos, count, shift, bits, start, total);
+  if ((int)threadIdx.x <= mask)
+    sh.gofs[threadIdx.x] = offsets[(long long)threadIdx.x * ntiles + blockIdx.x] - start;
   int *istage = reinterpret_cast<int *>(stage);
 #pragma unroll
   for (int i = 0; i < kEntItems; i++)
@@ -279,8 +210,8 @@ __global__ __launch_bounds__(kEntThreads) void k_entry_scatter(
 // ptr[b] = the first k with (keys[k] >> shift) >= b, for b in [0, nb]: the
 // bucket starts of sorted keys, by binary search (no atomics: counting 24 M
 // banded keys by atomic additions took 1053 us, and 4.8 M with hub rows 317).
-// Two threads find the ends of their workgroup's 256 buckets among all keys,
-// the others search between them.
+// Two waves find the ends of their workgroup's 256 buckets among all keys, 64
+// probes at a time; the threads then search between them.
 template <typename K>
 __device__ inline long long first_at_least(const K *__restrict__ keys, int shift, long long lo,
                                            long long hi, long long b) {
@@ -298,9 +229,21 @@ __global__ __launch_bounds__(kBlock) void k_bucket_starts(const K *__restrict__ 
                                                           int *__restrict__ ptr) {
   __shared__ long long ends[2];
   const long long b0 = (long long)blockIdx.x * kBlock, b = b0 + threadIdx.x;
-  if (threadIdx.x % kWave == 0 && threadIdx.x < 2 * kWave)
-    ends[threadIdx.x / kWave] =
-        first_at_least(keys, shift, 0, n, threadIdx.x ? b0 + kBlock : b0);
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  if (wave < 2) {
+    const long long want = b0 + wave * kBlock;
+    long long lo = 0, hi = n;  // the answer lies in [lo, hi]
+    while (hi - lo > kWave) {
+      const long long step = (hi - lo) / kWave, at = lo + lane * step;
+      const unsigned long long less = __ballot((long long)(keys[at] >> shift) < want);
+      const int m = __popcll(less);  // probes below `want`: lanes 0 .. m - 1
+      if (m < kWave) hi = lo + m * step;
+      lo = m ? lo + (m - 1) * step + 1 : lo;
+    }
+    const unsigned long long less =
+        __ballot(lo + lane < hi && (long long)(keys[min(lo + lane, n - 1)] >> shift) < want);
+    if (lane == 0) ends[wave] = lo + __popcll(less);
+  }
   __syncthreads();
   if (b <= nb) ptr[b] = (int)first_at_least(keys, shift, ends[0], ends[1], b);
 }
@@ -373,12 +316,12 @@ int bits_for(long long v) {
 
 template <typename K, typename Src>
 static int radix_sort_from(const Src *first, K **keys, int **payload, long long n, int key_bits,
-                           hipStream_t s) {
+                           hipStream_t s, int low = 0) {
   typedef SortTile<K> T;
   if (n <= 0) return TBSLA_HIP_SUCCESS;
   const long long ntiles = (n + T::elems - 1) / T::elems;
-  const int passes = std::max(1, (key_bits + 7) / 8);
-  const int bits = std::max(1, (key_bits + passes - 1) / passes);
+  const int passes = std::max(1, (key_bits - low + 7) / 8);
+  const int bits = std::max(1, (key_bits - low + passes - 1) / passes);
   const long long hist_n = (1LL << bits) * ntiles;
   K *keys_alt = nullptr;
   int *pay_alt = nullptr, *hist = nullptr;
@@ -399,7 +342,7 @@ static int radix_sort_from(const Src *first, K **keys, int **payload, long long 
     return st;
   }
   for (int p = 0; p < passes; p++) {
-    const int shift = bits * p, b = std::min(bits, std::max(1, key_bits - shift));
+    const int shift = low + bits * p, b = std::min(bits, std::max(1, key_bits - shift));
     const K *kin = *keys;
     if (p == 0 && first)
       k_digit_hist<T><<<(unsigned)ntiles, T::threads, 0, s>>>(*first, n, shift, (1 << b) - 1,
@@ -426,18 +369,18 @@ static int radix_sort_from(const Src *first, K **keys, int **payload, long long 
 }
 
 template <typename K>
-int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s) {
-  return radix_sort_from<K, const K *>(nullptr, keys, payload, n, key_bits, s);
+int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s, int low) {
+  return radix_sort_from<K, const K *>(nullptr, keys, payload, n, key_bits, s, low);
 }
 
 int radix_sort_columns(const ColumnKeys &src, unsigned **keys, int **payload, long long n,
-                       int key_bits, hipStream_t s) {
-  return radix_sort_from<unsigned, ColumnKeys>(&src, keys, payload, n, key_bits, s);
+                       int key_bits, hipStream_t s, int low) {
+  return radix_sort_from<unsigned, ColumnKeys>(&src, keys, payload, n, key_bits, s, low);
 }
 
-template int radix_sort_pairs<unsigned>(unsigned **, int **, long long, int, hipStream_t);
+template int radix_sort_pairs<unsigned>(unsigned **, int **, long long, int, hipStream_t, int);
 template int radix_sort_pairs<unsigned long long>(unsigned long long **, int **, long long, int,
-                                                  hipStream_t);
+                                                  hipStream_t, int);
 
 template <typename K>
 int bucket_starts(const K *keys, long long n, int shift, long long nb, int *ptr, hipStream_t s) {
