@@ -208,6 +208,44 @@ __device__ inline double group_sum(double v) {
   return v;
 }
 
+// v[k] of lane l (of 4 or 2 adjacent ones) <-> v[l] of lane k: a load of N
+// consecutive entries per lane turned so that each of the N values lies beside
+// its neighbours' in the lanes.  A gather by those columns then touches a few
+// lines per instruction, as the columns of consecutive entries are near each other,
+// where strides of N entries between the lanes cost the address unit a lookup for
+// every second lane.  Quad permutes and selects: 3 instructions a pair and word.
+template <int N>
+__device__ inline void lane_transpose(int (&v)[N]) {
+  static_assert(N == 2 || N == 4, "adjacent lanes");
+  const bool odd = threadIdx.x & 1, high = threadIdx.x & 2;
+#pragma unroll
+  for (int k = 0; k < N; k += 2) {  // lanes l, l ^ 1
+    const int t = __builtin_amdgcn_mov_dpp(odd ? v[k] : v[k + 1], 0xB1, 0xf, 0xf, true);
+    v[k] = odd ? t : v[k];
+    v[k + 1] = odd ? v[k + 1] : t;
+  }
+  if constexpr (N == 4)
+#pragma unroll
+    for (int k = 0; k < 2; k++) {  // lanes l, l ^ 2
+      const int t = __builtin_amdgcn_mov_dpp(high ? v[k] : v[k + 2], 0x4E, 0xf, 0xf, true);
+      v[k] = high ? t : v[k];
+      v[k + 2] = high ? v[k + 2] : t;
+    }
+}
+template <int N>
+__device__ inline void lane_transpose(double (&v)[N]) {
+  int lo[N], hi[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    lo[k] = __double2loint(v[k]);
+    hi[k] = __double2hiint(v[k]);
+  }
+  lane_transpose<N>(lo);
+  lane_transpose<N>(hi);
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = __hiloint2double(hi[k], lo[k]);
+}
+
 // Inside a kernel that must round a*b+c twice, as the reference's loops do
 // (HIP compiles with fp-contract=fast, which would fuse them).
 #define TBSLA_NO_FMA _Pragma("clang fp contract(off)")

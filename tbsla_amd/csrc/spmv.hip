@@ -329,27 +329,30 @@ int coo_rowptr(tbsla_hip_matrix_s *m, long long n, bool *ok, hipStream_t s) {
 }
 
 // The row kernel for a mean row length.  Every compiled kernel was timed on
-// cqmats (q = 0.1) of 20,000 to 2.5 M rows with 3 to 34 entries, three matrices
+// cqmats (q = 0.1) of 3,000 to 2.5 M rows with 3 to 1000 entries, three matrices
 // in turn; the line lies where the neighbours meet, and each choice is within
-// 6 % of the best at 10^6 rows.  A quad of entries per lane (V = 4) makes a
-// row's lines whole per instruction, and pays from ten entries on; below, the
-// quads of short rows are mostly slack.  One million rows, against V = 1 with
-// two entries per lane, four rows in flight and the non-temporal hint (the rule
-// before): 5 entries 32 -> 22 us, 8: 44 -> 29, 12: 63 -> 40, 17: 99 -> 72, 24:
-// 109 -> 73, 34: 183 -> 120.  The hint pays (3 to 5 %) only where the entries
-// are more than the 256 MB MALL keeps from one product to the next, and not for
-// short rows, whose lines are shared between instructions.
+// 6 % of the best at 300,000 rows and more.  A quad of entries per lane (V = 4),
+// turned for the gather, pays from ten entries on; below, the quads of short rows
+// are mostly slack.  A group takes about a row's entries and a few more per trip.
+// One million rows, against V = 1 with two entries per lane, four rows in flight
+// and the non-temporal hint (the rule before): 3 entries 21 -> 16 us, 5: 32 -> 21,
+// 8: 44 -> 30, 12: 63 -> 40, 17: 99 -> 57, 24: 109 -> 74, 34: 183 -> 108.  The hint
+// pays (3 to 5 %) only where the entries are more than the 256 MB MALL keeps from
+// one product to the next, and where a trip reads a row's lines whole: with rows
+// split over two it costs up to half (17 entries, 16 to a trip, n = 2.5 M: 143 ->
+// 213 us).  Long rows, against a wavefront per row: n = 300,007, 200 entries 224 ->
+// 163 us, n = 10,007, 400 entries 18 -> 12.
 CsrKernel csr_default(double mean, double entries) {
   const int nt = 12.0 * entries > 256e6 && mean >= 8 ? 1 : 0;
   if (mean < 2.5) return {1, mean <= 2 ? 1 : 2, 4, 1};  // hypersparse: not timed, as before
-  if (mean < 4) return {1, 4, 2, nt};
+  if (mean < 4) return {1, 4, 4, nt};
   if (mean < 10) return {2, 4, 2, nt};
   if (mean < 15) return {4, 4, 2, nt};
-  if (mean < 20) return {4, 4, 1, nt};
-  if (mean < 28) return {4, 8, 2, nt};
-  if (mean < 48) return {4, 8, 1, nt};
-  if (mean < 128) return {4, 16, 1, nt};
-  return {1, 64, 1, 1};  // long rows: a wavefront per row, as before
+  if (mean < 20) return {4, 8, 2, 0};
+  if (mean < 32) return {4, 8, 2, nt};
+  if (mean < 48) return {4, 16, 2, 0};
+  if (mean < 128) return {4, 16, 1, 0};
+  return {2, 32, 1, 0};
 }
 
 CsrKernel pick_csr(const tbsla_hip_matrix_s *m) {
@@ -390,9 +393,17 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf
        t0 += (long long)gridDim.x * kBlock, buf ^= 1) {
     const long long k = t0 + threadIdx.x;
     const double old = k < a.n_rows ? a.x[k] : 0.0;
+    // a lane's row of the wavefront's 64; the groups take theirs from there
+    const int beg = k < a.n_rows ? a.rowptr[k] : 0, end = k < a.n_rows ? a.rowptr[k + 1] : 0;
     for (int q = 0; q < kWave; q += G * R) {
       double sum[R];
-      csr_row_sums<V, L, R, 0>(a, t0 + wave * kWave + q, lane, g, sum);
+      int rb[R], re[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        rb[r] = __shfl(beg, q + r * G + g, kWave);
+        re[r] = __shfl(end, q + r * G + g, kWave);
+      }
+      csr_row_sums<V, L, R, 0>(a, rb, re, lane, sum);
 #pragma unroll
       for (int r = 0; r < R; r++)
         if (lane == 0) y[buf][wave * kWave + q + r * G + g] = sum[r];

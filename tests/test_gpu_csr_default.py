@@ -7,7 +7,7 @@ import tbsla_amd as T
 
 pytestmark = pytest.mark.gpu
 
-LINES = [2, 2.5, 4, 10, 15, 20, 28, 48, 128]
+LINES = [2, 2.5, 4, 10, 15, 20, 28, 32, 48, 128]
 
 
 @pytest.mark.parametrize("fmt", [T.CSR, T.COO])
