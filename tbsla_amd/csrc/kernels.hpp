@@ -85,12 +85,26 @@ struct PrFuse {
   double *p_err, *p_sum;
 };
 int split_pr_blocks(const tbsla_hip_matrix_s *m);
+// A PageRank solve's state
+struct PrState {
+  double S;      // sum of the current iterate
+  double err;    // last L1 change
+  int iters;     // iterations done (reference counting)
+  int done;      // set when the solve has finished
+};
+constexpr int kPrBlocks = 1024;  // most workgroups (partials) of an update
 // The same on the CSR row kernel (spmv.hip): for a square block on the diagonal
 // whose row kernel has a fused form; nb workgroups and partials, those of
-// k_pr_update on its grid of nb
+// k_pr_update on its grid of nb.  q_err, q_sum: the step before's partials, whose
+// finalisation (k_pr_finalize's) this step makes, or null when it has been made.
+struct PrPrev {
+  const double *q_err, *q_sum;
+  int NC;
+  double epsilon;
+};
 bool csr_pr_fits(const tbsla_hip_matrix_s *m);
-int csr_pr_launch(const tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf, const int *done,
-                  unsigned nb, hipStream_t s);
+int csr_pr_launch(const tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf,
+                  const PrPrev &prev, PrState *st, unsigned nb, hipStream_t s);
 int split_launch_pr(tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf, const int *done,
                     hipStream_t s);
 // The row pointer of a COO / SCOO block's n row-sorted triplets over their

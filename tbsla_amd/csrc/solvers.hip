@@ -20,14 +20,9 @@ namespace tbsla_hip {
 namespace {
 
 // reduction grid (fixed: the partial layout is part of the order)
-constexpr int kRedBlocks = 2048;
+constexpr int kRedBlocks = kPrBlocks;
 
-struct SolverState {
-  double S;      // sum of the current iterate
-  double err;    // last L1 change
-  int iters;     // iterations done (reference counting)
-  int done;      // set when the solve has finished
-};
+typedef PrState SolverState;
 
 __device__ inline double block_sum(double v) {
   __shared__ double lds[kBlock / kWave];
@@ -635,7 +630,7 @@ extern "C" int tbsla_hip_page_rank(tbsla_hip_matrix_t m, double beta, double eps
   TBSLA_TRY(bufA.alloc(ln_col));
   TBSLA_TRY(bufB.alloc(ln_col));
   if (!fused && !rows_fused) TBSLA_TRY(y.alloc(ylen));
-  TBSLA_TRY(part.alloc(2 * np + 8));
+  TBSLA_TRY(part.alloc(4 * np + 8));
   TBSLA_TRY(st.alloc(1));
   TBSLA_TRY(launch_fill(bufA.p, ln_col, 1.0, s));  // b = 1 (Matrix.cpp:549-552)
   SolverState h{};
@@ -644,16 +639,34 @@ extern "C" int tbsla_hip_page_rank(tbsla_hip_matrix_t m, double beta, double eps
   const unsigned nb = red_grid(ln_col);
   double *buf[2] = {bufA.p, bufB.p};
   int launched = 0;
+  double before = 0.0;  // the error at the last test of the host's, and the steps since
+  int last = 0;
   while (launched < max_iterations) {
-    const int batch = std::min(16, max_iterations - launched);
+    // steps to the next test: 8 twice, then as many as the error's decay over the
+    // last ones asks for (a test costs as much as 20 steps that find the solve done)
+    double want = 8;
+    if (launched > 8) {
+      const double rate = std::log(h.err / before) / last;
+      want = rate < 0 && epsilon > 0 ? std::log(epsilon / h.err) / rate + 2 : 16;
+    }
+    before = h.err;
+    const int steps = want >= 8 && want <= 64 ? (int)want : (want > 64 ? 64 : 8);
+    const int batch = std::min(steps, max_iterations - launched);
+    last = batch;
     for (int i = 0; i < batch; i++, launched++) {
       double *bt = buf[launched % 2], *bn = buf[(launched + 1) % 2];
       if (fused) {
         const PrFuse pf{bn, &st.p->S, beta, (double)m->n_col, part.p, part.p + np};
         TBSLA_TRY(split_launch_pr(m, bt, pf, &st.p->done, s));
       } else if (rows_fused) {
-        const PrFuse pf{bn, &st.p->S, beta, (double)m->n_col, part.p, part.p + np};
-        TBSLA_TRY(csr_pr_launch(m, bt, pf, &st.p->done, nb, s));
+        // the step before's partials are this one's to finalise, except a batch's last
+        double *mine = part.p + (i % 2) * 2 * np, *its = part.p + (1 - i % 2) * 2 * np;
+        const PrFuse pf{bn, &st.p->S, beta, (double)m->n_col, mine, mine + np};
+        const PrPrev prev{i ? its : nullptr, i ? its + np : nullptr, m->NC, epsilon};
+        TBSLA_TRY(csr_pr_launch(m, bt, pf, prev, st.p, nb, s));
+        if (i + 1 == batch)
+          k_pr_finalize<<<1, kBlock, 0, s>>>(st.p, mine, mine + np, (int)nb, m->NC, epsilon);
+        continue;
       } else {
         TBSLA_TRY(spmv_launch(m, y.p, bt, 0, true, s, &st.p->done));
         k_pr_update<<<nb, kBlock, 0, s>>>(ln_col, y.p, bt, bn, r_start, s_start, length, beta,

@@ -374,19 +374,36 @@ CsrKernel pick_csr(const tbsla_hip_matrix_s *m) {
 // so thread t updates the rows that k_pr_update's thread t of workgroup b does,
 // in the same order, and leaves the same partials; a tile's row sums (those of
 // k_csr_rows for the same V and L) pass through LDS instead of y.  A launch and
-// 16 bytes a row less: n = 200,003, c = 12: 9.3 + 4.5 us -> 10.2.
+// 16 bytes a row less: n = 200,003, c = 12: 9.3 + 4.5 us -> 10.2.  The sums of
+// the step before (k_pr_finalize's, bit for bit) are taken by every workgroup,
+// their loads issued before the rows': a launch less again.  All told a step of the
+// solve takes 15.7 us where it took 27 (n = 3,000, 8 to a row: 8.0 and 15.0; n =
+// 600,011, 24 to a row: 49 and 82).
 template <int V, int L, int R>
-__global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf) {
+__global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf, PrPrev prev,
+                                                        PrState *__restrict__ st) {
   TBSLA_NO_FMA
-  if (*a.done) return;
   __shared__ double y[2][kBlock];
   __shared__ double lds[2][kBlock / kWave];
+  __shared__ int s_done;
+  constexpr int Q = kPrBlocks / kBlock;
+  double qs[2][Q];
+  const int nq = prev.q_err ? (int)gridDim.x : 0;
+  const int done = __hip_atomic_load(&st->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (nq) {
+#pragma unroll
+    for (int i = 0; i < Q; i++) {
+      if (i * kBlock >= nq) break;
+      const int k = min((int)threadIdx.x + i * kBlock, nq - 1);
+      qs[0][i] = prev.q_err[k];
+      qs[1][i] = prev.q_sum[k];
+    }
+  }
   constexpr int G = kWave / L;
   const int lane = threadIdx.x & (L - 1);
   const int wl = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int g = wl / L;
-  const double S = *pf.S;
-  const double t_sum = S * ((1 - pf.beta) / pf.n_col);
+  double S = 0.0, t_sum = 0.0;
   double e = 0.0, sm = 0.0;
   int buf = 0;
   for (long long t0 = (long long)blockIdx.x * kBlock; t0 < a.n_rows;
@@ -408,6 +425,46 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf
       for (int r = 0; r < R; r++)
         if (lane == 0) y[buf][wave * kWave + q + r * G + g] = sum[r];
     }
+    if (t0 == (long long)blockIdx.x * kBlock) {  // the first tile
+      // one answer for the workgroup: another may be writing the flag
+      if (threadIdx.x == 0) s_done = done;
+      if (nq) {
+        double v[2] = {0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < Q; i++)
+          if ((int)threadIdx.x + i * kBlock < nq) {
+            v[0] += qs[0][i];
+            v[1] += qs[1][i];
+          }
+        v[0] = group_sum<kWave>(v[0]);
+        v[1] = group_sum<kWave>(v[1]);
+        if (wl == 0) {
+          lds[0][wave] = v[0];
+          lds[1][wave] = v[1];
+        }
+      }
+      __syncthreads();
+      if (s_done) return;
+      if (nq) {
+        double pe = 0.0;
+        for (int w = 0; w < kBlock / kWave; w++) {
+          pe += lds[0][w];
+          S += lds[1][w];
+        }
+        pe /= prev.NC;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          st->err = pe;
+          st->S = S;
+          st->iters += 1;
+          if (pe < prev.epsilon)
+            __hip_atomic_store(&st->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (pe < prev.epsilon) return;  // in every workgroup: the same sums
+      } else {
+        S = st->S;
+      }
+      t_sum = S * ((1 - pf.beta) / pf.n_col);
+    }
     __syncthreads();  // y of this tile is there; the other buffer is free
     if (k < a.n_rows) {
       double v = y[buf][threadIdx.x];
@@ -420,6 +477,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf
   }
   e = group_sum<kWave>(e);
   sm = group_sum<kWave>(sm);
+  __syncthreads();
   if (wl == 0) {
     lds[0][wave] = e;
     lds[1][wave] = sm;
@@ -432,11 +490,14 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf
   }
 }
 
-// rows a group keeps in flight: two, while a wavefront's pass is at most its
-// 64 rows of a tile and the registers stay few
+// rows a group keeps in flight: four of the shortest, so that a wavefront goes
+// through its 64 rows of a tile once (65,536 rows of 6: 8.0 -> 7.4 us a step),
+// else two (200,003 rows of 12, where four take the registers of two
+// wavefronts: 15.7 us a step, not 16.9)
 template <int V, int L>
-void csr_pr_go(const CsrRowsArgs &a, const PrFuse &pf, unsigned nb, hipStream_t s) {
-  k_csr_rows_pr<V, L, 2><<<nb, kBlock, 0, s>>>(a, pf);
+void csr_pr_go(const CsrRowsArgs &a, const PrFuse &pf, const PrPrev &prev, PrState *st,
+               unsigned nb, hipStream_t s) {
+  k_csr_rows_pr<V, L, L == 4 && V < 4 ? 4 : 2><<<nb, kBlock, 0, s>>>(a, pf, prev, st);
 }
 
 bool csr_pr_fits(const tbsla_hip_matrix_s *m) {
@@ -445,23 +506,23 @@ bool csr_pr_fits(const tbsla_hip_matrix_s *m) {
   return k.L >= 4 && (k.V == 1 ? k.L <= 32 : true);
 }
 
-int csr_pr_launch(const tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf, const int *done,
-                  unsigned nb, hipStream_t s) {
-  const CsrRowsArgs a{m->ln_row, m->rowptr, m->colidx, m->values, bt, m->f_col, nullptr, done,
+int csr_pr_launch(const tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf,
+                  const PrPrev &prev, PrState *st, unsigned nb, hipStream_t s) {
+  const CsrRowsArgs a{m->ln_row, m->rowptr, m->colidx, m->values, bt, m->f_col, nullptr, nullptr,
                       nullptr};
   const CsrKernel k = pick_csr(m);
   switch (k.V * 100 + k.L) {
-    case 104: csr_pr_go<1, 4>(a, pf, nb, s); break;
-    case 108: csr_pr_go<1, 8>(a, pf, nb, s); break;
-    case 116: csr_pr_go<1, 16>(a, pf, nb, s); break;
-    case 132: csr_pr_go<1, 32>(a, pf, nb, s); break;
-    case 204: csr_pr_go<2, 4>(a, pf, nb, s); break;
-    case 208: csr_pr_go<2, 8>(a, pf, nb, s); break;
-    case 216: csr_pr_go<2, 16>(a, pf, nb, s); break;
-    case 232: csr_pr_go<2, 32>(a, pf, nb, s); break;
-    case 404: csr_pr_go<4, 4>(a, pf, nb, s); break;
-    case 408: csr_pr_go<4, 8>(a, pf, nb, s); break;
-    case 416: csr_pr_go<4, 16>(a, pf, nb, s); break;
+    case 104: csr_pr_go<1, 4>(a, pf, prev, st, nb, s); break;
+    case 108: csr_pr_go<1, 8>(a, pf, prev, st, nb, s); break;
+    case 116: csr_pr_go<1, 16>(a, pf, prev, st, nb, s); break;
+    case 132: csr_pr_go<1, 32>(a, pf, prev, st, nb, s); break;
+    case 204: csr_pr_go<2, 4>(a, pf, prev, st, nb, s); break;
+    case 208: csr_pr_go<2, 8>(a, pf, prev, st, nb, s); break;
+    case 216: csr_pr_go<2, 16>(a, pf, prev, st, nb, s); break;
+    case 232: csr_pr_go<2, 32>(a, pf, prev, st, nb, s); break;
+    case 404: csr_pr_go<4, 4>(a, pf, prev, st, nb, s); break;
+    case 408: csr_pr_go<4, 8>(a, pf, prev, st, nb, s); break;
+    case 416: csr_pr_go<4, 16>(a, pf, prev, st, nb, s); break;
     default: return fail(TBSLA_HIP_ERR_INVALID, "no fused PageRank kernel for this row kernel");
   }
   TBSLA_HIP_LAUNCH_CHECK();
