@@ -336,7 +336,9 @@ struct RowPrefetch {
 // first entry rounded down to a multiple of 4 of its system's entries (so that a
 // system is summed alike alone and in a batch, where its quads may lie on any
 // 4-byte boundary); lane l's quads are l and l + L, so a row's lines are read
-// whole by one instruction instead of 4 L bytes at a time.  Slots outside the row
+// whole by one instruction instead of 4 L bytes at a time (but for the lines that
+// two rows share: no nontemporal hint, which had them fetched twice; 96 systems
+// of 85 M entries, mixed, K1b: 252 -> 230 us).  Slots outside the row
 // have column 0 of the block and are not summed.  Longer rows continue with the
 // entries from `rest` on.
 template <int L, typename V>
@@ -363,7 +365,6 @@ struct CgRow {
   }
   // the entries, clamped into the arrays (the last quad may end up to three
   // entries after the last one: device_alloc's blocks have room for them)
-  template <bool NT>
   __device__ inline void load(const int *__restrict__ ci, const V *__restrict__ va, int nnz,
                               int f_col, int lane) {
     if constexpr (L == 1) {
@@ -375,24 +376,23 @@ struct CgRow {
       }
     } else {
 #pragma unroll
-      for (int h = 0; h < 2; h++) quad<NT>(ci, va, min(at(lane, 4 * h), nnz - 1), 4 * h);
+      for (int h = 0; h < 2; h++) quad(ci, va, min(at(lane, 4 * h), nnz - 1), 4 * h);
     }
 #pragma unroll
     for (int k = 0; k < P; k++) col[k] = in(lane, k) ? col[k] - f_col : 0;
   }
-  template <bool NT>
   __device__ inline void quad(const int *__restrict__ ci, const V *__restrict__ va, int j, int k) {
     typedef int vi __attribute__((ext_vector_type(4), aligned(4)));
     constexpr int W = 16 / sizeof(V);  // values per 16 bytes
     typedef V vv __attribute__((ext_vector_type(W), aligned(sizeof(V))));
     const vi *pc = reinterpret_cast<const vi *>(ci + j);
-    const vi c = NT ? __builtin_nontemporal_load(pc) : *pc;
+    const vi c = *pc;
 #pragma unroll
     for (int q = 0; q < 4; q++) col[k + q] = c[q];
 #pragma unroll
     for (int q = 0; q < 4; q += W) {
       const vv *pv = reinterpret_cast<const vv *>(va + j + q);
-      const vv x = NT ? __builtin_nontemporal_load(pv) : *pv;
+      const vv x = *pv;
 #pragma unroll
       for (int w = 0; w < W; w++) v[k + q + w] = x[w];
     }
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
   double fs[P], ft[P];
   f.extent(a.rowptr, rowc, sg.ent0);
   const double own_z = zv[rowc], own_p = po[rowc];
-  f.template load<false>(a.colidx, val, a.a_nnz, a.f_col, lane);
+  f.load(a.colidx, val, a.a_nnz, a.f_col, lane);
   const int flag = __atomic_load_n(&S->done, __ATOMIC_RELAXED);
   SegLoad sl;
   seg_issue(CG_AT(prz, par ^ 1), CG_AT(prz, par), CG_AT(prr, par ^ 1), NP, b0, b1, sl);
@@ -595,7 +595,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
       op[r] = po[rw[r]];
     }
 #pragma unroll
-    for (int r = 0; r < R2; r++) g[r].template load<false>(a.colidx, val, a.a_nnz, a.f_col, lane);
+    for (int r = 0; r < R2; r++) g[r].load(a.colidx, val, a.a_nnz, a.f_col, lane);
 #pragma unroll
     for (int r = 0; r < R2; r++)
 #pragma unroll
@@ -692,7 +692,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
       own[r] = pn[rw[r]];
     }
 #pragma unroll
-    for (int r = 0; r < R2; r++) w[r].template load<L != 1>(a.colidx, val, a.a_nnz, a.f_col, lane);
+    for (int r = 0; r < R2; r++) w[r].load(a.colidx, val, a.a_nnz, a.f_col, lane);
 #pragma unroll
     for (int r = 0; r < R2; r++)
 #pragma unroll
@@ -1590,7 +1590,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_ax(CG_ARGS, int par_g, int mode) 
   for (int row = r0 + (int)threadIdx.x / L; row < r1; row += PASS) {
     Row w;
     w.extent(a.rowptr, row, sg.ent0);
-    w.template load<false>(a.colidx, a.val64, a.a_nnz, a.f_col, lane);
+    w.load(a.colidx, a.val64, a.a_nnz, a.f_col, lane);
     double g[Row::P];
 #pragma unroll
     for (int k = 0; k < Row::P; k++) g[k] = a.x[w.col[k]];
