@@ -750,7 +750,11 @@ __device__ inline T ldi(const T *__restrict__ base, long long i) {
 // at 64^3, FP64: 9.7 -> 8.0 us an iteration (KD and the early loads, 0.9; global
 // loads for flat ones, 0.8); 10^6 rows, mixed: 19.4 -> 17.1.  Two rows in flight per
 // thread were slower (8.3 and 18.6: 204 registers, half the wavefronts).
-template <bool MIX, bool ZBUF, int KD>
+// SYM: the layout's values are symmetric bit for bit, and a slot below the main
+// diagonal is read as its mirror image, from lines that other rows read anyway:
+// half the values from memory (64^3, FP64: 7.8 -> 6.9 us; 10^6 rows, mixed: as
+// before, 15.1).
+template <bool MIX, bool ZBUF, int KD, bool SYM>
 __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int check,
                                                         int check_only) {
   TBSLA_NO_FMA
@@ -787,7 +791,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
 #pragma unroll
       for (int i = 0; i < U; i++) {
         const unsigned c = (unsigned)min(max(row + CG_OFF(doff8, i), 0), a.ncol - 1);
-        w.v[i] = ld32(dv, at + i * kWave);
+        if (SYM && i < KD / 2)  // its mirror image's (unused where there is none)
+          w.v[i] = ld32(dv, c / kWave * (kWave * KD) + (KD - 1 - i) * kWave + c % kWave);
+        else
+          w.v[i] = ld32(dv, at + i * kWave);
         w.z[i] = ld32(zv, c);
         w.p[i] = ld32(po, c);
       }
@@ -823,10 +830,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
   const double beta = rz_new / fmax(rz_old, sg.near_zero);
   double *pn = CG_AT(p, par ^ 1);
   double pap = 0.0;
-  auto add = [&](const Row &w, int k0, V acc) {
+  auto add = [&](const Row &w, int row, int k0, V acc) {
 #pragma unroll
     for (int i = 0; i < U; i++) {
-      if ((KD > 0 || k0 + i < a.ndiag) && w.v[i] != (V)0) {
+      const bool none = SYM && i < KD / 2 && row + CG_OFF(doff8, i) < 0;
+      if ((KD > 0 || k0 + i < a.ndiag) && !none && w.v[i] != (V)0) {
         const double pc = w.z[i] + beta * w.p[i];
         if (MIX) acc = fmaf((float)w.v[i], (float)pc, (float)acc);
         else acc = fma((double)w.v[i], pc, (double)acc);
@@ -842,14 +850,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dia(CG_ARGS, int par_g, int 
   if (KD > 0) {
     for (int row = row_first; row < r1; row += kBlock) {
       if (row != row_first) load(row, 0, f);
-      store(row, f.oz + beta * f.op, add(f, 0, (V)0));
+      store(row, f.oz + beta * f.op, add(f, row, 0, (V)0));
     }
   } else {
     for (int row = row_first; row < r1; row += kBlock) {
       V acc = 0;
       for (int k = 0; k < a.ndiag; k += U) {
         load(row, k, f);
-        acc = add(f, k, acc);
+        acc = add(f, row, k, acc);
       }
       store(row, zv[row] + beta * po[row], acc);
     }
@@ -1834,6 +1842,7 @@ struct Plan {
   int L, pre, mixed, replace, verify, stall;
   bool dia;   // K1 reads A's diagonal layout
   int dkd;    // its kernel's diagonals: 3, 5 or 7, or 0 for any number
+  bool sym;   // and those below the main one read as their mirror images
   bool two;   // K1 in two passes (k_cg_pnew, then k_cg_ap) on A's CSR rows
   bool gdia;  // M = G G^T applied from G's diagonals
   int gkd;    // their kernels' capacity: 4 or 8 diagonals
@@ -1855,15 +1864,15 @@ void launch_k1(const Plan &p, int par, int check, int check_only) {
   if (!check_only) k_cg_ap<L, MIX><<<p.nblocks, kBlock, 0, p.s>>>(p.args, p.multi, par);
 }
 
-template <int KD>
+template <int KD, bool SYM>
 void launch_k1_dia(const Plan &p, bool zbuf, int par, int check, int check_only) {
   const int g = p.nblocks;
   if (p.mixed) {
-    if (zbuf) k_cg_spmv_dia<true, true, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
-    else k_cg_spmv_dia<true, false, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+    if (zbuf) k_cg_spmv_dia<true, true, KD, SYM><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+    else k_cg_spmv_dia<true, false, KD, SYM><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
   } else {
-    if (zbuf) k_cg_spmv_dia<false, true, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
-    else k_cg_spmv_dia<false, false, KD><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+    if (zbuf) k_cg_spmv_dia<false, true, KD, SYM><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
+    else k_cg_spmv_dia<false, false, KD, SYM><<<g, kBlock, 0, p.s>>>(p.args, p.multi, par, check, check_only);
   }
 }
 
@@ -1871,11 +1880,14 @@ template <int L>
 void launch_k1_l(const Plan &p, int par, int check, int check_only) {
   const bool zbuf = p.pre != 0;
   if (p.dia) {
-    switch (p.dkd) {
-      case 3: launch_k1_dia<3>(p, zbuf, par, check, check_only); break;
-      case 5: launch_k1_dia<5>(p, zbuf, par, check, check_only); break;
-      case 7: launch_k1_dia<7>(p, zbuf, par, check, check_only); break;
-      default: launch_k1_dia<0>(p, zbuf, par, check, check_only); break;
+    switch (p.dkd + (p.sym ? 10 : 0)) {
+      case 3: launch_k1_dia<3, false>(p, zbuf, par, check, check_only); break;
+      case 5: launch_k1_dia<5, false>(p, zbuf, par, check, check_only); break;
+      case 7: launch_k1_dia<7, false>(p, zbuf, par, check, check_only); break;
+      case 13: launch_k1_dia<3, true>(p, zbuf, par, check, check_only); break;
+      case 15: launch_k1_dia<5, true>(p, zbuf, par, check, check_only); break;
+      case 17: launch_k1_dia<7, true>(p, zbuf, par, check, check_only); break;
+      default: launch_k1_dia<0, false>(p, zbuf, par, check, check_only); break;
     }
     return;
   }
@@ -2314,10 +2326,10 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   // A in the diagonal layout with no remote entries: K1 reads its diagonals
   const int *d_off = nullptr, *h_off = nullptr;
   const double *d_v = nullptr;
-  int ndiag = 0;
+  int ndiag = 0, symmetric = 0;
   long long dv_len = 0;
   unsigned long long build = 0;
-  const bool dia = split_diag_only(m, &d_off, &h_off, &d_v, &ndiag, &dv_len, &build) && m->ln_col > 0;
+  const bool dia = split_diag_only(m, &d_off, &h_off, &d_v, &ndiag, &dv_len, &build, &symmetric) && m->ln_col > 0;
   // K1 on CSR rows in two passes: asked for, or picked for large blocks,
   // whose gathers of z and p miss the caches (a random column then costs
   // one line fill instead of two)
@@ -2383,6 +2395,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   const long long most = 1LL << 32;
   const bool narrow_a = (n + kWave) * std::max(ndiag, 1) * 8 < most;
   p.dkd = dia && narrow_a && (ndiag == 3 || ndiag == 5 || ndiag == 7) ? ndiag : 0;
+  p.sym = p.dkd > 0 && symmetric;
   p.wide = (n + kWave) * std::max(gndiag, 1) * 8 >= most;
   p.two = two;
   p.gdia = gdia;
@@ -2457,7 +2470,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   key.nblocks = nblocks;
   key.multi = p.multi;
   key.verify = p.verify;
-  key.dia = p.dia ? 1 + p.dkd : 0;
+  key.dia = p.dia ? 1 + p.dkd + (p.sym ? 10 : 0) : 0;
   key.gdia = p.gdia ? p.gkd + (p.wide ? 16 : 0) : 0;
   key.two = p.two ? 1 : 0;
   // the graph set of this plan, captured and instantiated once; the least

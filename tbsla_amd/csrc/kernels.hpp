@@ -112,11 +112,13 @@ int split_launch_pr(tbsla_hip_matrix_s *m, const double *bt, const PrFuse &pf, c
 // triplets are not sorted by row
 int coo_rowptr(tbsla_hip_matrix_s *m, long long n, bool *ok, hipStream_t s);
 // The diagonal layout's arrays when it holds every entry (no remote part):
-// offsets (device and host), tiled values (dia_at), count, values' length, and the build's
-// id (unique in the process: a copy made from one build is stale for any
-// other, even one whose arrays reuse the same addresses); else 0.
+// offsets (device and host), tiled values (dia_at), count, values' length, the
+// build's id (unique in the process: a copy made from one build is stale for any
+// other, even one whose arrays reuse the same addresses), and whether the values
+// are symmetric bit for bit; else 0.
 int split_diag_only(const tbsla_hip_matrix_s *m, const int **doff, const int **hoff,
-                    const double **dv, int *ndiag, long long *dv_len, unsigned long long *build_id);
+                    const double **dv, int *ndiag, long long *dv_len, unsigned long long *build_id,
+                    int *symmetric);
 
 // solvers.hip: after the values of m changed in place: rebuild the split
 // layout (it holds a copy of the values), mark copies of the old values

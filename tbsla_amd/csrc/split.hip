@@ -76,6 +76,7 @@ struct SplitCsr {
   int *lrp = nullptr, *lci = nullptr, *sr = nullptr, *sc = nullptr, *boff = nullptr;
   int *doff = nullptr;  // their offsets c - r, ascending
   std::vector<int> hoff;  // the same on the host
+  bool symmetric = false; // and dv holds a symmetric matrix, bit for bit
   double *lv = nullptr, *sv = nullptr, *P = nullptr, *R = nullptr;
   double *dv = nullptr;  // dv[k n + r]: row r's entry on diagonal k, or 0
   std::vector<long long> soff;  // slice boundaries (host)
@@ -731,6 +732,22 @@ int bits_of(long long v) {
   return b;
 }
 
+// *differ = 1 unless every slot equals its mirror image: row r's on diagonal k and
+// row r + doff[k]'s on diagonal ndiag - 1 - k (offsets in pairs of opposite sign)
+__global__ __launch_bounds__(kBlock) void k_dia_differ(long long n, int ndiag,
+                                                       const int *__restrict__ doff,
+                                                       const double *__restrict__ dv,
+                                                       int *__restrict__ differ) {
+  for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r < n;
+       r += (long long)gridDim.x * kBlock)
+    for (int k = 0; k < ndiag / 2; k++) {
+      const long long c = r + doff[k];
+      const double lower = dv[dia_at(r, k, ndiag)];
+      const double upper = c >= 0 ? dv[dia_at(c, ndiag - 1 - k, ndiag)] : 0.0;
+      if (!(lower == upper)) *differ = 1;
+    }
+}
+
 }  // namespace
 
 int split_pr_blocks(const tbsla_hip_matrix_s *m) {
@@ -770,13 +787,14 @@ int split_lds_block_rows(const tbsla_hip_matrix_s *m) {
 }
 
 int split_diag_only(const tbsla_hip_matrix_s *m, const int **doff, const int **hoff,
-                    const double **dv, int *ndiag, long long *dv_len,
-                    unsigned long long *build_id) {
+                    const double **dv, int *ndiag, long long *dv_len, unsigned long long *build_id,
+                    int *symmetric) {
   const SplitCsr *sp = static_cast<const SplitCsr *>(m->split);
   if (!sp || sp->layout != TBSLA_HIP_CSR_DIAG || sp->nr != 0 || sp->ndiag == 0) return 0;
   *build_id = sp->build_id;
   *doff = sp->doff;
   *hoff = sp->hoff.data();
+  *symmetric = sp->symmetric ? 1 : 0;
   *dv = sp->dv;
   *ndiag = sp->ndiag;
   *dv_len = (long long)sp->ndiag * ((layout_rows(m).n + kWave - 1) / kWave) * kWave;
@@ -1039,10 +1057,21 @@ int split_build(tbsla_hip_matrix_s *m, int window, int slices, hipStream_t s, in
   if (sp->nr > 0)
     k_split_place<<<sgrid(sp->nr), kBlock, 0, s>>>(sp->nr, keys, rb, pay, rc, rv, sp->sr, sp->sc,
                                                    sp->sv);
+  // one value for both of a symmetric pair (CG's K1 then reads half of them)
+  int differ = 1;
+  bool pairs = diag && sp->nr == 0 && n == nc && n > 0;
+  for (int k = 0; pairs && k < sp->ndiag; k++)
+    pairs = sp->hoff[k] == -sp->hoff[sp->ndiag - 1 - k];
+  if (pairs) {
+    (void)hipMemsetAsync(hist, 0, 4, s);
+    k_dia_differ<<<sgrid(n), kBlock, 0, s>>>(n, sp->ndiag, sp->doff, sp->dv, hist);
+    (void)hipMemcpyAsync(&differ, hist, 4, hipMemcpyDeviceToHost, s);
+  }
   std::vector<int> hc(slices + 1, 0);
   if (hipMemcpyAsync(hc.data(), scount, (size_t)slices * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return failed(fail(TBSLA_HIP_ERR_HIP, "split layout: slice counts"));
+  sp->symmetric = pairs && !differ;
   sp->soff.assign(slices + 1, 0);
   for (int k = 0; k < slices; k++) sp->soff[k + 1] = sp->soff[k] + hc[k];
   long long *d_soff = reinterpret_cast<long long *>(sp->P + nr1);

@@ -67,6 +67,24 @@ def test_stencils_in_the_diagonal_layout(grid, pre, precision):
     check(m, A, its, preconditioner=pre, precision=precision)
 
 
+@pytest.mark.parametrize("precision", [T.CG_FP64, T.CG_MIXED])
+@pytest.mark.parametrize("at", [(1, 0), (0, 1), (299, 300), (511, 510)])
+def test_one_entry_off_symmetry(at, precision):
+    """Not read as half of a symmetric matrix, before or after the entry changes."""
+    m = T.Matrix(T.CSR).fill_poisson3d(512, 1, 1, kappa=T.lognormal_field(512, 1, 1, seed=3))
+    A = dense(m)
+    rp, ci, va = m.arrays()
+    m.set_csr_layout(T.CSR_DIAG, 65536, 8)
+    check(m, A, precision=precision)
+    A[at] *= 1.25
+    k = rp[at[0]] + int(np.flatnonzero(ci[rp[at[0]]:rp[at[0] + 1]] == at[1])[0])
+    va = va.copy()
+    va[k] *= 1.25
+    T.check(T.lib().tbsla_hip_memcpy_htod(m.device_arrays()[2], va.ctypes.data, va.nbytes, None))
+    m.values_changed()
+    check(m, A, precision=precision)
+
+
 @pytest.mark.parametrize("offsets", [(0,), (0, 3), (0, 1, 2, 7), (0, 1, 5, 6, 40, 41)])
 def test_other_diagonal_counts(offsets):
     n = 700
