@@ -299,51 +299,63 @@ __global__ __launch_bounds__(kBlock) void k_aggregate(long long n, const int *__
 }
 
 // C[n x N] (+)= A[n x K] B[K x N] with A row-major BF16 and B given as Bt
-// (N x K, row-major BF16), FP32 result.  Workgroup: 64 rows, 4 waves of 16
-// rows; each wave holds N/16 16x16 tiles (v_mfma_f32_16x16x32_bf16:
-// lane l holds A[l%16][8(l/16)..+8], Bt[l%16][8(l/16)..+8] and
-// D[4(l/16)..+4][l%16]).  Epilogue: add the existing C, then zero where
-// mask <= 0 (the ReLU derivative).
+// (N x K, row-major BF16), FP32 result.  Workgroup: kGemmRows rows, 4 waves of
+// kGemmRows / 4; each wave holds N/16 16x16 tiles per 16 rows
+// (v_mfma_f32_16x16x32_bf16 with Bt's rows as its first operand: lane l holds
+// Bt[l%16][8(l/16)..+8], A[l%16][8(l/16)..+8] and 4 consecutive outputs
+// 4(l/16)..+4 of row l%16, stored as 16 bytes).  Epilogue: add the existing C,
+// then zero where mask <= 0 (the ReLU derivative).  Bound by
+// C's bytes: 979,700 rows, 64 -> 128, 203 us with 16 rows a wave and 4-byte stores,
+// 149 so (4.2 TB/s); 262,144 rows, 128 -> 64 with C added and masked, 74 -> 53.
+constexpr int kGemmRows = 128;
+
 template <int K, int N>
 __global__ __launch_bounds__(kBlock) void k_gemm_rows(long long n, const bf16_t *__restrict__ A,
                                                       const bf16_t *__restrict__ Bt,
                                                       float *__restrict__ C, int add,
                                                       const float *__restrict__ mask) {
-  constexpr int NT = N / 16;
+  constexpr int NT = N / 16, RT = kGemmRows / 64;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  const long long r0 = (long long)blockIdx.x * 64 + wave * 16;
+  const long long r0 = (long long)blockIdx.x * kGemmRows + wave * 16 * RT;
   if (r0 >= n) return;
-  floatx4 acc[NT];
+  floatx4 acc[RT][NT];
 #pragma unroll
-  for (int t = 0; t < NT; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int u = 0; u < RT; u++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
   const long long ar = r0 + (lane & 15);
   const int kq = (lane >> 4) * 8;
 #pragma unroll
   for (int kb = 0; kb < K; kb += 32) {
-    bf16x8 a;
-    if (ar < n) {
-      a = *reinterpret_cast<const bf16x8 *>(A + ar * K + kb + kq);
-    } else {
-      a = bf16x8{};
-    }
+    bf16x8 a[RT];
+#pragma unroll
+    for (int u = 0; u < RT; u++)
+      a[u] = *reinterpret_cast<const bf16x8 *>(A + min(ar + 16 * u, n - 1) * K + kb + kq);
 #pragma unroll
     for (int t = 0; t < NT; t++) {
       const bf16x8 b = *reinterpret_cast<const bf16x8 *>(Bt + (long long)(t * 16 + (lane & 15)) * K + kb + kq);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < RT; u++)
+        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[u], acc[u][t], 0, 0, 0);
     }
   }
 #pragma unroll
-  for (int t = 0; t < NT; t++) {
+  for (int u = 0; u < RT; u++) {
+    const long long r = ar + 16 * u;
+    if (r >= n) break;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const long long r = r0 + (lane >> 4) * 4 + q;
-      if (r >= n) continue;
-      const long long o = r * N + t * 16 + (lane & 15);
-      float v = acc[t][q];
-      if (add) v += C[o];
-      if (mask && !(mask[o] > 0.f)) v = 0.f;
-      C[o] = v;
+    for (int t = 0; t < NT; t++) {
+      const long long o = r * N + t * 16 + (lane >> 4) * 4;
+      floatx4 v = acc[u][t];
+      if (add) v += *reinterpret_cast<const floatx4 *>(C + o);
+      if (mask) {
+        const floatx4 m = *reinterpret_cast<const floatx4 *>(mask + o);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (!(m[q] > 0.f)) v[q] = 0.f;
+      }
+      *reinterpret_cast<floatx4 *>(C + o) = v;
     }
   }
 }
@@ -428,7 +440,8 @@ __global__ __launch_bounds__(kBlock) void k_gemm_wgrad(long long n, const bf16_t
 }
 
 // edge head: four rows per wavefront, 16 lanes per row, four channels per
-// lane; the row's lower edges one at a time
+// lane; the gathers of four of the row's lower edges in flight (979,700 rows: 250
+// us one at a time, 216 so)
 __global__ __launch_bounds__(kBlock) void k_edge_head(long long n, const int *__restrict__ erp,
                                                       const int *__restrict__ eci,
                                                       const float *__restrict__ ev,
@@ -449,17 +462,30 @@ __global__ __launch_bounds__(kBlock) void k_edge_head(long long n, const int *__
   for (long long i = (long long)blockIdx.x * (kBlock / 16) + threadIdx.x / 16; i < n; i += groups) {
     const floatq pi = *reinterpret_cast<const floatq *>(P + i * H2 + 4 * q);
     const int lo = nlow[i], g0 = grp[i];
-    for (int k = 0; k < lo; k++) {
-      const int j = eci[erp[i] + k];
-      const float e = ev[erp[i] + k];
-      const floatq pj = *reinterpret_cast<const floatq *>(P + (long long)j * H2 + H + 4 * q);
-      const floatq sv = pi + pj + e * ve + cc;
-      float g = wo.x * fmaxf(sv.x, 0.f) + wo.y * fmaxf(sv.y, 0.f) + wo.z * fmaxf(sv.z, 0.f) +
-                wo.w * fmaxf(sv.w, 0.f);
-      g = group_sumf<16>(g) + bo;
-      if (q == 0) {
-        ghat[g0 + k] = g;
-        if (gval) gval[g0 + k] = s[i] * (double)g;
+    const int beg = erp[i];
+    for (int k0 = 0; k0 < lo; k0 += 4) {
+      floatq pj[4];
+      float e[4];
+      long long j[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        j[k] = eci[beg + min(k0 + k, lo - 1)];
+        e[k] = ev[beg + min(k0 + k, lo - 1)];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        pj[k] = *reinterpret_cast<const floatq *>(P + j[k] * H2 + H + 4 * q);
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (k0 + k >= lo) break;
+        const floatq sv = pi + pj[k] + e[k] * ve + cc;
+        float g = wo.x * fmaxf(sv.x, 0.f) + wo.y * fmaxf(sv.y, 0.f) + wo.z * fmaxf(sv.z, 0.f) +
+                  wo.w * fmaxf(sv.w, 0.f);
+        g = group_sumf<16>(g) + bo;
+        if (q == 0) {
+          ghat[g0 + k0 + k] = g;
+          if (gval) gval[g0 + k0 + k] = s[i] * (double)g;
+        }
       }
     }
     if (q == 0) {
@@ -983,7 +1009,7 @@ int forward(tbsla_hip_precond_net_s *net, double *gval, hipStream_t s) {
   TBSLA_TRY(net->P.ensure(n * H2));
   TBSLA_TRY(net->gdiag.ensure(n));
   TBSLA_TRY(net->ghat.ensure(net->ng));
-  const unsigned gg = (unsigned)((n + 63) / 64);
+  const unsigned gg = (unsigned)((n + kGemmRows - 1) / kGemmRows);
   const unsigned qg = (unsigned)std::min<long long>(4096, (n + 15) / 16);  // 16 nodes per workgroup
   const float *th = net->th.p;
   k_layer0<<<(unsigned)((n + 63) / 64), kBlock, 0, s>>>(n, net->erp.p, net->eci.p, net->ev.p,
@@ -1044,7 +1070,7 @@ int loss_and_dghat(tbsla_hip_precond_net_s *net, int k, unsigned long long seed,
 int backward(tbsla_hip_precond_net_s *net, hipStream_t s) {
   const long long n = net->n;
   const unsigned rg = row_grid(n);
-  const unsigned gg = (unsigned)((n + 63) / 64);
+  const unsigned gg = (unsigned)((n + kGemmRows - 1) / kGemmRows);
   const unsigned wg = (unsigned)((n + kWgRows - 1) / kWgRows);
   TBSLA_TRY(net->dh.ensure(n * H));
   TBSLA_TRY(net->dPb.ensure(n * H2));
