@@ -490,7 +490,8 @@ int tbsla_hip_personalized_page_rank(tbsla_hip_matrix_t m, double beta, double e
 
 /* CSR SpMV schedule (no reference counterpart): `lanes` cooperating on one
  * row (1..64, power of two) and `rows` each lane group keeps in flight
- * (1, 2 or 4); 0 restores the choice from the mean row length. */
+ * (1, 2 or 4); 0 restores the choice from the mean row length (both 0: the
+ * default kernel, with its vec and nontemporal below). */
 int tbsla_hip_set_csr_schedule(tbsla_hip_matrix_t m, int lanes, int rows);
 int tbsla_hip_get_csr_schedule(tbsla_hip_matrix_t m, int *lanes, int *rows);
 /* The full CSR row-kernel choice (no reference counterpart): the schedule

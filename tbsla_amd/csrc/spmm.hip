@@ -9,6 +9,7 @@
 #include <climits>
 #include <cstdint>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "common.hpp"
@@ -19,7 +20,8 @@ namespace tbsla_hip {
 namespace {
 
 // C = A B.  A group of LPR lanes takes one row and one chunk of LPR V columns (V
-// doubles per lane load), up to eight entries' pieces of B in flight.  Every
+// doubles per lane load), up to 16 entries' pieces of B in flight (8 where LPR is
+// not 16).  Every
 // entry gathers its row's chunk of B, so the kernel is bound by where those come
 // from, and the chunk is narrow: 32 columns (256 bytes, two lines) keep the
 // chunk's slice of B small enough to be met again in a cache.  Chunks are the
@@ -50,6 +52,19 @@ constexpr int kSpmmXcdCols = 65536;
 
 // E entries from j on: their pieces of B are in flight together, the products
 // are added in entry order
+// lane K of each group of 16, in every lane of the group (row_newbcast reads
+// a lane of the lane's own row, so every lane has a source; bound_ctrl set
+// lets the compiler give the broadcast straight to the instruction using it,
+// as the address add does)
+template <int K>
+__device__ __forceinline__ int qbc(int v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, true);
+}
+template <int K>
+__device__ __forceinline__ double qbc_d(double v) {
+  return __hiloint2double(qbc<K>(__double2hiint(v)), qbc<K>(__double2loint(v)));
+}
+
 template <int E, int V>
 __device__ inline void spmm_step(const SpmmArgs &a, int j, int col, bool on, double (&acc)[V]) {
   TBSLA_NO_FMA
@@ -81,10 +96,8 @@ __device__ inline void spmm_step(const SpmmArgs &a, int j, int col, bool on, dou
       if (in[e]) acc[q] = acc[q] + v[e] * x[e][q];
 }
 
-template <int LPR, int V>
-__global__ __launch_bounds__(kBlock) void k_csr_spmm(SpmmArgs a) {
-  typedef double vd __attribute__((ext_vector_type(V)));
-  unsigned chunk, rb;
+// the chunk and the row block of a workgroup
+__device__ inline void spmm_place(const SpmmArgs &a, unsigned &chunk, unsigned &rb) {
   if (a.xcd && a.nchunks >= 8) {  // nchunks a multiple of 8
     const unsigned i = blockIdx.x / 8;
     chunk = blockIdx.x % 8 + 8 * (i / a.rblocks);
@@ -97,6 +110,103 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmm(SpmmArgs a) {
     chunk = a.chunk0 + blockIdx.y;
     rb = blockIdx.x;
   }
+}
+
+// entries E0 + K of the 16 that a row's lanes hold: their columns, and the pieces
+// of B's rows they name (nothing for an entry outside the row or the block)
+template <int E0, int V, int... K>
+__device__ inline void spmm16_gather(std::integer_sequence<int, K...>, const SpmmArgs &a, int c,
+                                     bool on, int col, int (&ce)[8], double (&x)[8][V]) {
+  typedef double vd __attribute__((ext_vector_type(V)));
+  ((ce[K] = qbc<E0 + K>(c)), ...);
+  auto one = [&](int e) {
+    const double *bp = a.B + (size_t)max(ce[e], 0) * a.k + col;
+    const bool get = on && ce[e] >= 0;
+    if constexpr (V == 1) {
+      x[e][0] = get ? *bp : 0.0;
+    } else {
+      const vd b = get ? *reinterpret_cast<const vd *>(bp) : vd{};
+#pragma unroll
+      for (int q = 0; q < V; q++) x[e][q] = b[q];
+    }
+  };
+  (one(K), ...);
+}
+
+template <int E0, int V, int... K>
+__device__ inline void spmm16_add(std::integer_sequence<int, K...>, double v, const int (&ce)[8],
+                                  const double (&x)[8][V], double (&acc)[V]) {
+  TBSLA_NO_FMA
+  auto one = [&](double ve, int e) {
+    TBSLA_NO_FMA
+#pragma unroll
+    for (int q = 0; q < V; q++)
+      if (ce[e] >= 0) acc[q] = acc[q] + ve * x[e][q];
+  };
+  (one(qbc_d<E0 + K>(v), K), ...);
+}
+
+// 16 lanes per row: each loads one of the row's next 16 entries, one trip for
+// columns and values, and hands it to the others by row broadcasts; the pieces of
+// B of all 16 are then in flight together, with the entries after them.  A row of
+// ten took two trips for entries and two for B where this takes one each (cqmats,
+// q = 0.1: n = 200,003, 10 to a row, k = 512: 709 -> 660 us; n = 50,021, 30, k =
+// 128: 82 -> 59; n = 300,007, 16, k = 15: 65 -> 45; random columns as before,
+// bound by the MALL).
+template <int V>
+__global__ __launch_bounds__(kBlock) void k_csr_spmm16(SpmmArgs a) {
+  typedef double vd __attribute__((ext_vector_type(V)));
+  constexpr int LPR = 16;
+  unsigned chunk, rb;
+  spmm_place(a, chunk, rb);
+  const long long row = (long long)rb * (kBlock / LPR) + threadIdx.x / LPR;
+  if (rb >= a.rblocks || row >= a.n_rows) return;
+  const int lane = threadIdx.x & (LPR - 1);
+  const int col = ((int)chunk * LPR + lane) * V;
+  const bool on = col < a.k;  // V = 2: k is even
+  double acc[V];
+#pragma unroll
+  for (int q = 0; q < V; q++) acc[q] = 0.0;
+  int j = a.rowptr[row];
+  const int end = a.rowptr[row + 1];
+  int c = -1;
+  double v = 0.0;
+  auto entries = [&](int j0, int &cn, double &vn) {
+    const int e = min(j0 + lane, end - 1);
+    const unsigned cc = (unsigned)(a.colidx[e] - a.f_col);
+    vn = a.vals[e];
+    cn = j0 + lane < end && cc < (unsigned)a.ln_col ? (int)cc : -1;  // block filter (:19)
+  };
+  if (j < end) entries(j, c, v);
+  const std::make_integer_sequence<int, 8> eight{};
+  for (; j < end; j += LPR) {
+    int c0[8], c1[8], cn = -1;
+    double x0[8][V], x1[8][V], vn = 0.0;
+    spmm16_gather<0, V>(eight, a, c, on, col, c0, x0);
+    if (j + 8 < end) spmm16_gather<8, V>(eight, a, c, on, col, c1, x1);
+    if (j + LPR < end) entries(j + LPR, cn, vn);
+    spmm16_add<0, V>(eight, v, c0, x0, acc);
+    if (j + 8 < end) spmm16_add<8, V>(eight, v, c1, x1, acc);
+    c = cn;
+    v = vn;
+  }
+  if (!on) return;
+  double *out = a.C + (size_t)row * a.k + col;
+  if constexpr (V == 1) {
+    __builtin_nontemporal_store(acc[0], out);
+  } else {
+    vd o;
+#pragma unroll
+    for (int q = 0; q < V; q++) o[q] = acc[q];
+    __builtin_nontemporal_store(o, reinterpret_cast<vd *>(out));
+  }
+}
+
+template <int LPR, int V>
+__global__ __launch_bounds__(kBlock) void k_csr_spmm(SpmmArgs a) {
+  typedef double vd __attribute__((ext_vector_type(V)));
+  unsigned chunk, rb;
+  spmm_place(a, chunk, rb);
   const long long row = (long long)rb * (kBlock / LPR) + threadIdx.x / LPR;
   if (rb >= a.rblocks || row >= a.n_rows) return;
   const int col = (int)chunk * LPR * V + (threadIdx.x & (LPR - 1)) * V;
@@ -128,6 +238,12 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmm(SpmmArgs a) {
   }
 }
 
+template <int LPR, int V>
+void spmm_run(const SpmmArgs &a, dim3 grid, hipStream_t s) {
+  if constexpr (LPR == 16) k_csr_spmm16<V><<<grid, kBlock, 0, s>>>(a);
+  else k_csr_spmm<LPR, V><<<grid, kBlock, 0, s>>>(a);
+}
+
 // the launch of one (LPR, V)
 template <int LPR, int V>
 int spmm_go(SpmmArgs a, hipStream_t s) {
@@ -140,13 +256,13 @@ int spmm_go(SpmmArgs a, hipStream_t s) {
     const unsigned share = a.nchunks < 8 ? 8 / a.nchunks : 1;  // XCDs to a chunk
     const unsigned grid =
         a.nchunks < 8 ? 8 * ((a.rblocks + share - 1) / share) : a.rblocks * a.nchunks;
-    k_csr_spmm<LPR, V><<<grid, kBlock, 0, s>>>(a);
+    spmm_run<LPR, V>(a, dim3(grid), s);
     TBSLA_HIP_LAUNCH_CHECK();
     return TBSLA_HIP_SUCCESS;
   }
   constexpr unsigned kMostY = 65535;
   for (a.chunk0 = 0; a.chunk0 < a.nchunks; a.chunk0 += kMostY) {
-    k_csr_spmm<LPR, V><<<dim3(a.rblocks, std::min(kMostY, a.nchunks - a.chunk0)), kBlock, 0, s>>>(a);
+    spmm_run<LPR, V>(a, dim3(a.rblocks, std::min(kMostY, a.nchunks - a.chunk0)), s);
     TBSLA_HIP_LAUNCH_CHECK();
   }
   return TBSLA_HIP_SUCCESS;
@@ -351,19 +467,6 @@ __device__ __forceinline__ void ring_store(const PprArgs &a, bool tile_ok, int j
 constexpr int kQuadLanes = 16;
 constexpr int kQuadRows = kWave / kQuadLanes;  // rows per wavefront step
 constexpr int kQuadEnt = 2 * kQuadLanes;       // entries per row in the pipeline
-
-// lane K of each group of 16, in every lane of the group (row_newbcast reads
-// a lane of the lane's own row, so every lane has a source; bound_ctrl set
-// lets the compiler give the broadcast straight to the instruction using it,
-// as the address add does)
-template <int K>
-__device__ __forceinline__ int qbc(int v) {
-  return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, true);
-}
-template <int K>
-__device__ __forceinline__ double qbc_d(double v) {
-  return __hiloint2double(qbc<K>(__double2hiint(v)), qbc<K>(__double2loint(v)));
-}
 
 // a quad slot: four rows (row q of each group), this lane's part
 template <int S>
