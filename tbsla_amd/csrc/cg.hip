@@ -70,6 +70,7 @@ struct CgCom {
   int ndone;     // systems finished for good
   int npending;  // systems waiting for the true-residual test
   long long t0;  // wall clock at the start of the iteration
+  double ratio;  // the first system's |r| over its threshold at its last test
 };
 
 struct CgArgs {
@@ -479,6 +480,7 @@ __device__ inline int k1_test(const CgArgs &a, CgSeg *S, const CgPart &sg, int b
     fin = kBreakdown;
   if (b == sg.blk0 && threadIdx.x == 0) {
     S->rnorm = rn;
+    if (S == a.seg) a.com->ratio = rn / sg.stop;
     if (fin != kRunning) {
       S->stop_par = par;
       S->t_done = wall_clock64();
@@ -2496,7 +2498,7 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
         if (e == hipSuccess) {
           for (int k = 0; k < B; k++) {
             const bool last = k == B - 1;
-            enqueue_iteration(p, (v == 1 && last) ? B * p.replace : 1 + k, last);
+            enqueue_iteration(p, (v == 1 && last) ? B * p.replace : 1 + k, false);
           }
           e = hipStreamEndCapture(s, &graph);
         }
@@ -2526,11 +2528,23 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   // tail (or when no graph is used).
   int batches = 0;
   bool finished = false;
+  // settle waiting systems after a batch (a replacement step does): a lone
+  // system's batches leave that out while its residual, by its decay over the last
+  // batch, is more than three batches from the threshold (five kernels that find
+  // nothing to do: 30 of 455 us a batch at 10^6 rows, mixed, factored).  Were it
+  // to get there sooner, the status of that batch would tell, and it would wait
+  // for one more.
+  bool near = true;
+  double ratio = 0.0;
   while (it < max_it && !finished) {
     if (B > 0 && it + B <= max_it) {
       const int last = it + B - 1;  // the batch's last iteration
       const bool rep = p.replace > 0 && last % p.replace == 0;
       TBSLA_HIP_CHECK(hipGraphLaunch(gs->exec[rep ? 1 : 0], s));
+      if (p.verify && !rep && near) {
+        true_residual(p, last & 1, kVerify);
+        k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, p.multi, (last + 1) & 1);
+      }
       it += B;
     } else {
       const int stop = std::min(max_it, it + poll_every);
@@ -2550,6 +2564,9 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
         TBSLA_HIP_LAUNCH_CHECK();
       }
       if (h.ndone >= nactive) finished = true;
+      const double decay = std::max(ratio / h.ratio, 1.0);
+      near = multi || !(ratio > 0 && h.ratio > 4 * decay * decay * decay);
+      ratio = h.ratio;
     }
     batches++;
   }
