@@ -177,8 +177,10 @@ __device__ inline int cg_block(int multi) {
 // offset i < 8 of A's or of G's diagonals
 #define CG_OFF(field, i) ((TBSLA_CONST CgBlock *)pa_)->args.field[i]
 // The system of workgroup b: S, and in sg what a kernel of the iteration reads
-// of it and none of that launch writes (K1's test aside, which only writes iters
-// where it does not read it).  A lone system's is read at once, with the
+// of it and none of that launch writes: every wavefront reads it for itself.  K1's
+// test writes `done`, and `iters` where it does not read it, so the kernels that
+// make the test take `done` from seg_finish alone, one answer for the workgroup;
+// sg.done is for those that do not.  A lone system's is read at once, with the
 // arguments: CG_HAND names those a kernel needs first, so that the compiler asks
 // for all of them before it waits.
 #define CG_SYSTEM(b, ...)                                                              \
@@ -626,7 +628,6 @@ __global__ __launch_bounds__(kBlock) void k_cg_pnew(CG_ARGS, int par_g, int chec
   __shared__ SegShared sh;
   const int b = cg_block(multi_);
   CG_SYSTEM(b);
-  if (multi_ && sg.done != kRunning) return;  // finished before this launch
   const int par = (par_g ^ sg.shift) & 1;
   const int b0 = sg.blk0, b1 = sg.blk1;
   const int r0 = sg.row0 + (b - b0) * sg.rpb;

@@ -119,3 +119,32 @@ def test_ragged_rows_under_every_lane_count(lanes, precision):
     m = matrix(A)
     x = [check(m, A, lanes_per_row=lanes, precision=precision, spmv_passes=p) for p in (1, 2)]
     assert np.array_equal(x[0], x[1])
+
+
+@pytest.mark.parametrize("precision", [T.CG_FP64, T.CG_MIXED])
+@pytest.mark.parametrize("pre", [T.PRECOND_NONE, T.PRECOND_JACOBI])
+def test_two_passes_of_uneven_systems(pre, precision):
+    """Systems of 1 to 236 workgroups that finish at different iterations, so that a
+    launch meets running systems, the one it ends and those ended before: bit for
+    bit as in one pass, and each as it is alone."""
+    sizes = [(60401, 6), (300, 9), (9000, 40), (1, 3), (33000, 17), (5003, 2)]
+    parts = [T.Matrix(T.CSR).fill_sym_cqmat(n, c, 0.1, 1, value_seed=k)
+             for k, (n, c) in enumerate(sizes)]
+    bd = T.Matrix.block_diag(parts)
+    offs = np.concatenate([[0], np.cumsum([n for n, _ in sizes])]).astype(np.int32)
+    rhs = np.random.default_rng(2).standard_normal(int(offs[-1]))
+    kw = dict(tolerance=1e-10, relative=True, precision=precision, preconditioner=pre,
+              lanes_per_row=4, replace_every=20 if precision == T.CG_MIXED else 0,
+              max_blocks_per_system=256, max_iterations=300)
+    x, res = bd.cg_batched(offs, rhs, bd.cg_options(spmv_passes=2, **kw))
+    assert len({r.iterations for r in res}) >= 4
+    x1, res1 = bd.cg_batched(offs, rhs, bd.cg_options(spmv_passes=1, **kw))
+    of = [[(r.status, r.iterations, r.res_norm) for r in rs] for rs in (res, res1)]
+    assert of[0] == of[1]
+    assert np.array_equal(x, x1)
+    if precision == T.CG_MIXED:
+        return
+    for k, p in enumerate(parts):
+        xs, its, rs = p.cg(rhs[offs[k]:offs[k + 1]], spmv_passes=2, **kw)
+        assert (res[k].iterations, res[k].res_norm) == (its, rs)
+        assert np.array_equal(x[offs[k]:offs[k + 1]], xs)
