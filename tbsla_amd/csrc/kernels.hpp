@@ -39,14 +39,14 @@ int launch_axpy_inplace(double *y, const double *x, long long n, hipStream_t s);
 template <typename K>
 int radix_sort_pairs(K **keys, int **payload, long long n, int key_bits, hipStream_t s,
                      int low = 0);
-// Keys taken from column indices: the local column, or ln_col outside the block.
+// Keys taken from column indices: the local column, or `none` outside the block.
 struct ColumnKeys {
   const int *cols;
   int f_col;
-  unsigned ln_col;
+  unsigned ln_col, none;
   __device__ inline unsigned operator[](long long i) const {
     const unsigned c = (unsigned)(cols[i] - f_col);
-    return c < ln_col ? c : ln_col;
+    return c < ln_col ? c : none;
   }
 };
 // radix_sort_pairs<unsigned> of src's n keys, read by the first pass in place of

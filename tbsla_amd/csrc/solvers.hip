@@ -55,19 +55,21 @@ unsigned red_grid(long long n) {
 // array by the first pass; ELL: row-major slot i*max_col+j, here).  Entries
 // the reference skips -- ELL slots whose value is not positive
 // (MatrixELL.cpp:812), which include the padding (column 0, possibly left of
-// the block) -- and any column outside [0, ln_col) get the key ln_col, a
-// bucket after the last column that no sum reads.
+// the block) -- and any column outside [0, ln_col) get the key `none`, in a
+// bucket after the last column's (buckets being what the sort tells apart) that
+// no workgroup reads: a block with a few long rows is mostly padding.
 __global__ __launch_bounds__(kBlock) void k_ell_colkeys(long long n, long long ln_row,
                                                         long long ln_col, int max_col,
                                                         const int *__restrict__ cols,
                                                         const double *__restrict__ vals, int f_col,
+                                                        unsigned none,
                                                         unsigned *__restrict__ keys) {
   long long p = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (p >= n) return;
   const long long src = (p % max_col) * ln_row + p / max_col;
   const long long c = (long long)cols[src] - f_col;
   const bool keep = c >= 0 && c < ln_col && vals[src] > 0;
-  keys[p] = keep ? (unsigned)c : (unsigned)ln_col;
+  keys[p] = keep ? (unsigned)c : none;
 }
 
 // s[c] += the column's values in reference order (one thread per column):
@@ -95,8 +97,8 @@ __global__ __launch_bounds__(kSumThreads) void k_col_sums(
   const int first = starts[blockIdx.x], last = starts[blockIdx.x + 1];
   const int sub = tile_sub<kSumItems>();
   double acc = live ? s[c] : 0.0;
-  for (int b = first; b < last; b += kSumChunk) {
-    const int count = min(kSumChunk, last - b);
+  for (int b = first, count; b < last; b += count) {
+    count = min(kSumChunk, last - b);
     unsigned key[kSumItems];
     long long p[kSumItems];
     double v[kSumItems];
@@ -545,27 +547,38 @@ extern "C" int tbsla_hip_get_col_sums(tbsla_hip_matrix_t m, double *d_s, void *s
   DevBuf<int> pos, colptr;
   TBSLA_TRY(keys.alloc(n));
   TBSLA_TRY(pos.alloc(n));
-  int bits = 1;
-  while (bits < 32 && (1LL << bits) <= ln_col) bits++;  // keys <= ln_col < 2^bits
   // the bits left to the sums: as many as spare the sort a pass, then as few as
-  // give a workgroup half a chunk or more
+  // give a workgroup half a chunk or more; the other bits tell the workgroups'
+  // buckets from each other and from the skipped entries' after them (which
+  // costs a pass more where 256 columns a bucket fill 8 or 16 bits: 65,281 to
+  // 65,535 columns, 16,776,961 to 16,777,215)
+  auto buckets = [&](int low) { return (ln_col + (1LL << low) - 1) >> low; };
+  auto bits_above = [&](int low) {
+    int b = 1;
+    while ((1LL << b) <= buckets(low)) b++;
+    return b;
+  };
+  const int bits = bits_above(0);  // of the local columns
   const int passes = std::max(1, (bits - 1) / 8);
   int low = std::min(8, bits - 1);
-  while (low > std::max(0, bits - 8 * passes) && ((n << low) / std::max(ln_col, 1LL)) > 3 * kSumChunk / 4)
+  while (low > 0 && bits_above(low - 1) <= 8 * passes &&
+         ((n << low) / std::max(ln_col, 1LL)) > 3 * kSumChunk / 4)
     low--;
-  const long long nb = (ln_col >> low) + 1;
+  const long long nb = buckets(low);
+  const unsigned none = (unsigned)(nb << low);
+  const int key_bits = low + bits_above(low);
   TBSLA_TRY(colptr.alloc(nb + 1));
   if (fmt == TBSLA_HIP_ELL) {
     k_ell_colkeys<<<grid_for(n), kBlock, 0, s>>>(n, m->ln_row, ln_col, m->max_col, m->colidx,
-                                                 m->values, m->f_col, keys.p);
+                                                 m->values, m->f_col, none, keys.p);
     TBSLA_HIP_LAUNCH_CHECK();
-    TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, bits, s, low));
+    TBSLA_TRY(radix_sort_pairs<unsigned>(&keys.p, &pos.p, n, key_bits, s, low));
   } else {
-    const ColumnKeys src{m->colidx, m->f_col, (unsigned)ln_col};
-    TBSLA_TRY(radix_sort_columns(src, &keys.p, &pos.p, n, bits, s, low));
+    const ColumnKeys src{m->colidx, m->f_col, (unsigned)ln_col, none};
+    TBSLA_TRY(radix_sort_columns(src, &keys.p, &pos.p, n, key_bits, s, low));
   }
   TBSLA_TRY(bucket_starts<unsigned>(keys.p, n, low, nb, colptr.p, s));
-  if (ln_col > 0) {
+  if (nb > 0) {
     k_col_sums<<<(unsigned)nb, kSumThreads, 0, s>>>(ln_col, fmt, m->ln_row, m->max_col, low,
                                                     colptr.p, keys.p, pos.p, m->values, d_s);
     TBSLA_HIP_LAUNCH_CHECK();
