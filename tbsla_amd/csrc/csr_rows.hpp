@@ -7,12 +7,15 @@
 // column indices and one 8 V-byte load of values), starting from the row's
 // first entry rounded down to a multiple of V, so the vector loads stay
 // aligned; they may reach V - 1 entries past the row, and past the arrays
-// (device_alloc's blocks have room for them).  The entries are then turned in
-// groups of V lanes (lane_transpose), so that x is gathered by neighbouring
-// columns; what lies outside the row is not summed (17 entries a row, a load per
-// entry at the row's end before: n = 2.5 M 176 -> 143 us, n = 10^6 71 -> 57).  Lanes add their entries in
-// trip order and the group adds its lanes by a fixed xor tree, so results are
-// deterministic and within rounding of the sequential row sum.
+// (device_alloc's blocks have room for them).  In a batch of instances (SEG) the
+// multiple is counted from the instance's first entry, so that a row is summed
+// as in a block of the instance alone; the loads then lie on any entry.  The
+// entries are turned in groups of V lanes (lane_transpose), so that x is gathered
+// by neighbouring columns; what lies outside the row is not summed (17 entries a
+// row, a load per entry at the row's end before: n = 2.5 M 176 -> 143 us, n = 10^6
+// 71 -> 57).  Lanes add their entries in trip order and the group adds its lanes
+// by a fixed xor tree, so results are deterministic and within rounding of the
+// sequential row sum.
 //
 // NT selects the nontemporal load (the line is not kept in L2 for later
 // use): it pays when every line is read whole by one instruction, and
@@ -54,11 +57,12 @@ __device__ inline int seg_of_row(const int *offs, int nseg, long long row) {
   return lo;
 }
 
-template <int V, int NT>
+// ANY: j need not be a multiple of V
+template <int V, int NT, bool ANY>
 __device__ inline void csr_load(const int *ci, const double *va, int j, int (&c)[V],
                                 double (&v)[V]) {
-  typedef int vi __attribute__((ext_vector_type(V)));
-  typedef double vd __attribute__((ext_vector_type(V)));
+  typedef int vi __attribute__((ext_vector_type(V), aligned((ANY ? 1 : V) * sizeof(int))));
+  typedef double vd __attribute__((ext_vector_type(V), aligned((ANY ? 1 : V) * sizeof(double))));
   if (V == 1) {
     c[0] = NT ? __builtin_nontemporal_load(ci + j) : ci[j];
     v[0] = NT ? __builtin_nontemporal_load(va + j) : va[j];
@@ -76,13 +80,17 @@ __device__ inline void csr_load(const int *ci, const double *va, int j, int (&c)
 }
 
 // The sums of the R rows [beg[r], end[r]) of this lane's group, in every lane of
-// the group
-template <int V, int L, int R, int NT>
+// the group; ent0[r] (SEG): the entry that row r's loads are counted from
+template <int V, int L, int R, int NT, bool SEG = false>
 __device__ inline void csr_row_sums(const CsrRowsArgs &a, const int (&beg)[R], const int (&end)[R],
-                                    int lane, double (&sum)[R]) {
+                                    int lane, double (&sum)[R], const int (&ent0)[R]) {
+  auto down = [&](int e, int r) {  // e rounded down to a load's first entry
+    if constexpr (SEG) return e - ((e - ent0[r]) & (V - 1));
+    else return e & ~(V - 1);
+  };
   int len = 0;
 #pragma unroll
-  for (int r = 0; r < R; r++) len = max(len, end[r] - (beg[r] & ~(V - 1)));
+  for (int r = 0; r < R; r++) len = max(len, end[r] - down(beg[r], r));
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) len = max(len, __shfl_xor(len, off, kWave));
   const int trips = (len + V * L - 1) / (V * L);
@@ -97,14 +105,14 @@ __device__ inline void csr_row_sums(const CsrRowsArgs &a, const int (&beg)[R], c
     bool in[R][V];
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      const int first = (beg[r] & ~(V - 1)) + V * t * L;
+      const int first = down(beg[r], r) + V * t * L;
       // lanes past the row read its last entries again
-      const int j = max(min(first + V * lane, (end[r] - 1) & ~(V - 1)), 0);
-      csr_load<V, NT>(a.colidx, a.vals, j, c[r], v[r]);
+      const int j = max(min(first + V * lane, down(end[r] - 1, r)), 0);
+      csr_load<V, NT, SEG>(a.colidx, a.vals, j, c[r], v[r]);
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      const int first = (beg[r] & ~(V - 1)) + V * t * L;
+      const int first = down(beg[r], r) + V * t * L;
       if constexpr (V > 1) {
         lane_transpose<V>(c[r]);
         lane_transpose<V>(v[r]);
@@ -125,7 +133,7 @@ __device__ inline void csr_row_sums(const CsrRowsArgs &a, const int (&beg)[R], c
   for (int r = 0; r < R; r++) sum[r] = group_sum<L>(sum[r]);
 }
 
-template <int V, int L, int R, int NT, bool SPLIT>
+template <int V, int L, int R, int NT, bool SPLIT, bool SEG>
 __global__ __launch_bounds__(kBlock) void k_csr_rows(CsrRowsArgs a) {
   if (a.done && *a.done) return;
   constexpr int G = kWave / L;
@@ -134,24 +142,36 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows(CsrRowsArgs a) {
   const long long wave = ((long long)blockIdx.x * kBlock + threadIdx.x) / kWave;
   const long long base = wave * (G * R);
   if (base >= a.n_rows) return;
+  int seg = 0, seg_end = 0, seg_ent0 = 0;
   if (a.seg_offs) {  // wave-uniform
     const long long last = min(base + G * R, a.n_rows) - 1;
-    const int k0 = seg_of_row(a.seg_offs, a.nseg, base);
-    if (a.seg_done[k0] && (last < a.seg_offs[k0 + 1])) return;
+    seg = seg_of_row(a.seg_offs, a.nseg, __builtin_amdgcn_readfirstlane((int)base));
+    seg_end = a.seg_offs[seg + 1];
+    if constexpr (SEG) seg_ent0 = a.rowptr[a.seg_offs[seg]];
+    if (a.seg_done[seg] && last < seg_end) return;
   }
-  int beg[R], end[R];
+  int beg[R], end[R], ent0[R];
 #pragma unroll
   for (int r = 0; r < R; r++) {
     const long long row = base + r * G + g;
+    ent0[r] = 0;
     if (row < a.n_rows) {
       beg[r] = a.rowptr[row];
       end[r] = a.rowptr[row + 1];
+      if constexpr (SEG) {
+        if (row >= seg_end) {  // a later segment: from the row before's on
+          do seg_end = a.seg_offs[++seg + 1];
+          while (row >= seg_end);
+          seg_ent0 = a.rowptr[a.seg_offs[seg]];
+        }
+        ent0[r] = seg_ent0;
+      }
     } else {
       beg[r] = end[r] = 0;
     }
   }
   double sum[R];
-  csr_row_sums<V, L, R, NT>(a, beg, end, lane, sum);
+  csr_row_sums<V, L, R, NT, SEG>(a, beg, end, lane, sum, ent0);
 #pragma unroll
   for (int r = 0; r < R; r++) {
     const long long row = base + r * G + g;
@@ -175,7 +195,13 @@ template <bool SPLIT, int V, int L, int R, int NT>
 void csr_rows_go(const CsrRowsArgs &a, hipStream_t s) {
   const long long rows_per_wave = (long long)(kWave / L) * R;
   const long long waves = (a.n_rows + rows_per_wave - 1) / rows_per_wave;
-  k_csr_rows<V, L, R, NT, SPLIT><<<grid_for(waves * kWave), kBlock, 0, s>>>(a);
+  const unsigned grid = grid_for(waves * kWave);
+  if constexpr (V > 1 && !SPLIT)  // one entry a load: no multiple to count
+    if (a.seg_offs) {
+      k_csr_rows<V, L, R, NT, false, true><<<grid, kBlock, 0, s>>>(a);
+      return;
+    }
+  k_csr_rows<V, L, R, NT, SPLIT, false><<<grid, kBlock, 0, s>>>(a);
 }
 
 template <bool SPLIT, int V, int L, int R>

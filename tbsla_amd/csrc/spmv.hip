@@ -415,12 +415,13 @@ __global__ __launch_bounds__(kBlock) void k_csr_rows_pr(CsrRowsArgs a, PrFuse pf
     for (int q = 0; q < kWave; q += G * R) {
       double sum[R];
       int rb[R], re[R];
+      const int ent0[R] = {};
 #pragma unroll
       for (int r = 0; r < R; r++) {
         rb[r] = __shfl(beg, q + r * G + g, kWave);
         re[r] = __shfl(end, q + r * G + g, kWave);
       }
-      csr_row_sums<V, L, R, 0>(a, rb, re, lane, sum);
+      csr_row_sums<V, L, R, 0>(a, rb, re, lane, sum, ent0);
 #pragma unroll
       for (int r = 0; r < R; r++)
         if (lane == 0) y[buf][wave * kWave + q + r * G + g] = sum[r];
