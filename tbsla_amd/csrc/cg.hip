@@ -1583,7 +1583,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_vcheck(CG_ARGS, int j) {
 
 // ax = A x (FP64 matrix) for the rows of the systems the mode selects, in
 // the engine's workgroup layout (workgroups of other systems return at
-// once); L lanes per row.
+// once); L lanes per row.  kStart: before k_cg_start has stored ent0.
 template <int L>
 __global__ __launch_bounds__(kBlock) void k_cg_ax(CG_ARGS, int par_g, int mode) {
   CG_BIND;
@@ -1596,11 +1596,12 @@ __global__ __launch_bounds__(kBlock) void k_cg_ax(CG_ARGS, int par_g, int mode) 
   const int r0 = sg.row0 + (b - sg.blk0) * sg.rpb;
   const int r1 = min(sg.row1, r0 + sg.rpb);
   const int lane = threadIdx.x & (L - 1);
+  const int ent0 = mode == kStart ? a.rowptr[sg.row0] : sg.ent0;
   typedef CgRow<L, double> Row;
   constexpr int PASS = kBlock / L;
   for (int row = r0 + (int)threadIdx.x / L; row < r1; row += PASS) {
     Row w;
-    w.extent(a.rowptr, row, sg.ent0);
+    w.extent(a.rowptr, row, ent0);
     w.load(a.colidx, a.val64, a.a_nnz, a.f_col, lane);
     double g[Row::P];
 #pragma unroll
@@ -2429,7 +2430,8 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   if (pre == TBSLA_HIP_PRECOND_JACOBI)
     k_csr_dinv<<<sgrid(n), kBlock, 0, s>>>(n, m->f_row, m->f_col, m->rowptr, m->colidx, m->values,
                                           c.dinv.p);
-  if (o.use_initial_guess) TBSLA_TRY(spmv_launch(m, c.ax.p, c.x.p, 0, true, s));
+  // A x by the engine's own rows: a system alone and in a batch starts alike
+  if (o.use_initial_guess) launch_ax(p, 0, kStart);
   launch_residual(p, o.use_initial_guess ? 1 : 0, 0, kStart, o.use_initial_guess ? 0 : 1);
   if (pre == TBSLA_HIP_PRECOND_FACTORED) {
     launch_gtr(p, 0, kStart);

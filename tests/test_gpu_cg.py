@@ -236,6 +236,33 @@ def test_batched_equals_single(pre):
     assert t[np.argmax(its)] >= t[np.argmin(its)]
 
 
+@pytest.mark.parametrize("lanes", [1, 8])
+@pytest.mark.parametrize("precision", [T.CG_FP64, T.CG_MIXED])
+def test_batched_from_a_guess_equals_single(precision, lanes):
+    """The residual of the guess is a system's own too, whatever the mean row length
+    of the batch and wherever its entries start."""
+    sizes = [(777, 31), (4097, 8), (3, 2), (9001, 20), (1200, 3)]
+    parts, bd, offs = make_batch(sizes, seed=5)
+    assert len(set(bd.arrays()[0][offs[:-1]] % 4)) > 1
+    n = int(offs[-1])
+    rhs, x0 = 2 * O.unit_vector(4, n) - 1, 2 * O.unit_vector(9, n) - 1
+    kw = dict(tolerance=1e-9, relative=True, preconditioner=T.PRECOND_JACOBI, precision=precision,
+              replace_every=16 if precision else 0, lanes_per_row=lanes, max_blocks_per_system=256,
+              max_iterations=12)
+    opt = bd.cg_options(use_initial_guess=True, **kw)
+    x, res = bd.cg_batched(offs, rhs, opt, x0=x0)
+    for k, p in enumerate(parts):
+        at = slice(offs[k], offs[k + 1])
+        xs, its, rs = p.cg(rhs[at], x0=x0[at], **kw)
+        assert (res[k].iterations, res[k].res_norm) == (its, rs)
+        assert np.array_equal(x[at], xs)
+    # an inactive system keeps its guess
+    x, res = bd.cg_batched(offs, rhs, opt, active=[1, 0, 1, 1, 0], x0=x0)
+    for k in (1, 4):
+        assert res[k].status == T.CG_INACTIVE
+        assert np.array_equal(x[offs[k]:offs[k + 1]], x0[offs[k]:offs[k + 1]])
+
+
 def test_batched_inactive_and_mixed():
     sizes = [(3000, 10), (5000, 24), (2500, 8)]
     parts, bd, offs = make_batch(sizes, seed=7)
