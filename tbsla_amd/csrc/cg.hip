@@ -2535,16 +2535,22 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
   // system's batches leave that out while its residual, by its decay over the last
   // batch, is more than three batches from the threshold (five kernels that find
   // nothing to do: 30 of 455 us a batch at 10^6 rows, mixed, factored).  Were it
-  // to get there sooner, the status of that batch would tell, and it would wait
-  // for one more.
+  // to get there sooner, the status of that batch would tell.  The batch then in
+  // flight finds it waiting and does nothing, so that batch is taken back: the
+  // iterations are numbered, and end at max_it, as if it had been settled at once.
   bool near = true;
+  bool left_out[2] = {false, false};  // of the batch behind each status copy
   double ratio = 0.0;
   while (it < max_it && !finished) {
+    const int slot = batches & 1;
+    left_out[slot] = false;
     if (B > 0 && it + B <= max_it) {
       const int last = it + B - 1;  // the batch's last iteration
       const bool rep = p.replace > 0 && last % p.replace == 0;
       TBSLA_HIP_CHECK(hipGraphLaunch(gs->exec[rep ? 1 : 0], s));
-      if (p.verify && !rep && near) {
+      // only a whole batch can be taken back: one comes after
+      left_out[slot] = p.verify && !rep && !near && it + 2 * B <= max_it;
+      if (p.verify && !rep && !left_out[slot]) {
         true_residual(p, last & 1, kVerify);
         k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, p.multi, (last + 1) & 1);
       }
@@ -2554,7 +2560,6 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
       for (; it < stop; it++) enqueue_iteration(p, it, it == stop - 1);
     }
     TBSLA_HIP_LAUNCH_CHECK();
-    const int slot = batches & 1;
     TBSLA_HIP_CHECK(hipMemcpyAsync(c.h_com + slot, a.com, sizeof(CgCom), hipMemcpyDeviceToHost, s));
     TBSLA_HIP_CHECK(hipEventRecord(c.ev[slot], s));
     if (batches > 0) {
@@ -2562,6 +2567,10 @@ int cg_solve_on(tbsla_hip_matrix_s *m, int nsys, const int *h_rows, const int *h
       TBSLA_HIP_CHECK(hipEventSynchronize(c.ev[prev]));
       const CgCom h = c.h_com[prev];
       if (h.npending > 0 && p.verify) {
+        if (left_out[prev]) {
+          it -= B;
+          left_out[slot] = false;  // settled here
+        }
         true_residual(p, 0, kVerify);
         k_cg_vcheck<<<nblocks, kBlock, 0, s>>>(p.args, p.multi, it);
         TBSLA_HIP_LAUNCH_CHECK();

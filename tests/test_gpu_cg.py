@@ -196,6 +196,28 @@ def test_graph_and_direct_launches_identical(sym, pre):
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[0], c[0]) and np.array_equal(a[0], d[0])
 
 
+@pytest.mark.parametrize("replace", [0, 32, 50])
+@pytest.mark.parametrize("most", [100, 112, 113, 120, 127, 128, 129, 140, 150, 160, 161, 250])
+def test_a_residual_that_falls_at_once(most, replace):
+    """A chain of n from a unit vector at its end: |r| falls by less than a fifth a batch and
+    to its rounding errors at step n, far from where its decay puts the threshold, with a
+    true residual above it.  The solve goes on from that one, at the same iterations
+    under graphs, which settle such a system late, as under direct launches."""
+    n = 100
+    A = sp.diags([np.full(n - 1, -1 / 3), np.full(n, 2 / 3), np.full(n - 1, -1 / 3)], [-1, 0, 1])
+    A = sp.csr_matrix(A)
+    g = to_gpu(O.csr_from_arrays(n, n, A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data))
+    b = np.zeros(n)
+    b[0] = 1.0
+    out = [g.cg(b, tolerance=3e-8, relative=True, precision=T.CG_MIXED, replace_every=replace,
+                max_iterations=most, graph_batch=k) for k in (0, -1)]
+    (xg, itg, rg), (xd, itd, rd) = out
+    assert (itg, rg) == (itd, rd)
+    assert np.array_equal(xg, xd)
+    if replace == 0 and most == 250:  # it did go on after step n
+        assert itg > n + 1 and rg < 3e-8
+
+
 def test_max_iterations_count(sym):
     o, g = sym
     n = o.geom["ln_row"]
