@@ -57,6 +57,7 @@ struct CgSeg {
   long long t_done;  // wall clock when the system finished
   int iters;         // reference counting
   int done;          // SegDone
+  int left;          // K2 found the system not running (K1 may leave at once)
   int shift;         // buffer parity of this system relative to the global iteration
   int true_res;      // the current r.r partials belong to a true residual b - A x
   int stop_par;      // buffer parity at the test that ended the recurrence
@@ -180,9 +181,10 @@ __device__ inline int cg_block(int multi) {
 // of it and none of that launch writes: every wavefront reads it for itself.  K1's
 // test writes `done`, and `iters` where it does not read it, so the kernels that
 // make the test take `done` from seg_finish alone, one answer for the workgroup;
-// sg.done is for those that do not.  A lone system's is read at once, with the
-// arguments: CG_HAND names those a kernel needs first, so that the compiler asks
-// for all of them before it waits.
+// sg.done is for those that do not, and `left`, which K2 writes, for K1's first pass
+// (96 systems: 9.00 ms by the shared flag alone, 8.80 with it).  A lone system's is
+// read at once, with the arguments: CG_HAND names those a kernel needs first, so
+// that the compiler asks for all of them before it waits.
 #define CG_SYSTEM(b, ...)                                                              \
   CgPart sg = cg_part(&((TBSLA_CONST CgBlock *)pa_)->seg);                             \
   CG_HAND("s"(sg.shift), "s"(sg.row0), "s"(sg.row1), "s"(sg.blk0), "s"(sg.blk1),       \
@@ -196,12 +198,12 @@ __device__ inline int cg_block(int multi) {
 
 struct CgPart {
   double stop, near_zero, rnorm0;
-  int iters, shift, true_res, stop_par, done;
+  int iters, shift, true_res, stop_par, done, left;
   int row0, row1, blk0, blk1, rpb, ent0;
 };
 
 __device__ inline CgPart cg_part(TBSLA_CONST CgSeg *c) {
-  return CgPart{c->stop, c->near_zero, c->rnorm0, c->iters, c->shift, c->true_res, c->stop_par, c->done,
+  return CgPart{c->stop, c->near_zero, c->rnorm0, c->iters, c->shift, c->true_res, c->stop_par, c->done, c->left,
                 c->row0, c->row1, c->blk0, c->blk1, c->rpb, c->ent0};
 }
 
@@ -628,6 +630,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_pnew(CG_ARGS, int par_g, int chec
   __shared__ SegShared sh;
   const int b = cg_block(multi_);
   CG_SYSTEM(b);
+  if (multi_ && sg.left) return;  // finished before the last K2
   const int par = (par_g ^ sg.shift) & 1;
   const int b0 = sg.blk0, b1 = sg.blk1;
   const int r0 = sg.row0 + (b - b0) * sg.rpb;
@@ -883,7 +886,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CG_ARGS, int par_g, int co
   CG_SYSTEM(b, "s"(a.p[0]), "s"(a.p[1]), "s"(a.prz[0]), "s"(a.prz[1]), "s"(a.prr[0]),
             "s"(a.prr[1]), "s"(a.r[0]), "s"(a.r[1]), "s"(a.x), "s"(a.ap), "s"(a.ppap),
             "s"(a.dinv));
-  if (multi_ && sg.done != kRunning) return;  // finished before this launch
+  if (multi_ && sg.done != kRunning) {  // finished before this launch
+    if (b == sg.blk0 && threadIdx.x == 0) S->left = 1;
+    return;
+  }
   const int par = (par_g ^ sg.shift) & 1;
   const int b0 = sg.blk0, b1 = sg.blk1;
   const double *rc = CG_AT(r, par);
@@ -1075,7 +1081,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_gdia(CG_ARGS, int par_g, i
             "s"(a.ncol), "s"(a.gndiag), "s"(MIX ? (const void *)a.gd32 : (const void *)a.gd64),
             "s"(CG_OFF(gdoff8, 0)), "s"(CG_OFF(gdoff8, 1)), "s"(CG_OFF(gdoff8, 2)),
             "s"(CG_OFF(gdoff8, 3)));
-  if (multi_ && sg.done != kRunning) return;  // finished before this launch
+  if (multi_ && sg.done != kRunning) {  // finished before this launch
+    if (b == sg.blk0 && threadIdx.x == 0) S->left = 1;
+    return;
+  }
   const int par = (par_g ^ sg.shift) & 1;
   const int b0 = sg.blk0, b1 = sg.blk1;
   const double *rc = CG_AT(r, par);
@@ -1571,6 +1580,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_vcheck(CG_ARGS, int j) {
       // (beta = 0 at the next iteration: an infinite "old r.z")
       S->shift = (j ^ sg.stop_par) & 1;
       S->done = kRunning;
+      S->left = 0;
     }
   }
   __syncthreads();

@@ -1,6 +1,7 @@
 """The CG kernels' reads of a system's state, from the source: a kernel whose
 first workgroup records a system's end (k1_test stores `done`) must not branch on
-the wavefronts' own plain reads of `done`, which may differ within a workgroup."""
+the wavefronts' own plain reads of `done`, which may differ within a workgroup; nor
+a kernel that writes `left` on its own reads of that."""
 import os
 import re
 
@@ -21,3 +22,11 @@ def test_kernels_that_make_the_test_share_one_flag():
     for name in makes:
         assert "sg.done" not in found[name], name
         assert "seg_finish(" in found[name], name
+
+
+def test_left_is_not_read_where_it_is_written():
+    found = kernels()
+    reads = {name for name, text in found.items() if "sg.left" in text}
+    writes = {name for name, text in found.items() if "S->left" in text}
+    assert reads == {"k_cg_pnew"}
+    assert writes == {"k_cg_update", "k_cg_update_gdia", "k_cg_vcheck"}
