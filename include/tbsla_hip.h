@@ -77,6 +77,14 @@ int tbsla_hip_version(void);
 /* ---- memory helpers (for callers without their own allocator) ----------- */
 int tbsla_hip_malloc(void **d_ptr, size_t bytes);
 int tbsla_hip_free(void *d_ptr);
+/* Device memory that the library's own objects give back (a destroyed handle's
+ * arrays, a call's work space) is kept for its next ones, at most 4 GiB.  It goes
+ * back to the device when 512 later allocations of the library's have not taken
+ * it or one of them fails, and so not while the library is idle.  This call
+ * returns all of it now, for another allocator or process; *released (nullable)
+ * receives the bytes.  Any thread may call it.  The states that CG keeps for
+ * later solves stay. */
+int tbsla_hip_release_memory(size_t *released);
 int tbsla_hip_memcpy_htod(void *d_dst, const void *h_src, size_t bytes, void *stream);
 int tbsla_hip_memcpy_dtoh(void *h_dst, const void *d_src, size_t bytes, void *stream);
 int tbsla_hip_memcpy_dtod(void *d_dst, const void *d_src, size_t bytes, void *stream);
@@ -94,6 +102,7 @@ int tbsla_hip_device_count(int *count);
 /* C_CPP_Matrix<FMT>_create / _destroy (cpp/interface/c/include/tbsla/cpp/
  * MatrixCSR.h:10-11). */
 int tbsla_hip_create(tbsla_hip_matrix_t *out, int format);
+/* The handle's device memory is kept for later ones (tbsla_hip_release_memory). */
 int tbsla_hip_destroy(tbsla_hip_matrix_t m);
 int tbsla_hip_get_geometry(tbsla_hip_matrix_t m, tbsla_hip_geometry *out);
 

@@ -62,6 +62,7 @@ SIGNATURES = [
     ("tbsla_hip_version", C.c_int, []),
     ("tbsla_hip_malloc", C.c_int, [C.POINTER(C.c_void_p), C.c_size_t]),
     ("tbsla_hip_free", C.c_int, [_vp]),
+    ("tbsla_hip_release_memory", C.c_int, [C.POINTER(C.c_size_t)]),
     ("tbsla_hip_memcpy_htod", C.c_int, [_vp, _vp, C.c_size_t, _vp]),
     ("tbsla_hip_memcpy_dtoh", C.c_int, [_vp, _vp, C.c_size_t, _vp]),
     ("tbsla_hip_memcpy_dtod", C.c_int, [_vp, _vp, C.c_size_t, _vp]),
@@ -226,6 +227,14 @@ class DeviceBuffer:
         assert a.nbytes <= self.nbytes
         if a.nbytes:
             check(lib().tbsla_hip_memcpy_htod(self.ptr, a.ctypes.data, a.nbytes, None))
+
+
+def release_memory() -> int:
+    """Returns the idle device memory that the library keeps for its next objects to the
+    device; the bytes returned."""
+    n = C.c_size_t()
+    check(lib().tbsla_hip_release_memory(C.byref(n)))
+    return n.value
 
 
 def lognormal_field(nx, ny, nz, mu=0.0, sigma=1.0, corr_len=4.0, seed=0) -> DeviceBuffer:

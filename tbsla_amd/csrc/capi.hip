@@ -35,7 +35,8 @@ int fail(int status, const std::string &msg) {
 // (device_free waits for the device, as hipFree does), so any stream and thread
 // may take it.  Bounds: at most kPoolBytes idle (the oldest go first), no block
 // idle for more than kPoolAge later allocations, nothing kept when an
-// allocation fails; a block serves requests down to three quarters of its size.
+// allocation fails or the caller asks for it back (tbsla_hip_release_memory); a
+// block serves requests down to three quarters of its size.
 namespace {
 
 constexpr size_t kPoolBytes = size_t(4) << 30;  // of 288 GB
@@ -296,6 +297,13 @@ int tbsla_hip_malloc(void **d_ptr, size_t bytes) {
     *d_ptr = nullptr;
     return alloc_failed(bytes, e);
   }
+  return TBSLA_HIP_SUCCESS;
+}
+
+int tbsla_hip_release_memory(size_t *released) {
+  std::lock_guard<std::mutex> g(pool().mu);
+  if (released) *released = pool().idle_bytes;
+  pool().drop(pool().idle.size());
   return TBSLA_HIP_SUCCESS;
 }
 

@@ -1,10 +1,11 @@
 """Handles built and dropped over and over, from several threads at once: the
 device memory that one leaves behind serves the next, and every result is that
-of a fresh block."""
+of a fresh block.  What is left behind goes back to the device when asked for."""
 import threading
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 import tbsla_amd as T
@@ -37,6 +38,35 @@ def test_reused_memory_gives_fresh_results(threads):
           for k in range(threads)]
     for t in ts:
         t.start()
+    for t in ts:
+        t.join()
+    assert not errors, errors[0]
+
+
+def test_idle_memory_goes_back_to_the_device():
+    n, c = 1000000, 16
+    held = 12 * n * c  # an int and a double an entry
+    T.Matrix(T.CSR).fill_cqmat(1000, 1000, 3, 0.2, 0).spmv(np.ones(1000))  # code is loaded
+    T.release_memory()
+    free = torch.cuda.mem_get_info()[0]
+    g = T.Matrix(T.CSR).fill_cqmat(n, n, c, 0.2, 0)
+    del g
+    assert torch.cuda.mem_get_info()[0] <= free - held  # kept
+    assert T.release_memory() >= held
+    assert torch.cuda.mem_get_info()[0] >= free
+    assert T.release_memory() == 0
+
+
+def test_release_while_others_build():
+    errors = []
+    sizes = [(500, 3), (40000, 16), (9000, 31), (41000, 16)]
+    ts = [threading.Thread(target=build_and_check, args=(k, sizes[k:] + sizes[:k], errors))
+          for k in range(3)]
+    for t in ts:
+        t.start()
+    while any(t.is_alive() for t in ts):
+        T.release_memory()
+        ts[0].join(0.001)
     for t in ts:
         t.join()
     assert not errors, errors[0]
