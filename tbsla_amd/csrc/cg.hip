@@ -345,7 +345,8 @@ struct RowPrefetch {
 // two rows share: no nontemporal hint, which had them fetched twice; 96 systems
 // of 85 M entries, mixed, K1b: 252 -> 230 us).  Slots outside the row
 // have column 0 of the block and are not summed.  Longer rows continue with the
-// entries from `rest` on.
+// entries from `rest` on.  Entry positions are unsigned: slots reach some hundred
+// past the row, and a block may end at entry 2^31 - 2.
 template <int L, typename V>
 struct CgRow {
   static constexpr int P = 8;
@@ -358,15 +359,15 @@ struct CgRow {
     end = rowptr[row + 1];
     first = L == 1 ? beg : beg - ((beg - ent0) & 3);
   }
-  __device__ inline int at(int lane, int k) const {
-    return L == 1 ? beg + k : first + 4 * (lane + (k >> 2) * L) + (k & 3);
+  __device__ inline unsigned at(int lane, int k) const {
+    return L == 1 ? (unsigned)beg + k : (unsigned)first + (4 * (lane + (k >> 2) * L) + (k & 3));
   }
   __device__ inline bool in(int lane, int k) const {
-    const int e = at(lane, k);
-    return e >= beg && e < end;
+    const unsigned e = at(lane, k);
+    return e >= (unsigned)beg && e < (unsigned)end;
   }
-  __device__ inline int rest(int lane) const {
-    return L == 1 ? beg + P : first + 4 * (lane + 2 * L);
+  __device__ inline unsigned rest(int lane) const {
+    return L == 1 ? (unsigned)beg + P : (unsigned)first + 4 * (lane + 2 * L);
   }
   // the entries, clamped into the arrays (the last quad may end up to three
   // entries after the last one: device_alloc's blocks have room for them)
@@ -375,13 +376,13 @@ struct CgRow {
     if constexpr (L == 1) {
 #pragma unroll
       for (int k = 0; k < P; k++) {
-        const int j = min(at(lane, k), nnz - 1);
+        const int j = (int)min(at(lane, k), (unsigned)nnz - 1);
         col[k] = ci[j];
         v[k] = va[j];
       }
     } else {
 #pragma unroll
-      for (int h = 0; h < 2; h++) quad(ci, va, min(at(lane, 4 * h), nnz - 1), 4 * h);
+      for (int h = 0; h < 2; h++) quad(ci, va, (int)min(at(lane, 4 * h), (unsigned)nnz - 1), 4 * h);
     }
 #pragma unroll
     for (int k = 0; k < P; k++) col[k] = in(lane, k) ? col[k] - f_col : 0;
@@ -570,10 +571,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_p(CG_ARGS, int par_g, int ch
     for (int k = 0; k < P; k++)
       if (w.in(lane, k)) term(w.v[k], sv[k], tv[k]);
     constexpr int Q = L == 1 ? 1 : 4;  // consecutive entries of a lane
-    for (int j = w.rest(lane); j < w.end; j += Q * L)
+    for (unsigned j = w.rest(lane); j < (unsigned)w.end; j += Q * L)
 #pragma unroll
       for (int q = 0; q < Q; q++)
-        if (j + q < w.end) {
+        if (j + q < (unsigned)w.end) {
           const int c = a.colidx[j + q] - a.f_col;
           term(val[j + q], zv[c], po[c]);
         }
@@ -715,10 +716,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_ap(CG_ARGS, int par_g) {
       for (int k = 0; k < P; k++)
         if (w[r].in(lane, k)) term(w[r].v[k], g[r][k]);
       constexpr int Q = L == 1 ? 1 : 4;
-      for (int j = w[r].rest(lane); j < w[r].end; j += Q * L)
+      for (unsigned j = w[r].rest(lane); j < (unsigned)w[r].end; j += Q * L)
 #pragma unroll
         for (int q = 0; q < Q; q++)
-          if (j + q < w[r].end) term(val[j + q], pn[a.colidx[j + q] - a.f_col]);
+          if (j + q < (unsigned)w[r].end) term(val[j + q], pn[a.colidx[j + q] - a.f_col]);
       acc = lane_sum<L>(acc);
       if (lane == 0) {
         a.ap[rw[r]] = (double)acc;
@@ -1621,10 +1622,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_ax(CG_ARGS, int par_g, int mode) 
     for (int k = 0; k < Row::P; k++)
       if (w.in(lane, k)) acc = fma(w.v[k], g[k], acc);
     constexpr int Q = L == 1 ? 1 : 4;
-    for (int j = w.rest(lane); j < w.end; j += Q * L)
+    for (unsigned j = w.rest(lane); j < (unsigned)w.end; j += Q * L)
 #pragma unroll
       for (int q = 0; q < Q; q++)
-        if (j + q < w.end) acc = fma(a.val64[j + q], a.x[a.colidx[j + q] - a.f_col], acc);
+        if (j + q < (unsigned)w.end) acc = fma(a.val64[j + q], a.x[a.colidx[j + q] - a.f_col], acc);
     acc = lane_sum<L>(acc);
     if (lane == 0) ax[row] = acc;
   }

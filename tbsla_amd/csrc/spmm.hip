@@ -167,12 +167,13 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmm16(SpmmArgs a) {
   double acc[V];
 #pragma unroll
   for (int q = 0; q < V; q++) acc[q] = 0.0;
-  int j = a.rowptr[row];
-  const int end = a.rowptr[row + 1];
+  // unsigned: j passes the row's end by up to 15
+  unsigned j = a.rowptr[row];
+  const unsigned end = a.rowptr[row + 1];
   int c = -1;
   double v = 0.0;
-  auto entries = [&](int j0, int &cn, double &vn) {
-    const int e = min(j0 + lane, end - 1);
+  auto entries = [&](unsigned j0, int &cn, double &vn) {
+    const unsigned e = min(j0 + lane, end - 1);
     const unsigned cc = (unsigned)(a.colidx[e] - a.f_col);
     vn = a.vals[e];
     cn = j0 + lane < end && cc < (unsigned)a.ln_col ? (int)cc : -1;  // block filter (:19)
@@ -216,12 +217,12 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmm(SpmmArgs a) {
   for (int q = 0; q < V; q++) acc[q] = 0.0;
   int j = a.rowptr[row];
   const int end = a.rowptr[row + 1];
-  for (; j + 8 <= end; j += 8) spmm_step<8, V>(a, j, col, on, acc);
-  if (j + 4 <= end) {
+  for (; end - j >= 8; j += 8) spmm_step<8, V>(a, j, col, on, acc);
+  if (end - j >= 4) {
     spmm_step<4, V>(a, j, col, on, acc);
     j += 4;
   }
-  if (j + 2 <= end) {
+  if (end - j >= 2) {
     spmm_step<2, V>(a, j, col, on, acc);
     j += 2;
   }
