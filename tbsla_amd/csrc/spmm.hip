@@ -21,19 +21,18 @@ namespace {
 
 // C = A B.  A group of LPR lanes takes one row and one chunk of LPR V columns (V
 // doubles per lane load), up to 16 entries' pieces of B in flight (8 where LPR is
-// not 16).  Every
-// entry gathers its row's chunk of B, so the kernel is bound by where those come
-// from, and the chunk is narrow: 32 columns (256 bytes, two lines) keep the
-// chunk's slice of B small enough to be met again in a cache.  Chunks are the
-// outer order of the grid: the whole chip works on one slice (MALL: 51 MB at
-// 200,003 columns, where whole rows of 512 doubles are 819 MB).  Up to
+// not 16).  Every entry gathers its row's chunk of B, so the kernel is bound by
+// where those come from, and the chunk is narrow: 32 columns (256 bytes, two
+// lines) keep the chunk's slice of B small enough to be met again in a cache.
+// Chunks are the outer order of the grid: the whole chip works on one slice (MALL:
+// 51 MB at 200,003 columns, where whole rows of 512 doubles are 819 MB).  Up to
 // kSpmmXcdCols columns, whose slices are a few times an XCD's 4 MB L2 at most,
-// each XCD (workgroup b runs on XCD b mod 8) takes its own chunks instead,
-// when the chunks divide evenly.  Ten random columns per row, k = 512, whole
-// rows against this: n = 5,003: 28 -> 14 us, 20,011: 114 -> 65, 50,021: 308 ->
-// 245, 100,003: 648 -> 579, 200,003: 1229 -> 1091 (7.5 TB/s gathered); a chunk
-// of 16 columns took 81, 297, 670 and 1380 (one line per gather).  C is written
-// past the caches (1 to 5 %): nothing here reads it again.
+// each XCD (workgroup b runs on XCD b mod 8) takes its own chunks instead, when
+// the chunks divide evenly.  Ten random columns per row, k = 512, whole rows
+// against this: n = 5,003: 28 -> 14 us, 20,011: 114 -> 65, 50,021: 308 -> 245,
+// 100,003: 648 -> 579, 200,003: 1229 -> 1091 (7.5 TB/s gathered); a chunk of 16
+// columns took 81, 297, 670 and 1380 at the last four (one line per gather).  C is
+// written past the caches (1 to 5 %): nothing here reads it again.
 struct SpmmArgs {
   long long n_rows;
   int k, f_col, ln_col;
@@ -50,8 +49,6 @@ struct SpmmArgs {
 
 constexpr int kSpmmXcdCols = 65536;
 
-// E entries from j on: their pieces of B are in flight together, the products
-// are added in entry order
 // lane K of each group of 16, in every lane of the group (row_newbcast reads
 // a lane of the lane's own row, so every lane has a source; bound_ctrl set
 // lets the compiler give the broadcast straight to the instruction using it,
@@ -65,6 +62,8 @@ __device__ __forceinline__ double qbc_d(double v) {
   return __hiloint2double(qbc<K>(__double2hiint(v)), qbc<K>(__double2loint(v)));
 }
 
+// E entries from j on: their pieces of B are in flight together, the products
+// are added in entry order
 template <int E, int V>
 __device__ inline void spmm_step(const SpmmArgs &a, int j, int col, bool on, double (&acc)[V]) {
   TBSLA_NO_FMA

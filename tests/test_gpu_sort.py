@@ -1,6 +1,7 @@
-"""The radix sort behind the conversions and the column sums, at the edges of
-its tiles (8192 32-bit keys, 4096 64-bit keys) and of the column sums' chunks
-(4096 entries of 256 columns), against numpy's stable sort and serial sums."""
+"""The radix sort behind the conversions, the column sums and the transpose, at the
+edges of its tiles (4096 entries of a conversion, 8192 32-bit keys of the sums, 4096
+64-bit keys of the transpose) and of the column sums' chunks (4096 entries of 256
+columns), against numpy's stable sort and serial sums."""
 import numpy as np
 import pytest
 
@@ -25,7 +26,7 @@ def triplets(n_row, n_col, nnz, hub, seed=3):
 
 
 @pytest.mark.parametrize("hub", [False, True])
-@pytest.mark.parametrize("n", [7, 40000, 3000000])  # 32-bit keys, twice 64-bit
+@pytest.mark.parametrize("n", [7, 40000, 3000000])  # one, two and three passes an index
 @pytest.mark.parametrize("nnz", [1, 63, 64, 65, 4095, 4096, 4097, 8191, 8192, 8193, 20011])
 def test_convert_sorts_stably(n, nnz, hub):
     r, c, v = triplets(n, n, nnz, hub)
@@ -57,6 +58,17 @@ def test_col_sums_serial_order(fmt, nnz, n_col, hub):
         cols, vals = cols[vals > 0], vals[vals > 0]
     np.add.at(want, cols, vals)  # unbuffered: entry by entry, in order
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("nnz", [1, 4095, 4096, 4097, 8193])
+def test_transpose_at_a_tiles_edges(nnz):
+    n_row, n_col = 3000, 700
+    r, c, v = triplets(n_row, n_col, nnz, True)
+    g = T.Matrix.from_arrays(T.COO, geom(n_row, n_col, nnz), r, c, v).to(T.CSR)
+    trp, tci, tva = g.transpose().arrays()
+    p = np.lexsort((r, c))  # by column, then row, then the triplets' order
+    assert np.array_equal(trp, np.concatenate([[0], np.cumsum(np.bincount(c, minlength=n_col))]))
+    assert np.array_equal(tci, r[p]) and np.array_equal(tva, v[p])
 
 
 def test_transpose_and_row_sums_past_one_tile():
