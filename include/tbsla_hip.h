@@ -509,7 +509,7 @@ int tbsla_hip_get_csr_schedule(tbsla_hip_matrix_t m, int *lanes, int *rows);
  * keep their lines in L2).  Compiled kernels: vec 1 with lanes 1..64 and
  * rows 1, 2, 4; vec 2 with lanes 4..32 and vec 4 with lanes 4..16, both with
  * rows 1, 2.  tbsla_hip_set_csr_schedule resets vec to 1 and nontemporal to
- * 1. */
+ * 1, or with lanes and rows both 0 to the default kernel's. */
 int tbsla_hip_set_csr_kernel(tbsla_hip_matrix_t m, int lanes, int rows, int vec,
                              int nontemporal);
 int tbsla_hip_get_csr_kernel(tbsla_hip_matrix_t m, int *lanes, int *rows, int *vec,

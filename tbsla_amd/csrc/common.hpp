@@ -276,7 +276,7 @@ struct tbsla_hip_matrix_s {
   int *colidx = nullptr;     // CSR: stored;  ELL: max_col * ln_row, column-major
   int *rowidx = nullptr;     // COO/SCOO: stored
   double *values = nullptr;  // CSR/COO/SCOO: stored; ELL: column-major; DENSE: row-major
-  // SpMV schedule
+  // SpMV schedule; lanes_per_row and rows_per_group both 0: csr_default's
   int lanes_per_row = 0;     // CSR: 0 = pick from the mean row length
   int rows_per_group = 0;    // CSR: rows each lane group keeps in flight (0 = pick)
   int csr_vec = 0;           // CSR: entries per lane load (0 = 1)
