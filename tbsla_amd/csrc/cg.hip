@@ -57,7 +57,6 @@ struct CgSeg {
   long long t_done;  // wall clock when the system finished
   int iters;         // reference counting
   int done;          // SegDone
-  int left;          // K2 found the system not running (K1 may leave at once)
   int shift;         // buffer parity of this system relative to the global iteration
   int true_res;      // the current r.r partials belong to a true residual b - A x
   int stop_par;      // buffer parity at the test that ended the recurrence
@@ -65,6 +64,7 @@ struct CgSeg {
   int blk0, blk1;    // workgroups of the system (same in every kernel)
   int rpb;           // rows per workgroup
   int ent0;          // the first entry of row0
+  int left;          // K2 found the system not running (K1 may leave at once)
 };
 
 struct CgCom {
@@ -198,13 +198,13 @@ __device__ inline int cg_block(int multi) {
 
 struct CgPart {
   double stop, near_zero, rnorm0;
-  int iters, shift, true_res, stop_par, done, left;
-  int row0, row1, blk0, blk1, rpb, ent0;
+  int iters, shift, true_res, stop_par, done;
+  int row0, row1, blk0, blk1, rpb, ent0, left;
 };
 
 __device__ inline CgPart cg_part(TBSLA_CONST CgSeg *c) {
-  return CgPart{c->stop, c->near_zero, c->rnorm0, c->iters, c->shift, c->true_res, c->stop_par, c->done, c->left,
-                c->row0, c->row1, c->blk0, c->blk1, c->rpb, c->ent0};
+  return CgPart{c->stop, c->near_zero, c->rnorm0, c->iters, c->shift, c->true_res, c->stop_par, c->done,
+                c->row0, c->row1, c->blk0, c->blk1, c->rpb, c->ent0, c->left};
 }
 
 // the block's other fields
