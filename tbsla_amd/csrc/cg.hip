@@ -64,7 +64,9 @@ struct CgSeg {
   int blk0, blk1;    // workgroups of the system (same in every kernel)
   int rpb;           // rows per workgroup
   int ent0;          // the first entry of row0
-  int left;          // K2 found the system not running (K1 may leave at once)
+  // K2 found the system not running: K1 may leave at once (last here: among the
+  // fields that a lone system loads together it cost its solve 0.4 %)
+  int left;
 };
 
 struct CgCom {
